@@ -10,7 +10,7 @@
 // from the row-major matrix makes every group of lanes touch 16 different cache lines per instruction and
 // ran at about a third of the bandwidth.)
 //
-// Two kernels share the format.  The dense kernel (w8a16_gemm4_kernel, described where it is defined) loads weight
+// Three kernels share the format.  Many rows run on tiles (w8a16_tile_kernel).  The skinny dense kernel (w8a16_gemm4_kernel, described where it is defined) loads weight
 // tiles straight into MFMA operand registers, shares one LDS-staged activation tile among the waves of a workgroup
 // and serves the decode layer's projections; its epilogue, or the split-K reduce kernels, carry the fused variants
 // (gate/up + SiLU*mul, residual + RMSNorm,
@@ -25,6 +25,7 @@
 // MFMAs of a k-step take bytes 0-7 and 8-15 of each lane's 16 weight bytes, and the activation operand is
 // gathered in the same k order.
 #include "common.h"
+#include "w8a16_tile_gemm.h"
 
 namespace {
 
@@ -56,23 +57,25 @@ __device__ __forceinline__ float dequant_bias(float acc, float scale, const uint
 template <typename T>
 __device__ __forceinline__ void store4(uint16_t* y, const uint16_t* bias, const uint16_t* residual,
                                        const float* scale, int64_t row_off, int n, int N, f32x4 acc) {
-    float o[4];
+    if (n + 3 < N && ((row_off + n) & 3) == 0) {              // residual and result as one 8-byte access each
+        u32x2 r = {0u, 0u};
+        if (residual) r = *(const u32x2*)(residual + row_off + n);
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o[i] = dequant_bias<T>(acc[i], scale ? scale[n + i] : 1.0f, bias, n + i);   // no scale: already applied
+            if (residual) o[i] = __fadd_rn(T::to_float(T::from_float(o[i])), T::to_float((uint16_t)(r[i >> 1] >> (16 * (i & 1)))));
+        }
+        *(u32x2*)(y + row_off + n) = (u32x2){pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if (n + i < N) {
-            float v = dequant_bias<T>(acc[i], scale ? scale[n + i] : 1.0f, bias, n + i);   // no scale: already applied
+            float v = dequant_bias<T>(acc[i], scale ? scale[n + i] : 1.0f, bias, n + i);
             if (residual) v = __fadd_rn(T::to_float(T::from_float(v)), T::to_float(residual[row_off + n + i]));
-            o[i] = v;
-        } else {
-            o[i] = 0.f;
+            y[row_off + n + i] = T::from_float(v);
         }
-    }
-    if (n + 3 < N && ((row_off + n) & 3) == 0) {
-        *(u32x2*)(y + row_off + n) = (u32x2){pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (n + i < N) y[row_off + n + i] = T::from_float(o[i]);
     }
 }
 
@@ -510,6 +513,177 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 3 : 1) void w8a16_gemm4_ke
     }
 }
 
+// ---- many rows ---------------------------------------------------------------------------------------------------------
+// More rows than two or three passes of the skinny kernel: tiles of 128 rows x 256 channels (w8a16_tile_gemm.h).
+// Workgroup id -> (row block, channel block, part of K).  Ids below `full` are whole tiles in whole rounds of the device:
+// ids go to the XCDs in turn, so XCD j is given the tiles [j * full / 8, (j + 1) * full / 8) and the workgroups that run
+// on it at one time share row and channel blocks in its L2.  The tiles left over are cut into `split` parts of K each.
+struct TileGrid {
+    int m_blocks, n_blocks, full, split, steps_per_split;
+};
+constexpr int TG_PANEL = 4;                                   // row blocks walked together along the channels
+__device__ __forceinline__ void tg_locate(const TileGrid& g, int id, int& mb, int& nb, int& part, int& slot) {
+    int t;
+    if (id < g.full) {
+        t = (id & 7) * (g.full >> 3) + (id >> 3);
+        part = slot = 0;
+    } else {
+        slot = id - g.full;
+        t = g.full + slot / g.split;
+        part = slot % g.split;
+    }
+    const int panel = t / (TG_PANEL * g.n_blocks), in = t - panel * TG_PANEL * g.n_blocks;
+    const int rows = min(TG_PANEL, g.m_blocks - panel * TG_PANEL);
+    nb = in / rows;
+    mb = panel * TG_PANEL + in - nb * rows;
+}
+// the lanes of a wave exchange values through LDS: its own instructions stay in order
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Output of one wave: 64 channels from n0 on, 32 rows at a time.  The channels of a row lie spread over the accumulators of
+// two lanes, so the values (dequantised, with bias, gated where asked, rounded to T) go through LDS and leave as whole
+// 128-byte (gated: 64-byte) pieces of rows; the residual is read the same way.  Rounding points as in store4 / store_gated.
+// (8-byte stores straight from the accumulators, each waiting for its own scales: 4096 x 4096 at 1536 rows 69.8 us against
+// 54.3, 24576 x 1536 at 129 rows 42.3 against 25.6.)  N is a multiple of 16.
+template <typename T>
+struct TileOut {
+    static constexpr int ROW = 144;                           // bytes of a staged row: 16-byte slots spread over the banks
+    uint16_t* y;
+    const uint16_t *bias, *residual;
+    int M, N, gated, aligned;
+
+    // scale and bias of channels 8q + 4h .. + 3 of 32-channel block nt
+    __device__ __forceinline__ void load(const float* scale, int n0, int nt, int q, f32x4& sc, f32x4& bi) const {
+        const int n = min(n0 + 32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1), N - 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            sc[i] = scale[n + i];
+            bi[i] = bias ? T::to_float(bias[n + i]) : 0.f;
+        }
+    }
+    // these channels of a row into the stage
+    __device__ __forceinline__ void put(f32x4 v, f32x4 sc, f32x4 bi, int nt, int q, uint8_t* stage) const {
+        const int r = threadIdx.x & 31, c = 32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1);
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o[i] = __fmul_rn(v[i], sc[i]);
+            if (bias) o[i] = __fadd_rn(o[i], bi[i]);
+        }
+        if (gated) {
+            float a[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float gv = T::to_float(T::from_float(o[2 * e])), uv = T::to_float(T::from_float(o[2 * e + 1]));
+                a[e] = T::to_float(T::from_float(silu_f(gv))) * uv;
+            }
+            *(uint32_t*)(stage + r * ROW + c) = pack2<T>(a[0], a[1]);
+        } else {
+            *(u32x2*)(stage + r * ROW + 2 * c) = (u32x2){pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
+        }
+    }
+    // the 32 staged rows to memory, by `threads` threads of which this is number t
+    __device__ __forceinline__ void flush(int m0, int n0, const uint8_t* stage, int t, int threads) const {
+        const int cols = gated ? N >> 1 : N, c0 = gated ? n0 >> 1 : n0, per = gated ? 4 : 8;   // 16-byte pieces of a row
+        const int row = t / per, c = c0 + 8 * (t - row * per), step = threads / per;
+        for (int j = row; j < 32; j += step) {
+            const int m = m0 + j;
+            if (m >= M || c >= cols) continue;
+            u32x4 v = *(const u32x4*)(stage + j * ROW + 2 * (c - c0));
+            const int64_t at = (int64_t)m * cols + c;
+            if (residual) {
+                float f[8], g[8];
+                u32x4 rr;
+                if (aligned) rr = *(const u32x4*)(residual + at);
+                else
+                    for (int i = 0; i < 4; ++i) rr[i] = residual[at + 2 * i] | (uint32_t)residual[at + 2 * i + 1] << 16;
+                unpack8<T>(v, f);
+                unpack8<T>(rr, g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = pack2<T>(__fadd_rn(f[2 * i], g[2 * i]), __fadd_rn(f[2 * i + 1], g[2 * i + 1]));
+            }
+            if (aligned) *(u32x4*)(y + at) = v;
+            else
+                for (int i = 0; i < 8; ++i) y[at + i] = (uint16_t)(v[i >> 1] >> (16 * (i & 1)));
+        }
+    }
+};
+
+template <typename T, int MT>
+__global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
+    uint16_t* __restrict__ y, float* __restrict__ partial, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp,
+    const float* __restrict__ scale, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N,
+    int K, int gated, int aligned, TileGrid g) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * 32 * MT * 128];
+    static_assert(tg::WAVES * 32 * TileOut<T>::ROW <= (int)sizeof(smem), "the output stage reuses the operand stages");
+    int mb, nb, part, slot;
+    tg_locate(g, blockIdx.x, mb, nb, part, slot);
+    const bool whole = blockIdx.x < g.full || g.split == 1;
+    const int KS = K / tg::KSTEP, s0 = part * g.steps_per_split;
+    const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int m0 = mb * 32 * MT, n0 = nb * tg::BN + 64 * wv;
+    float* pt = partial + (int64_t)slot * (32 * MT * tg::BN) + (wv * MT * 8 * 64 + lane) * 4;
+    const TileOut<T> out{y, bias, residual, M, N, gated, aligned};
+    f32x4 sc[8], bi[8];
+    uint8_t* stage = smem + wv * 32 * TileOut<T>::ROW;
+    tg::tile<T, MT>(x, wp, M, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const f32x16 (&acc)[2]) {
+        constexpr int mt = decltype(mtc)::value;
+        if (whole) {
+            if (mt == 0) {
+                __syncthreads();                              // every wave has read its last operands
+#pragma unroll
+                for (int e = 0; e < 8; ++e) out.load(scale, n0, e >> 2, e & 3, sc[e], bi[e]);
+            }
+            wave_lds_order();
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                out.put((f32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
+                                acc[e >> 2][4 * (e & 3) + 3]}, sc[e], bi[e], e >> 2, e & 3, stage);
+            wave_lds_order();
+            out.flush(m0 + 32 * mt, n0, stage, lane, 64);
+        } else {                                              // accumulator order: whole cache lines
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                *(f32x4*)(pt + (mt * 8 + e) * 256) = (f32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1],
+                                                             acc[e >> 2][4 * (e & 3) + 2], acc[e >> 2][4 * (e & 3) + 3]};
+        }
+    });
+}
+
+// Sums the parts of the tiles that were cut along K, in order: a workgroup per 32 rows x 64 channels, a quarter of the
+// channels per wave.
+template <typename T, int MT>
+__global__ __launch_bounds__(256) void w8a16_tile_reduce_kernel(
+    uint16_t* __restrict__ y, const float* __restrict__ partial, const float* __restrict__ scale,
+    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N, int gated, int aligned, TileGrid g) {
+    __shared__ __attribute__((aligned(16))) uint8_t stage[32 * TileOut<T>::ROW];
+    constexpr int ITEMS = tg::WAVES * MT;                     // workgroups per tile
+    constexpr int64_t PART = 32 * MT * tg::BN;
+    const int tile = blockIdx.x / ITEMS, item = blockIdx.x - tile * ITEMS, wv = item / MT, mt = item - wv * MT;
+    int mb, nb, part, slot;
+    tg_locate(g, g.full + tile * g.split, mb, nb, part, slot);
+    const int m0 = mb * 32 * MT + 32 * mt, n0 = nb * tg::BN + 64 * wv;
+    if (m0 >= M || n0 >= N) return;
+    const int lane = threadIdx.x & 63, e0 = 2 * (threadIdx.x >> 6);
+    const float* p = partial + slot * PART + ((wv * MT + mt) * 8 * 64 + lane) * 4;
+    const TileOut<T> out{y, bias, residual, M, N, gated, aligned};
+    f32x4 sc[2], bi[2], v[2] = {(f32x4)(0.f), (f32x4)(0.f)};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) out.load(scale, n0, (e0 + e) >> 2, (e0 + e) & 3, sc[e], bi[e]);
+#pragma unroll 8
+    for (int s = 0; s < g.split; ++s)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) v[e] += *(const f32x4*)(p + s * PART + (e0 + e) * 256);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) out.put(v[e], sc[e], bi[e], (e0 + e) >> 2, (e0 + e) & 3, stage);
+    __syncthreads();
+    out.flush(m0, n0, stage, threadIdx.x, 256);
+}
+
 // Grouped (experts): grid = (ceil(N/64), n_experts).  Rows offsets[e] .. offsets[e+1] of x use expert e's
 // packed weights and scale[e]; experts with no rows exit at once.  One pass over the expert's weights serves up to
 // 64 rows (decode batches route a handful of tokens to each expert: 16 rows per pass there); experts with more rows
@@ -846,6 +1020,47 @@ struct GemmPlan {
     int steps_per_split;
 };
 
+// Tile plan of the many-row kernel.  Measured, a 64-wide k-step of a tile takes TG_STEP_ALONE us on a compute unit of its
+// own and a pair of tiles on one compute unit takes TG_STEP_PAIR us a step (the clock follows the power draw).  Whole
+// tiles fill whole multiples of the 256 compute units; what is left over would hold a few of them for a whole tile's
+// time, so it is cut along K where the shorter tail pays for writing and summing the fp32 parts
+// (4137 x 4096 x 14336: 16 of 528 tiles left, 531 us uncut, 423 us in 8 parts).
+constexpr int TG_MT = 4;
+constexpr float TG_STEP_ALONE = 0.75f, TG_STEP_PAIR = 1.72f, TG_REDUCE = 5.f, TG_PART = 0.065f, TG_FIXED = 6.f;
+
+TileGrid plan_tiles(int m, int n, int k, float* us = nullptr) {
+    TileGrid g;
+    g.m_blocks = (m + 32 * TG_MT - 1) / (32 * TG_MT);
+    g.n_blocks = (n + tg::BN - 1) / tg::BN;
+    const int tiles = g.m_blocks * g.n_blocks, steps = k / tg::KSTEP;
+    const int rows = tiles / 256, rem = tiles % 256;
+    float best = 0.f;
+    g.split = 1;
+    for (int s = 1; s <= 16; s *= 2) {
+        if (s > 1 && (rem == 0 || steps / s < 4)) break;
+        const int part = (steps + s - 1) / s;
+        float t = (rows / 2) * steps * TG_STEP_PAIR;
+        if (s == 1) {
+            const int tail = (rows & 1) * 256 + rem;
+            t += tail == 0 ? 0.f : steps * (tail <= 256 ? TG_STEP_ALONE : TG_STEP_PAIR);
+        } else {
+            const int left = rem * s;
+            if (rows & 1) t += steps * TG_STEP_ALONE + (left + 255) / 256 * part * (TG_STEP_PAIR - TG_STEP_ALONE);
+            else t += left <= 256 ? part * TG_STEP_ALONE : (left + 511) / 512 * part * TG_STEP_PAIR;
+            t += TG_REDUCE + left * TG_PART;
+        }
+        if (s == 1 || t < best) {
+            best = t;
+            g.split = s;
+        }
+    }
+    g.steps_per_split = (steps + g.split - 1) / g.split;
+    g.split = (steps + g.steps_per_split - 1) / g.steps_per_split;
+    g.full = g.split > 1 ? tiles - rem : tiles / 8 * 8;       // a multiple of 8 (see tg_locate)
+    if (us) *us = best + TG_FIXED;
+    return g;
+}
+
 GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
     GemmPlan p;
     p.mt = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
@@ -872,19 +1087,37 @@ GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
     return p;
 }
 
+// Tiles against passes of 64 rows of the skinny kernel (more than 64 rows, K of whole steps, N of whole 16-byte pieces, gated
+// too).  Measured, a k-step of a round of 256 skinny workgroups takes 0.40 us: 28672 x 4096 at 65 / 256 / 4137 rows runs in
+// 41 / 65 / 787 us on tiles against 51 / 103 / 1447 us, 4096 x 4096 at 128 / 256 / 700 rows in 18 / 26 / 48 against 17 / 20 / 47.
+bool use_tiles(int m, int n, int k) {
+    if (m <= 64 || k % tg::KSTEP != 0 || n % 16 != 0) return false;
+    float us;
+    plan_tiles(m, n, k, &us);
+    const GemmPlan p = plan_w8a16(m, n, k);
+    const int rounds = (p.n_blocks * p.m_blocks * p.split_k + 255) / 256;
+    return us < 0.40f * rounds * p.steps_per_split + 4.f + (p.split_k > 1 ? TG_REDUCE : 0.f);
+}
+
 template <typename T>
-int launch_w8a16(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias,
-                 const void* residual, int m, int n, int k, int gated, void* workspace, hipStream_t st,
-                 void* norm_out = nullptr, const void* gamma = nullptr, float eps = 0.f, int gamma_dtype = MF_FP32,
-                 const RopeCacheArgs* rc_args = nullptr, int w4_group = -1, int norm_cols = 0) {
-    // norm_cols: columns the norm in norm_out covers (the leading ones; 0 = the whole row)
-    if (norm_cols <= 0) norm_cols = n;
-    // w4_group >= 0: 4-bit weights; 0 = `scale` holds one value per channel, 64 / 128 = one per channel and group
-    // ([K / group][N]), applied inside the kernel (the epilogues then see no scale)
-    const GemmPlan p = plan_w8a16(m, n, k, w4_group == 128 ? 2 : 1);
-    const float* gscale = w4_group > 0 ? scale : nullptr;
-    if (w4_group > 0) scale = nullptr;
-    float* partial = p.split_k > 1 ? (float*)workspace : nullptr;
+void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias, const void* residual, int m,
+                  int n, int k, int gated, void* workspace, hipStream_t st) {
+    const TileGrid g = plan_tiles(m, n, k);
+    const int cut = g.m_blocks * g.n_blocks - g.full;
+    const int aligned = (((uintptr_t)y | (uintptr_t)residual) & 15) == 0;
+    hipLaunchKernelGGL((w8a16_tile_kernel<T, TG_MT>), dim3(g.full + cut * g.split), dim3(256), 0, st, (uint16_t*)y,
+                       (float*)workspace, (const uint16_t*)x, wp, scale, (const uint16_t*)bias, (const uint16_t*)residual, m,
+                       n, k, gated, aligned, g);
+    if (g.split > 1)
+        hipLaunchKernelGGL((w8a16_tile_reduce_kernel<T, TG_MT>), dim3(cut * tg::WAVES * TG_MT), dim3(256), 0, st,
+                           (uint16_t*)y, (const float*)workspace, scale, (const uint16_t*)bias, (const uint16_t*)residual, m,
+                           n, gated, aligned, g);
+}
+
+template <typename T>
+void launch_skinny(const GemmPlan& p, void* y, float* partial, const void* x, const uint8_t* wp, const float* scale,
+                   const float* gscale, const void* bias, const void* residual, int m, int n, int k, int gated, int w4_group,
+                   hipStream_t st) {
     const int split_major = p.split_k % 8 == 0;
     dim3 grid(split_major ? p.split_k : p.n_blocks, split_major ? p.n_blocks : p.split_k, p.m_blocks);
     const bool ktail = (k % GW_KSTEP) != 0;
@@ -911,6 +1144,24 @@ int launch_w8a16(void* y, const void* x, const uint8_t* wp, const float* scale, 
 #undef GW4_LAUNCH
 #undef GW4_LAUNCH_W4
 #undef GW4_W4_BY_GROUP
+}
+
+template <typename T>
+int launch_w8a16(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias,
+                 const void* residual, int m, int n, int k, int gated, void* workspace, hipStream_t st,
+                 void* norm_out = nullptr, const void* gamma = nullptr, float eps = 0.f, int gamma_dtype = MF_FP32,
+                 const RopeCacheArgs* rc_args = nullptr, int w4_group = -1, int norm_cols = 0) {
+    // norm_cols: columns the norm in norm_out covers (the leading ones; 0 = the whole row)
+    if (norm_cols <= 0) norm_cols = n;
+    // w4_group >= 0: 4-bit weights; 0 = `scale` holds one value per channel, 64 / 128 = one per channel and group
+    // ([K / group][N]), applied inside the kernel (the epilogues then see no scale)
+    const bool tiles = w4_group < 0 && use_tiles(m, n, k);
+    const GemmPlan p = tiles ? GemmPlan{} : plan_w8a16(m, n, k, w4_group == 128 ? 2 : 1);
+    const float* gscale = w4_group > 0 ? scale : nullptr;
+    if (w4_group > 0) scale = nullptr;
+    float* partial = p.split_k > 1 ? (float*)workspace : nullptr;   // the tile kernel sums its own parts
+    if (tiles) launch_tiles<T>(y, x, wp, scale, bias, residual, m, n, k, gated, workspace, st);
+    else launch_skinny<T>(p, y, partial, x, wp, scale, gscale, bias, residual, m, n, k, gated, w4_group, st);
     int rc = MF_LAUNCH_CHECK();
     if (rc) return rc;
     if (rc_args && partial) {                                 // reduce + RoPE + cache scatter in one kernel
@@ -983,6 +1234,10 @@ extern "C" int mf_w8a16_pack_weight(void* packed, const int8_t* w, int n, int k,
 
 extern "C" size_t mf_w8a16_workspace_bytes(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
+    if (use_tiles(m, n, k)) {
+        const TileGrid g = plan_tiles(m, n, k);
+        return g.split > 1 ? (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * TG_MT * tg::BN) * sizeof(float) : 0;
+    }
     const GemmPlan p = plan_w8a16(m, n, k);
     return p.split_k > 1 ? (size_t)p.split_k * m * n * sizeof(float) : 0;
 }
@@ -1224,3 +1479,4 @@ extern "C" int mf_w4a16_gemm(void* y, const void* x, const void* w_packed, const
     return launch_w8a16<FP16>(y, x, (const uint8_t*)w_packed, scale, bias, residual, m, n, k, 0, workspace,
                               (hipStream_t)stream, nullptr, nullptr, 0.f, MF_FP32, nullptr, group_size);
 }
+

@@ -1029,6 +1029,43 @@ def test_w8a16_qkv_rope_and_quant_cache_equals_unfused(dtype, t, n_head, n_kv, d
     assert not torch.equal(kc1, init)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,bias,residual", [
+    (513, 8208, 704, True, True),          # one row and one 16-channel piece past whole tiles, an odd number of k-steps
+    (129, 28672, 4096, False, False),      # whole channel blocks, no cut along K
+    (65, 12304, 8192, True, False),        # every tile cut along K
+    (1100, 2064, 4096, False, True),       # whole tiles and cut ones
+    (2305, 4096, 4160, True, True)])       # a full round, the tiles left over in parts of unequal length
+def test_w8a16_many_rows(dtype, m, n, k, bias, residual):
+    """The tile kernel against float64 on the device.  Both roundings (the projection, then the sum with the residual) are
+    to nearest, off by at most EPS (half a step) of the value; fp32 accumulation in any order adds at most K * 2^-24 of the sum of magnitudes."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    w = torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+    s = (torch.rand(n, generator=g, device="cuda") + 0.5) * (k ** -0.5 / 73)
+    b = torch.randn(n, generator=g, device="cuda").to(dtype) if bias else None
+    r = torch.randn(m, n, generator=g, device="cuda").to(dtype) if residual else None
+    packed = ops.pack_w8a16(w, s)
+    y = ops.w8a16_linear(x, packed, bias=b, residual=r)
+    v = x.double() @ w.double().t() * s.double()
+    mag = x.double().abs() @ w.double().abs().t() * s.double()
+    if bias:
+        v += b.double()
+    ref = v + r.double() if residual else v
+    tol = EPS[dtype] * (ref.abs() + (v.abs() if residual else 0)) * 1.01 + k * 2.0 ** -24 * mag + 1e-7
+    assert bool(((y.double() - ref).abs() <= tol).all())
+    if not residual:
+        gamma = torch.rand(n, generator=g, device="cuda")
+        res = torch.randn(m, n, generator=g, device="cuda").to(dtype)
+        if n <= 16384:
+            h, norm = ops.w8a16_linear_add_rmsnorm(x, packed, res, gamma, 1e-5, bias=b)
+            assert torch.equal(h, ops.w8a16_linear(x, packed, bias=b, residual=res)) and torch.equal(norm, ops.rms_norm(h, gamma, 1e-5))
+        inter = ops.interleave_gate_up(b, "halves") if bias else None
+        fused = ops.w8a16_gated_linear(x, ops.pack_w8a16_gated(w, s, "halves"), inter)
+        assert torch.equal(fused, ops.silu_mul(y))
+
+
 def test_w8a16_exact_on_integer_grid():
     """Power-of-two scales and small-integer activations make every product and sum exact: the kernel must
     return exactly the integer matmul (catches a dropped k-step, a wrong row/column or a transposed operand)."""
