@@ -1,0 +1,113 @@
+// Work distribution of the many-row GEMMs (W8A16 and W8A8): output tiles in whole rounds of the device, the rest cut along K.
+#pragma once
+#include "common.h"
+
+// Workgroup id -> (row block, channel block, part of K).  Ids below `full` are whole tiles: ids go to the XCDs in turn, so
+// XCD j is given the tiles [j * full / 8, (j + 1) * full / 8) and the workgroups that run on it at one time share row and
+// channel blocks in its L2.  The tiles left over are cut into `split` parts of K each.
+struct TileGrid {
+    int m_blocks, n_blocks, full, split, steps_per_split;
+};
+constexpr int TG_PANEL = 4;                                   // row blocks walked together along the channels
+__device__ __forceinline__ void tg_locate(const TileGrid& g, int id, int& mb, int& nb, int& part, int& slot) {
+    int t;
+    if (id < g.full) {
+        t = (id & 7) * (g.full >> 3) + (id >> 3);
+        part = slot = 0;
+    } else {
+        slot = id - g.full;
+        t = g.full + slot / g.split;
+        part = slot % g.split;
+    }
+    const int panel = t / (TG_PANEL * g.n_blocks), in = t - panel * TG_PANEL * g.n_blocks;
+    const int rows = min(TG_PANEL, g.m_blocks - panel * TG_PANEL);
+    nb = in / rows;
+    mb = panel * TG_PANEL + in - nb * rows;
+}
+inline int tg_workgroups(const TileGrid& g) { return g.full + (g.m_blocks * g.n_blocks - g.full) * g.split; }
+
+// Measured times (us): a k-step of a tile on a compute unit of its own, of a pair of tiles on one compute unit (the clock
+// follows the power draw), what a launch and a tile's start and end take, the reduce launch, and one part's share of
+// writing and summing the parts.
+struct TileCost {
+    float alone, pair, fixed, reduce, part;
+};
+// Whole tiles fill whole multiples of the 256 compute units; what is left over would hold a few of them for a whole tile's
+// time, so it is cut along K where the shorter tail pays for its parts.
+inline TileGrid tg_plan(int m_blocks, int n_blocks, int steps, const TileCost& c, float* us) {
+    TileGrid g;
+    g.m_blocks = m_blocks;
+    g.n_blocks = n_blocks;
+    const int tiles = m_blocks * n_blocks, rounds = tiles / 256, rem = tiles % 256;
+    float best = 0.f;
+    g.split = 1;
+    for (int s = 1; s <= 16; s *= 2) {
+        if (s > 1 && (rem == 0 || steps / s < 4)) break;
+        const int part = (steps + s - 1) / s;
+        float t = (rounds / 2) * steps * c.pair;
+        if (s == 1) {
+            const int tail = (rounds & 1) * 256 + rem;
+            t += tail == 0 ? 0.f : steps * (tail <= 256 ? c.alone : c.pair);
+        } else {
+            const int left = rem * s;
+            if (rounds & 1) t += steps * c.alone + (left + 255) / 256 * part * (c.pair - c.alone);
+            else t += left <= 256 ? part * c.alone : (left + 511) / 512 * part * c.pair;
+            t += c.reduce + left * c.part;
+        }
+        if (s == 1 || t < best) {
+            best = t;
+            g.split = s;
+        }
+    }
+    g.steps_per_split = (steps + g.split - 1) / g.split;
+    g.split = (steps + g.steps_per_split - 1) / g.steps_per_split;
+    g.full = g.split > 1 ? tiles - rem : tiles / 8 * 8;       // a multiple of 8 (see tg_locate)
+    *us = best + c.fixed;
+    return g;
+}
+
+// acc * a (* b) (+ bias), every operation rounded by itself: the epilogues of the many-row kernels are straight-line code in
+// which the compiler would contract the last product and the sum, and the other kernels' results are to be met bit for bit
+__device__ __forceinline__ float scaled_bias(float acc, float a, float b, bool two, float bias, bool with_bias) {
+#pragma clang fp contract(off)
+    float v = acc * a;
+    if (two) v = v * b;
+    if (with_bias) v = v + bias;
+    return v;
+}
+
+// the lanes of a wave exchange values through LDS: its own instructions stay in order
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// 32 staged rows of up to 64 channels (144 bytes a row: 16-byte slots spread over the banks) to memory as whole 16-byte pieces
+// of rows, by `threads` threads of which this is number t; the residual, read the same way, is added to the rounded values.
+// cols = row length of y, c0 = first channel, per = 16-byte pieces of a staged row.
+constexpr int TG_STAGE_ROW = 144;
+template <typename T>
+__device__ __forceinline__ void tg_flush(uint16_t* y, const uint16_t* residual, const uint8_t* stage, int m0, int M, int c0,
+                                         int cols, int per, bool aligned, int t, int threads) {
+    const int row = t / per, c = c0 + 8 * (t - row * per), step = threads / per;
+    for (int j = row; j < 32; j += step) {
+        const int m = m0 + j;
+        if (m >= M || c >= cols) continue;
+        u32x4 v = *(const u32x4*)(stage + j * TG_STAGE_ROW + 2 * (c - c0));
+        const int64_t at = (int64_t)m * cols + c;
+        if (residual) {
+            float f[8], g[8];
+            u32x4 rr;
+            if (aligned) rr = *(const u32x4*)(residual + at);
+            else
+                for (int i = 0; i < 4; ++i) rr[i] = residual[at + 2 * i] | (uint32_t)residual[at + 2 * i + 1] << 16;
+            unpack8<T>(v, f);
+            unpack8<T>(rr, g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = pack2<T>(__fadd_rn(f[2 * i], g[2 * i]), __fadd_rn(f[2 * i + 1], g[2 * i + 1]));
+        }
+        if (aligned) *(u32x4*)(y + at) = v;
+        else
+            for (int i = 0; i < 8; ++i) y[at + i] = (uint16_t)(v[i >> 1] >> (16 * (i & 1)));
+    }
+}

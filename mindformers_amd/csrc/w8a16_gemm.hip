@@ -25,6 +25,7 @@
 // MFMAs of a k-step take bytes 0-7 and 8-15 of each lane's 16 weight bytes, and the activation operand is
 // gathered in the same k order.
 #include "common.h"
+#include "tile_grid.h"
 #include "w8a16_tile_gemm.h"
 
 namespace {
@@ -515,34 +516,6 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 3 : 1) void w8a16_gemm4_ke
 
 // ---- many rows ---------------------------------------------------------------------------------------------------------
 // More rows than two or three passes of the skinny kernel: tiles of 128 rows x 256 channels (w8a16_tile_gemm.h).
-// Workgroup id -> (row block, channel block, part of K).  Ids below `full` are whole tiles in whole rounds of the device:
-// ids go to the XCDs in turn, so XCD j is given the tiles [j * full / 8, (j + 1) * full / 8) and the workgroups that run
-// on it at one time share row and channel blocks in its L2.  The tiles left over are cut into `split` parts of K each.
-struct TileGrid {
-    int m_blocks, n_blocks, full, split, steps_per_split;
-};
-constexpr int TG_PANEL = 4;                                   // row blocks walked together along the channels
-__device__ __forceinline__ void tg_locate(const TileGrid& g, int id, int& mb, int& nb, int& part, int& slot) {
-    int t;
-    if (id < g.full) {
-        t = (id & 7) * (g.full >> 3) + (id >> 3);
-        part = slot = 0;
-    } else {
-        slot = id - g.full;
-        t = g.full + slot / g.split;
-        part = slot % g.split;
-    }
-    const int panel = t / (TG_PANEL * g.n_blocks), in = t - panel * TG_PANEL * g.n_blocks;
-    const int rows = min(TG_PANEL, g.m_blocks - panel * TG_PANEL);
-    nb = in / rows;
-    mb = panel * TG_PANEL + in - nb * rows;
-}
-// the lanes of a wave exchange values through LDS: its own instructions stay in order
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Output of one wave: 64 channels from n0 on, 32 rows at a time.  The channels of a row lie spread over the accumulators of
 // two lanes, so the values (dequantised, with bias, gated where asked, rounded to T) go through LDS and leave as whole
 // 128-byte (gated: 64-byte) pieces of rows; the residual is read the same way.  Rounding points as in store4 / store_gated.
@@ -550,7 +523,7 @@ __device__ __forceinline__ void wave_lds_order() {
 // 54.3, 24576 x 1536 at 129 rows 42.3 against 25.6.)  N is a multiple of 16.
 template <typename T>
 struct TileOut {
-    static constexpr int ROW = 144;                           // bytes of a staged row: 16-byte slots spread over the banks
+    static constexpr int ROW = TG_STAGE_ROW;
     uint16_t* y;
     const uint16_t *bias, *residual;
     int M, N, gated, aligned;
@@ -569,10 +542,7 @@ struct TileOut {
         const int r = threadIdx.x & 31, c = 32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1);
         float o[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[i] = __fmul_rn(v[i], sc[i]);
-            if (bias) o[i] = __fadd_rn(o[i], bi[i]);
-        }
+        for (int i = 0; i < 4; ++i) o[i] = scaled_bias(v[i], sc[i], 1.f, false, bi[i], bias != nullptr);
         if (gated) {
             float a[2];
 #pragma unroll
@@ -587,28 +557,7 @@ struct TileOut {
     }
     // the 32 staged rows to memory, by `threads` threads of which this is number t
     __device__ __forceinline__ void flush(int m0, int n0, const uint8_t* stage, int t, int threads) const {
-        const int cols = gated ? N >> 1 : N, c0 = gated ? n0 >> 1 : n0, per = gated ? 4 : 8;   // 16-byte pieces of a row
-        const int row = t / per, c = c0 + 8 * (t - row * per), step = threads / per;
-        for (int j = row; j < 32; j += step) {
-            const int m = m0 + j;
-            if (m >= M || c >= cols) continue;
-            u32x4 v = *(const u32x4*)(stage + j * ROW + 2 * (c - c0));
-            const int64_t at = (int64_t)m * cols + c;
-            if (residual) {
-                float f[8], g[8];
-                u32x4 rr;
-                if (aligned) rr = *(const u32x4*)(residual + at);
-                else
-                    for (int i = 0; i < 4; ++i) rr[i] = residual[at + 2 * i] | (uint32_t)residual[at + 2 * i + 1] << 16;
-                unpack8<T>(v, f);
-                unpack8<T>(rr, g);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = pack2<T>(__fadd_rn(f[2 * i], g[2 * i]), __fadd_rn(f[2 * i + 1], g[2 * i + 1]));
-            }
-            if (aligned) *(u32x4*)(y + at) = v;
-            else
-                for (int i = 0; i < 8; ++i) y[at + i] = (uint16_t)(v[i >> 1] >> (16 * (i & 1)));
-        }
+        tg_flush<T>(y, residual, stage, m0, M, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? 4 : 8, aligned, t, threads);
     }
 };
 
@@ -1020,45 +969,12 @@ struct GemmPlan {
     int steps_per_split;
 };
 
-// Tile plan of the many-row kernel.  Measured, a 64-wide k-step of a tile takes TG_STEP_ALONE us on a compute unit of its
-// own and a pair of tiles on one compute unit takes TG_STEP_PAIR us a step (the clock follows the power draw).  Whole
-// tiles fill whole multiples of the 256 compute units; what is left over would hold a few of them for a whole tile's
-// time, so it is cut along K where the shorter tail pays for writing and summing the fp32 parts
-// (4137 x 4096 x 14336: 16 of 528 tiles left, 531 us uncut, 423 us in 8 parts).
+// Tile plan of the many-row kernel (4137 x 4096 x 14336: 16 of 528 tiles left over by whole rounds, 531 us uncut, 423 us in
+// 8 parts).
 constexpr int TG_MT = 4;
-constexpr float TG_STEP_ALONE = 0.75f, TG_STEP_PAIR = 1.72f, TG_REDUCE = 5.f, TG_PART = 0.065f, TG_FIXED = 6.f;
-
-TileGrid plan_tiles(int m, int n, int k, float* us = nullptr) {
-    TileGrid g;
-    g.m_blocks = (m + 32 * TG_MT - 1) / (32 * TG_MT);
-    g.n_blocks = (n + tg::BN - 1) / tg::BN;
-    const int tiles = g.m_blocks * g.n_blocks, steps = k / tg::KSTEP;
-    const int rows = tiles / 256, rem = tiles % 256;
-    float best = 0.f;
-    g.split = 1;
-    for (int s = 1; s <= 16; s *= 2) {
-        if (s > 1 && (rem == 0 || steps / s < 4)) break;
-        const int part = (steps + s - 1) / s;
-        float t = (rows / 2) * steps * TG_STEP_PAIR;
-        if (s == 1) {
-            const int tail = (rows & 1) * 256 + rem;
-            t += tail == 0 ? 0.f : steps * (tail <= 256 ? TG_STEP_ALONE : TG_STEP_PAIR);
-        } else {
-            const int left = rem * s;
-            if (rows & 1) t += steps * TG_STEP_ALONE + (left + 255) / 256 * part * (TG_STEP_PAIR - TG_STEP_ALONE);
-            else t += left <= 256 ? part * TG_STEP_ALONE : (left + 511) / 512 * part * TG_STEP_PAIR;
-            t += TG_REDUCE + left * TG_PART;
-        }
-        if (s == 1 || t < best) {
-            best = t;
-            g.split = s;
-        }
-    }
-    g.steps_per_split = (steps + g.split - 1) / g.split;
-    g.split = (steps + g.steps_per_split - 1) / g.steps_per_split;
-    g.full = g.split > 1 ? tiles - rem : tiles / 8 * 8;       // a multiple of 8 (see tg_locate)
-    if (us) *us = best + TG_FIXED;
-    return g;
+constexpr TileCost TG_COST = {0.75f, 1.72f, 6.f, 5.f, 0.065f};
+TileGrid plan_tiles(int m, int n, int k, float* us) {
+    return tg_plan((m + 32 * TG_MT - 1) / (32 * TG_MT), (n + tg::BN - 1) / tg::BN, k / tg::KSTEP, TG_COST, us);
 }
 
 GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
@@ -1096,20 +1012,20 @@ bool use_tiles(int m, int n, int k) {
     plan_tiles(m, n, k, &us);
     const GemmPlan p = plan_w8a16(m, n, k);
     const int rounds = (p.n_blocks * p.m_blocks * p.split_k + 255) / 256;
-    return us < 0.40f * rounds * p.steps_per_split + 4.f + (p.split_k > 1 ? TG_REDUCE : 0.f);
+    return us < 0.40f * rounds * p.steps_per_split + 4.f + (p.split_k > 1 ? TG_COST.reduce : 0.f);
 }
 
 template <typename T>
 void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias, const void* residual, int m,
                   int n, int k, int gated, void* workspace, hipStream_t st) {
-    const TileGrid g = plan_tiles(m, n, k);
-    const int cut = g.m_blocks * g.n_blocks - g.full;
+    float us;
+    const TileGrid g = plan_tiles(m, n, k, &us);
     const int aligned = (((uintptr_t)y | (uintptr_t)residual) & 15) == 0;
-    hipLaunchKernelGGL((w8a16_tile_kernel<T, TG_MT>), dim3(g.full + cut * g.split), dim3(256), 0, st, (uint16_t*)y,
+    hipLaunchKernelGGL((w8a16_tile_kernel<T, TG_MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y,
                        (float*)workspace, (const uint16_t*)x, wp, scale, (const uint16_t*)bias, (const uint16_t*)residual, m,
                        n, k, gated, aligned, g);
     if (g.split > 1)
-        hipLaunchKernelGGL((w8a16_tile_reduce_kernel<T, TG_MT>), dim3(cut * tg::WAVES * TG_MT), dim3(256), 0, st,
+        hipLaunchKernelGGL((w8a16_tile_reduce_kernel<T, TG_MT>), dim3((g.m_blocks * g.n_blocks - g.full) * tg::WAVES * TG_MT), dim3(256), 0, st,
                            (uint16_t*)y, (const float*)workspace, scale, (const uint16_t*)bias, (const uint16_t*)residual, m,
                            n, gated, aligned, g);
 }
@@ -1139,8 +1055,7 @@ void launch_skinny(const GemmPlan& p, void* y, float* partial, const void* x, co
     } else
     if (p.mt == 1) { if (ktail) GW4_LAUNCH(1, 4, true); else GW4_LAUNCH(1, 4, false); }
     else if (p.mt == 2) { if (ktail) GW4_LAUNCH(2, 4, true); else GW4_LAUNCH(2, 4, false); }
-    else if (p.waves == 8) { if (ktail) GW4_LAUNCH(4, 8, true); else GW4_LAUNCH(4, 8, false); }
-    else { if (ktail) GW4_LAUNCH(4, 4, true); else GW4_LAUNCH(4, 4, false); }
+    else { if (ktail) GW4_LAUNCH(4, 8, true); else GW4_LAUNCH(4, 8, false); }
 #undef GW4_LAUNCH
 #undef GW4_LAUNCH_W4
 #undef GW4_W4_BY_GROUP
@@ -1235,7 +1150,8 @@ extern "C" int mf_w8a16_pack_weight(void* packed, const int8_t* w, int n, int k,
 extern "C" size_t mf_w8a16_workspace_bytes(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
     if (use_tiles(m, n, k)) {
-        const TileGrid g = plan_tiles(m, n, k);
+        float us;
+        const TileGrid g = plan_tiles(m, n, k, &us);
         return g.split > 1 ? (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * TG_MT * tg::BN) * sizeof(float) : 0;
     }
     const GemmPlan p = plan_w8a16(m, n, k);

@@ -20,10 +20,13 @@
 // applied on the global-address side, which makes the operand reads bank-conflict free.
 // Small N cannot fill the chip with output tiles alone: K is then split across workgroups, which write exact
 // int32 partial tiles that a second kernel sums (integer sums do not depend on the order).
-// Two more kernels serve the shapes where that one is not the best: a register-streaming kernel for narrow outputs
-// at 65+ rows (w8a8_regs_kernel) and, for very wide outputs at 129+ rows, 256 x 192 tiles on 8 waves with the
-// full-rate v_mfma_i32_32x32x32_i8 and a coalesced, LDS-turned epilogue (w8a8_wide_kernel).
+// More kernels serve the shapes where that one is not the best: from 65 rows on with tiled activations 128 x 256 tiles with
+// the full-rate v_mfma_i32_32x32x32_i8 (w8a8_tile_kernel); where those leave a part of a round over, for narrow outputs and
+// few rows, a register-streaming kernel (w8a8_regs_kernel) and, for very wide outputs at 129 - 256 rows, 256 x 192 tiles on 8
+// waves with a coalesced, LDS-turned epilogue (w8a8_wide_kernel).
 #include "common.h"
+#include "tile_grid.h"
+#include "w8a8_tile_gemm.h"
 
 namespace {
 
@@ -90,8 +93,7 @@ __device__ __forceinline__ void q2_store4(uint16_t* y, int32_t* acc_out, const f
     for (int i = 0; i < 4; ++i) {
         v[i] = 0.f;
         if (n + i < N) {
-            float t = (float)a[i] * xs * w_scale[n + i];
-            if (bias) t += T::to_float(bias[n + i]);
+            float t = scaled_bias((float)a[i], xs, w_scale[n + i], true, bias ? T::to_float(bias[n + i]) : 0.f, bias != nullptr);
             if (residual) t = T::to_float(T::from_float(t)) + T::to_float(residual[o + i]);
             v[i] = t;
         }
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(
 // flight per workgroup) and a main loop that is nothing but loads and matrix instructions.
 constexpr int QR_DEPTH = 3;
 
-// ---- wide outputs at 129+ rows: 256 x 192 tiles on 8 waves with mfma_i32_32x32x32_i8 ----------------------------
+// ---- wide outputs at 129 - 256 rows: 256 x 192 tiles on 8 waves with mfma_i32_32x32x32_i8 ----------------------------
 // On gfx950 the 16x16x64 int8 instruction issues at half the rate of the 32x32x32 one (measured: 2.4 against
 // 4.4 POP/s with independent accumulators), so the kernel that is bound by the matrix cores uses the latter.
 // The packed tile format serves it unchanged: rows 32 b .. 32 b + 31 of a k-step are two consecutive 1 KiB
@@ -746,6 +748,107 @@ __global__ __launch_bounds__(QRC_THREADS) void w8a8_reduce_rope_cache_kernel(
     }
 }
 
+// ---- many rows (tiled activations): 128 x 256 tiles, w8a8_tile_gemm.h ------------------------------------------------
+// Output of one wave, 32 rows x 64 channels at a time, through LDS as whole pieces of rows (tg_flush); rounding points as in
+// q2_store4.  N is a multiple of 16.
+template <typename T>
+struct QTileOut {
+    const float *x_scale, *w_scale;
+    const uint16_t* bias;
+    int M, N;
+    __device__ __forceinline__ void load(int n0, int nt, int q, f32x4& ws, f32x4& bi) const {
+        const int n = min(n0 + 32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1), N - 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            ws[i] = w_scale[n + i];
+            bi[i] = bias ? T::to_float(bias[n + i]) : 0.f;
+        }
+    }
+    __device__ __forceinline__ void put(i32x4 a, float xs, f32x4 ws, f32x4 bi, int nt, int q, uint8_t* stage) const {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = scaled_bias((float)a[i], xs, ws[i], true, bi[i], bias != nullptr);
+        *(u32x2*)(stage + (threadIdx.x & 31) * TG_STAGE_ROW + 2 * (32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1))) =
+            (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+    }
+};
+
+template <typename T, int MT>
+__global__ __launch_bounds__(256, 2) void w8a8_tile_kernel(
+    uint16_t* __restrict__ y, int32_t* __restrict__ partial, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
+    const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const uint16_t* __restrict__ bias,
+    const uint16_t* __restrict__ residual, int M, int N, int K, int aligned, TileGrid g) {
+    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW, OPS = tq::LDS_BYTES<MT>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
+    int mb, nb, part, slot;
+    tg_locate(g, blockIdx.x, mb, nb, part, slot);
+    const bool whole = blockIdx.x < g.full || g.split == 1;
+    const int KS = (K + Q_KSTEP - 1) / Q_KSTEP, s0 = part * g.steps_per_split;
+    const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int m0 = mb * 32 * MT, n0 = nb * tq::BN + 64 * wv;
+    int32_t* pt = partial + (int64_t)slot * (32 * MT * tq::BN) + (wv * MT * 8 * 64 + lane) * 4;
+    const QTileOut<T> out{x_scale, w_scale, bias, M, N};
+    f32x4 ws[8], bi[8];
+    uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
+    tq::tile<MT>((const uint8_t*)xq, wp, m0 >> 4, (M + 15) >> 4, nb * (tq::BN / 16), (N + 15) >> 4, s0, s_end, smem,
+                 [&](auto mtc, const i32x16 (&acc)[2]) {
+        constexpr int mt = decltype(mtc)::value;
+        if (whole) {
+            if (mt == 0) {
+                __syncthreads();                              // every wave has read its last operands
+#pragma unroll
+                for (int e = 0; e < 8; ++e) out.load(n0, e >> 2, e & 3, ws[e], bi[e]);
+            }
+            const float xs = x_scale[min(m0 + 32 * mt + (lane & 31), M - 1)];
+            wave_lds_order();
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                out.put((i32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
+                                acc[e >> 2][4 * (e & 3) + 3]}, xs, ws[e], bi[e], e >> 2, e & 3, stage);
+            wave_lds_order();
+            tg_flush<T>(y, residual, stage, m0 + 32 * mt, M, n0, N, 8, aligned, lane, 64);
+        } else {                                              // accumulator order: whole cache lines
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                *(i32x4*)(pt + (mt * 8 + e) * 256) = (i32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1],
+                                                             acc[e >> 2][4 * (e & 3) + 2], acc[e >> 2][4 * (e & 3) + 3]};
+        }
+    });
+}
+
+// Sums the parts of the tiles that were cut along K: a workgroup per 32 rows x 64 channels, a quarter of the channels per wave.
+template <typename T, int MT>
+__global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
+    uint16_t* __restrict__ y, const int32_t* __restrict__ partial, const float* __restrict__ x_scale,
+    const float* __restrict__ w_scale, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N,
+    int aligned, TileGrid g) {
+    __shared__ __attribute__((aligned(16))) uint8_t stage[32 * TG_STAGE_ROW];
+    constexpr int ITEMS = tq::WAVES * MT;                     // workgroups per tile
+    constexpr int64_t PART = 32 * MT * tq::BN;
+    const int tile = blockIdx.x / ITEMS, item = blockIdx.x - tile * ITEMS, wv = item / MT, mt = item - wv * MT;
+    int mb, nb, part, slot;
+    tg_locate(g, g.full + tile * g.split, mb, nb, part, slot);
+    const int m0 = mb * 32 * MT + 32 * mt, n0 = nb * tq::BN + 64 * wv;
+    if (m0 >= M || n0 >= N) return;
+    const int lane = threadIdx.x & 63, e0 = 2 * (threadIdx.x >> 6);
+    const int32_t* p = partial + slot * PART + ((wv * MT + mt) * 8 * 64 + lane) * 4;
+    const QTileOut<T> out{x_scale, w_scale, bias, M, N};
+    const float xs = x_scale[min(m0 + (lane & 31), M - 1)];
+    f32x4 ws[2], bi[2];
+    i32x4 v[2] = {(i32x4)(0), (i32x4)(0)};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) out.load(n0, (e0 + e) >> 2, (e0 + e) & 3, ws[e], bi[e]);
+#pragma unroll 8
+    for (int s = 0; s < g.split; ++s)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) v[e] += *(const i32x4*)(p + s * PART + (e0 + e) * 256);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) out.put(v[e], xs, ws[e], bi[e], (e0 + e) >> 2, (e0 + e) & 3, stage);
+    __syncthreads();
+    tg_flush<T>(y, residual, stage, m0, M, n0, N, 8, aligned, threadIdx.x, 256);
+}
+
 // ---- grouped (experts): rows offsets[e] .. offsets[e+1] of the quantised activations use expert e's weights --------
 // grid = (ceil(N / 64), n_experts); a workgroup of 4 waves owns 64 output channels of one expert for all of its
 // rows.  Decode batches route a handful of tokens to each expert, so the kernel is a weight stream: the waves
@@ -911,7 +1014,7 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
         p.nt = n >= 16384 ? 5 : 4;
         // very wide outputs: 256 x 192 tiles on 8 waves, one workgroup per CU (one staged activation tile serves
         // more channels, and the 32 x 32 x 32 instruction runs at twice the rate of the 16 x 16 x 64 one)
-        p.wide = x_tiled && n >= 16384 && m > 128;
+        p.wide = x_tiled && n >= 16384 && m > 128 && m <= 256;
         p.m_blocks = (m + 255) / 256;
     } else {
         p.nt = 2;
@@ -932,12 +1035,48 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
     return p;
 }
 
+// Many rows, tiled activations: 128 x 256 tiles against the kernels above.  Measured, a 64-wide step of a round of 256
+// workgroups takes 0.32 us in the register-streaming kernel and 0.78 us in the wide one.  37888 x 3584 at 65 / 257 / 1531 rows
+// runs in 32 / 57 / 250 us on tiles against 49 / 86 / 275 (256 rows: 296 tiles, 40 more than units, 52 us against 48 on 198
+// wide tiles), 28672 x 4096 at 256 rows in 40 against 51, 3584 x 18944 at 1531 rows in 120 against 181, 3584 x 3584 at 448
+// rows in 27 against 20.  `fused`: the sum of the register-streaming kernel's parts carries what follows, which is a kernel of
+// its own behind tiles.
+constexpr int TQ_MT = 4;
+constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f};
+bool plan_q_tiles(int m, int n, int k, bool fused, TileGrid& g) {
+    if (m <= 64 || n % 16 != 0) return false;
+    float us;
+    g = tg_plan((m + 32 * TQ_MT - 1) / (32 * TQ_MT), (n + tq::BN - 1) / tq::BN, (k + Q_KSTEP - 1) / Q_KSTEP, TQ_COST, &us);
+    const QPlan p = plan_w8a8(m, n, k, true);
+    if (!p.regs && !p.wide) return true;                      // the LDS-staged kernel on the half-rate instruction
+    const int rounds = (p.n_blocks * p.m_blocks * p.split_k + 255) / 256;
+    const float old = (p.wide ? 0.78f : 0.32f) * rounds * p.steps_per_split + 5.f + (p.split_k > 1 ? TQ_COST.reduce : 0.f);
+    return us + (fused && p.split_k > 1 ? 6.f : 0.f) < old;
+}
+
+template <typename T>
+void launch_q_tiles(const TileGrid& g, void* y, const int8_t* xq, const float* x_scale, const uint8_t* wp,
+                    const float* w_scale, const void* bias, const void* residual, int m, int n, int k, void* workspace,
+                    hipStream_t st) {
+    const int aligned = (((uintptr_t)y | (uintptr_t)residual) & 15) == 0;
+    hipLaunchKernelGGL((w8a8_tile_kernel<T, TQ_MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y,
+                       (int32_t*)workspace, xq, x_scale, wp, w_scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n,
+                       k, aligned, g);
+    if (g.split > 1)
+        hipLaunchKernelGGL((w8a8_tile_reduce_kernel<T, TQ_MT>), dim3((g.m_blocks * g.n_blocks - g.full) * tq::WAVES * TQ_MT),
+                           dim3(256), 0, st, (uint16_t*)y, (const int32_t*)workspace, x_scale, w_scale,
+                           (const uint16_t*)bias, (const uint16_t*)residual, m, n, aligned, g);
+}
+
 template <typename T>
 int launch_w8a8(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale, const uint8_t* wp,
                 const float* w_scale, const void* bias, const void* residual, int m, int n, int k, bool x_tiled,
                 void* workspace, hipStream_t st, const QNormQuantArgs* nq = nullptr,
                 const QRopeCacheArgs* rc = nullptr) {
-    const QPlan p = plan_w8a8(m, n, k, x_tiled);
+    QPlan p = plan_w8a8(m, n, k, x_tiled);
+    TileGrid g;
+    const bool tiles = x_tiled && y && !acc_out && plan_q_tiles(m, n, k, nq || rc, g);
+    if (tiles) p.split_k = 1;                                 // the tile kernel sums its own parts
     int32_t* partial = p.split_k > 1 ? (int32_t*)workspace : nullptr;
     dim3 grid(p.n_blocks, p.split_k, p.m_blocks);
     const bool ktail = (k % Q_KSTEP) != 0;
@@ -968,7 +1107,8 @@ int launch_w8a8(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scal
     hipLaunchKernelGGL((w8a8_regs_kernel<T, WMV, MTV, NTV>), grid, dim3(256), 0, st, (uint16_t*)y, acc_out, partial, \
                        xq, x_scale, wp, w_scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k,          \
                        p.steps_per_split)
-    if (p.regs == 1) QR_LAUNCH(4, 4, 4);
+    if (tiles) launch_q_tiles<T>(g, y, xq, x_scale, wp, w_scale, bias, residual, m, n, k, workspace, st);
+    else if (p.regs == 1) QR_LAUNCH(4, 4, 4);
     else if (!p.msplit) Q_LAUNCH_KT(2, 0, 4);
     else if (p.wide) {
         static bool configured[MF_MAX_DEVICES] = {};
@@ -1030,6 +1170,11 @@ extern "C" size_t mf_w8a8_workspace_bytes(int m, int n, int k) {
     for (int tiled = 0; tiled < 2; ++tiled) {
         const QPlan p = plan_w8a8(m, n, k, tiled != 0);
         const size_t b = p.split_k > 1 ? (size_t)p.split_k * m * n * sizeof(int32_t) : 0;
+        need = b > need ? b : need;
+    }
+    TileGrid g;
+    if (plan_q_tiles(m, n, k, false, g) && g.split > 1) {     // enough for either kernel
+        const size_t b = (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * TQ_MT * tq::BN) * sizeof(int32_t);
         need = b > need ? b : need;
     }
     return need;

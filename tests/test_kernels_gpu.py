@@ -1251,6 +1251,37 @@ def test_w8a8_gemm_int32_bit_exact(m, n, k):
     assert_within(to_np(y), ref, np.abs(ref) + np.abs(b), dtype, ulps=1.0, extra=1e-6, what="w8a8 dequant")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,bias,residual", [
+    (129, 8208, 208, True, True),          # one row and one 16-channel piece past whole tiles, a short last k-step
+    (65, 16384, 4160, False, False),       # one row block, an odd number of k-steps
+    (513, 3584, 9472, True, True),         # every tile cut along K
+    (1100, 9216, 1088, True, False),       # whole tiles and cut ones
+    (2100, 4608, 320, False, True)])       # more than a round of whole tiles, few k-steps
+def test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, bias, residual):
+    """The tile kernel (tiled activations) gives the bits of the row-major kernel on the same integers, whose int32
+    accumulators are exact; the dequantisation against float64: three roundings to fp32, one to the output type and one of
+    the sum with the residual."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    w = torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+    ws = (torch.rand(n, generator=g, device="cuda") + 0.5) * (k ** -0.5 / 73)
+    b = torch.randn(n, generator=g, device="cuda").to(dtype) if bias else None
+    r = torch.randn(m, n, generator=g, device="cuda").to(dtype) if residual else None
+    packed = ops.pack_w8a16(w, ws)
+    xt, xs = ops.dynamic_quant(x, None, tiled=True)
+    xr, _ = ops.dynamic_quant(x, None)
+    y = ops.w8a8_linear(xt, xs, packed, out_dtype=dtype, bias=b, residual=r)
+    assert torch.equal(y, ops.w8a8_linear(xr, xs, packed, out_dtype=dtype, bias=b, residual=r))
+    v = (xr.double() @ w.double().t()) * xs.double()[:, None] * ws.double()
+    if bias:
+        v += b.double()
+    ref = v + r.double() if residual else v
+    tol = EPS[dtype] * (ref.abs() + (v.abs() if residual else 0)) * 1.01 + 4 * 2.0 ** -24 * (v.abs() + 1) + 1e-7
+    assert bool(((y.double() - ref).abs() <= tol).all())
+
+
 @pytest.mark.parametrize("m,k", [(256, 3584), (37, 1376), (1, 64), (130, 208)])
 def test_dynamic_quant_tiled_layout_bit_exact(m, k):
     """The tiled output holds exactly the row-major result, at the positions the int8 GEMM reads."""
