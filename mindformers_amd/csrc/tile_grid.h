@@ -66,13 +66,63 @@ inline TileGrid tg_plan(int m_blocks, int n_blocks, int steps, const TileCost& c
     return g;
 }
 
+// Grouped rows (experts): the row blocks of all experts, in order, times the channel blocks.  Their number is known on the
+// device only (offsets [n_experts + 1]), so the launch covers what the total allows and each workgroup finds its own by a
+// scan of the offsets.  Ids go to the XCDs in turn; XCD j is given the j-th eighth of the row blocks, all channel blocks of
+// one side by side, so that an expert's activations are read into one L2 and the weights of an expert with several row blocks
+// are met there by all of them.  False: nothing to do.
+constexpr int TG_GROUP_ROWS = 128;
+inline unsigned tg_group_workgroups(int total_rows, int n_experts, int n_blocks) {
+    const int64_t m_blocks = (int64_t)total_rows / TG_GROUP_ROWS + min(n_experts, total_rows);
+    return (unsigned)((m_blocks + 7) / 8 * 8 * n_blocks);
+}
+__device__ __forceinline__ bool tg_group_locate(const int32_t* __restrict__ offsets, int n_experts, int total_rows,
+                                                int n_blocks, int& expert, int& m0, int& row0, int& rows, int& nb) {
+    const int lane = threadIdx.x & 63;
+    auto span = [&](int e, int& r0) {
+        if (e >= n_experts) return 0;
+        r0 = max(0, min(offsets[e], total_rows));
+        return max(r0, min(offsets[e + 1], total_rows)) - r0;
+    };
+    int total = 0, r0 = 0;
+    for (int e = lane; e < n_experts; e += 64) total += (span(e, r0) + TG_GROUP_ROWS - 1) / TG_GROUP_ROWS;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+    const int id = blockIdx.x, per_xcd = (total + 7) / 8, at = (id >> 3) / n_blocks;
+    nb = (id >> 3) - at * n_blocks;
+    int want = (id & 7) * per_xcd + at;
+    if (at >= per_xcd || want >= total) return false;
+    for (int base = 0; base < n_experts; base += 64) {
+        const int n = span(base + lane, r0), blocks = (n + TG_GROUP_ROWS - 1) / TG_GROUP_ROWS;
+        int upto = blocks;                                    // blocks of the experts up to this lane's
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += up;
+        }
+        const uint64_t past = __ballot(upto > want);
+        if (past) {
+            const int l = __ffsll((unsigned long long)past) - 1;
+            expert = __builtin_amdgcn_readfirstlane(base + l);
+            row0 = __builtin_amdgcn_readfirstlane(__shfl(r0, l, 64));
+            rows = __builtin_amdgcn_readfirstlane(__shfl(n, l, 64));
+            m0 = __builtin_amdgcn_readfirstlane(TG_GROUP_ROWS * (want - __shfl(upto - blocks, l, 64)));
+            return true;
+        }
+        want -= __builtin_amdgcn_readfirstlane(__shfl(upto, 63, 64));
+    }
+    return false;
+}
+
 // acc * a (* b) (+ bias), every operation rounded by itself: the epilogues of the many-row kernels are straight-line code in
-// which the compiler would contract the last product and the sum, and the other kernels' results are to be met bit for bit
+// which the compiler would contract the last product and the sum, or (without a bias) round the last product to fp16 at once
+// (v_fma_mixlo_f16), and the other kernels' results are to be met bit for bit
 __device__ __forceinline__ float scaled_bias(float acc, float a, float b, bool two, float bias, bool with_bias) {
 #pragma clang fp contract(off)
     float v = acc * a;
     if (two) v = v * b;
     if (with_bias) v = v + bias;
+    asm("" : "+v"(v));                                        // a float32 value of its own
     return v;
 }
 

@@ -633,6 +633,10 @@ __global__ __launch_bounds__(256) void w8a16_tile_reduce_kernel(
     out.flush(m0, n0, stage, threadIdx.x, 256);
 }
 
+// Groups that average more rows take w8a16_group_tile_kernel.  256 experts of 4096 x 7168 (gated) / 7168 x 2048, us, passes |
+// tiles: 12 rows a group 1151 + 725 | 1210 + 662, 16: 1196 + 780 | 1216 + 681, 32: 1515 + 941 | 1258 + 731.
+constexpr int GW_GROUP_TILE_ROWS = 12;
+
 // Grouped (experts): grid = (ceil(N/64), n_experts).  Rows offsets[e] .. offsets[e+1] of x use expert e's
 // packed weights and scale[e]; experts with no rows exit at once.  One pass over the expert's weights serves up to
 // 64 rows (decode batches route a handful of tokens to each expert: 16 rows per pass there); experts with more rows
@@ -667,6 +671,56 @@ __global__ __launch_bounds__(GW_WAVES * 64, 2) void w8a16_grouped_kernel(
             __syncthreads();                                  // the LDS tile is reused by the next pass
         }
     }
+}
+
+// Groups of prompt size: tiles of up to 128 rows x 256 channels of one expert (w8a16_tile_gemm.h; fewer 32-row tiles where the
+// expert's rows end), the row blocks of all experts dealt to the XCDs as tg_group_locate says.  Bound by the stream of the
+// expert weights: 256 experts of 65 rows, 4096 x 7168 (gated): 2644 us in passes of 64 rows, 1439 here (5.2 TB/s of weights);
+// 7168 x 2048: 1564 / 804.
+template <typename T, int MT>
+__device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* xe, const uint8_t* we, const float* se, int rows,
+                                                 int m0, int nb, int N, int K, int gated, int aligned, uint8_t* smem) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int n0 = nb * tg::BN + 64 * wv;
+    const TileOut<T> out{y, nullptr, nullptr, rows, N, gated, aligned};
+    f32x4 sc[8], bi[8];
+    uint8_t* stage = smem + wv * 32 * TileOut<T>::ROW;
+    tg::tile<T, MT>(xe, we, rows, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, 0, K / tg::KSTEP, smem,
+                    [&](auto mtc, const f32x16 (&acc)[2]) {
+        constexpr int mt = decltype(mtc)::value;
+        if (mt == 0) {
+            __syncthreads();                                  // every wave has read its last operands
+#pragma unroll
+            for (int e = 0; e < 8; ++e) out.load(se, n0, e >> 2, e & 3, sc[e], bi[e]);
+        }
+        wave_lds_order();
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            out.put((f32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
+                            acc[e >> 2][4 * (e & 3) + 3]}, sc[e], bi[e], e >> 2, e & 3, stage);
+        wave_lds_order();
+        out.flush(m0 + 32 * mt, n0, stage, lane, 64);
+    });
+}
+
+template <typename T>
+__global__ __launch_bounds__(256, 2) void w8a16_group_tile_kernel(
+    uint16_t* __restrict__ y, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, const float* __restrict__ scale,
+    const int32_t* __restrict__ offsets, int n_experts, int total_rows, int N, int K, int64_t expert_bytes, int gated,
+    int aligned) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * 128 * 128];
+    static_assert(tg::WAVES * 32 * TileOut<T>::ROW <= (int)sizeof(smem), "the output stage reuses the operand stages");
+    int e, m0, row0, rows, nb;
+    if (!tg_group_locate(offsets, n_experts, total_rows, (N + tg::BN - 1) / tg::BN, e, m0, row0, rows, nb)) return;
+    uint16_t* ye = y + (int64_t)row0 * (gated ? N >> 1 : N);
+    const uint16_t* xe = x + (int64_t)row0 * K;
+    const uint8_t* we = wp + (int64_t)e * expert_bytes;
+    const float* se = scale + (int64_t)e * N;
+    const int left = rows - m0;
+    if (left <= 32) w8a16_group_tile<T, 1>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
+    else if (left <= 64) w8a16_group_tile<T, 2>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
+    else if (left <= 96) w8a16_group_tile<T, 3>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
+    else w8a16_group_tile<T, 4>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
 }
 
 template <typename T>
@@ -1324,6 +1378,18 @@ static int grouped_w8a16_entry(const char* who, void* y, const void* x, const vo
     MF_REQUIRE(!gated || n % 4 == 0, "%s: N (%d) must be a multiple of 4 (gate / up pairs)", who, n);
     MF_REQUIRE((((uintptr_t)x | (uintptr_t)w_packed) & 15) == 0, "%s: x and w_packed must be 16-byte aligned", who);
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
+    if (n % 16 == 0 && k % tg::KSTEP == 0 && total_rows > GW_GROUP_TILE_ROWS * (int64_t)n_experts) {
+        const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tg::BN - 1) / tg::BN));
+        const int aligned = ((uintptr_t)y & 15) == 0;
+#define GGT_LAUNCH(TT)                                                                                            \
+    hipLaunchKernelGGL((w8a16_group_tile_kernel<TT>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y,        \
+                       (const uint16_t*)x, (const uint8_t*)w_packed, scale, offsets, n_experts, total_rows, n, k,    \
+                       expert_bytes, gated, aligned)
+        if (dtype == MF_BF16) GGT_LAUNCH(BF16);
+        else GGT_LAUNCH(FP16);
+#undef GGT_LAUNCH
+        return MF_LAUNCH_CHECK();
+    }
     dim3 grid((n + GW_BN - 1) / GW_BN, n_experts);
 #define GG_LAUNCH(TT, KT)                                                                                        \
     hipLaunchKernelGGL((w8a16_grouped_kernel<TT, KT>), grid, dim3(GW_WAVES * 64), 0, (hipStream_t)stream,           \

@@ -791,8 +791,8 @@ __global__ __launch_bounds__(256, 2) void w8a8_tile_kernel(
     const QTileOut<T> out{x_scale, w_scale, bias, M, N};
     f32x4 ws[8], bi[8];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
-    tq::tile<MT>((const uint8_t*)xq, wp, m0 >> 4, (M + 15) >> 4, nb * (tq::BN / 16), (N + 15) >> 4, s0, s_end, smem,
-                 [&](auto mtc, const i32x16 (&acc)[2]) {
+    const tq::TiledRows<MT / 2> rows((const uint8_t*)xq, m0 >> 4, (M + 15) >> 4);
+    tq::tile<MT>(rows, wp, nb * (tq::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const i32x16 (&acc)[2]) {
         constexpr int mt = decltype(mtc)::value;
         if (whole) {
             if (mt == 0) {
@@ -862,6 +862,9 @@ __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
 constexpr int QG_WAVES = 4;
 constexpr int QG_NT = 4;                                      // 16-channel weight tiles per wave and step
 constexpr int QG_BN = 16 * QG_NT;
+// Groups that average more rows take w8a8_group_tile_kernel.  256 experts of 4096 x 7168 / 7168 x 2048, us, passes | tiles:
+// 12 rows a group 1219 + 655 | 1218 + 657, 16: 1236 + 689 | 1222 + 677, 32: 1459 + 856 | 1268 + 726.
+constexpr int QG_TILE_ROWS = 12;
 template <int MTMAX>
 constexpr int QG_SMEM = QG_WAVES * 16 * MTMAX * QG_BN * 4;    // MTMAX 16-row activation tiles per pass
 
@@ -970,6 +973,55 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
         for (int m0 = 0; m0 < rows; m0 += 16 * MTMAX)
             w8a8_group_pass<T, MTMAX>(ye, ae, xe, xse, we, se, rows, N, K, n0, m0, red);
     }
+}
+
+// Groups of prompt size: tiles of up to 128 rows x 256 channels of one expert (w8a8_tile_gemm.h on row-major rows, 64-row
+// tiles where the expert has no more), the row blocks of all experts dealt to the XCDs as tg_group_locate says.  Bound by the
+// stream of the expert weights: 256 experts of 65 rows, 4096 x 7168: 2258 us in passes of 64 rows by 64-channel workgroups
+// (each fetching the rows anew, a second pass for every second expert), 1435 here (5.2 TB/s of weights); 7168 x 2048: 1280 / 817.
+template <typename T, int MT>
+__device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, const float* xs, const uint8_t* we,
+                                                const float* ws, int rows, int m0, int nb, int N, int K, int aligned,
+                                                uint8_t* smem) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int n0 = nb * tq::BN + 64 * wv;
+    const QTileOut<T> out{xs, ws, nullptr, rows, N};
+    f32x4 wsv[8], bi[8];
+    uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
+    const tq::PlainRows<MT / 2> src(xe, m0, rows, K);
+    tq::tile<MT>(src, we, nb * (tq::BN / 16), (N + 15) >> 4, 0, (K + Q_KSTEP - 1) / Q_KSTEP, smem,
+                 [&](auto mtc, const i32x16 (&acc)[2]) {
+        constexpr int mt = decltype(mtc)::value;
+        if (mt == 0) {
+            __syncthreads();                                  // every wave has read its last operands
+#pragma unroll
+            for (int e = 0; e < 8; ++e) out.load(n0, e >> 2, e & 3, wsv[e], bi[e]);
+        }
+        const float x1 = xs[min(m0 + 32 * mt + (lane & 31), rows - 1)];
+        wave_lds_order();
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            out.put((i32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
+                            acc[e >> 2][4 * (e & 3) + 3]}, x1, wsv[e], bi[e], e >> 2, e & 3, stage);
+        wave_lds_order();
+        tg_flush<T>(y, nullptr, stage, m0 + 32 * mt, rows, n0, N, 8, aligned, lane, 64);
+    });
+}
+
+template <typename T>
+__global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
+    uint16_t* __restrict__ y, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
+    const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const int32_t* __restrict__ offsets, int n_experts,
+    int total_rows, int N, int K, int64_t expert_bytes, int aligned) {
+    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW, OPS = tq::LDS_BYTES<4>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
+    int e, m0, row0, rows, nb;
+    if (!tg_group_locate(offsets, n_experts, total_rows, (N + tq::BN - 1) / tq::BN, e, m0, row0, rows, nb)) return;
+    uint16_t* ye = y + (int64_t)row0 * N;
+    const uint8_t *xe = (const uint8_t*)xq + (int64_t)row0 * K, *we = wp + (int64_t)e * expert_bytes;
+    const float *xs = x_scale + row0, *ws = w_scale + (int64_t)e * N;
+    if (rows - m0 <= 64) w8a8_group_tile<T, 2>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
+    else w8a8_group_tile<T, 4>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
 }
 
 // What may follow the GEMM in the same call, fused with the split-K reduce where K is split.
@@ -1278,6 +1330,17 @@ extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq,
                "grouped_w8a8_gemm: xq and w_packed must be 16-byte aligned");
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
     dim3 grid((n + QG_BN - 1) / QG_BN, n_experts);
+    if (y && !acc_out && n % 16 == 0 && total_rows > QG_TILE_ROWS * (int64_t)n_experts) {
+        const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tq::BN - 1) / tq::BN));
+        const int aligned = ((uintptr_t)y & 15) == 0;
+#define QGT_LAUNCH(TT)                                                                                           \
+    hipLaunchKernelGGL((w8a8_group_tile_kernel<TT>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y, xq, x_scale, \
+                       (const uint8_t*)w_packed, w_scale, offsets, n_experts, total_rows, n, k, expert_bytes, aligned)
+        if (out_dtype == MF_BF16) QGT_LAUNCH(BF16);
+        else QGT_LAUNCH(FP16);
+#undef QGT_LAUNCH
+        return MF_LAUNCH_CHECK();
+    }
     // groups that average more than 16 rows (prefill-sized) take the 64-row passes; both builds serve any row count
     const bool big = (int64_t)total_rows > 16 * (int64_t)n_experts;
 #define QG_LAUNCH(TT, MTV)                                                                                      \

@@ -24,23 +24,46 @@ constexpr int D = 3;                                          // register sets
 template <int MT>
 constexpr int LDS_BYTES = 2 * 32 * MT * KSTEP;
 
-// xq in tile order; m_tile0 / tile0: first 16-row tile of the activations / weights, *_tiles: tiles of a step
-template <int MT, typename Epilogue>
-__device__ __forceinline__ void tile(const uint8_t* __restrict__ xq, const uint8_t* __restrict__ wp, int m_tile0, int m_tiles,
-                                     int tile0, int n_tiles, int s_begin, int s_end, uint8_t* smem, Epilogue&& epilogue) {
+// Where the activations come from: 16-row tile 4i + wave of the workgroup is load i of a wave, lane (r, g) of it row r, columns
+// 16g .. + 15 of the step.
+template <int XL>
+struct TiledRows {                                            // tile order: whole KiB, m_tiles of them a step
+    const uint8_t* p[XL];
+    int64_t step;
+    __device__ __forceinline__ TiledRows(const uint8_t* xq, int m_tile0, int m_tiles) : step((int64_t)m_tiles * 1024) {
+#pragma unroll
+        for (int i = 0; i < XL; ++i)
+            p[i] = xq + (int64_t)min(m_tile0 + 4 * i + (int)(threadIdx.x >> 6), m_tiles - 1) * 1024 + (threadIdx.x & 63) * 16;
+    }
+    __device__ __forceinline__ i32x4 load(int i, int s) const { return *(const i32x4*)(p[i] + s * step); }
+};
+template <int XL>
+struct PlainRows {                                            // rows m0 .. of `rows` rows of K (a multiple of 16) bytes
+    const uint8_t* p[XL];
+    int last;                                                 // columns past K are clamped: their weights are zero
+    __device__ __forceinline__ PlainRows(const uint8_t* xq, int m0, int rows, int K) {
+        const int r = threadIdx.x & 15, c = 16 * ((threadIdx.x >> 4) & 3);
+#pragma unroll
+        for (int i = 0; i < XL; ++i)
+            p[i] = xq + (int64_t)min(m0 + 16 * (4 * i + (int)(threadIdx.x >> 6)) + r, rows - 1) * K + c;
+        last = K - 16 - c;
+    }
+    __device__ __forceinline__ i32x4 load(int i, int s) const { return *(const i32x4*)(p[i] + min(s * KSTEP, last)); }
+};
+
+// tile0: first 16-channel tile of the weights, n_tiles: tiles of a step
+template <int MT, typename Rows, typename Epilogue>
+__device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ wp, int tile0, int n_tiles, int s_begin,
+                                     int s_end, uint8_t* smem, Epilogue&& epilogue) {
     static_assert(MT % 2 == 0, "the activation tiles of a step are dealt over the four waves");
     constexpr int STAGE = 32 * MT * KSTEP, XL = MT / 2;       // 16-row tiles loaded per wave and step
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int h = lane >> 5;
     const int s_last = s_end - 1;
-    const uint8_t* xbase[XL];
-#pragma unroll
-    for (int i = 0; i < XL; ++i) xbase[i] = xq + (int64_t)min(m_tile0 + 4 * i + wv, m_tiles - 1) * 1024 + lane * 16;
     i32x4 xreg[D][XL], wreg[D][2][2];
     auto load_x = [&](auto setc, int s) {
-        const int64_t off = (int64_t)min(s, s_last) * m_tiles * 1024;
 #pragma unroll
-        for (int i = 0; i < XL; ++i) xreg[decltype(setc)::value][i] = *(const i32x4*)(xbase[i] + off);
+        for (int i = 0; i < XL; ++i) xreg[decltype(setc)::value][i] = x.load(i, min(s, s_last));
     };
     auto write_x = [&](auto setc, int stage) {
 #pragma unroll

@@ -1618,6 +1618,37 @@ def test_grouped_w8a8_accumulators_bit_exact(counts, n, k):
         assert np.all(np.abs(got_y[r0:r1] - yref) <= 1.01 * EPS[torch.bfloat16] * np.abs(yref) + 1e-6), ex
 
 
+@pytest.mark.parametrize("counts,n,k", [
+    ([0, 1, 32, 33, 64, 65, 96, 97, 128, 129, 0, 300], 272, 192),   # both sides of every row-tile edge, a ragged last tile
+    ([20] * 70 + [0] * 3 + [17], 48, 64),                       # more experts than lanes, one step of K
+    ([0, 0, 400], 1024, 1040),                                  # one expert only; K ends inside a step (int8 activations)
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_grouped_gemms_at_prompt_sizes(counts, n, k, dtype):
+    """Groups that average more than 12 rows (the tiled kernels).  int8 activations: the bits of the register-streaming
+    kernel, whose exact accumulators are checked above.  16-bit activations: the oracle, an fp32 sum of K products (an ulp
+    of the output and 2^-18 of the sum of magnitudes), and the gated form as silu_mul of the plain one."""
+    rng = np.random.default_rng(n + k)
+    counts, off = _ragged_groups(rng, counts)
+    e, rows = len(counts), int(counts.sum())
+    od = torch.from_numpy(off).cuda()
+    wq = rng.integers(-127, 128, (e, n, k)).astype(np.int8)
+    ws = rng.uniform(1e-4, 5e-4, (e, n)).astype(np.float32)
+    qd, sd = torch.from_numpy(wq).cuda(), torch.from_numpy(ws).cuda()
+    w = ops.pack_w8a16(qd, sd)
+    x = rounded(rng.normal(size=(rows, k)), dtype)
+    xq, xs = ops.dynamic_quant(dev(x, dtype))
+    y8 = ops.grouped_w8a8_linear(xq, xs, w, od, out_dtype=dtype)
+    y8_ref, _ = ops.grouped_w8a8_linear(xq, xs, w, od, out_dtype=dtype, return_acc=True)
+    assert torch.equal(y8, y8_ref)
+    y = ops.grouped_w8a16_linear(dev(x, dtype), w, od)
+    deq = np.transpose(wq.astype(np.float64) * ws[..., None], (0, 2, 1))
+    ref, mag = O.grouped_matmul(x, deq, counts), O.grouped_matmul(np.abs(x), np.abs(deq), counts)
+    assert_within(to_np(y), ref, np.abs(ref), dtype, ulps=1.0, extra=2.0 ** -18 * mag + 1e-9, what="grouped gemm, prompts")
+    fused = ops.grouped_w8a16_linear(dev(x, dtype), ops.pack_w8a16_gated(qd, sd, "halves"), od)
+    assert torch.equal(fused, ops.silu_mul(y))
+
+
 # ------------------------------------------------------------------------------------------- MLA absorbed projections
 @pytest.mark.parametrize("dtype,t,h,k,n,strided", [
     (torch.bfloat16, 64, 128, 128, 512, True),     # query side at DeepSeek-V3 geometry: q_no_pe inside [T, H, 192]
