@@ -534,6 +534,13 @@ int mf_moe_permute(void* permuted_x, int32_t* row_map, int64_t* counts, int32_t*
                    const int32_t* expert_index, int tokens, int k, int n_experts, int hidden, int dtype,
                    void* stream);
 
+/* mf_moe_permute of rows quantised before it: x int8 [tokens, hidden] (hidden % 16 == 0) and its scales x_scale
+ * [tokens] as mf_dynamic_quant_per_token / mf_static_quant_per_tensor write them row-major; permuted_x int8 [T*k, H],
+ * permuted_scale [T*k].  The same values as quantising the permuted rows, each token quantised once. */
+int mf_moe_permute_int8(int8_t* permuted_x, float* permuted_scale, int32_t* row_map, int64_t* counts, int32_t* offsets,
+                        const int8_t* x, const float* x_scale, const int32_t* expert_index, int tokens, int k,
+                        int n_experts, int hidden, void* stream);
+
 /* GroupedMatmulV4(split_item=3, group_type=0, group_list_type=1) with int8 expert weights —
  * mindformers/parallel_core/inference/transformer/moe/experts.py:116-117,136-137.
  * Rows offsets[e]..offsets[e+1] of x use expert e: y = (x . w[e]^T) * scale[e].  w_packed holds the E experts

@@ -128,88 +128,96 @@ __global__ __launch_bounds__(64) void moe_route_kernel(uint16_t* __restrict__ we
     }
 }
 
-// Histogram + exclusive scan + stable rank.  One workgroup of 1024 threads; pairs p = t*k + j.
-__global__ __launch_bounds__(1024) void moe_sort_kernel(int32_t* __restrict__ row_map, int64_t* __restrict__ counts,
-                                                        int32_t* __restrict__ offsets,
-                                                        const int32_t* __restrict__ expert_index, int pairs,
-                                                        int E) {
-    __shared__ int s_cnt[RT_MAX_E];
-    __shared__ int s_cur[RT_MAX_E];
-    const int tid = threadIdx.x;
-    for (int e = tid; e < E; e += blockDim.x) s_cnt[e] = 0;
+// Stable counting sort of the pairs p = t*k + j by expert; a workgroup of 1024 threads places SORT_CHUNK pairs.  Every
+// workgroup counts all the pairs itself (the indices are at most 256 KB, read from the L2), those in front of its chunk apart
+// from the rest, so that no second launch, workspace or order among workgroups is needed: a pair's row is its expert's first
+// row + the expert's pairs in earlier chunks + those of earlier waves of the chunk + those of lower lanes of its wave.
+// What bounds it: the latency of a few dependent passes.  16616 pairs on 256 experts: 129 us in one workgroup that
+// walked the pairs 64 at a time, 8 us here.
+constexpr int SORT_CHUNK = 1024;
+__global__ __launch_bounds__(SORT_CHUNK) void moe_sort_kernel(int32_t* __restrict__ row_map, int64_t* __restrict__ counts,
+                                                              int32_t* __restrict__ offsets,
+                                                              const int32_t* __restrict__ expert_index, int pairs,
+                                                              int E) {
+    __shared__ int s_before[RT_MAX_E], s_rest[RT_MAX_E], s_cur[RT_MAX_E];
+    __shared__ uint8_t s_wave[SORT_CHUNK / 64][RT_MAX_E];     // pairs of the wave for the expert: at most 64
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int chunk0 = blockIdx.x * SORT_CHUNK;
+    for (int e = tid; e < E; e += SORT_CHUNK) s_before[e] = s_rest[e] = 0;
+    for (int i = tid; i < (int)sizeof(s_wave) / 16; i += SORT_CHUNK) ((u32x4*)s_wave)[i] = (u32x4){0u, 0u, 0u, 0u};
     __syncthreads();
-    for (int p = tid; p < pairs; p += blockDim.x) {
-        const int e = expert_index[p];
-        if (e >= 0 && e < E) atomicAdd(&s_cnt[e], 1);
+    const int p = chunk0 + tid;
+    int e = p < pairs ? expert_index[p] : -1;
+    if (e >= E) e = -1;
+    for (int base = 0; base < pairs; base += 4 * SORT_CHUNK) {
+        int v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int q = base + i * SORT_CHUNK + tid;
+            v[i] = q < pairs ? expert_index[q] : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (v[i] >= 0 && v[i] < E) atomicAdd(base + i * SORT_CHUNK < chunk0 ? &s_before[v[i]] : &s_rest[v[i]], 1);
     }
+    // lanes holding the same expert (10 index bits + validity)
+    uint64_t same = __ballot(e >= 0);
+#pragma unroll
+    for (int bit = 0; bit < 10; ++bit) {
+        const uint64_t bm = __ballot((e >> bit) & 1);
+        same &= ((e >> bit) & 1) ? bm : ~bm;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    if (e >= 0 && rank == 0) s_wave[wv][e] = (uint8_t)__popcll(same);
     __syncthreads();
-    if (tid < 64) {                                           // exclusive scan: a chunk of experts per lane of wave 0
+    if (wv == 0) {                                            // exclusive scan: a run of experts per lane of wave 0
         const int per = (E + 63) / 64;
-        const int e0 = tid * per;
+        const int e0 = lane * per;
         int local = 0;
         for (int i = 0; i < per; ++i)
-            if (e0 + i < E) local += s_cnt[e0 + i];
+            if (e0 + i < E) local += s_before[e0 + i] + s_rest[e0 + i];
         int incl = local;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const int up = __shfl_up(incl, o, 64);
-            if (tid >= o) incl += up;
+            if (lane >= o) incl += up;
         }
         int run = incl - local;
         for (int i = 0; i < per; ++i) {
-            const int e = e0 + i;
-            if (e < E) {
-                const int c = s_cnt[e];
-                s_cur[e] = run;
-                offsets[e] = run;
-                counts[e] = c;
+            const int x = e0 + i;
+            if (x < E) {
+                const int c = s_before[x] + s_rest[x];
+                s_cur[x] = run + s_before[x];
+                if (blockIdx.x == 0) {
+                    offsets[x] = run;
+                    counts[x] = c;
+                }
                 run += c;
             }
         }
-        if (tid == 63) offsets[E] = incl;
+        if (blockIdx.x == 0 && lane == 63) offsets[E] = incl;
     }
     __syncthreads();
-    // stable placement: wave 0 walks the pairs in order, 64 at a time
-    if (tid < 64) {
-        const int lane = tid;
-        for (int base = 0; base < pairs; base += 64) {
-            const int p = base + lane;
-            const bool live = p < pairs;
-            int e = live ? expert_index[p] : -1;
-            const bool ok = live && e >= 0 && e < E;
-            if (!ok) e = -1;
-            // lanes holding the same expert (10 index bits + validity)
-            uint64_t same = __ballot(ok);
-#pragma unroll
-            for (int bit = 0; bit < 10; ++bit) {
-                const uint64_t bm = __ballot((e >> bit) & 1);
-                same &= ((e >> bit) & 1) ? bm : ~bm;
-            }
-            if (ok) {
-                const uint64_t below = same & ((1ull << lane) - 1ull);
-                const int rank = __popcll(below);
-                const int dst = s_cur[e] + rank;
-                row_map[p] = dst;
-            } else if (live) {
-                row_map[p] = -1;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (ok && (same & ((1ull << lane) - 1ull)) == 0) s_cur[e] += __popcll(same);   // group leader
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        }
+    if (p >= pairs) return;
+    int dst = -1;
+    if (e >= 0) {
+        dst = s_cur[e] + rank;
+        for (int w = 0; w < wv; ++w) dst += s_wave[w][e];
     }
+    row_map[p] = dst;
 }
 
-// permuted_x[row_map[p]] = x[p / k]; one workgroup per pair.
-__global__ void moe_gather_kernel(uint16_t* __restrict__ permuted, const uint16_t* __restrict__ x,
+// permuted_x[row_map[p]] = x[p / k]; one workgroup per pair.  Rows of int8 values come as `hidden` pairs of them, with their
+// scales in x_scale (else null).
+__global__ void moe_gather_kernel(uint16_t* __restrict__ permuted, float* __restrict__ permuted_scale,
+                                  const uint16_t* __restrict__ x, const float* __restrict__ x_scale,
                                   const int32_t* __restrict__ row_map, int k, int hidden, int pairs) {
     const int p = blockIdx.x;
     const int dst = row_map[p];
     if (dst < 0 || dst >= pairs) return;
     const uint16_t* src = x + (int64_t)(p / k) * hidden;
     uint16_t* d = permuted + (int64_t)dst * hidden;
+    if (x_scale && threadIdx.x == 0) permuted_scale[dst] = x_scale[p / k];
     for (int i = threadIdx.x * 8; i < hidden; i += blockDim.x * 8) *(u32x4*)(d + i) = *(const u32x4*)(src + i);
 }
 
@@ -381,6 +389,19 @@ GatePlan plan_router_gate(int tokens, int E, int H) {
     return p;
 }
 
+int permute(uint16_t* permuted, float* permuted_scale, int32_t* row_map, int64_t* counts, int32_t* offsets, const uint16_t* x,
+            const float* x_scale, const int32_t* expert_index, int tokens, int k, int n_experts, int hidden,
+            hipStream_t stream) {
+    const int pairs = tokens * k, chunks = pairs > SORT_CHUNK ? (pairs + SORT_CHUNK - 1) / SORT_CHUNK : 1;
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(chunks), dim3(SORT_CHUNK), 0, stream, row_map, counts, offsets, expert_index,
+                       pairs, n_experts);
+    int rc = MF_LAUNCH_CHECK();
+    if (rc || pairs == 0) return rc;
+    hipLaunchKernelGGL(moe_gather_kernel, dim3(pairs), dim3(256), 0, stream, permuted, permuted_scale, x, x_scale, row_map, k,
+                       hidden, pairs);
+    return MF_LAUNCH_CHECK();
+}
+
 }  // namespace
 
 extern "C" int mf_moe_route(void* weights_out, int32_t* index_out, const float* logits, const float* bias,
@@ -458,14 +479,21 @@ extern "C" int mf_moe_permute(void* permuted_x, int32_t* row_map, int64_t* count
     MF_REQUIRE(tokens >= 0 && k > 0 && (int64_t)tokens * k <= 65536, "moe_permute: tokens*k must be <= 65536");
     MF_REQUIRE(hidden > 0 && hidden % 8 == 0, "moe_permute: hidden (%d) must be a multiple of 8", hidden);
     MF_REQUIRE((((uintptr_t)permuted_x | (uintptr_t)x) & 15) == 0, "moe_permute: rows must be 16-byte aligned");
-    const int pairs = tokens * k;
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, row_map, counts, offsets,
-                       expert_index, pairs, n_experts);
-    int rc = MF_LAUNCH_CHECK();
-    if (rc || pairs == 0) return rc;
-    hipLaunchKernelGGL(moe_gather_kernel, dim3(pairs), dim3(256), 0, (hipStream_t)stream, (uint16_t*)permuted_x,
-                       (const uint16_t*)x, row_map, k, hidden, pairs);
-    return MF_LAUNCH_CHECK();
+    return permute((uint16_t*)permuted_x, nullptr, row_map, counts, offsets, (const uint16_t*)x, nullptr, expert_index, tokens,
+                   k, n_experts, hidden, (hipStream_t)stream);
+}
+
+extern "C" int mf_moe_permute_int8(int8_t* permuted_x, float* permuted_scale, int32_t* row_map, int64_t* counts,
+                                   int32_t* offsets, const int8_t* x, const float* x_scale, const int32_t* expert_index,
+                                   int tokens, int k, int n_experts, int hidden, void* stream) {
+    MF_REQUIRE(permuted_x && permuted_scale && row_map && counts && offsets && x && x_scale && expert_index,
+               "moe_permute_int8: null argument");
+    MF_REQUIRE(n_experts > 0 && n_experts <= RT_MAX_E, "moe_permute_int8: n_experts (%d) must be in 1..%d", n_experts, RT_MAX_E);
+    MF_REQUIRE(tokens >= 0 && k > 0 && (int64_t)tokens * k <= 65536, "moe_permute_int8: tokens*k must be <= 65536");
+    MF_REQUIRE(hidden > 0 && hidden % 16 == 0, "moe_permute_int8: hidden (%d) must be a multiple of 16", hidden);
+    MF_REQUIRE((((uintptr_t)permuted_x | (uintptr_t)x) & 15) == 0, "moe_permute_int8: rows must be 16-byte aligned");
+    return permute((uint16_t*)permuted_x, permuted_scale, row_map, counts, offsets, (const uint16_t*)x, x_scale, expert_index,
+                   tokens, k, n_experts, hidden / 2, (hipStream_t)stream);
 }
 
 extern "C" int mf_moe_unpermute(void* out, const void* y, const int32_t* row_map, const void* probs,

@@ -1143,6 +1143,27 @@ def moe_permute(x, expert_index, n_experts):
     return px, row_map, counts, offsets
 
 
+def moe_permute_int8(xq, x_scale, expert_index, n_experts):
+    """``moe_permute`` of rows that are quantised already (``dynamic_quant`` of the tokens): returns (permuted_xq int8
+    [T*k,H], permuted_scale fp32 [T*k], row_map, counts, offsets)."""
+    lib = _lib.load()
+    dev = _dev_ok(xq, x_scale, expert_index)
+    _need(xq.dtype == torch.int8 and xq.dim() == 2, "xq must be int8 [T, H]")
+    _need(x_scale.dtype == torch.float32 and x_scale.numel() == xq.shape[0], "x_scale must be fp32 [T]")
+    _need(expert_index.dtype == torch.int32 and expert_index.dim() == 2 and expert_index.shape[0] == xq.shape[0],
+          "expert_index must be int32 [T, k]")
+    t, h = xq.shape
+    k = expert_index.shape[1]
+    px = torch.empty(t * k, h, dtype=torch.int8, device=dev)
+    ps = torch.empty(t * k, dtype=torch.float32, device=dev)
+    row_map = torch.empty(t * k, dtype=torch.int32, device=dev)
+    counts = torch.empty(n_experts, dtype=torch.int64, device=dev)
+    offsets = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
+    check(lib.mf_moe_permute_int8(ptr(px), ptr(ps), ptr(row_map), ptr(counts), ptr(offsets), ptr(xq), ptr(x_scale),
+                                  ptr(expert_index), t, k, n_experts, h, stream_ptr(dev)), "mf_moe_permute_int8")
+    return px, ps, row_map, counts, offsets
+
+
 def grouped_w8a16_linear(x, w, offsets, scale=None):
     """GroupedMatmulV4 over expert row groups.  x [R, K]; ``w`` a PackedInt8Weight of [E, N, K] (or a raw int8
     [E, N, K] tensor with ``scale`` [E, N], packed on every call); offsets int32 [E+1].  A weight packed with

@@ -1530,6 +1530,32 @@ def test_moe_permute_unpermute_shapes(t, h, e, k):
         assert_within(to_np(out), ref, mag, dtype, ulps=1.0, extra=2.0 ** -9 * EPS[dtype] * mag + 1e-9, what="unpermute")
 
 
+@pytest.mark.parametrize("t,h,e,k", [(1, 16, 8, 8), (128, 64, 256, 8), (205, 48, 1024, 5), (341, 16, 3, 3), (2077, 32, 256, 8),
+                                     (8192, 16, 64, 8)])
+def test_moe_permute_int8_rows(t, h, e, k):
+    """Rows quantised before the permute: the sort around its 1024-pair chunks (1, 1023, 1024, 1025 pairs, many, the limit), a
+    crowded expert, pairs without an expert (they take no row); rows and scales move as they are."""
+    rng = np.random.default_rng(t + e)
+    xq = rng.integers(-128, 128, (t, h)).astype(np.int8)
+    xs = rng.uniform(0.01, 1.0, t).astype(np.float32)
+    idx = rng.integers(0, e, (t, k)).astype(np.int32)
+    idx[:, 0] = 1
+    idx[t // 2, k - 1] = -1
+    idx[t // 3, k - 1] = e
+    flat = idx.reshape(-1)
+    ok = (flat >= 0) & (flat < e)
+    order = np.flatnonzero(ok)[np.argsort(flat[ok], kind="stable")]
+    map_ref = np.full(t * k, -1, np.int32)
+    map_ref[order] = np.arange(order.size)
+    cnt_ref = np.bincount(flat[ok], minlength=e)
+    px, ps, row_map, counts, offsets = ops.moe_permute_int8(torch.from_numpy(xq).cuda(), torch.from_numpy(xs).cuda(),
+                                                            torch.from_numpy(idx).cuda(), e)
+    assert np.array_equal(to_np(row_map), map_ref) and np.array_equal(to_np(counts), cnt_ref)
+    assert np.array_equal(to_np(offsets), np.concatenate(([0], np.cumsum(cnt_ref))).astype(np.int32))
+    assert np.array_equal(px.cpu().numpy()[:order.size], xq[order // k])
+    assert np.array_equal(ps.cpu().numpy()[:order.size], xs[order // k])
+
+
 def test_moe_permute_grouped_unpermute():
     rng = np.random.default_rng(14)
     dtype = torch.bfloat16
