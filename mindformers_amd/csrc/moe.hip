@@ -302,6 +302,7 @@ __device__ __forceinline__ float rg_round(float v) {
     else return WT::to_float(WT::from_float(v));
 }
 
+constexpr int RG_TILE_MIN = 256;   // more tokens than this: tiles (see there)
 constexpr int RG_TT = 4;                                      // token tiles of 16 per workgroup
 
 template <typename T, typename WT>
@@ -365,6 +366,78 @@ __global__ __launch_bounds__(256) void router_gate_kernel(float* __restrict__ ou
         if (e + i < E) dst[i] = partial ? v[i] : rg_round<WT>(v[i]);
 }
 
+// The same product for many tokens: a workgroup owns 64 tokens x 64 experts and a slice of H, a wave 32 x 32 of them on the
+// 32 x 32 x 2 instruction.  64 columns of both operands at a time are staged in LDS as fp32 (whole rows of 256 bytes are
+// fetched; the next 64 columns are in registers meanwhile), and lane half h takes columns 32 h .. 32 h + 31 of its row.
+// What bounds it: the fp32 matrix instruction (157 TFLOP/s nominal).  2077 x 256 x 7168: 236 us with operands fetched
+// into registers 16 rows at a time, where every 16 experts fetched the tokens anew, 97 us here;
+// the difference to a float64 product is half of that kernel's (two shorter chains).  Up to 256 tokens the latter is as fast (28 us at
+// 256, both) or faster (18 and 20 us at 128): it slices H further and reads the weight once.
+constexpr int RGT = 64;                                       // tokens, experts and columns of a step
+constexpr int RGT_ROW = RGT + 4;                              // floats of a staged row: 16-byte pieces of 8 rows meet all banks
+template <typename T, typename WT>
+__global__ __launch_bounds__(256) void router_gate_tile_kernel(float* __restrict__ out, float* __restrict__ partial,
+                                                               const uint16_t* __restrict__ x, const void* __restrict__ w,
+                                                               int tokens, int E, int H, int k_per_split) {
+    __shared__ float sw[RGT * RGT_ROW], sx[RGT * RGT_ROW];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = lane & 31, h = lane >> 5;
+    const int e0 = blockIdx.x * RGT, t0 = blockIdx.z * RGT;
+    const int k_begin = blockIdx.y * k_per_split, k_end = min(H, k_begin + k_per_split);
+    // load i of a thread: columns 4 c .. 4 c + 3 of row lr + 16 i; rows past the matrix re-read the last one, never stored
+    const int lr = threadIdx.x >> 4, lc = 4 * (threadIdx.x & 15);
+    int64_t wrow[4], xrow[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        wrow[i] = (int64_t)min(e0 + lr + 16 * i, E - 1) * H;
+        xrow[i] = (int64_t)min(t0 + lr + 16 * i, tokens - 1) * H;
+    }
+    f32x4 wr[4], xr[4];
+    auto load = [&](int k0) {
+        const int k = k0 + lc;
+        const bool in = k < k_end;                            // H and the slices are multiples of 4
+        const int kc = in ? k : k_begin;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            wr[i] = rg_load4<WT>(w, wrow[i] + kc);
+            xr[i] = rg_load4<T>(x, xrow[i] + kc);
+            if (!in) wr[i] = xr[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    f32x16 acc[2] = {(f32x16)(0.f), (f32x16)(0.f)};          // two shorter chains: a smaller rounding error
+    const float* pw = sw + (32 * (wv & 1) + r) * RGT_ROW + 32 * h;
+    const float* px = sx + (32 * (wv >> 1) + r) * RGT_ROW + 32 * h;
+    load(k_begin);
+    for (int k0 = k_begin; k0 < k_end; k0 += RGT) {
+        __syncthreads();                                      // the step before has been read
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            *(f32x4*)(sw + (lr + 16 * i) * RGT_ROW + lc) = wr[i];
+            *(f32x4*)(sx + (lr + 16 * i) * RGT_ROW + lc) = xr[i];
+        }
+        __syncthreads();
+        if (k0 + RGT < k_end) load(k0 + RGT);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const f32x4 a = *(const f32x4*)(pw + 4 * j), b = *(const f32x4*)(px + 4 * j);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], acc[i & 1], 0, 0, 0);
+        }
+    }
+    acc[0] += acc[1];
+    // lane (r, h) holds token r, experts 8 q + 4 h .. + 3 in elements 4 q .. 4 q + 3
+    const int t = t0 + 32 * (wv >> 1) + r;
+    if (t >= tokens) return;
+    float* dst = partial ? partial + ((int64_t)blockIdx.y * tokens + t) * E : out + (int64_t)t * E;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = e0 + 32 * (wv & 1) + 8 * q + 4 * h + i;
+            if (e < E) dst[e] = partial ? acc[0][4 * q + i] : rg_round<WT>(acc[0][4 * q + i]);
+        }
+}
+
 template <typename WT>
 __global__ void router_gate_reduce_kernel(float* __restrict__ out, const float* __restrict__ partial, int64_t n,
                                           int splits) {
@@ -376,14 +449,16 @@ __global__ void router_gate_reduce_kernel(float* __restrict__ out, const float* 
 }
 
 struct GatePlan {
-    int splits, k_per_split;
+    int tile, splits, k_per_split;
 };
 GatePlan plan_router_gate(int tokens, int E, int H) {
-    const int wgs = ((E + 15) / 16) * ((tokens + 16 * RG_TT - 1) / (16 * RG_TT));
-    int s = 512 / wgs;
-    const int max_s = H / 256 < 1 ? 1 : H / 256;              // at least one chunk per wave
-    s = s < 1 ? 1 : (s > max_s ? max_s : s);
     GatePlan p;
+    p.tile = tokens > RG_TILE_MIN;
+    const int te = p.tile ? RGT : 16;
+    const int wgs = ((E + te - 1) / te) * ((tokens + 16 * RG_TT - 1) / (16 * RG_TT));
+    int s = p.tile ? 1024 / wgs : 512 / wgs;
+    const int max_s = H / 256 < 1 ? 1 : H / 256;              // at least one chunk per wave, or four steps of a tile
+    s = s < 1 ? 1 : (s > max_s ? max_s : s);
     p.k_per_split = ((H + s - 1) / s + 63) / 64 * 64;
     p.splits = (H + p.k_per_split - 1) / p.k_per_split;
     return p;
@@ -447,13 +522,15 @@ extern "C" int mf_router_gate_gemm(float* logits, const void* x, const void* w, 
     MF_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), "router_gate_gemm: workspace of %zu bytes needed, %zu given",
                need, workspace_bytes);
     float* partial = p.splits > 1 ? (float*)workspace : nullptr;
-    const dim3 grid((n_experts + 15) / 16, p.splits, (tokens + 16 * RG_TT - 1) / (16 * RG_TT));
+    const int te = p.tile ? RGT : 16;
+    const dim3 grid((n_experts + te - 1) / te, p.splits, (tokens + 16 * RG_TT - 1) / (16 * RG_TT));
     const int64_t n = (int64_t)tokens * n_experts;
     const dim3 rgrid((unsigned)((n + 255) / 256));
 #define RG_LAUNCH(TT_, WT_)                                                                                      \
     {                                                                                                            \
-        hipLaunchKernelGGL((router_gate_kernel<TT_, WT_>), grid, dim3(256), 0, (hipStream_t)stream, logits, partial, \
-                           (const uint16_t*)x, w, tokens, n_experts, hidden, p.k_per_split);                     \
+        hipLaunchKernelGGL((p.tile ? router_gate_tile_kernel<TT_, WT_> : router_gate_kernel<TT_, WT_>), grid, dim3(256), 0, \
+                           (hipStream_t)stream, logits, partial, (const uint16_t*)x, w, tokens, n_experts, hidden,   \
+                           p.k_per_split);                                                                       \
         if (partial) {                                                                                           \
             int rc = MF_LAUNCH_CHECK();                                                                          \
             if (rc) return rc;                                                                                   \

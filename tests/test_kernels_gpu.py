@@ -1480,6 +1480,14 @@ def test_router_gate_projection(dtype, t, e, h, wdt):
     assert np.array_equal(got_i, want)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("t,e,h,wdt", [(257, 256, 7168, "fp32"), (320, 65, 260, "fp32"), (300, 3, 4, "fp32"), (257, 129, 324, "same"),
+                                       (1100, 64, 2048, "same")])
+def test_router_gate_projection_tiles(dtype, t, e, h, wdt):
+    """The same bounds on the 64 x 64 tiles (more than 256 tokens): ragged rows, experts and columns, one step, one slice."""
+    test_router_gate_projection(dtype, t, e, h, wdt)
+
+
 @pytest.mark.parametrize("t,e,k,ng,tg", [(128, 256, 8, 8, 4), (16, 8, 2, 2, 2), (33, 64, 6, 8, 3), (5, 16, 4, 1, 1), (7, 96, 3, 4, 1),
                                          (9, 96, 4, 3, 2), (6, 60, 5, 6, 2), (4, 1024, 32, 16, 8), (3, 640, 7, 64, 9)])
 def test_moe_route(t, e, k, ng, tg):
