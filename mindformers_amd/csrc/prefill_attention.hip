@@ -588,10 +588,10 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
     int rc = MF_LAUNCH_CHECK();
     if (rc) return rc;
     if (plan.max_parts > 1) {
-        hipLaunchKernelGGL((paged_attention_reduce_kernel<T, DV, true>), dim3(n_heads, total_q),
-                           dim3(PA_REDUCE_THREADS<DV>), 0, st,
-                           (uint16_t*)out, part_out, part_ml, context_lens, n_heads, plan.max_parts,
-                           plan.part_tokens, q_starts, batch, contiguous, max_blocks * block_size);
+        const dim3 grid((unsigned)total_q, (unsigned)((n_heads * DV + 4 * PF_REDUCE_THREADS - 1) / (4 * PF_REDUCE_THREADS)));
+        hipLaunchKernelGGL((prefill_reduce_kernel<T, DV>), grid, dim3(PF_REDUCE_THREADS), 0, st, (uint16_t*)out, part_out,
+                           part_ml, context_lens, n_heads, plan.max_parts, plan.part_tokens, q_starts, batch, contiguous,
+                           max_blocks * block_size, total_q);
         rc = MF_LAUNCH_CHECK();
     }
     return rc;
