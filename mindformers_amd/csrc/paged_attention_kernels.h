@@ -1,6 +1,6 @@
 // Kernels shared by the decode and the prefill side of paged attention on gfx950: the 16-column kernel (decode: one
-// query row per sequence; also the prefill path of int8 caches) and the partition-combine kernels.  Included by
-// paged_attention.hip (decode entry points) and prefill_attention.hip (prefill entry points).
+// query row per sequence; also the prefill path of int8 caches with per-token scales) and the partition-combine
+// kernels.  Included by paged_attention.hip (decode entry points) and prefill_attention.hip (prefill entry points).
 //
 // Decode: work decomposition
 //   grid = batch * max_partitions * n_kv_heads * head_groups (1-D); one workgroup of 4 wavefronts owns one

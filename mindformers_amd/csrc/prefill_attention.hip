@@ -1,5 +1,6 @@
 // GQA paged attention for gfx950, prefill side (several causal query rows per sequence): the 32-column kernel,
-// its launch rule and entry points.  int8 caches go through the 16-column kernel of paged_attention_kernels.h.
+// its launch rule and entry points.  int8 caches with per-token scales go through the 16-column kernel of
+// paged_attention_kernels.h.
 #include "paged_attention_kernels.h"
 
 namespace {
@@ -27,6 +28,11 @@ namespace {
 // compute unit (48 KB of LDS, at most 168 registers), so a SIMD holds three waves whose matrix and vector phases
 // overlap; a version that interleaved the phases of neighbouring tiles inside a wave needed 216 registers and was
 // no faster with two.
+// int8 caches with per-channel scales (KVQ = 1) cannot go straight into LDS: a thread loads 16 bytes of a K and of a V row
+// one tile ahead into registers and writes them, widened to T (exactly), to the same places of the ring; the matrix
+// path is the same.  The key scale is folded into the query, the key offset drops out of the softmax, value scale and
+// offset are applied once to the (accumulator, sum) pair.  Two 512-row chunks beside 24 decoding sequences of 512 to 4096
+// tokens (32 heads on 8): 235 us on the 16-column kernel, which widens a tile for 16 columns, 140 us here.
 // A wave owns its columns over the whole partition, so there is no merge: it writes final rows (single partition) or
 // fp32 partials for the reduce kernel.
 constexpr int PF_COLS = 128;                                  // columns per workgroup
@@ -68,16 +74,17 @@ struct PfSmem {
 // Three workgroups per compute unit; two at 192-wide heads (72 KB of LDS and 96 accumulator registers each).
 // DV: width of a value head and of an output head.  DV < D (the prefill of multi-latent attention: 192-wide queries
 // and keys, 128-wide values, packed rows only) loads and multiplies the first sub-tile of the value rows only.
-template <typename T, int D, bool TIB, int DV = D>
+template <typename T, int D, bool TIB, int DV = D, int KVQ = 0>
 __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_attention_kernel(
     uint16_t* __restrict__ out, float* __restrict__ part_out, float* __restrict__ part_ml,
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, int n_heads, int n_kv,
     int n_rep, int block_size, int max_blocks, int num_blocks, int max_parts, float scale_log2, int64_t q_stride,
     int batch, const int32_t* __restrict__ q_starts, int part_tokens, int64_t kv_stride, int rows,
-    int64_t v_stride) {
+    int64_t v_stride, const float* __restrict__ kv_scale, const float* __restrict__ kv_offset) {
     using vec8 = typename T::vec8;
     using S = PfSmem<D>;
+    static_assert(KVQ == 0 || (KVQ == 1 && DV == D && S::W1 == 0), "int8 caches: per-channel scales, power-of-two heads");
     static_assert(DV == D || DV == S::W0, "value heads as wide as the key heads, or as their first sub-tile");
     constexpr int KS = D / 16;                                // k-steps of the score product
     constexpr int DB = DV / 32;                               // 32-row blocks of O^T
@@ -175,6 +182,14 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
         for (int j = 0; j < KS; ++j) {
             u32x4 v = {0u, 0u, 0u, 0u};
             if (col_ok) v = *(const u32x4*)(qp + 16 * j);
+            if constexpr (KVQ == 1) {                         // fold the per-channel key scale into the query
+                float f[8];
+                unpack8<T>(v, f);
+                const float* ks = kv_scale + kvh * D + 16 * j + 8 * h;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] *= ks[e];
+                v = (u32x4){pack2<T>(f[0], f[1]), pack2<T>(f[2], f[3]), pack2<T>(f[4], f[5]), pack2<T>(f[6], f[7])};
+            }
             qreg[j] = bitcast<vec8>(v);
         }
     }
@@ -274,6 +289,45 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)vp,
                                                  (__attribute__((address_space(3))) void*)(dst + S::KBYTES), 16, 0, 0);
         });
+    };
+
+    // ---- int8 tiles: thread (row prow, 16-byte piece pc) of the first PF_TOK * D / 16 threads
+    constexpr int PCS = D / 16;                               // 16-byte pieces of an int8 row
+    const bool piece = tid < PF_TOK * PCS;
+    const int prow = tid / PCS, pc = tid - prow * PCS;
+    [[maybe_unused]] u32x4 kraw, vraw;
+    auto load_regs = [&](int t) {
+        if (!piece) return;
+        const int ts = part_start + t * PF_TOK;
+        const int rc = min(prow, Lwg - 1 - ts);               // rows past the group's range re-read its last row
+        int64_t slot;
+        if constexpr (TIB) {
+            const int bi = ts / block_size;
+            int blk = table[bi];
+            blk = (blk < 0 || blk >= num_blocks) ? 0 : blk;
+            slot = (int64_t)blk * block_size + (ts - bi * block_size) + rc;
+        } else {
+            const int tok = ts + rc;
+            const int bi = tok / block_size;
+            int blk = table[bi];
+            blk = (blk < 0 || blk >= num_blocks) ? 0 : blk;
+            slot = (int64_t)blk * block_size + (tok - bi * block_size);
+        }
+        const int64_t off = slot * kv_stride + kvh * D + 16 * pc;      // bytes: one per element
+        kraw = *(const u32x4*)((const uint8_t*)kc + off);
+        vraw = *(const u32x4*)((const uint8_t*)vc + off);
+    };
+    auto write_regs = [&](int t) {
+        if (!piece) return;
+        const int key = (prow / S0::RPB) & (S0::CPR - 1), key4 = (prow / S0::RPB) & (S0::CPR / 4 - 1);
+        uint8_t* kdst = pf_smem + (t % PF_RING) * S::BUF + prow * S0::ROWB;
+        uint8_t* vdst = kdst + S::KBYTES;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int c = 2 * pc + i;
+            *(vec8*)(kdst + 16 * (c ^ key)) = dequant8<T>(kraw[2 * i], kraw[2 * i + 1]);
+            *(vec8*)(vdst + 16 * ((c + 4 * key4) & (S0::CPR - 1))) = dequant8<T>(vraw[2 * i], vraw[2 * i + 1]);
+        }
     };
 
     // ---- operand read addresses within a ring buffer (the buffer is a compile-time offset of the read)
@@ -405,14 +459,28 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
         }
     };
 
-    issue_tile(0);
-    if (ntiles > 1) issue_tile(1);
+    if constexpr (KVQ == 1) {
+        load_regs(0);
+        write_regs(0);
+        if (ntiles > 1) load_regs(1);
+    } else {
+        issue_tile(0);
+        if (ntiles > 1) issue_tile(1);
+    }
 #pragma unroll
     for (int j = 0; j < KS; ++j) asm volatile("" : "+v"(qreg[j]));   // the query is complete before the loop
     // tile t has landed for every wave (tile t + 1 may still be on its way), and every wave is done with tile t - 1,
     // whose buffer takes tile t + 2
     auto sync_issue = [&](int t) {
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (KVQ == 1) {                             // tile t was written one step ahead; t + 1 is in registers
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            if (t + 1 < ntiles) write_regs(t + 1);
+            if (t + 2 < ntiles) load_regs(t + 2);
+            return;
+        }
         if (t + 1 < ntiles) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NI + NIV) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -444,6 +512,17 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     // ---- every lane writes its column's values: 4 consecutive d per accumulator quad
     l_run += __shfl_xor(l_run, 32, 64);
     if (!col_ok) return;
+    if constexpr (KVQ == 1) {                                 // value dequantisation, linear in (acc, l_run)
+        const float* vs = kv_scale + n_kv * D + kvh * D + 4 * h;
+        const float* vo = kv_offset ? kv_offset + n_kv * D + kvh * D + 4 * h : nullptr;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int d = 32 * db + 8 * (i >> 2) + (i & 3);
+                acc[db][i] = vs[d] * (acc[db][i] - (vo ? vo[d] : 0.f) * l_run);
+            }
+    }
     const int64_t gh = (int64_t)(q_start + qi) * n_heads + kvh * n_rep + hcol;
     if (max_parts == 1) {
         const float inv = 1.0f / l_run;
@@ -473,7 +552,7 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
 
 // ---- prefill --------------------------------------------------------------------------------------------------
 // Partitioning rule shared by the workspace query and the launch.  A workgroup serves 128 (query, head) columns of
-// one kv head (16 with an int8 cache); when the query rows alone give the chip enough workgroups one partition spans the
+// one kv head (16 with an int8 cache of per-token scales); when the query rows alone give the chip enough workgroups one partition spans the
 // whole context and no partials are written, otherwise the context is cut so that at least 512 workgroups exist.
 struct PfPlan {
     int part_tokens;
@@ -536,8 +615,8 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
     float* part_out = plan.max_parts > 1 ? (float*)workspace : nullptr;
     float* part_ml = part_out ? part_out + (int64_t)total_q * n_heads * plan.max_parts * DV : nullptr;
     const float scale_log2 = scale * 1.4426950408889634f;
-    constexpr bool KV8 = KVQ != 0;
-    const int64_t wgs = (KV8 ? plan.col_groups16 : plan.col_groups128) * n_kv * plan.max_parts;
+    constexpr bool COLS16 = KVQ == 2;
+    const int64_t wgs = (COLS16 ? plan.col_groups16 : plan.col_groups128) * n_kv * plan.max_parts;
     if (wgs > 0x7fffffffLL) {
         mf_set_error("paged_attention_prefill: %lld workgroups exceed the grid limit", (long long)wgs);
         return 1;
@@ -548,7 +627,7 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
         int rc = MF_LAUNCH_CHECK();
         if (rc) return rc;
     }
-    if constexpr (KV8) {
+    if constexpr (COLS16) {
         const bool tib = block_size % PA_TILE == 0;           // a 32-token tile never straddles two blocks
 #define PF_LAUNCH(TIBV)                                                                                           \
     hipLaunchKernelGGL((paged_attention_kernel<T, D, 2, true, KVQ, TIBV>), dim3((unsigned)wgs),                    \
@@ -568,7 +647,7 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
         if (e != hipSuccess) return (int)e;
 #define PF_LAUNCH(TIBV)                                                                                           \
     {                                                                                                             \
-        auto kern = prefill_attention_kernel<T, D, TIBV, DV>;                                                     \
+        auto kern = prefill_attention_kernel<T, D, TIBV, DV, KVQ>;                                                    \
         if (dev < 0 || dev >= MF_MAX_DEVICES || !lds_set[TIBV][dev]) {                                            \
             e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,                \
                                     PfSmem<D>::BYTES);                                                            \
@@ -579,7 +658,7 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
                            part_out, part_ml, (const uint16_t*)query, (const uint16_t*)key_cache,                 \
                            (const uint16_t*)value_cache, block_tables, context_lens, n_heads, n_kv, n_rep,        \
                            block_size, max_blocks, num_blocks, plan.max_parts, scale_log2, q_stride, batch,       \
-                           q_starts, plan.part_tokens, kv_stride, total_q, v_stride);                             \
+                           q_starts, plan.part_tokens, kv_stride, total_q, v_stride, kv_scale, kv_offset);        \
     }
         if (tib) PF_LAUNCH(true)
         else PF_LAUNCH(false)

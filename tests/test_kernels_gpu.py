@@ -682,6 +682,29 @@ def test_paged_prefill_int8kv_vs_oracle():
     assert_within(to_np(out), ref, mag, dtype, ulps=3.0, what="prefill over an int8 cache")
 
 
+@pytest.mark.parametrize("dtype,nh,nkv,d,bs,lens,q_lens,with_offset", [
+    (torch.bfloat16, 7, 1, 128, 128, [33, 1, 640], [33, 1, 19], False),           # 7 heads a kv head, one-row sequences
+    (torch.float16, 4, 4, 64, 16, [95, 64, 31], [95, 32, 1], True),               # blocks that a 32-token tile straddles
+    (torch.bfloat16, 8, 2, 32, 48, [97, 290], [97, 65], True),                    # likewise, narrow heads
+    (torch.float16, 8, 1, 128, 32, [32, 65], [32, 65], True),                     # whole tiles and one token more
+    (torch.bfloat16, 32, 8, 128, 128, [2200, 2049], [1100, 1030], False),         # many rows: one partition, written at once
+])
+def test_paged_prefill_int8kv_shapes(dtype, nh, nkv, d, bs, lens, q_lens, with_offset):
+    """The 128-column kernel over an int8 cache, at the bound of the decode side."""
+    rng = np.random.default_rng(nh + d + bs)
+    lens, q_lens = np.array(lens), np.array(q_lens)
+    k8, v8, kf, vf, tables, nb, scale, offset = _kv8_case(rng, dtype, len(lens), nh, nkv, d, bs, lens, with_offset)
+    q = rounded(rng.normal(size=(int(q_lens.sum()), nh * d)), dtype)
+    sc = 1.0 / np.sqrt(d)
+    out = ops.paged_attention_int8kv(dev(q, dtype), torch.from_numpy(k8).cuda(), torch.from_numpy(v8).cuda(),
+                                     dev(tables, torch.int32), dev(lens.astype(np.int32), torch.int32),
+                                     dev(scale, torch.float32), None if offset is None else dev(offset, torch.float32),
+                                     nh, nkv, sc, q_starts=dev(_starts(q_lens), torch.int32))
+    ref = O.paged_attention_prefill(q, kf, vf, tables, lens, q_lens, nh, nkv, sc)
+    mag = O.paged_attention_prefill(q, kf, np.abs(vf), tables, lens, q_lens, nh, nkv, sc)
+    assert_within(to_np(out), ref, mag, dtype, ulps=3.0, what="prefill over an int8 cache")
+
+
 def _kv8_token_case(rng, dtype, b, nkv, d, bs, lens, max_blocks=None, poison=True):
     """Random 16-bit caches quantised per token by the oracle: int8 caches, the float caches they stand for, the scale
     caches [blocks, block_size] and the tables.  With ``poison`` the scales of every slot that holds no token of a
