@@ -189,17 +189,54 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 }
 
 
+// Division by a row's scale.  The grid point that is chosen has to equal the CPU statement's, rint(v / s) with a true IEEE
+// division, at five instructions a value where the compiler's division takes about ten and a quarter-rate reciprocal.
+// Markstein's correction (IBM J. Res. Dev. 34, 1990): with inv = RN(1 / s) and q within one ulp of v / s the residual
+// fma(-q, s, v) is exact and fma(residual, inv, q) = RN(v / s).  RN(v * inv) is within 1.5 ulp, so the correction is made twice.
+// It needs |v| <= 128 s (infinities and NaN aside, which make s infinite or leave q NaN either way) and residuals that do
+// not underflow; `exact` rows (scales that do not come from the row's own maximum, or outside 2^+-60) divide.
+struct QuantScale {
+    float s, inv;
+    bool exact;
+};
+__device__ __forceinline__ QuantScale quant_scale(float safe, bool from_row) {
+    const int exact = !(from_row && safe > 0x1p-60f && safe < 0x1p60f);
+    return {safe, __fdiv_rn(1.0f, safe), __builtin_amdgcn_readfirstlane(exact) != 0};   // the same in every lane
+}
+__device__ __forceinline__ float quant_div(float v, const QuantScale& d) {
+    float q = __fmul_rn(v, d.inv);
+    q = __fmaf_rn(__fmaf_rn(-q, d.s, v), d.inv, q);
+    return __fmaf_rn(__fmaf_rn(-q, d.s, v), d.inv, q);
+}
+
+// Workgroup -> row for the kernels that quantise a row per workgroup into the tiled layout.  A row is 16 bytes of every 128
+// there, so eight consecutive rows fill a cache line between them; workgroups go to the XCDs in turn, and with row =
+// workgroup each of the eight would leave its piece in another L2, to be written to memory by itself.  Within every whole
+// 64 rows the eight rows of a line are given to one XCD.
+__device__ __forceinline__ int quant_row(int id, int rows, int tiled) {
+    return tiled && (id | 63) < rows ? (id & ~63) | (id & 7) << 3 | ((id >> 3) & 7) : id;
+}
+
 // 8 values of row m, columns k .. k+7, quantised with the row's scale and written in the chosen layout.
-// The division is a true IEEE division so that the grid point chosen equals the CPU statement.
-__device__ __forceinline__ void quant_store8(int8_t* __restrict__ xq, const float* v, float safe, int m, int k, int cols,
-                                             int rows, int tiled) {
-    uint32_t o[2] = {0u, 0u};
+__device__ __forceinline__ void quant_store8(int8_t* __restrict__ xq, const float* v, const QuantScale& d, int m, int k,
+                                             int cols, int rows, int tiled) {
+    float q[8];
+    if (d.exact) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float qf = rintf(__fdiv_rn(v[i], safe));
-        qf = fminf(fmaxf(qf, -128.f), 127.f);
-        o[i >> 2] |= ((uint32_t)((int)qf & 0xff)) << (8 * (i & 3));
+        for (int i = 0; i < 8; ++i) q[i] = __fdiv_rn(v[i], d.s);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q[i] = quant_div(v[i], d);
     }
+    uint32_t b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)                               // NaN -> -128; + 1.5 * 2^23 rounds to an integer, ties to even
+        b[i] = __float_as_uint(__fadd_rn(fminf(fmaxf(q[i], -128.f), 127.f), 12582912.f));
+    uint32_t o[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)                               // the low bytes
+        o[i] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(b[4 * i + 3], b[4 * i + 2], 0x0c0c0400u),
+                                     __builtin_amdgcn_perm(b[4 * i + 1], b[4 * i], 0x0c0c0400u), 0x05040100u);
     if (tiled) {
         // 1 KiB tiles of 16 rows x 64 columns, [column step][row tile], 16 consecutive columns per lane
         // (lane = 16*(column/16 % 4) + row % 16): the operand order of the int8 matrix instructions

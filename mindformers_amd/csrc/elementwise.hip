@@ -182,8 +182,9 @@ __global__ __launch_bounds__(THREADS) void dynamic_quant_kernel(int8_t* __restri
                                                                int tiled, const float* __restrict__ static_scale,
                                                                RowGroups rg) {
     __shared__ float red[THREADS / 64];
-    const float* smooth = smooth_of_row(smooth_table, rg, blockIdx.x, cols);
-    const int64_t row = (int64_t)blockIdx.x * cols;
+    const int m = quant_row(blockIdx.x, gridDim.x, tiled);
+    const float* smooth = smooth_of_row(smooth_table, rg, m, cols);
+    const int64_t row = (int64_t)m * cols;
     const int nvec = cols >> 3;
     constexpr int ROW_THREADS = THREADS;
     constexpr int MAXV = ROW_MAX_COLS / 8 / THREADS;
@@ -204,12 +205,12 @@ __global__ __launch_bounds__(THREADS) void dynamic_quant_kernel(int8_t* __restri
         amax = block_max(amax, red);
         s = __fdiv_rn(amax, 127.0f);
     }
-    const float safe = s > 0.f ? s : 1.0f;
-    if (threadIdx.x == 0) x_scale[blockIdx.x] = s;
+    const QuantScale d = quant_scale(s > 0.f ? s : 1.0f, !static_scale);
+    if (threadIdx.x == 0) x_scale[m] = s;
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
         const int c = threadIdx.x + it * ROW_THREADS;
-        if (c < nvec) quant_store8(xq, v[it], safe, blockIdx.x, 8 * c, cols, gridDim.x, tiled);
+        if (c < nvec) quant_store8(xq, v[it], d, m, 8 * c, cols, gridDim.x, tiled);
     }
 }
 
@@ -233,7 +234,8 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual, const void* __restrict__ gamma,
     const float* __restrict__ smooth, float eps, int cols, int gamma_dtype, int tiled, PartialRow pr) {
     __shared__ float red[NORM_THREADS / 64];
-    const int64_t row = (int64_t)blockIdx.x * cols;
+    const int m = quant_row(blockIdx.x, gridDim.x, tiled);
+    const int64_t row = (int64_t)m * cols;
     const int nvec = cols >> 3;
     float v[NORM_MAX_VEC][8], gm[NORM_MAX_VEC][8];
     float ss = 0.f;
@@ -261,7 +263,7 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
                             hi += b[q];
                         }
                 }
-                const float xs = pr.row_scale[blockIdx.x];
+                const float xs = pr.row_scale[m];
                 const f32x4 w_lo = *(const f32x4*)(pr.col_scale + 8 * c), w_hi = *(const f32x4*)(pr.col_scale + 8 * c + 4);
                 float t[8];
 #pragma unroll
@@ -315,12 +317,12 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
     }
     amax = block_max(amax, red);
     const float s = __fdiv_rn(amax, 127.0f);
-    const float safe = s > 0.f ? s : 1.0f;
-    if (threadIdx.x == 0) x_scale[blockIdx.x] = s;
+    const QuantScale d = quant_scale(s > 0.f ? s : 1.0f, true);
+    if (threadIdx.x == 0) x_scale[m] = s;
 #pragma unroll
     for (int it = 0; it < NORM_MAX_VEC; ++it) {
         const int c = threadIdx.x + it * NORM_THREADS;
-        if (c < nvec) quant_store8(xq, v[it], safe, blockIdx.x, 8 * c, cols, gridDim.x, tiled);
+        if (c < nvec) quant_store8(xq, v[it], d, m, 8 * c, cols, gridDim.x, tiled);
     }
 }
 
@@ -332,13 +334,14 @@ __global__ __launch_bounds__(THREADS) void silu_mul_quant_kernel(int8_t* __restr
                                                                 const float* __restrict__ smooth_table, int cols,
                                                                 int layout, int tiled, RowGroups rg) {
     __shared__ float red[THREADS / 64];
-    const float* smooth = smooth_of_row(smooth_table, rg, blockIdx.x, cols);
+    const int m = quant_row(blockIdx.x, gridDim.x, tiled);
+    const float* smooth = smooth_of_row(smooth_table, rg, m, cols);
     const int nvec = cols >> 3;
     constexpr int ROW_THREADS = THREADS;
     constexpr int MAXV = ROW_MAX_COLS / 8 / THREADS;
     float v[MAXV][8];
     float amax = 0.f;
-    const uint16_t* base = gu + (int64_t)blockIdx.x * 2 * cols;
+    const uint16_t* base = gu + (int64_t)m * 2 * cols;
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
         const int cv = threadIdx.x + it * ROW_THREADS;
@@ -371,12 +374,12 @@ __global__ __launch_bounds__(THREADS) void silu_mul_quant_kernel(int8_t* __restr
     }
     amax = block_max(amax, red);
     const float s = __fdiv_rn(amax, 127.0f);
-    const float safe = s > 0.f ? s : 1.0f;
-    if (threadIdx.x == 0) x_scale[blockIdx.x] = s;
+    const QuantScale d = quant_scale(s > 0.f ? s : 1.0f, true);
+    if (threadIdx.x == 0) x_scale[m] = s;
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
         const int cv = threadIdx.x + it * ROW_THREADS;
-        if (cv < nvec) quant_store8(xq, v[it], safe, blockIdx.x, 8 * cv, cols, gridDim.x, tiled);
+        if (cv < nvec) quant_store8(xq, v[it], d, m, 8 * cv, cols, gridDim.x, tiled);
     }
 }
 

@@ -762,7 +762,7 @@ __global__ __launch_bounds__(PA_RQ_THREADS) void paged_attention_reduce_quant_ke
     const float* __restrict__ part_out, const float* __restrict__ part_ml, const int32_t* __restrict__ ctx_lens,
     const float* __restrict__ smooth, int n_heads, int max_parts, int part_tokens, int tiled) {
     __shared__ float red[PA_RQ_THREADS / 64];
-    const int b = blockIdx.x;
+    const int b = quant_row(blockIdx.x, gridDim.x, tiled);
     const int cols = n_heads * D;
     const int c = threadIdx.x;                                // 8-element piece of the row
     const bool on_row = c * 8 < cols;
@@ -808,9 +808,9 @@ __global__ __launch_bounds__(PA_RQ_THREADS) void paged_attention_reduce_quant_ke
     }
     amax = block_max(amax, red);
     const float s = __fdiv_rn(amax, 127.0f);
-    const float safe = s > 0.f ? s : 1.0f;
+    const QuantScale d = quant_scale(s > 0.f ? s : 1.0f, true);
     if (threadIdx.x == 0) x_scale[b] = s;
-    if (on_row) quant_store8(xq, v, safe, b, c * 8, cols, gridDim.x, tiled);
+    if (on_row) quant_store8(xq, v, d, b, c * 8, cols, gridDim.x, tiled);
 }
 
 }  // namespace

@@ -1317,6 +1317,24 @@ def test_dynamic_quant_tiled_layout_bit_exact(m, k):
     assert np.array_equal(untile_int8(to_np(xt.data), m, k), q_ref)
 
 
+@pytest.mark.parametrize("m", [64, 65, 127, 200])
+@pytest.mark.parametrize("dtype,lo,hi", [(torch.bfloat16, -110, 110), (torch.float16, -14, 8)])
+def test_dynamic_quant_at_rounding_edges(dtype, lo, hi, m):
+    """Quotients at half grid points and up to three float32 steps beside them, row scales from far below to far above the
+    range in which the quotient is formed without a division, row counts around the 64 rows that are dealt out together."""
+    rng = np.random.default_rng(m)
+    k = 2048
+    x = np.ldexp(np.ones((m, k), np.float32), rng.integers(lo, hi + 1, (m, 1)))
+    amax = np.float32(rng.uniform(1, 2) * 127)
+    sm = (rng.integers(-127, 127, k) + 0.5).astype(np.float32) * (amax / np.float32(127))
+    sm = (sm.view(np.int32) + rng.integers(-3, 4, k).astype(np.int32)).view(np.float32)
+    sm[0] = amax
+    xt, xs = ops.dynamic_quant(dev(x, dtype), torch.from_numpy(sm).cuda(), tiled=True)
+    q_ref, s_ref = O.dynamic_quant_per_token(x, sm)
+    assert np.array_equal(to_np(xs), s_ref)
+    assert np.array_equal(untile_int8(to_np(xt.data), m, k), q_ref)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("tiled", [False, True])
 @pytest.mark.parametrize("counts,k", [([5, 0, 17, 1, 0, 40], 256), ([0, 0, 3], 7168), ([64] * 16, 2048), ([1], 64)])
