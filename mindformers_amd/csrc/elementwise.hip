@@ -8,8 +8,6 @@
 
 namespace {
 
-constexpr int ROW_THREADS = 256;   // per-token quantisation: threads per row for narrow rows ...
-constexpr int ROW_THREADS_WIDE = 1024;   // ... and for wide ones (one workgroup per row either way: more waves in flight)
 constexpr int ROW_MAX_COLS = 24576;
 constexpr int NORM_THREADS = 512;  // RMSNorm: the geometry (and summation order) shared with the GEMM-fused norm
 constexpr int NORM_MAX_VEC = 4;    // up to 4 x (8 elements) per thread: cols <= 512*4*8 = 16384
@@ -24,7 +22,13 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     __syncthreads();
     return t;
 }
-template <typename T>
+// The row kernels are built for the number of 8-element pieces a thread holds (NV, MAXV): registers for more would only cost
+// waves in flight.  Pieces past the row's end are the last one once more (maxima do not change, sums leave them out) and
+// only the stores ask for the end: loads behind a branch per piece would each wait for the one before.  Bound by the
+// latency of load, reduction and store per workgroup, i.e. by the waves in flight; built for the widest row (12 pieces
+// behind branches) | as here: SiLU * up + quantise 1531 x 18944 54.5 | 45.3 us, 16616 x 2048 60.7 | 48.3, quantise
+// 2077 x 7168 29.9 | 16.0, 1531 x 3584 10.5 | 8.0, norm + quantise 1531 x 3584 14.4 | 13.1, norm 4137 x 4096 18.4 | 15.7.
+template <typename T, int NV>
 __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_kernel(uint16_t* __restrict__ y,
                                                              uint16_t* __restrict__ sum_out,
                                                              const uint16_t* __restrict__ x,
@@ -35,34 +39,41 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_kernel(uint16_t* __restr
     __shared__ float red[NORM_THREADS / 64];
     const int64_t row = (int64_t)blockIdx.x * cols;
     const int nvec = cols >> 3;
-    float v[NORM_MAX_VEC][8], gm[NORM_MAX_VEC][8];
+    float v[NV][8], gm[NV][8];
     float ss = 0.f;
+    u32x4 raw[NV], rraw[NV];
 #pragma unroll
-    for (int it = 0; it < NORM_MAX_VEC; ++it) {
+    for (int it = 0; it < NV; ++it)
+        raw[it] = *(const u32x4*)(x + (int64_t)blockIdx.x * x_stride + 8 * min((int)threadIdx.x + it * NORM_THREADS, nvec - 1));
+    if (residual) {
+#pragma unroll
+        for (int it = 0; it < NV; ++it)
+            rraw[it] = *(const u32x4*)(residual + row + 8 * min((int)threadIdx.x + it * NORM_THREADS, nvec - 1));
+    }
+#pragma unroll
+    for (int it = 0; it < NV; ++it) {
         const int c = threadIdx.x + it * NORM_THREADS;
-        if (c < nvec) {
-            u32x4 raw = *(const u32x4*)(x + (int64_t)blockIdx.x * x_stride + 8 * c);
-            u32x4 rraw;
-            if (residual) rraw = *(const u32x4*)(residual + row + 8 * c);
-            load8_as_float(gamma, 8 * c, gamma_dtype, gm[it]);   // in flight together with the row, used after the sum
-            unpack8<T>(raw, v[it]);
-            if (residual) {
-                float rr[8];
-                unpack8<T>(rraw, rr);
-                u32x4 s;
+        const bool on = c < nvec;
+        load8_as_float(gamma, 8 * min(c, nvec - 1), gamma_dtype, gm[it]);   // used after the sum
+        unpack8<T>(raw[it], v[it]);
+        if (residual) {
+            float rr[8];
+            unpack8<T>(rraw[it], rr);
+            u32x4 s;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) s[i] = pack2<T>(v[it][2 * i] + rr[2 * i], v[it][2 * i + 1] + rr[2 * i + 1]);
-                *(u32x4*)(sum_out + row + 8 * c) = s;
-                unpack8<T>(s, v[it]);                          // normalise the rounded sum, as two ops would
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) ss = __fmaf_rn(v[it][i], v[it][i], ss);
+            for (int i = 0; i < 4; ++i) s[i] = pack2<T>(v[it][2 * i] + rr[2 * i], v[it][2 * i + 1] + rr[2 * i + 1]);
+            if (on) *(u32x4*)(sum_out + row + 8 * c) = s;
+            unpack8<T>(s, v[it]);                              // normalise the rounded sum, as two ops would
         }
+        float t = ss;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t = __fmaf_rn(v[it][i], v[it][i], t);
+        ss = on ? t : ss;
     }
     ss = rmsnorm_block_sum<NORM_THREADS>(ss, red);
     const float inv = rsqrtf(ss / (float)cols + eps);
 #pragma unroll
-    for (int it = 0; it < NORM_MAX_VEC; ++it) {
+    for (int it = 0; it < NV; ++it) {
         const int c = threadIdx.x + it * NORM_THREADS;
         if (c < nvec) {
             u32x4 o;
@@ -175,28 +186,27 @@ __device__ __forceinline__ const float* smooth_of_row(const float* smooth, RowGr
 // Per-token dynamic int8: xs = x*smooth; s = max|xs|/127; q = clip(rint(xs/s), -128, 127).
 // With static_scale (one float on the device: a calibrated per-tensor activation scale) s is that value for every
 // row and no maximum is taken; x_scale still receives s per row, which is what the int8 GEMM's epilogue reads.
-template <typename T, int THREADS>
-__global__ __launch_bounds__(THREADS) void dynamic_quant_kernel(int8_t* __restrict__ xq, float* __restrict__ x_scale,
+template <typename T, int THREADS, int MAXV>
+__global__ __launch_bounds__(THREADS, THREADS == 1024 ? 8 : 4) void dynamic_quant_kernel(int8_t* __restrict__ xq, float* __restrict__ x_scale,
                                                                const uint16_t* __restrict__ x,
                                                                const float* __restrict__ smooth_table, int cols,
                                                                int tiled, const float* __restrict__ static_scale,
                                                                RowGroups rg) {
     __shared__ float red[THREADS / 64];
     const int m = quant_row(blockIdx.x, gridDim.x, tiled);
-    const float* smooth = smooth_of_row(smooth_table, rg, m, cols);
     const int64_t row = (int64_t)m * cols;
-    const int nvec = cols >> 3;
-    constexpr int ROW_THREADS = THREADS;
-    constexpr int MAXV = ROW_MAX_COLS / 8 / THREADS;
+    const int nvec = cols >> 3, first = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
+    u32x4 raw[MAXV];
+#pragma unroll
+    for (int it = 0; it < MAXV; ++it) raw[it] = *(const u32x4*)(x + row + 8 * min((int)threadIdx.x + it * THREADS, nvec - 1));
+    const float* smooth = smooth_of_row(smooth_table, rg, m, cols);
     float v[MAXV][8];
     float amax = 0.f;
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
-        const int c = threadIdx.x + it * ROW_THREADS;
-        if (c < nvec) {
-            unpack8<T>(*(const u32x4*)(x + row + 8 * c), v[it]);
-            amax = fmaxf(amax, smooth_absmax8(v[it], smooth, 8 * c));
-        }
+        if (first + it * THREADS >= nvec) break;               // the whole wave is past the end
+        unpack8<T>(raw[it], v[it]);
+        amax = fmaxf(amax, smooth_absmax8(v[it], smooth, 8 * min((int)threadIdx.x + it * THREADS, nvec - 1)));
     }
     float s;
     if (static_scale) {
@@ -209,7 +219,7 @@ __global__ __launch_bounds__(THREADS) void dynamic_quant_kernel(int8_t* __restri
     if (threadIdx.x == 0) x_scale[m] = s;
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
-        const int c = threadIdx.x + it * ROW_THREADS;
+        const int c = threadIdx.x + it * THREADS;
         if (c < nvec) quant_store8(xq, v[it], d, m, 8 * c, cols, gridDim.x, tiled);
     }
 }
@@ -228,7 +238,7 @@ struct PartialRow {
     int split_k;
 };
 
-template <typename T, bool PARTIAL>
+template <typename T, bool PARTIAL, int NV>
 __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
     int8_t* __restrict__ xq, float* __restrict__ x_scale, uint16_t* __restrict__ sum_out,
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual, const void* __restrict__ gamma,
@@ -237,10 +247,20 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
     const int m = quant_row(blockIdx.x, gridDim.x, tiled);
     const int64_t row = (int64_t)m * cols;
     const int nvec = cols >> 3;
-    float v[NORM_MAX_VEC][8], gm[NORM_MAX_VEC][8];
+    float v[NV][8], gm[NV][8];
     float ss = 0.f;
+    u32x4 xraw[NV], rraw[NV];
+    auto piece = [&](int it) { return 8 * min((int)threadIdx.x + it * NORM_THREADS, nvec - 1); };
+    if constexpr (!PARTIAL) {
 #pragma unroll
-    for (int it = 0; it < NORM_MAX_VEC; ++it) {
+        for (int it = 0; it < NV; ++it) xraw[it] = *(const u32x4*)(x + row + piece(it));
+    }
+    if (residual) {
+#pragma unroll
+        for (int it = 0; it < NV; ++it) rraw[it] = *(const u32x4*)(residual + row + piece(it));
+    }
+#pragma unroll
+    for (int it = 0; it < NV; ++it) {
         const int c = threadIdx.x + it * NORM_THREADS;
         if (c < nvec) {
             u32x4 raw;
@@ -281,15 +301,13 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
                 for (int i = 0; i < 4; ++i) raw[i] = pack2<T>(t[2 * i], t[2 * i + 1]);
                 if (!residual && sum_out) *(u32x4*)(sum_out + row + 8 * c) = raw;
             } else {
-                raw = *(const u32x4*)(x + row + 8 * c);
+                raw = xraw[it];
             }
-            u32x4 rraw;
-            if (residual) rraw = *(const u32x4*)(residual + row + 8 * c);
             load8_as_float(gamma, 8 * c, gamma_dtype, gm[it]);
             unpack8<T>(raw, v[it]);
             if (residual) {
                 float rr[8];
-                unpack8<T>(rraw, rr);
+                unpack8<T>(rraw[it], rr);
                 u32x4 sm;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) sm[i] = pack2<T>(v[it][2 * i] + rr[2 * i], v[it][2 * i + 1] + rr[2 * i + 1]);
@@ -304,7 +322,7 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
     const float inv = rsqrtf(ss / (float)cols + eps);
     float amax = 0.f;
 #pragma unroll
-    for (int it = 0; it < NORM_MAX_VEC; ++it) {
+    for (int it = 0; it < NV; ++it) {
         const int c = threadIdx.x + it * NORM_THREADS;
         if (c < nvec) {
             u32x4 o;
@@ -320,7 +338,7 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
     const QuantScale d = quant_scale(s > 0.f ? s : 1.0f, true);
     if (threadIdx.x == 0) x_scale[m] = s;
 #pragma unroll
-    for (int it = 0; it < NORM_MAX_VEC; ++it) {
+    for (int it = 0; it < NV; ++it) {
         const int c = threadIdx.x + it * NORM_THREADS;
         if (c < nvec) quant_store8(xq, v[it], d, m, 8 * c, cols, gridDim.x, tiled);
     }
@@ -328,49 +346,51 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
 
 // act(gate) * up followed by the per-token quantisation of the product, which is not written.  One workgroup per
 // row; rounding points as silu_mul_kernel has them.
-template <typename T, int THREADS>
-__global__ __launch_bounds__(THREADS) void silu_mul_quant_kernel(int8_t* __restrict__ xq, float* __restrict__ x_scale,
+template <typename T, int THREADS, int MAXV>
+__global__ __launch_bounds__(THREADS, THREADS == 1024 ? 8 : 4) void silu_mul_quant_kernel(int8_t* __restrict__ xq, float* __restrict__ x_scale,
                                                                 const uint16_t* __restrict__ gu,
                                                                 const float* __restrict__ smooth_table, int cols,
                                                                 int layout, int tiled, RowGroups rg) {
     __shared__ float red[THREADS / 64];
     const int m = quant_row(blockIdx.x, gridDim.x, tiled);
-    const float* smooth = smooth_of_row(smooth_table, rg, m, cols);
-    const int nvec = cols >> 3;
-    constexpr int ROW_THREADS = THREADS;
-    constexpr int MAXV = ROW_MAX_COLS / 8 / THREADS;
-    float v[MAXV][8];
-    float amax = 0.f;
+    const int nvec = cols >> 3, first = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
     const uint16_t* base = gu + (int64_t)m * 2 * cols;
+    u32x4 lo[MAXV], hi[MAXV];                                 // layout 0: gate and up; 1: two halves of the pairs
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
-        const int cv = threadIdx.x + it * ROW_THREADS;
-        if (cv < nvec) {
-            const int c = 8 * cv;
-            float g[8], u[8];
-            if (layout == 0) {
-                unpack8<T>(*(const u32x4*)(base + c), g);
-                unpack8<T>(*(const u32x4*)(base + cols + c), u);
-            } else {
-                float a[8], b[8];
-                unpack8<T>(*(const u32x4*)(base + 2 * c), a);
-                unpack8<T>(*(const u32x4*)(base + 2 * c + 8), b);
+        const int c = 8 * min((int)threadIdx.x + it * THREADS, nvec - 1);
+        lo[it] = *(const u32x4*)(base + (layout == 0 ? c : 2 * c));
+        hi[it] = *(const u32x4*)(base + (layout == 0 ? cols + c : 2 * c + 8));
+    }
+    const float* smooth = smooth_of_row(smooth_table, rg, m, cols);
+    float v[MAXV][8];
+    float amax = 0.f;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    g[j] = a[2 * j]; u[j] = a[2 * j + 1];
-                    g[4 + j] = b[2 * j]; u[4 + j] = b[2 * j + 1];
-                }
-            }
-            u32x4 o;
+    for (int it = 0; it < MAXV; ++it) {
+        if (first + it * THREADS >= nvec) break;               // the whole wave is past the end
+        float g[8], u[8];
+        if (layout == 0) {
+            unpack8<T>(lo[it], g);
+            unpack8<T>(hi[it], u);
+        } else {
+            float a[8], b[8];
+            unpack8<T>(lo[it], a);
+            unpack8<T>(hi[it], b);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float a0 = T::to_float(T::from_float(silu_f(g[2 * j])));
-                const float a1 = T::to_float(T::from_float(silu_f(g[2 * j + 1])));
-                o[j] = pack2<T>(a0 * u[2 * j], a1 * u[2 * j + 1]);
+                g[j] = a[2 * j]; u[j] = a[2 * j + 1];
+                g[4 + j] = b[2 * j]; u[4 + j] = b[2 * j + 1];
             }
-            unpack8<T>(o, v[it]);                              // the rounded product, as the next kernel would read it
-            amax = fmaxf(amax, smooth_absmax8(v[it], smooth, c));
         }
+        u32x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float a0 = T::to_float(T::from_float(silu_f(g[2 * j])));
+            const float a1 = T::to_float(T::from_float(silu_f(g[2 * j + 1])));
+            o[j] = pack2<T>(a0 * u[2 * j], a1 * u[2 * j + 1]);
+        }
+        unpack8<T>(o, v[it]);                                  // the rounded product, as the next kernel would read it
+        amax = fmaxf(amax, smooth_absmax8(v[it], smooth, 8 * min((int)threadIdx.x + it * THREADS, nvec - 1)));
     }
     amax = block_max(amax, red);
     const float s = __fdiv_rn(amax, 127.0f);
@@ -378,12 +398,35 @@ __global__ __launch_bounds__(THREADS) void silu_mul_quant_kernel(int8_t* __restr
     if (threadIdx.x == 0) x_scale[m] = s;
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
-        const int cv = threadIdx.x + it * ROW_THREADS;
+        const int cv = threadIdx.x + it * THREADS;
         if (cv < nvec) quant_store8(xq, v[it], d, m, 8 * cv, cols, gridDim.x, tiled);
     }
 }
 
 }  // namespace
+
+// one launch per (type, 8-element pieces a thread of the norm kernels holds)
+#define NORM_PIECES(dtype, cols, L)                                                                                \
+    do {                                                                                                           \
+        const int nv_ = (cols) <= NORM_THREADS * 8 ? 1 : (cols) <= NORM_THREADS * 16 ? 2 : NORM_MAX_VEC;             \
+        if ((dtype) == MF_BF16) {                                                                                  \
+            if (nv_ == 1) L(BF16, 1); else if (nv_ == 2) L(BF16, 2); else L(BF16, NORM_MAX_VEC);                     \
+        } else {                                                                                                   \
+            if (nv_ == 1) L(FP16, 1); else if (nv_ == 2) L(FP16, 2); else L(FP16, NORM_MAX_VEC);                     \
+        }                                                                                                          \
+    } while (0)
+// (type, threads per row, pieces a thread holds) of the quantisation kernels.  Up to 8192 columns few waves a row, with two
+// pieces each (1531 x 3584: 8.0 us, 11.2 with 512 threads of one piece); the widest rows keep 64 registers, so that two
+// workgroups of 16 waves share a compute unit (1531 x 18944: 45.3 us, 59.6 with one).
+#define QUANT_SHAPES(TT, cols, L)                                                                                  \
+    do {                                                                                                           \
+        if ((cols) <= 4096) L(TT, 256, 2); else if ((cols) <= 8192) L(TT, 512, 2); else L(TT, 1024, 3);              \
+    } while (0)
+#define QUANT_PIECES(dtype, cols, L)                                                                               \
+    do {                                                                                                           \
+        if ((dtype) == MF_BF16) QUANT_SHAPES(BF16, cols, L); else QUANT_SHAPES(FP16, cols, L);                       \
+    } while (0)
+static_assert(ROW_MAX_COLS == 1024 * 3 * 8, "the widest build covers every row");
 
 static int rmsnorm_entry(void* y, void* sum_out, const void* x, int64_t x_row_stride, const void* residual,
                          const void* gamma, float eps, int rows, int cols, int dtype, int gamma_dtype, void* stream) {
@@ -399,14 +442,12 @@ static int rmsnorm_entry(void* y, void* sum_out, const void* x, int64_t x_row_st
                (long long)x_row_stride);
     MF_REQUIRE((((uintptr_t)y | (uintptr_t)x | (uintptr_t)residual | (uintptr_t)sum_out | (uintptr_t)gamma) & 15) == 0,
                "rmsnorm: pointers must be 16-byte aligned");
-    if (dtype == MF_BF16)
-        hipLaunchKernelGGL(rmsnorm_kernel<BF16>, dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, (uint16_t*)y,
-                           (uint16_t*)sum_out, (const uint16_t*)x, (const uint16_t*)residual, gamma, eps, cols,
-                           gamma_dtype, x_row_stride);
-    else
-        hipLaunchKernelGGL(rmsnorm_kernel<FP16>, dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, (uint16_t*)y,
-                           (uint16_t*)sum_out, (const uint16_t*)x, (const uint16_t*)residual, gamma, eps, cols,
-                           gamma_dtype, x_row_stride);
+#define RN_LAUNCH(TT, NV)                                                                                          \
+    hipLaunchKernelGGL((rmsnorm_kernel<TT, NV>), dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, (uint16_t*)y, \
+                       (uint16_t*)sum_out, (const uint16_t*)x, (const uint16_t*)residual, gamma, eps, cols,           \
+                       gamma_dtype, x_row_stride)
+    NORM_PIECES(dtype, cols, RN_LAUNCH);
+#undef RN_LAUNCH
     return MF_LAUNCH_CHECK();
 }
 
@@ -502,15 +543,10 @@ static int quant_rows_entry(int8_t* xq, float* x_scale, const void* x, const flo
     MF_REQUIRE((((uintptr_t)xq & 7) | ((uintptr_t)x & 15) | ((uintptr_t)smooth & 15)) == 0,
                "dynamic_quant: x/smooth must be 16-byte aligned, xq 8-byte aligned");
     if (m <= 0) return 0;
-#define DQ_LAUNCH(TT, TH)                                                                                        \
-    hipLaunchKernelGGL((dynamic_quant_kernel<TT, TH>), dim3(m), dim3(TH), 0, (hipStream_t)stream, xq, x_scale,    \
+#define DQ_LAUNCH(TT, TH, NV)                                                                                        \
+    hipLaunchKernelGGL((dynamic_quant_kernel<TT, TH, NV>), dim3(m), dim3(TH), 0, (hipStream_t)stream, xq, x_scale,    \
                        (const uint16_t*)x, smooth, k, layout, static_scale, rg)
-    const bool wide = k > 4096;
-    if (dtype == MF_BF16) {
-        if (wide) DQ_LAUNCH(BF16, ROW_THREADS_WIDE); else DQ_LAUNCH(BF16, ROW_THREADS);
-    } else {
-        if (wide) DQ_LAUNCH(FP16, ROW_THREADS_WIDE); else DQ_LAUNCH(FP16, ROW_THREADS);
-    }
+    QUANT_PIECES(dtype, k, DQ_LAUNCH);
 #undef DQ_LAUNCH
     return MF_LAUNCH_CHECK();
 }
@@ -532,14 +568,12 @@ extern "C" int mf_rmsnorm_dynamic_quant(int8_t* xq, float* x_scale, void* sum_ou
                    ((uintptr_t)xq & 7) == 0,
                "rmsnorm_dynamic_quant: pointers must be 16-byte aligned, xq 8-byte aligned");
     const PartialRow none = {nullptr, nullptr, nullptr, nullptr, 0};
-    if (dtype == MF_BF16)
-        hipLaunchKernelGGL((rmsnorm_quant_kernel<BF16, false>), dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, xq,
-                           x_scale, (uint16_t*)sum_out, (const uint16_t*)x, (const uint16_t*)residual, gamma, smooth, eps,
-                           cols, gamma_dtype, layout, none);
-    else
-        hipLaunchKernelGGL((rmsnorm_quant_kernel<FP16, false>), dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, xq,
-                           x_scale, (uint16_t*)sum_out, (const uint16_t*)x, (const uint16_t*)residual, gamma, smooth, eps,
-                           cols, gamma_dtype, layout, none);
+#define RQ_LAUNCH(TT, NV) \
+    hipLaunchKernelGGL((rmsnorm_quant_kernel<TT, false, NV>), dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, xq, \
+                       x_scale, (uint16_t*)sum_out, (const uint16_t*)x, (const uint16_t*)residual, gamma, smooth, eps, \
+                       cols, gamma_dtype, layout, none)
+    NORM_PIECES(dtype, cols, RQ_LAUNCH);
+#undef RQ_LAUNCH
     return MF_LAUNCH_CHECK();
 }
 
@@ -550,14 +584,12 @@ int mf_detail_rmsnorm_quant_from_partial(int8_t* xq, float* x_scale, void* sum_o
                                          const void* residual, const void* gamma, const float* smooth, float eps,
                                          int rows, int cols, int dtype, int gamma_dtype, int layout, void* stream) {
     const PartialRow pr = {partial, row_scale, col_scale, (const uint16_t*)bias, split_k};
-    if (dtype == MF_BF16)
-        hipLaunchKernelGGL((rmsnorm_quant_kernel<BF16, true>), dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, xq,
-                           x_scale, (uint16_t*)sum_out, nullptr, (const uint16_t*)residual, gamma, smooth, eps, cols,
-                           gamma_dtype, layout, pr);
-    else
-        hipLaunchKernelGGL((rmsnorm_quant_kernel<FP16, true>), dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, xq,
-                           x_scale, (uint16_t*)sum_out, nullptr, (const uint16_t*)residual, gamma, smooth, eps, cols,
-                           gamma_dtype, layout, pr);
+#define RQ_LAUNCH(TT, NV) \
+    hipLaunchKernelGGL((rmsnorm_quant_kernel<TT, true, NV>), dim3(rows), dim3(NORM_THREADS), 0, (hipStream_t)stream, xq, \
+                       x_scale, (uint16_t*)sum_out, nullptr, (const uint16_t*)residual, gamma, smooth, eps, cols, \
+                       gamma_dtype, layout, pr)
+    NORM_PIECES(dtype, cols, RQ_LAUNCH);
+#undef RQ_LAUNCH
     return MF_LAUNCH_CHECK();
 }
 
@@ -576,15 +608,10 @@ static int silu_mul_quant_entry(int8_t* xq, float* x_scale, const void* gate_up,
                "silu_mul_dynamic_quant: cols (%d) must be a multiple of 8, <= %d", cols, ROW_MAX_COLS);
     MF_REQUIRE((((uintptr_t)gate_up | (uintptr_t)smooth) & 15) == 0 && ((uintptr_t)xq & 7) == 0,
                "silu_mul_dynamic_quant: gate_up/smooth must be 16-byte aligned, xq 8-byte aligned");
-#define SQ_LAUNCH(TT, TH)                                                                                        \
-    hipLaunchKernelGGL((silu_mul_quant_kernel<TT, TH>), dim3(rows), dim3(TH), 0, (hipStream_t)stream, xq, x_scale, \
+#define SQ_LAUNCH(TT, TH, NV)                                                                                        \
+    hipLaunchKernelGGL((silu_mul_quant_kernel<TT, TH, NV>), dim3(rows), dim3(TH), 0, (hipStream_t)stream, xq, x_scale, \
                        (const uint16_t*)gate_up, smooth, cols, gate_up_layout, layout, rg)
-    const bool wide = cols > 4096;
-    if (dtype == MF_BF16) {
-        if (wide) SQ_LAUNCH(BF16, ROW_THREADS_WIDE); else SQ_LAUNCH(BF16, ROW_THREADS);
-    } else {
-        if (wide) SQ_LAUNCH(FP16, ROW_THREADS_WIDE); else SQ_LAUNCH(FP16, ROW_THREADS);
-    }
+    QUANT_PIECES(dtype, cols, SQ_LAUNCH);
 #undef SQ_LAUNCH
     return MF_LAUNCH_CHECK();
 }

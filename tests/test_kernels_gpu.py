@@ -1317,6 +1317,33 @@ def test_dynamic_quant_tiled_layout_bit_exact(m, k):
     assert np.array_equal(untile_int8(to_np(xt.data), m, k), q_ref)
 
 
+@pytest.mark.parametrize("cols", [2040, 2056, 4096, 4104, 8192, 8200, 16384])
+def test_row_kernels_around_their_widths(cols):
+    """Widths on both sides of every build of the row kernels (threads a row, pieces a thread): the norm against float64, the
+    quantisation against the oracle, the fused forms against the separate ones, bit for bit."""
+    dtype, m = torch.bfloat16, 67
+    rng = np.random.default_rng(cols)
+    x, r, gu = (rounded(rng.normal(size=(m, c)), dtype) for c in (cols, cols, 2 * cols))
+    gm = rng.uniform(0.5, 1.5, cols).astype(np.float32)
+    sm = rng.uniform(0.5, 2.0, cols).astype(np.float32)
+    gd, sd = torch.from_numpy(gm).cuda(), torch.from_numpy(sm).cuda()
+    y, h = ops.rms_norm(dev(x, dtype), gd, 1e-5, residual=dev(r, dtype))
+    hs = to_np(h).astype(np.float64)
+    assert np.array_equal(to_np(h), rounded(x + r, dtype))
+    ref = hs / np.sqrt((hs * hs).mean(1, keepdims=True) + 1e-5) * gm
+    assert_within(to_np(y), ref, np.abs(ref), dtype, ulps=1.0, extra=1e-5 * np.abs(ref) + 1e-7, what="norm")
+    q, s = ops.dynamic_quant(y, sd, tiled=True)
+    q_ref, s_ref = O.dynamic_quant_per_token(to_np(y), sm)
+    assert np.array_equal(to_np(s), s_ref) and np.array_equal(untile_int8(to_np(q.data), m, cols), q_ref)
+    fq, fs, fh = ops.rms_norm_dynamic_quant(dev(x, dtype), gd, 1e-5, sd, residual=dev(r, dtype), tiled=True)
+    assert torch.equal(fh, h)
+    assert torch.equal(fs, s) and np.array_equal(untile_int8(to_np(fq.data), m, cols), q_ref)
+    sq, ss = ops.silu_mul_dynamic_quant(dev(gu, dtype), sd, tiled=True)
+    act = to_np(ops.silu_mul(dev(gu, dtype)))
+    q_ref, s_ref = O.dynamic_quant_per_token(act, sm)
+    assert np.array_equal(to_np(ss), s_ref) and np.array_equal(untile_int8(to_np(sq.data), m, cols), q_ref)
+
+
 @pytest.mark.parametrize("m", [64, 65, 127, 200])
 @pytest.mark.parametrize("dtype,lo,hi", [(torch.bfloat16, -110, 110), (torch.float16, -14, 8)])
 def test_dynamic_quant_at_rounding_edges(dtype, lo, hi, m):
