@@ -80,6 +80,29 @@ def test_rope_half(dtype, table, t, nh, nkv, d):
         assert_within(to_np(got), ref, mag.reshape(t, n * d), dtype, ulps=1.0, what="rope")
 
 
+@pytest.mark.parametrize("dtype,table", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("t,nh,nkv,d,with_key", [(3, 32, 8, 128, True), (70, 5, 1, 16, True), (9, 7, 3, 48, False),
+                                                 (5, 33, 33, 64, True)])
+def test_rope_half_in_16_byte_pieces_equals_pairs(dtype, table, t, nh, nkv, d, with_key):
+    """Aligned rows (16-byte pieces, here column slices of a wider matrix) and rows that start 2 bytes off (a pair of
+    elements a lane) give the same bits, and the columns between the slices stay as they were."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(t * d)
+    n, nk = nh * d, nkv * d
+    wide = torch.randn(t, n + nk + 16, generator=g, device="cuda").to(dtype)
+    before = wide.clone()
+    q, k = wide[:, :n], wide[:, n + 8:n + 8 + nk]
+    c, s = (torch.randn(t, d, generator=g, device="cuda").to(table) for _ in range(2))
+    q1 = torch.empty(t * n + 8, dtype=dtype, device="cuda")[1:1 + t * n].view(t, n)
+    k1 = torch.empty(t * nk + 8, dtype=dtype, device="cuda")[1:1 + t * nk].view(t, nk)
+    q1.copy_(q)
+    k1.copy_(k)
+    ops.apply_rotary_pos_emb(q, k if with_key else None, c, s, nh, nkv, d)
+    ops.apply_rotary_pos_emb(q1, k1 if with_key else None, c, s, nh, nkv, d)
+    assert torch.equal(q, q1) and torch.equal(k, k1)
+    assert torch.equal(wide[:, n:n + 8], before[:, n:n + 8]) and torch.equal(wide[:, n + 8 + nk:], before[:, n + 8 + nk:])
+
+
 def test_rope_golden_decode_vectors(golden_dir):
     """The reference's own decode vectors (position 1, bf16 tables), through the kernel."""
     z = np.load(os.path.join(golden_dir, "rotary.npz"))
