@@ -54,6 +54,11 @@ int mf_rope_half(void* query, void* key, const void* cos, const void* sin, int n
                  int n_kv_heads, int head_dim, int64_t q_row_stride, int64_t k_row_stride, int dtype,
                  int table_dtype, void* stream);
 
+/* The rotary rows of a step: cos / sin [num_tokens, head_dim] (dtype) of positions[t] * inv_freq[i] (float32 product,
+ * inv_freq float32 [head_dim / 2]), the second half of a row repeating the first. */
+int mf_rope_rows(void* cos, void* sin, const int32_t* positions, const float* inv_freq, int num_tokens, int head_dim,
+                 int dtype, void* stream);
+
 /* RoPE on q and k followed by the cache scatter of rotated k and of v, one launch (the sequence
  * infer_attention.py:445,453 performs).  q and k are rotated in place. */
 int mf_rope_and_cache(void* query, void* key, const void* value, const void* cos, const void* sin,

@@ -21,6 +21,7 @@ SIGNATURES = {
     "mf_last_error": (_c.c_char_p, []),
     "mf_reshape_and_cache": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _P]),
     "mf_rope_half": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _L, _L, _I, _I, _P]),
+    "mf_rope_rows": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),
     "mf_rope_and_cache": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _L, _L, _L, _L, _I, _I, _P]),
     "mf_swap_blocks": (_I, [_P, _P, _P, _L, _L, _L, _L, _I, _P]),
     "mf_paged_attention_workspace_bytes": (_Z, [_I, _I, _I, _I]),

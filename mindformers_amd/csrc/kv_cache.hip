@@ -90,6 +90,26 @@ __global__ void rope_and_cache_kernel(uint16_t* __restrict__ q, uint16_t* __rest
     }
 }
 
+// One thread per (token, frequency).  The angle is a float32 product of its own, as the separate operations have it.
+template <typename T>
+__global__ __launch_bounds__(256) void rope_rows_kernel(uint16_t* __restrict__ cos, uint16_t* __restrict__ sin,
+                                                       const int32_t* __restrict__ positions,
+                                                       const float* __restrict__ inv_freq, int tokens, int D) {
+    const int half = D >> 1;
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= (int64_t)tokens * half) return;
+    const int64_t t = p / half;
+    const int i = (int)(p - t * half);
+    float a = __fmul_rn((float)positions[t], inv_freq[i]);
+    asm volatile("" : "+v"(a));
+    const uint16_t c = T::from_float(cosf(a)), s = T::from_float(sinf(a));
+    const int64_t at = t * D + i;
+    cos[at] = c;
+    cos[at + half] = c;
+    sin[at] = s;
+    sin[at + half] = s;
+}
+
 // Vector form of the fused rotate-and-scatter for head_dim % 16 == 0: one work item = 8 consecutive elements
 // of the first half of a head together with their partners in the second half (16-byte accesses), or one
 // 16-byte piece of the value row.  grid = (tokens, ceil(items / 256)).  Without slot_mapping (and v) it rotates only (1048
@@ -318,6 +338,22 @@ extern "C" int mf_rope_half(void* query, void* key, const void* cos, const void*
         hipLaunchKernelGGL(rope_kernel<FP16>, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, (uint16_t*)query,
                            (uint16_t*)key, cos, sin, n_heads, n_kv_heads, head_dim, table_dtype, q_row_stride,
                            k_row_stride);
+    return MF_LAUNCH_CHECK();
+}
+
+extern "C" int mf_rope_rows(void* cos, void* sin, const int32_t* positions, const float* inv_freq, int num_tokens,
+                            int head_dim, int dtype, void* stream) {
+    MF_REQUIRE(dtype == MF_BF16 || dtype == MF_FP16, "rope_rows: dtype must be bf16 or fp16");
+    if (num_tokens <= 0) return 0;
+    MF_REQUIRE(cos && sin && positions && inv_freq, "rope_rows: null argument");
+    MF_REQUIRE(head_dim > 0 && head_dim % 2 == 0, "rope_rows: head_dim must be even");
+    const unsigned blocks = (unsigned)(((int64_t)num_tokens * (head_dim / 2) + 255) / 256);
+    if (dtype == MF_BF16)
+        hipLaunchKernelGGL(rope_rows_kernel<BF16>, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (uint16_t*)cos,
+                           (uint16_t*)sin, positions, inv_freq, num_tokens, head_dim);
+    else
+        hipLaunchKernelGGL(rope_rows_kernel<FP16>, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (uint16_t*)cos,
+                           (uint16_t*)sin, positions, inv_freq, num_tokens, head_dim);
     return MF_LAUNCH_CHECK();
 }
 

@@ -118,6 +118,20 @@ def apply_rotary_pos_emb(query, key, cos, sin, n_heads, n_kv_heads, head_dim):
     return query, key
 
 
+def rope_rows(positions, inv_freq, dtype):
+    """Rotary rows of a step: (cos, sin), each [T, 2 * len(inv_freq)] in ``dtype``, of int32 ``positions`` [T] times the
+    fp32 ``inv_freq``; the second half of a row repeats the first."""
+    lib = _lib.load()
+    dev = _dev_ok(positions, inv_freq)
+    _need(positions.dtype == torch.int32 and inv_freq.dtype == torch.float32 and dtype in _ACT, "rope_rows dtypes")
+    t, d = positions.numel(), 2 * inv_freq.numel()
+    cos = torch.empty(t, d, dtype=dtype, device=dev)
+    sin = torch.empty_like(cos)
+    check(lib.mf_rope_rows(ptr(cos), ptr(sin), ptr(positions), ptr(inv_freq), t, d, dtype_code(dtype), stream_ptr(dev)),
+          "mf_rope_rows")
+    return cos, sin
+
+
 def rope_and_cache(query, key, value, cos, sin, key_cache, value_cache, slot_mapping, n_heads):
     """RoPE on q/k (in place) then scatter of rotated k and v into the caches, one launch."""
     lib = _lib.load()

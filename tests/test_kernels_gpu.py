@@ -103,6 +103,21 @@ def test_rope_half_in_16_byte_pieces_equals_pairs(dtype, table, t, nh, nkv, d, w
     assert torch.equal(wide[:, n:n + 8], before[:, n:n + 8]) and torch.equal(wide[:, n + 8 + nk:], before[:, n + 8 + nk:])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("t,d", [(1, 32), (4, 64), (301, 128), (2, 48)])
+def test_rope_rows(dtype, t, d):
+    """Rows against float64 cosines of the same float32 angles: one rounding to the type, 4 float32 steps for cosf / sinf."""
+    rng = np.random.default_rng(t + d)
+    pos = rng.integers(0, 1 << 17, t).astype(np.int32)
+    pos[0] = 0
+    inv = (1.0 / 10000.0 ** (np.arange(0, d, 2) / d)).astype(np.float32)
+    cos, sin = ops.rope_rows(torch.from_numpy(pos).cuda(), torch.from_numpy(inv).cuda(), dtype)
+    ang = (pos.astype(np.float32)[:, None] * inv).astype(np.float64)
+    for got, ref in ((cos, np.cos(ang)), (sin, np.sin(ang))):
+        ref = np.concatenate((ref, ref), 1)
+        assert (np.abs(to_np(got) - ref) <= EPS[dtype] * np.abs(ref) * 1.01 + 4 * 2.0 ** -24).all()
+
+
 def test_rope_golden_decode_vectors(golden_dir):
     """The reference's own decode vectors (position 1, bf16 tables), through the kernel."""
     z = np.load(os.path.join(golden_dir, "rotary.npz"))

@@ -234,3 +234,27 @@ def test_runner_sizes_and_runs_int8_caches_from_the_quantization_config():
     run.swap(np.array([[0, used[0]]]), False)
     torch.cuda.synchronize()
     assert torch.equal(run.key_cache[1][used[0]], before)
+
+
+def test_host_arrays_and_device_tensors_give_the_same_steps():
+    """Ten steps in a row without a wait, each with its own lengths, from numpy arrays (one copy a step, int64 and int32) and
+    from device tensors: the same bits, step by step."""
+    from mindformers_amd.runner import DecodeStackRunner
+    hidden, nh, nkv, d, bs, b = 512, 8, 2, 64, 16, 5
+    layers = _stack(1, hidden, nh, nkv, d, 1024, seed=3)
+    outs = []
+    for on_device in (False, True):
+        run = DecodeStackRunner(layers, npu_mem_size=0.002, cpu_mem_size=0, block_size=bs)
+        rng = np.random.default_rng(11)
+        x = dev(rounded(rng.normal(size=(b, hidden)), BF), BF)
+        tables = rng.permutation(run.npu_num_blocks)[:b * 4].reshape(b, 4)
+        got = []
+        for step in range(10):
+            lens = rng.integers(1, 4 * bs + 1, b)
+            slots = tables[np.arange(b), (lens - 1) // bs] * bs + (lens - 1) % bs
+            t, s = tables, slots.astype(np.int32)
+            if on_device:
+                t, s = torch.from_numpy(t.astype(np.int32)).cuda(), torch.from_numpy(s).cuda()
+            got.append(run.forward(x, lens, t, s, prefill=False))
+        outs.append([to_np(o) for o in got])
+    assert all(np.array_equal(a, c) for a, c in zip(*outs))
