@@ -791,7 +791,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_tile_kernel(
     const QTileOut<T> out{x_scale, w_scale, bias, M, N};
     f32x4 ws[8], bi[8];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
-    const tq::TiledRows<MT / 2> rows((const uint8_t*)xq, m0 >> 4, (M + 15) >> 4);
+    const tq::TiledRows<tq::XLOADS<MT>> rows((const uint8_t*)xq, m0 >> 4, (M + 15) >> 4);
     tq::tile<MT>(rows, wp, nb * (tq::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const i32x16 (&acc)[2]) {
         constexpr int mt = decltype(mtc)::value;
         if (whole) {
@@ -975,10 +975,12 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
     }
 }
 
-// Groups of prompt size: tiles of up to 128 rows x 256 channels of one expert (w8a8_tile_gemm.h on row-major rows, 64-row
-// tiles where the expert has no more), the row blocks of all experts dealt to the XCDs as tg_group_locate says.  Bound by the
+// Groups of prompt size: tiles of up to 128 rows x 256 channels of one expert (w8a8_tile_gemm.h on row-major rows, 64- or
+// 96-row tiles where the expert has no more), the row blocks of all experts dealt to the XCDs as tg_group_locate says.  Bound by the
 // stream of the expert weights: 256 experts of 65 rows, 4096 x 7168: 2258 us in passes of 64 rows by 64-channel workgroups
 // (each fetching the rows anew, a second pass for every second expert), 1435 here (5.2 TB/s of weights); 7168 x 2048: 1280 / 817.
+// With 128-row tiles for every expert of more than 64 rows the padding's matrix instructions counted: the two GEMMs of 256
+// experts of 65 rows on average 2323 us, 2167 with tiles of 96 rows for those up to 96.
 template <typename T, int MT>
 __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, const float* xs, const uint8_t* we,
                                                 const float* ws, int rows, int m0, int nb, int N, int K, int aligned,
@@ -988,7 +990,7 @@ __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, 
     const QTileOut<T> out{xs, ws, nullptr, rows, N};
     f32x4 wsv[8], bi[8];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
-    const tq::PlainRows<MT / 2> src(xe, m0, rows, K);
+    const tq::PlainRows<tq::XLOADS<MT>> src(xe, m0, rows, K);
     tq::tile<MT>(src, we, nb * (tq::BN / 16), (N + 15) >> 4, 0, (K + Q_KSTEP - 1) / Q_KSTEP, smem,
                  [&](auto mtc, const i32x16 (&acc)[2]) {
         constexpr int mt = decltype(mtc)::value;
@@ -1021,6 +1023,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
     const uint8_t *xe = (const uint8_t*)xq + (int64_t)row0 * K, *we = wp + (int64_t)e * expert_bytes;
     const float *xs = x_scale + row0, *ws = w_scale + (int64_t)e * N;
     if (rows - m0 <= 64) w8a8_group_tile<T, 2>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
+    else if (rows - m0 <= 96) w8a8_group_tile<T, 3>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
     else w8a8_group_tile<T, 4>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
 }
 

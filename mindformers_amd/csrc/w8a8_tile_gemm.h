@@ -21,8 +21,12 @@ constexpr int BN = 64 * WAVES;
 constexpr int KSTEP = 64;
 constexpr int D = 3;                                          // register sets
 
+// 16-row activation tiles that each of the four waves loads and stages per step (three 32-row blocks: as for four, the last
+// two tiles are not read back)
 template <int MT>
-constexpr int LDS_BYTES = 2 * 32 * MT * KSTEP;
+constexpr int XLOADS = (MT + 1) / 2;
+template <int MT>
+constexpr int LDS_BYTES = 2 * 64 * XLOADS<MT> * KSTEP;
 
 // Where the activations come from: 16-row tile 4i + wave of the workgroup is load i of a wave, lane (r, g) of it row r, columns
 // 16g .. + 15 of the step.
@@ -55,8 +59,7 @@ struct PlainRows {                                            // rows m0 .. of `
 template <int MT, typename Rows, typename Epilogue>
 __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ wp, int tile0, int n_tiles, int s_begin,
                                      int s_end, uint8_t* smem, Epilogue&& epilogue) {
-    static_assert(MT % 2 == 0, "the activation tiles of a step are dealt over the four waves");
-    constexpr int STAGE = 32 * MT * KSTEP, XL = MT / 2;       // 16-row tiles loaded per wave and step
+    constexpr int XL = XLOADS<MT>, STAGE = 64 * XL * KSTEP;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int h = lane >> 5;
     const int s_last = s_end - 1;
