@@ -41,8 +41,8 @@ class DecodeStackRunner:
         self.num_layers = len(layers)
         self.num_kv_heads, self.head_size, self.dtype = first.n_kv_head, first.head_dim, first.dtype
         self.block_size = int(block_size)
-        self.rope_theta = rope_theta
         self.device = torch.device(device)
+        self.rope_theta = rope_theta
         # the cache dtype follows the quantization config when it names one (model_runner.py:364-368); int8 caches
         # need every layer's dequantisation parameters (QuantDecodeLayer.set_kv_quant)
         kv_name = getattr(quantization_config, "kvcache_quant_dtype", None) if quantization_config is not None else None
@@ -72,7 +72,6 @@ class DecodeStackRunner:
         pin = self.cpu_num_blocks > 0
         self.key_host = [torch.zeros(host_shape, dtype=self.kvcache_dtype, pin_memory=pin) for _ in layers]
         self.value_host = [torch.zeros(host_shape, dtype=self.kvcache_dtype, pin_memory=pin) for _ in layers]
-        self._inv_freq = (None, None)                         # (theta, its frequencies)
         self.is_first_iteration = True
         self.phase = "prefill"
 
@@ -84,17 +83,22 @@ class DecodeStackRunner:
         self.is_first_iteration = bool(is_first_iteration)
         self.phase = "prefill" if self.is_first_iteration else "increment"
 
-    def _inverse_frequencies(self):
-        if self._inv_freq[0] != self.rope_theta:
-            d = self.head_size
-            self._inv_freq = (self.rope_theta, 1.0 / (self.rope_theta ** (torch.arange(
-                0, d, 2, dtype=torch.float32, device=self.device) / d)))
-        return self._inv_freq[1]
+    @property
+    def rope_theta(self):
+        return self._rope_theta
 
-    def _rope_rows(self, positions):
+    @rope_theta.setter
+    def rope_theta(self, theta):
+        # Computed by the device, as the separate operations would, and kept on the host: every step takes it over with its
+        # own arrays, so that steps on different streams or threads share no device memory that one of them writes.
+        d = self.head_size
+        inv = 1.0 / (theta ** (torch.arange(0, d, 2, dtype=torch.float32, device=self.device) / d))
+        self._rope_theta, self._inv_freq = theta, inv.cpu().numpy()
+
+    def _rope_rows(self, positions, inv_freq):
         if positions.dtype == torch.int32 and positions.is_contiguous():
-            return ops.rope_rows(positions, self._inverse_frequencies(), self.dtype)
-        ang = positions.to(torch.float32)[:, None] * self._inverse_frequencies()[None, :]
+            return ops.rope_rows(positions, inv_freq, self.dtype)
+        ang = positions.to(torch.float32)[:, None] * inv_freq[None, :]
         emb = torch.cat((ang, ang), dim=-1)
         return emb.cos().to(self.dtype), emb.sin().to(self.dtype)
 
@@ -141,7 +145,7 @@ class DecodeStackRunner:
             pos = np.concatenate([np.arange(l - q, l) for l, q in zip(lens, q_lens)]) if t else np.zeros(0, np.int64)
             q_starts = np.concatenate([[0], np.cumsum(q_lens)])
         # the scheduler's arrays go over in one copy; what it holds on the device, or in another form, goes by itself
-        host = {"lens": lens}
+        host = {"lens": lens, "freq": self._inv_freq.view(np.int32)}
         if position_ids is None:
             host["pos"] = pos
         if q_starts is not None:
@@ -155,7 +159,7 @@ class DecodeStackRunner:
                                                                             device=self.device)
         slots = there["slots"] if "slots" in there else torch.as_tensor(slot_mapping, dtype=torch.int32, device=self.device)
         pos_t = there["pos"] if "pos" in there else torch.as_tensor(position_ids, device=self.device).reshape(-1)
-        cos, sin = self._rope_rows(pos_t)
+        cos, sin = self._rope_rows(pos_t, there["freq"].view(torch.float32))
         h = hidden_states
         normed = None
         for i, layer in enumerate(self.layers):

@@ -258,3 +258,35 @@ def test_host_arrays_and_device_tensors_give_the_same_steps():
             got.append(run.forward(x, lens, t, s, prefill=False))
         outs.append([to_np(o) for o in got])
     assert all(np.array_equal(a, c) for a, c in zip(*outs))
+
+
+def test_first_steps_on_two_streams_equal_the_steps_on_one():
+    """The first step of a fresh runner waits behind other work on its stream while a step on a second stream runs through:
+    both give the bits of the same steps made one after the other, also after rope_theta was changed."""
+    from mindformers_amd.runner import DecodeStackRunner
+    hidden, nh, nkv, d, bs, b = 512, 8, 2, 64, 16, 4
+    layers = _stack(1, hidden, nh, nkv, d, 1024, seed=5)
+    rng = np.random.default_rng(2)
+    xs = [dev(rounded(rng.normal(size=(b, hidden)), BF), BF) for _ in range(2)]
+    lens = rng.integers(bs, 4 * bs, b)
+    tables = [rng.permutation(40)[:b * 4].reshape(b, 4) + 40 * i for i in range(2)]     # blocks of their own
+    slots = [t[np.arange(b), (lens - 1) // bs] * bs + (lens - 1) % bs for t in tables]
+    for theta in (10000.0, 500000.0):
+        ref, got = [], [None, None]
+        run = DecodeStackRunner(layers, npu_mem_size=0.002, cpu_mem_size=0, block_size=bs)
+        run.rope_theta = theta
+        for i in range(2):
+            ref.append(to_np(run.forward(xs[i], lens, tables[i], slots[i], prefill=False)))
+        refs_cache = [c.clone() for c in run.key_cache + run.value_cache]
+        run = DecodeStackRunner(layers, npu_mem_size=0.002, cpu_mem_size=0, block_size=bs)
+        run.rope_theta = theta
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        torch.cuda.synchronize()
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                if i == 0:
+                    torch.cuda._sleep(20_000_000)             # about 10 ms
+                got[i] = run.forward(xs[i], lens, tables[i], slots[i], prefill=False)
+        torch.cuda.synchronize()
+        assert all(np.array_equal(to_np(g), r) for g, r in zip(got, ref))
+        assert all(torch.equal(c, r) for c, r in zip(run.key_cache + run.value_cache, refs_cache))
