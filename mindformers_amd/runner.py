@@ -109,7 +109,7 @@ class DecodeStackRunner:
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("a step's host arrays cannot be captured: a replay would read them from a buffer given back")
         at = np.concatenate([[0], np.cumsum([(a.size + 15) // 16 * 16 for a in arrays])])   # 64-byte pieces
-        host = torch.empty(int(at[-1]), dtype=torch.int32, pin_memory=True)
+        host = torch.empty(int(at[-1]), dtype=torch.int32, pin_memory=True, device="cpu")   # whatever the default device
         flat = host.numpy()
         for a, o in zip(arrays, at):
             flat[o:o + a.size] = a.reshape(-1)

@@ -290,3 +290,24 @@ def test_first_steps_on_two_streams_equal_the_steps_on_one():
         torch.cuda.synchronize()
         assert all(np.array_equal(to_np(g), r) for g, r in zip(got, ref))
         assert all(torch.equal(c, r) for c, r in zip(run.key_cache + run.value_cache, refs_cache))
+
+
+def test_step_under_a_cuda_default_device():
+    """A program that runs with the GPU as torch's default device gets the same step."""
+    from mindformers_amd.runner import DecodeStackRunner
+    bs, b = 16, 3
+    layers = _stack(1, 512, 8, 2, 64, 1024, seed=6)
+    rng = np.random.default_rng(3)
+    x = dev(rounded(rng.normal(size=(b, 512)), BF), BF)
+    tables = np.arange(b * 2).reshape(b, 2)
+    lens = rng.integers(bs, 2 * bs, b)
+    slots = tables[np.arange(b), (lens - 1) // bs] * bs + (lens - 1) % bs
+    outs = []
+    for default in (None, "cuda"):
+        torch.set_default_device(default)
+        try:
+            run = DecodeStackRunner(layers, npu_mem_size=0.002, cpu_mem_size=0, block_size=bs)
+            outs.append(to_np(run.forward(x, lens, tables, slots, prefill=False)))
+        finally:
+            torch.set_default_device(None)
+    assert np.array_equal(*outs)
