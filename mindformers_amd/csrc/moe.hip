@@ -369,14 +369,18 @@ __global__ __launch_bounds__(256) void router_gate_kernel(float* __restrict__ ou
 // The same product for many tokens: a workgroup owns 64 tokens x 64 experts and a slice of H, a wave 32 x 32 of them on the
 // 32 x 32 x 2 instruction.  64 columns of both operands at a time are staged in LDS as fp32 (whole rows of 256 bytes are
 // fetched; the next 64 columns are in registers meanwhile), and lane half h takes columns 32 h .. 32 h + 31 of its row.
-// What bounds it: the fp32 matrix instruction (157 TFLOP/s nominal).  2077 x 256 x 7168: 236 us with operands fetched
-// into registers 16 rows at a time, where every 16 experts fetched the tokens anew, 97 us here;
-// the difference to a float64 product is half of that kernel's (two shorter chains).  Up to 256 tokens the latter is as fast (28 us at
-// 256, both) or faster (18 and 20 us at 128): it slices H further and reads the weight once.
+// What bounds it: the fp32 matrix instruction, half the rate of which is reached: at 2077 x 256 x 7168 (85 TFLOP/s of 157
+// nominal) the matrix pipes are busy 70 % of the time that a compute unit has work and LDS 18 % (no bank conflicts), and a
+// compute unit has work 77 % of the time (924 workgroups on 1024 places).  236 us there with operands fetched into registers 16
+// rows at a time, where every 16 experts fetched the tokens anew, 89 us here.  Rounding: four chains a slice as in that
+// kernel, and as many slices or more: RMS error against float64 2.9e-7 there (7 slices; 7.6e-7 in the kernel above, with one),
+// 7.6e-7 in both at 512 experts and 4200 tokens (one slice); two chains a slice would give 4.1e-7 and 10.7e-7.  Offsets of 32 bits from the tile's
+// rows keep it at 126 registers, four workgroups a compute unit (with three, 2077 x 256 x 7168 takes 102 us).  Up to 256
+// tokens the kernel above is as fast (28 us at 256, both) or faster (18 and 20 us at 128): it slices H further and reads the weight once.
 constexpr int RGT = 64;                                       // tokens, experts and columns of a step
 constexpr int RGT_ROW = RGT + 4;                              // floats of a staged row: 16-byte pieces of 8 rows meet all banks
 template <typename T, typename WT>
-__global__ __launch_bounds__(256) void router_gate_tile_kernel(float* __restrict__ out, float* __restrict__ partial,
+__global__ __launch_bounds__(256, 4) void router_gate_tile_kernel(float* __restrict__ out, float* __restrict__ partial,
                                                                const uint16_t* __restrict__ x, const void* __restrict__ w,
                                                                int tokens, int E, int H, int k_per_split) {
     __shared__ float sw[RGT * RGT_ROW], sx[RGT * RGT_ROW];
@@ -384,27 +388,32 @@ __global__ __launch_bounds__(256) void router_gate_tile_kernel(float* __restrict
     const int r = lane & 31, h = lane >> 5;
     const int e0 = blockIdx.x * RGT, t0 = blockIdx.z * RGT;
     const int k_begin = blockIdx.y * k_per_split, k_end = min(H, k_begin + k_per_split);
-    // load i of a thread: columns 4 c .. 4 c + 3 of row lr + 16 i; rows past the matrix re-read the last one, never stored
+    // load i of a thread: columns 4 c .. 4 c + 3 of row lr + 16 i; rows past the matrix re-read the last one, never stored.
+    // Byte offsets from the tile's first row: 64 rows of an operand are far below 4 GB
+    constexpr uint32_t WB = std::is_same<WT, RG_F32>::value ? 4 : 2;
+    const uint8_t *wt = (const uint8_t*)w + (int64_t)e0 * H * WB, *xt = (const uint8_t*)(x + (int64_t)t0 * H);
     const int lr = threadIdx.x >> 4, lc = 4 * (threadIdx.x & 15);
-    int64_t wrow[4], xrow[4];
+    uint32_t wrow[4], xrow[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        wrow[i] = (int64_t)min(e0 + lr + 16 * i, E - 1) * H;
-        xrow[i] = (int64_t)min(t0 + lr + 16 * i, tokens - 1) * H;
+        wrow[i] = (uint32_t)min(lr + 16 * i, E - 1 - e0) * (uint32_t)H * WB;
+        xrow[i] = (uint32_t)min(lr + 16 * i, tokens - 1 - t0) * (uint32_t)H * 2u;
     }
     f32x4 wr[4], xr[4];
     auto load = [&](int k0) {
         const int k = k0 + lc;
         const bool in = k < k_end;                            // H and the slices are multiples of 4
-        const int kc = in ? k : k_begin;
+        const uint32_t kc = in ? k : k_begin;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            wr[i] = rg_load4<WT>(w, wrow[i] + kc);
-            xr[i] = rg_load4<T>(x, xrow[i] + kc);
+            wr[i] = rg_load4<WT>(wt + (wrow[i] + kc * WB), 0);
+            xr[i] = rg_load4<T>(xt + (xrow[i] + kc * 2u), 0);
             if (!in) wr[i] = xr[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
         }
     };
-    f32x16 acc[2] = {(f32x16)(0.f), (f32x16)(0.f)};          // two shorter chains: a smaller rounding error
+    // four chains a slice, as the four waves of the kernel above make: the rounding error of a sum grows with the length of
+    // its chain, and there is one slice where the tiles alone fill the device
+    f32x16 acc[4] = {(f32x16)(0.f), (f32x16)(0.f), (f32x16)(0.f), (f32x16)(0.f)};
     const float* pw = sw + (32 * (wv & 1) + r) * RGT_ROW + 32 * h;
     const float* px = sx + (32 * (wv >> 1) + r) * RGT_ROW + 32 * h;
     load(k_begin);
@@ -421,10 +430,10 @@ __global__ __launch_bounds__(256) void router_gate_tile_kernel(float* __restrict
         for (int j = 0; j < 8; ++j) {
             const f32x4 a = *(const f32x4*)(pw + 4 * j), b = *(const f32x4*)(px + 4 * j);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], acc[i & 1], 0, 0, 0);
+            for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], acc[i], 0, 0, 0);
         }
     }
-    acc[0] += acc[1];
+    acc[0] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     // lane (r, h) holds token r, experts 8 q + 4 h .. + 3 in elements 4 q .. 4 q + 3
     const int t = t0 + 32 * (wv >> 1) + r;
     if (t >= tokens) return;
@@ -453,7 +462,7 @@ struct GatePlan {
 };
 GatePlan plan_router_gate(int tokens, int E, int H) {
     GatePlan p;
-    p.tile = tokens > RG_TILE_MIN;
+    p.tile = tokens > RG_TILE_MIN && H < (1 << 24);           // 64 rows within 32-bit offsets
     const int te = p.tile ? RGT : 16;
     const int wgs = ((E + te - 1) / te) * ((tokens + 16 * RG_TT - 1) / (16 * RG_TT));
     int s = p.tile ? 1024 / wgs : 512 / wgs;

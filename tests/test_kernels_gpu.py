@@ -1594,6 +1594,28 @@ def test_router_gate_projection_tiles(dtype, t, e, h, wdt):
     test_router_gate_projection(dtype, t, e, h, wdt)
 
 
+@pytest.mark.parametrize("t,e,h", [(4200, 512, 2048), (2100, 256, 256), (1100, 100, 5120)])
+def test_router_gate_tiles_round_no_more_than_four_chains(t, e, h):
+    """RMS error of the tile kernel against float64 (one slice of H, one slice of a short H, several slices): no more than
+    that of a sum in four fp32 chains of a quarter of H each, which is how the kernel for fewer tokens sums a slice.  Two
+    chains would show sqrt(2) of it; 1.15 leaves room for the sample of 48 rows."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(t + e + h)
+    x = torch.randn(t, h, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(e, h, generator=g, device="cuda") * 0.02
+    rows = torch.randperm(t, generator=g, device="cuda")[:48]
+    got = ops.router_gate(x, w)[rows].double().cpu()
+    xs, wd = x[rows].double().cpu(), w.double().cpu()
+    ref = xs @ wd.t()
+    sums = torch.zeros(4, len(rows), e)
+    for j in range(h // 4):                                   # one product of each chain, rounded once
+        for c in range(4):
+            sums[c] = (sums[c].double() + xs[:, 4 * j + c, None] * wd[None, :, 4 * j + c]).float()
+    chains = ((sums[0] + sums[1]) + (sums[2] + sums[3])).double()
+    rms = lambda v: float((v - ref).pow(2).mean().sqrt())
+    assert rms(got) <= 1.15 * rms(chains)
+
+
 @pytest.mark.parametrize("t,e,k,ng,tg", [(128, 256, 8, 8, 4), (16, 8, 2, 2, 2), (33, 64, 6, 8, 3), (5, 16, 4, 1, 1), (7, 96, 3, 4, 1),
                                          (9, 96, 4, 3, 2), (6, 60, 5, 6, 2), (4, 1024, 32, 16, 8), (3, 640, 7, 64, 9)])
 def test_moe_route(t, e, k, ng, tg):
