@@ -302,7 +302,6 @@ __device__ __forceinline__ float rg_round(float v) {
     else return WT::to_float(WT::from_float(v));
 }
 
-constexpr int RG_TILE_MIN = 256;   // more tokens than this: tiles (see there)
 constexpr int RG_TT = 4;                                      // token tiles of 16 per workgroup
 
 template <typename T, typename WT>
@@ -375,8 +374,8 @@ __global__ __launch_bounds__(256) void router_gate_kernel(float* __restrict__ ou
 // rows at a time, where every 16 experts fetched the tokens anew, 89 us here.  Rounding: four chains a slice as in that
 // kernel, and as many slices or more: RMS error against float64 2.9e-7 there (7 slices; 7.6e-7 in the kernel above, with one),
 // 7.6e-7 in both at 512 experts and 4200 tokens (one slice); two chains a slice would give 4.1e-7 and 10.7e-7.  Offsets of 32 bits from the tile's
-// rows keep it at 126 registers, four workgroups a compute unit (with three, 2077 x 256 x 7168 takes 102 us).  Up to 256
-// tokens the kernel above is as fast (28 us at 256, both) or faster (18 and 20 us at 128): it slices H further and reads the weight once.
+// rows keep it at 126 registers, four workgroups a compute unit (with three, 2077 x 256 x 7168 takes 102 us).  When it is
+// taken: plan_router_gate.
 constexpr int RGT = 64;                                       // tokens, experts and columns of a step
 constexpr int RGT_ROW = RGT + 4;                              // floats of a staged row: 16-byte pieces of 8 rows meet all banks
 template <typename T, typename WT>
@@ -462,7 +461,14 @@ struct GatePlan {
 };
 GatePlan plan_router_gate(int tokens, int E, int H) {
     GatePlan p;
-    p.tile = tokens > RG_TILE_MIN && H < (1 << 24);           // 64 rows within 32-bit offsets
+    // Tiles take over where there are enough of them, each with enough of H, to pay for their start and end; experts that fill
+    // less than three quarters of a tile of 64 need twice as many.  Measured on either side of the line, experts x H: tokens,
+    // us without | with tiles: 64 x 2048: 1024 12.5 | 14.4, 2077 21.5 | 18.9; 128 x 2048: 512 12.5 | 14.5,
+    // 1024 18.2 | 15.6; 160 x 5120: 384 22.1 | 22.8, 512 27.6 | 24.8; 256 x 7168: 256 27 | 28, 257 32.4 | 30.8, 2077 237 | 89;
+    // 256 x 256: 1024 5.7 | 10.3, 2077 11.2 | 10.5; 32 x 7168: 2077 29.2 | 33.3, 4200 57.8 | 48.8; 16 x 4096: 8192 28.8 | 45.0.
+    // Up to 256 tokens and with up to 16 experts the others always win: they read the weight once, at most 16 rows in vain.
+    // (H: 64 rows stay within 32-bit offsets.)
+    p.tile = tokens > 256 && E > 16 && H < (1 << 24) && (float)E * tokens > (E < 48 ? 2.f : 1.f) * (48e3f + 120e6f / H);
     const int te = p.tile ? RGT : 16;
     const int wgs = ((E + te - 1) / te) * ((tokens + 16 * RG_TT - 1) / (16 * RG_TT));
     int s = p.tile ? 1024 / wgs : 512 / wgs;

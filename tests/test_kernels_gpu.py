@@ -1594,6 +1594,15 @@ def test_router_gate_projection_tiles(dtype, t, e, h, wdt):
     test_router_gate_projection(dtype, t, e, h, wdt)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("t,e,h,wdt", [(1100, 65, 7172, "fp32"), (2000, 257, 260, "fp32"), (4000, 512, 64, "fp32"), (4100, 129, 324, "same"),
+                                       (3300, 40, 7168, "same")])
+def test_router_gate_projection_tiles_past_the_line(dtype, t, e, h, wdt):
+    """The same bounds at shapes that the tiles serve: ragged rows, experts and columns with and without slices of H, one step
+    of 64 columns, few experts."""
+    test_router_gate_projection(dtype, t, e, h, wdt)
+
+
 @pytest.mark.parametrize("t,e,h", [(4200, 512, 2048), (2100, 256, 256), (1100, 100, 5120)])
 def test_router_gate_tiles_round_no_more_than_four_chains(t, e, h):
     """RMS error of the tile kernel against float64 (one slice of H, one slice of a short H, several slices): no more than
