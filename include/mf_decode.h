@@ -171,6 +171,10 @@ int mf_paged_attention_prefill_int8kv(void* out, const void* query, const void* 
                                       int n_kv_heads, int head_dim, int block_size, int max_blocks_per_seq,
                                       int num_blocks, float scale, int64_t q_row_stride, int dtype,
                                       void* workspace, size_t workspace_bytes, void* stream);
+/* Columns (query row x head of a kv group) per workgroup that the call above takes for these sizes: 16 or 128; max_context =
+ * block_size * max_blocks_per_seq.  Host arithmetic only, for tests and tools. */
+int mf_paged_attention_prefill_int8kv_columns(int batch, int total_q, int n_heads, int n_kv_heads, int head_dim,
+                                              int max_context);
 
 /* int8 KV caches quantised per token (kvcache_quant_granularity per_token,
  * mindformers/utils/quantization_config.py:206-207,296-300: needs an int8 cache): the cache write, and the two

@@ -1,6 +1,6 @@
 // GQA paged attention for gfx950, prefill side (several causal query rows per sequence): the 32-column kernel,
-// its launch rule and entry points.  int8 caches with per-token scales go through the 16-column kernel of
-// paged_attention_kernels.h.
+// its launch rule and entry points.  int8 caches with per-token scales, and few rows over one with per-channel scales, go
+// through the 16-column kernel of paged_attention_kernels.h.
 #include "paged_attention_kernels.h"
 
 namespace {
@@ -552,8 +552,9 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
 
 // ---- prefill --------------------------------------------------------------------------------------------------
 // Partitioning rule shared by the workspace query and the launch.  A workgroup serves 128 (query, head) columns of
-// one kv head (16 with an int8 cache of per-token scales); when the query rows alone give the chip enough workgroups one partition spans the
-// whole context and no partials are written, otherwise the context is cut so that at least 512 workgroups exist.
+// one kv head (16 where pf_cols16 says so and with an int8 cache of per-token scales); when the query rows alone give the chip
+// enough workgroups one partition spans the whole context and no partials are written, otherwise the context is cut so that at
+// least 512 workgroups exist.
 struct PfPlan {
     int part_tokens;
     int max_parts;
@@ -576,6 +577,21 @@ static inline PfPlan pf_plan(int batch, int64_t total_q, int n_heads, int n_kv, 
     p.part_tokens = (int)pt;
     p.max_parts = (int)std::max<int64_t>(1, (max_ctx + pt - 1) / pt);
     return p;
+}
+
+// int8 caches with per-channel scales: the 16-column kernel or the 128-column one.  The 128-column kernel widens a tile for
+// 128 columns at once, but its workgroup walks the partition as one chain of tiles (four waves share them in the other) and a
+// group that one query row fills costs it more.  Measured over 0 to 48 decoding sequences beside a chunk of 0 to 1024 rows,
+// contexts up to 1024, 4096 and 16384, 32/8 and 28/4 heads of 128 and 8/2 of 64, both kernels' times follow 12 us + 8.6 ns
+// and 14 us + 13 ns for every token of a group's context (per compute unit, heads of 128), the latter + 22 ns for every token of a
+// partition; a sequence is taken to fill 0.6 of its table on average, a single one all of it.  The line below is chosen from those times: it
+// loses 0.5 % on average to the better kernel.  8 decoding sequences of up to 4096 tokens without | with a chunk of 64 and of 200
+// rows: 16 columns 21 | 45 and 77 us, 128 columns 40 | 49 and 55 us.
+static inline bool pf_cols16(const PfPlan& p, int batch, int n_kv, int head_dim, int64_t max_ctx) {
+    const float width = head_dim / 128.f;
+    const float per_group = n_kv * (max_ctx / 256.f) * width * (0.6f + 0.4f / batch);
+    return per_group * (p.col_groups16 - 1.4f * p.col_groups128) <=
+           200.f + 1.5f * std::min<int64_t>(p.part_tokens, max_ctx) * width;
 }
 
 // Zero the rows the single-partition prefill path never writes (rows of no sequence): one workgroup per sequence
@@ -611,12 +627,13 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
     if (v_stride <= 0) v_stride = kv_stride;
     const int n_rep = n_heads / n_kv;
     const bool contiguous = block_tables == nullptr;
-    const PfPlan plan = pf_plan(batch, total_q, n_heads, n_kv, contiguous ? total_q : (int64_t)max_blocks * block_size);
+    const int64_t max_ctx = contiguous ? total_q : (int64_t)max_blocks * block_size;
+    const PfPlan plan = pf_plan(batch, total_q, n_heads, n_kv, max_ctx);
     float* part_out = plan.max_parts > 1 ? (float*)workspace : nullptr;
     float* part_ml = part_out ? part_out + (int64_t)total_q * n_heads * plan.max_parts * DV : nullptr;
     const float scale_log2 = scale * 1.4426950408889634f;
-    constexpr bool COLS16 = KVQ == 2;
-    const int64_t wgs = (COLS16 ? plan.col_groups16 : plan.col_groups128) * n_kv * plan.max_parts;
+    const bool cols16 = KVQ == 2 || (KVQ == 1 && pf_cols16(plan, batch, n_kv, D, max_ctx));
+    const int64_t wgs = (cols16 ? plan.col_groups16 : plan.col_groups128) * n_kv * plan.max_parts;
     if (wgs > 0x7fffffffLL) {
         mf_set_error("paged_attention_prefill: %lld workgroups exceed the grid limit", (long long)wgs);
         return 1;
@@ -627,7 +644,7 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
         int rc = MF_LAUNCH_CHECK();
         if (rc) return rc;
     }
-    if constexpr (COLS16) {
+    if constexpr (KVQ != 0) if (cols16) {
         const bool tib = block_size % PA_TILE == 0;           // a 32-token tile never straddles two blocks
 #define PF_LAUNCH(TIBV)                                                                                           \
     hipLaunchKernelGGL((paged_attention_kernel<T, D, 2, true, KVQ, TIBV>), dim3((unsigned)wgs),                    \
@@ -639,7 +656,8 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
         if (tib) PF_LAUNCH(true);
         else PF_LAUNCH(false);
 #undef PF_LAUNCH
-    } else {
+    }
+    if constexpr (KVQ != 2) if (!cols16) {
         const bool tib = contiguous || block_size % PF_TOK == 0;   // a staged tile never straddles two blocks
         static bool lds_set[2][MF_MAX_DEVICES] = {};          // the tile buffers exceed the default dynamic LDS limit
         int dev = 0;
@@ -684,6 +702,13 @@ extern "C" size_t mf_paged_attention_prefill_workspace_bytes(int batch, int tota
     const PfPlan plan = pf_plan(batch, total_q, n_heads, n_kv_heads, max_context);
     if (plan.max_parts <= 1) return 0;
     return (size_t)total_q * n_heads * plan.max_parts * (head_dim + 2) * sizeof(float);
+}
+
+extern "C" int mf_paged_attention_prefill_int8kv_columns(int batch, int total_q, int n_heads, int n_kv_heads, int head_dim,
+                                                         int max_context) {
+    if (batch <= 0 || total_q <= 0 || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads) return 0;
+    const PfPlan plan = pf_plan(batch, total_q, n_heads, n_kv_heads, max_context);
+    return pf_cols16(plan, batch, n_kv_heads, head_dim, max_context) ? 16 : PF_COLS;
 }
 
 static int pa_prefill_entry(void* out, const void* query, const void* key_cache, const void* value_cache,

@@ -728,7 +728,7 @@ def test_paged_prefill_int8kv_vs_oracle():
     (torch.bfloat16, 32, 8, 128, 128, [2200, 2049], [1100, 1030], False),         # many rows: one partition, written at once
 ])
 def test_paged_prefill_int8kv_shapes(dtype, nh, nkv, d, bs, lens, q_lens, with_offset):
-    """The 128-column kernel over an int8 cache, at the bound of the decode side."""
+    """Prefill over an int8 cache (few rows: the 16-column kernel; 2130: the 128-column one), at the bound of the decode side."""
     rng = np.random.default_rng(nh + d + bs)
     lens, q_lens = np.array(lens), np.array(q_lens)
     k8, v8, kf, vf, tables, nb, scale, offset = _kv8_case(rng, dtype, len(lens), nh, nkv, d, bs, lens, with_offset)
@@ -741,6 +741,23 @@ def test_paged_prefill_int8kv_shapes(dtype, nh, nkv, d, bs, lens, q_lens, with_o
     ref = O.paged_attention_prefill(q, kf, vf, tables, lens, q_lens, nh, nkv, sc)
     mag = O.paged_attention_prefill(q, kf, np.abs(vf), tables, lens, q_lens, nh, nkv, sc)
     assert_within(to_np(out), ref, mag, dtype, ulps=3.0, what="prefill over an int8 cache")
+
+
+@pytest.mark.parametrize("dtype,nh,nkv,d,bs,lens,q_lens,with_offset", [
+    (torch.bfloat16, 7, 1, 128, 128, [900, 1, 1640], [433, 1, 319], False),       # 7 heads a kv head, one-row sequences
+    (torch.float16, 8, 4, 64, 16, [895, 464, 31], [595, 432, 1], True),           # blocks that a 32-token tile straddles
+    (torch.bfloat16, 16, 4, 32, 48, [1097, 1290], [665, 701], True),              # likewise, narrow heads
+    (torch.float16, 8, 1, 128, 32, [732, 565], [632, 465], True),                 # a column group of two sequences' ends
+])
+def test_paged_prefill_int8kv_many_rows(dtype, nh, nkv, d, bs, lens, q_lens, with_offset):
+    """Enough rows for the 128-column kernel, at the same bound; the same steps with their rows cut to the last 17 take the
+    16-column one."""
+    cap = (max(lens) + bs - 1) // bs * bs
+    columns = ops._lib.load().mf_paged_attention_prefill_int8kv_columns
+    few = [min(n, 17) for n in q_lens]
+    assert columns(len(lens), sum(q_lens), nh, nkv, d, cap) == 128 and columns(len(lens), sum(few), nh, nkv, d, cap) == 16
+    test_paged_prefill_int8kv_shapes(dtype, nh, nkv, d, bs, lens, q_lens, with_offset)
+    test_paged_prefill_int8kv_shapes(dtype, nh, nkv, d, bs, lens, few, with_offset)
 
 
 def _kv8_token_case(rng, dtype, b, nkv, d, bs, lens, max_blocks=None, poison=True):
