@@ -86,9 +86,10 @@ int launch_pa(void* out, const void* query, const void* key_cache, const void* v
         return MF_LAUNCH_CHECK();
     }
     if (max_parts > 1) {
-        hipLaunchKernelGGL((paged_attention_reduce_kernel<T, D>), dim3(n_heads, batch),
+        hipLaunchKernelGGL((paged_attention_reduce_kernel<T, D, false>), dim3(n_heads, batch),
                            dim3(PA_REDUCE_THREADS<D>), 0, st,
-                           (uint16_t*)out, part_out, part_ml, context_lens, n_heads, max_parts, part_tokens);
+                           (uint16_t*)out, part_out, part_ml, context_lens, n_heads, max_parts, part_tokens,
+                           (const int32_t*)nullptr, batch, false, 0);
         rc = MF_LAUNCH_CHECK();
         if (rc) return rc;
     }

@@ -585,7 +585,7 @@ __device__ inline int pf_row_limit(int row, const int32_t* __restrict__ q_starts
                                    int batch) {
     const int lane = threadIdx.x & 63;
     int lo = -1;                                              // last sequence with q_starts[s] <= row: all lanes call
-    for (int s0 = 0; s0 < batch; s0 += 64) {
+    for (int s0 = 0; s0 < batch && batch > 1; s0 += 64) {     // (one sequence: no read in front of its own)
         const uint64_t m = __ballot(s0 + lane < batch && q_starts[min(s0 + lane, batch - 1)] <= row);
         if (m) lo = s0 + 63 - __builtin_clzll(m);
     }
@@ -599,6 +599,8 @@ __device__ inline int pf_row_limit(int row, const int32_t* __restrict__ q_starts
 // Combine the partitions of one (sequence, head): out = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p.
 // One workgroup of D threads per (head, sequence).  The per-partition (max, sum) pairs are read one per lane
 // and reduced across the wave; the weighted accumulator sum runs 8 independent loads deep.
+// PF: blockIdx.y is a query row; its sequence is found in q_starts and its context is its causal limit.  Rows that
+// belong to no sequence (beyond q_starts[batch], or beyond a sequence's context) are written as zeros.
 // One output element from up to 16 partitions: (max, sum) pairs mv / lv and the partition accumulators pv of its
 // column (entries past the partition count hold PA_NEG, 0, 0 and contribute nothing).
 __device__ __forceinline__ float pa_combine16(const float* mv, const float* lv, const float* pv) {
@@ -621,18 +623,20 @@ __device__ __forceinline__ float pa_combine16(const float* mv, const float* lv, 
 template <int D>
 constexpr int PA_REDUCE_THREADS = D < 64 ? 64 : D;
 
-template <typename T, int D>
+template <typename T, int D, bool PF>
 __global__ __launch_bounds__(PA_REDUCE_THREADS<D>) void paged_attention_reduce_kernel(uint16_t* __restrict__ out,
                                                                   const float* __restrict__ part_out,
                                                                   const float* __restrict__ part_ml,
                                                                   const int32_t* __restrict__ ctx_lens, int n_heads,
-                                                                  int max_parts, int part_tokens) {
+                                                                  int max_parts, int part_tokens,
+                                                                  const int32_t* __restrict__ q_starts, int batch,
+                                                                  bool contiguous, int max_ctx) {
     __shared__ float s_f[64];
-    const int h = blockIdx.x, b = blockIdx.y;
+    const int h = blockIdx.x, b = blockIdx.y;                 // b: sequence (decode) or query row (PF)
     const bool own = (int)threadIdx.x < D;                    // this thread owns an output column
     const int d = own ? threadIdx.x : 0;
     const int lane = threadIdx.x & 63;
-    const int L = ctx_lens[b];
+    const int L = PF ? pf_row_limit(b, q_starts, ctx_lens, contiguous, gridDim.y, max_ctx, batch) : ctx_lens[b];
     const int64_t gh = (int64_t)b * n_heads + h;
     int np = L <= 0 ? 0 : (L + part_tokens - 1) / part_tokens;
     np = np < max_parts ? np : max_parts;
@@ -691,14 +695,13 @@ __global__ __launch_bounds__(PA_REDUCE_THREADS<D>) void paged_attention_reduce_k
     if (own) out[gh * D + d] = T::from_float(num / den);
 }
 
-// The combine of a prefill step: blockIdx.x is a query row, whose context is its causal limit; a thread owns 4 consecutive
-// elements of one head.  Rows that belong to no sequence (beyond q_starts[batch], or beyond a sequence's context) are written
-// as zeros.  What bounds it: with few partitions the latency of the dependent reads (sequence, limits, then all partitions at
-// once), so a workgroup serves 1024 elements and the sequence is found by one read a lane instead of a binary search:
-// 1531 rows of 28 heads, 2 partitions 42 us with a workgroup per (row, head), 12 us here; 1048 rows of 32 heads
-// 36 / 10 us.
+// The combine of a prefill step of many rows and up to NB partitions (launch_pf): blockIdx.x is a query row, whose context is its
+// causal limit; a thread owns 4 consecutive elements of one head.  What bounds it: the latency of the dependent reads
+// (sequence, limits, then all partitions at once), so a workgroup serves 1024 elements and the sequence is found by one read a
+// lane instead of a binary search: 1531 rows of 28 heads, 2 partitions 42 us with a workgroup per (row, head), 12 us here; 1048
+// rows of 32 heads 36 / 10 us.
 constexpr int PF_REDUCE_THREADS = 256;
-template <typename T, int D>
+template <typename T, int D, int NB>
 __global__ __launch_bounds__(PF_REDUCE_THREADS) void prefill_reduce_kernel(
     uint16_t* __restrict__ out, const float* __restrict__ part_out, const float* __restrict__ part_ml,
     const int32_t* __restrict__ ctx_lens, int n_heads, int max_parts, int part_tokens,
@@ -718,34 +721,26 @@ __global__ __launch_bounds__(PF_REDUCE_THREADS) void prefill_reduce_kernel(
     const int64_t gh = (int64_t)row * n_heads + h;
     const float* ml = part_ml + gh * max_parts * 2;
     const float* po = part_out + gh * max_parts * D + (c - h * D);
-    constexpr int NB = 4;                                     // partitions in flight
-    float M = PA_NEG, den = 0.f;
+    float mv[NB], lv[NB];
+    f32x4 pv[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {                            // past the end the last one again, then nothing in its place
+        const int p = min(i, np - 1);
+        mv[i] = ml[2 * p];
+        lv[i] = ml[2 * p + 1];
+        pv[i] = *(const f32x4*)(po + (int64_t)p * D);
+    }
+    float M = mv[0], den = 0.f;
     f32x4 num = {0.f, 0.f, 0.f, 0.f};
-    for (int p0 = 0; p0 < np; p0 += NB) {
-        float mv[NB], lv[NB];
-        f32x4 pv[NB];
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const bool on = p0 + i < np;
-            mv[i] = on ? ml[2 * (p0 + i)] : PA_NEG;
-            lv[i] = on ? ml[2 * (p0 + i) + 1] : 0.f;
-            pv[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
-            if (on) pv[i] = *(const f32x4*)(po + (int64_t)(p0 + i) * D);
-        }
-        float top = M;
+    for (int i = 1; i < NB; ++i) M = fmaxf(M, mv[i]);
 #pragma unroll
-        for (int i = 0; i < NB; ++i) top = fmaxf(top, mv[i]);
-        const float keep = __builtin_amdgcn_exp2f(M - top);   // 1 while the maximum stands
-        M = top;
-        den *= keep;
-        num *= keep;
+    for (int i = 0; i < NB; ++i) {
+        const bool on = i < np;
+        const float f = on ? __builtin_amdgcn_exp2f(mv[i] - M) : 0.f;
+        den = __fmaf_rn(f, on ? lv[i] : 0.f, den);
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const float f = __builtin_amdgcn_exp2f(mv[i] - M);
-            den = __fmaf_rn(f, lv[i], den);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) num[q] = __fmaf_rn(f, pv[i][q], num[q]);
-        }
+        for (int q = 0; q < 4; ++q) num[q] = __fmaf_rn(f, on ? pv[i][q] : 0.f, num[q]);
     }
     *(u32x2*)dst = (u32x2){pack2<T>(__fdiv_rn(num[0], den), __fdiv_rn(num[1], den)),
                            pack2<T>(__fdiv_rn(num[2], den), __fdiv_rn(num[3], den))};

@@ -376,6 +376,21 @@ def test_paged_prefill_many_short_sequences():
     assert_within(got, ref, mag, torch.bfloat16, ulps=1.5, what="paged prefill, 150 sequences")
 
 
+@pytest.mark.parametrize("dtype,nh,nkv,d,lens,q_lens", [
+    (torch.bfloat16, 4, 4, 32, [3000], [520]),                 # 1024 elements a workgroup: 12 partitions in flight
+    (torch.float16, 4, 4, 64, [900, 40, 300], [480, 0, 40]),   # 4 partitions, some rows with one
+    (torch.bfloat16, 12, 4, 128, [600, 300], [300, 50]),       # a row ends inside a workgroup
+    (torch.float16, 8, 2, 64, [9000, 60], [5, 3]),             # a workgroup per (row, head): 36 partitions
+])
+def test_paged_prefill_combine(dtype, nh, nkv, d, lens, q_lens):
+    """The partition combine of prefill steps, for many rows and for few, with rows that belong to no sequence."""
+    rng = np.random.default_rng(sum(lens))
+    got, ref, mag = _prefill_case(rng, dtype, nh, nkv, d, 32, np.asarray(lens), np.asarray(q_lens), pad_rows=5)
+    t = sum(q_lens)
+    assert_within(got[:t], ref, mag, dtype, ulps=1.5, what="prefill combine")
+    assert np.all(got[t:] == 0)
+
+
 def test_paged_prefill_rows_of_no_sequence_are_zero():
     """Rows past q_starts[batch] (padding of a fixed-size launch) come back as zeros, on both the single-partition
     path and the partitioned one; a sequence that claims more queries than context only gets its context's worth."""
