@@ -66,6 +66,15 @@ inline TileGrid tg_plan(int m_blocks, int n_blocks, int steps, const TileCost& c
     return g;
 }
 
+// Grouped rows (experts): rows a group must average for tiles of 256 channels to replace 64-channel workgroups.  `least` is where
+// the two meet when there are tiles enough.  With fewer tiles than compute units and a long K the units without one cost more than
+// the better tiles save, until the 64-channel workgroups need a second pass over the weights.  8 experts of 4096 x 14336 (128
+// tiles), W8A16 us without | with tiles: 16 rows a group 78 | 112, 33: 91 | 123, 48: 101 | 125, 65: 183 | 138; W8A8 20 rows 79 | 98,
+// 48: 101 | 110.  16 experts of 2048 x 1024 (128 tiles too): 16 rows 13.2 | 11.9.
+inline int tg_group_min_rows(int n_experts, int n_blocks, int k, int least) {
+    return k > 2048 && (int64_t)n_experts * n_blocks < 256 ? 64 : least;
+}
+
 // Grouped rows (experts): the row blocks of all experts, in order, times the channel blocks.  Their number is known on the
 // device only (offsets [n_experts + 1]), so the launch covers what the total allows and each workgroup finds its own by a
 // scan of the offsets.  Ids go to the XCDs in turn; XCD j is given the j-th eighth of the row blocks, all channel blocks of

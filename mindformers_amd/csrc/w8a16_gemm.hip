@@ -633,9 +633,13 @@ __global__ __launch_bounds__(256) void w8a16_tile_reduce_kernel(
     out.flush(m0, n0, stage, threadIdx.x, 256);
 }
 
-// Groups that average more rows take w8a16_group_tile_kernel.  256 experts of 4096 x 7168 (gated) / 7168 x 2048, us, passes |
-// tiles: 12 rows a group 1151 + 725 | 1210 + 662, 16: 1196 + 780 | 1216 + 681, 32: 1515 + 941 | 1258 + 731.
-constexpr int GW_GROUP_TILE_ROWS = 12;
+// Groups that average more rows take w8a16_group_tile_kernel (but see tg_group_min_rows).  256 experts of 4096 x 7168 (gated) /
+// 7168 x 2048, us, passes | tiles: 12 rows a group 1151 + 725 | 1210 + 662, 16: 1196 + 780 | 1216 + 681, 32: 1515 + 941 |
+// 1258 + 731: with a long K the passes' loads are the deeper ones (109 experts of 4096 x 7168: 13 rows 497 | 523, 20: 534 | 520; 8 of
+// 28672 x 4096: 13 rows 153 | 162, 20: 173 | 166).
+inline int gw_group_tile_rows(int n_experts, int n, int k) {
+    return tg_group_min_rows(n_experts, (n + tg::BN - 1) / tg::BN, k, k > 2048 ? 20 : 12);
+}
 
 // Grouped (experts): grid = (ceil(N/64), n_experts).  Rows offsets[e] .. offsets[e+1] of x use expert e's
 // packed weights and scale[e]; experts with no rows exit at once.  One pass over the expert's weights serves up to
@@ -1378,7 +1382,8 @@ static int grouped_w8a16_entry(const char* who, void* y, const void* x, const vo
     MF_REQUIRE(!gated || n % 4 == 0, "%s: N (%d) must be a multiple of 4 (gate / up pairs)", who, n);
     MF_REQUIRE((((uintptr_t)x | (uintptr_t)w_packed) & 15) == 0, "%s: x and w_packed must be 16-byte aligned", who);
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
-    if (n % 16 == 0 && k % tg::KSTEP == 0 && total_rows > GW_GROUP_TILE_ROWS * (int64_t)n_experts) {
+    if (n % 16 == 0 && k % tg::KSTEP == 0 &&
+        total_rows > gw_group_tile_rows(n_experts, n, k) * (int64_t)n_experts) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tg::BN - 1) / tg::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;
 #define GGT_LAUNCH(TT)                                                                                            \

@@ -862,7 +862,7 @@ __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
 constexpr int QG_WAVES = 4;
 constexpr int QG_NT = 4;                                      // 16-channel weight tiles per wave and step
 constexpr int QG_BN = 16 * QG_NT;
-// Groups that average more rows take w8a8_group_tile_kernel.  256 experts of 4096 x 7168 / 7168 x 2048, us, passes | tiles:
+// Groups that average more rows take w8a8_group_tile_kernel (but see tg_group_min_rows).  256 experts of 4096 x 7168 / 7168 x 2048, us, passes | tiles:
 // 12 rows a group 1219 + 655 | 1218 + 657, 16: 1236 + 689 | 1222 + 677, 32: 1459 + 856 | 1268 + 726.
 constexpr int QG_TILE_ROWS = 12;
 template <int MTMAX>
@@ -1333,7 +1333,8 @@ extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq,
                "grouped_w8a8_gemm: xq and w_packed must be 16-byte aligned");
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
     dim3 grid((n + QG_BN - 1) / QG_BN, n_experts);
-    if (y && !acc_out && n % 16 == 0 && total_rows > QG_TILE_ROWS * (int64_t)n_experts) {
+    if (y && !acc_out && n % 16 == 0 &&
+        total_rows > tg_group_min_rows(n_experts, (n + tq::BN - 1) / tq::BN, k, QG_TILE_ROWS) * (int64_t)n_experts) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tq::BN - 1) / tq::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;
 #define QGT_LAUNCH(TT)                                                                                           \

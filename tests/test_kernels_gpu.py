@@ -1852,6 +1852,15 @@ def test_grouped_gemms_at_prompt_sizes(counts, n, k, dtype):
     assert torch.equal(fused, ops.silu_mul(y))
 
 
+@pytest.mark.parametrize("counts,n", [
+    ([50, 80, 62], 48), ([65, 64, 66], 48),                     # few tiles: up to 64 rows a group the passes, above it tiles
+    ([20] * 255 + [8], 32), ([21] * 200 + [22] * 56, 32),       # tiles enough: 20 rows (16-bit activations; 12 with int8 ones)
+])
+def test_grouped_gemms_with_a_long_k(counts, n):
+    """The line between the passes and the tiles for a K above 2048, from both sides, at the same bounds."""
+    test_grouped_gemms_at_prompt_sizes(counts, n, 2112, torch.bfloat16)
+
+
 # ------------------------------------------------------------------------------------------- MLA absorbed projections
 @pytest.mark.parametrize("dtype,t,h,k,n,strided", [
     (torch.bfloat16, 64, 128, 128, 512, True),     # query side at DeepSeek-V3 geometry: q_no_pe inside [T, H, 192]
