@@ -343,6 +343,9 @@ size_t mf_w8a16_packed_bytes(int n, int k);
 int mf_w8a16_pack_weight(void* packed, const int8_t* w, int n, int k, void* stream);
 
 size_t mf_w8a16_workspace_bytes(int m, int n, int k);
+/* The kernel that serves an [m, k] x [n, k] product: 0 = passes of up to 64 rows, 1 = 128 x 256 tiles; *whole and *cut = its
+ * output blocks with all of K and those cut into *split parts of it.  Host arithmetic only, for tests and tools. */
+int mf_w8a16_plan(int m, int n, int k, int* whole, int* cut, int* split);
 
 /* golden-stick weight-only cell -> WeightQuantBatchMatmul, replacing P.MatMul(transpose_b=True) at
  *   mindformers/modules/layers.py:479,526; parallel_core/inference/tensor_parallel/layers.py:186,406
@@ -482,6 +485,9 @@ int mf_grouped_silu_mul_dynamic_quant(int8_t* xq, float* x_scale, const void* ga
  * are also written ([M,N] row-major); y may then be NULL.  K % 16 == 0.  workspace: mf_w8a8_workspace_bytes
  * bytes (int32 partial sums when K is split across workgroups; 0 for wide N). */
 size_t mf_w8a8_workspace_bytes(int m, int n, int k);
+/* As mf_w8a16_plan, for tiled activations (x_layout 1) and an output y without accumulators: 0 = LDS-staged, 1 =
+ * register-streaming, 2 = wide, 3 = 128 x 256 tiles; fused: a norm + quantisation or RoPE + cache form. */
+int mf_w8a8_plan(int m, int n, int k, int fused, int* whole, int* cut, int* split);
 int mf_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale, const void* w_packed,
                  const float* w_scale, const void* bias, const void* residual, int m, int n, int k, int dtype,
                  int x_layout, void* workspace, size_t workspace_bytes, void* stream);

@@ -57,6 +57,7 @@ SIGNATURES = {
     "mf_w8a16_packed_bytes": (_Z, [_I, _I]),
     "mf_w8a16_pack_weight": (_I, [_P, _P, _I, _I, _P]),
     "mf_w8a16_workspace_bytes": (_Z, [_I, _I, _I]),
+    "mf_w8a16_plan": (_I, [_I, _I, _I, _P, _P, _P]),
     "mf_w4a16_packed_bytes": (_Z, [_I, _I]),
     "mf_w4a16_pack_weight": (_I, [_P, _P, _I, _I, _P]),
     "mf_w4a16_workspace_bytes": (_Z, [_I, _I, _I, _I]),
@@ -72,6 +73,7 @@ SIGNATURES = {
     "mf_rmsnorm_dynamic_quant": (_I, [_P, _P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _I, _I, _P]),
     "mf_silu_mul_dynamic_quant": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "mf_w8a8_workspace_bytes": (_Z, [_I, _I, _I]),
+    "mf_w8a8_plan": (_I, [_I, _I, _I, _I, _P, _P, _P]),
     "mf_w8a8_gemm": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _Z, _P]),
     "mf_w8a8_gemm_add_rmsnorm_quant": (_I, [_P] * 11 + [_F] + [_I] * 7 + [_P, _Z, _P]),
     "mf_w8a8_qkv_rope_and_cache": (_I, [_P] * 11 + [_I] * 4 + [_L] + [_I] * 4 + [_P, _Z, _P]),

@@ -1216,6 +1216,23 @@ extern "C" size_t mf_w8a16_workspace_bytes(int m, int n, int k) {
     return p.split_k > 1 ? (size_t)p.split_k * m * n * sizeof(float) : 0;
 }
 
+extern "C" int mf_w8a16_plan(int m, int n, int k, int* whole, int* cut, int* split) {
+    if (m <= 0 || n <= 0 || k <= 0 || !whole || !cut || !split) return -1;
+    if (use_tiles(m, n, k)) {
+        float us;
+        const TileGrid g = plan_tiles(m, n, k, &us);
+        *split = g.split;
+        *whole = g.split > 1 ? g.full : g.m_blocks * g.n_blocks;
+        *cut = g.m_blocks * g.n_blocks - *whole;
+        return 1;
+    }
+    const GemmPlan p = plan_w8a16(m, n, k);
+    *split = p.split_k;
+    *whole = p.split_k > 1 ? 0 : p.n_blocks * p.m_blocks;
+    *cut = p.split_k > 1 ? p.n_blocks * p.m_blocks : 0;
+    return 0;
+}
+
 static int w8a16_gemm_entry(const char* who, void* y, const void* x, const void* w_packed, const float* scale,
                             const void* bias, const void* residual, int m, int n, int k, int dtype, int gated,
                             void* workspace, size_t workspace_bytes, void* stream) {

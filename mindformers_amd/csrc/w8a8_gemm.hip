@@ -22,8 +22,9 @@
 // int32 partial tiles that a second kernel sums (integer sums do not depend on the order).
 // More kernels serve the shapes where that one is not the best: from 65 rows on with tiled activations 128 x 256 tiles with
 // the full-rate v_mfma_i32_32x32x32_i8 (w8a8_tile_kernel); where those leave a part of a round over, for narrow outputs and
-// few rows, a register-streaming kernel (w8a8_regs_kernel) and, for very wide outputs at 129 - 256 rows, 256 x 192 tiles on 8
-// waves with a coalesced, LDS-turned epilogue (w8a8_wide_kernel).
+// few rows, a register-streaming kernel (w8a8_regs_kernel) and, for very wide outputs at 129+ rows (also where the tiles cannot
+// serve the call: accumulators asked for, N not a multiple of 16), 256 x 192 tiles on 8 waves with a coalesced, LDS-turned
+// epilogue (w8a8_wide_kernel).
 #include "common.h"
 #include "tile_grid.h"
 #include "w8a8_tile_gemm.h"
@@ -285,7 +286,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(
 // flight per workgroup) and a main loop that is nothing but loads and matrix instructions.
 constexpr int QR_DEPTH = 3;
 
-// ---- wide outputs at 129 - 256 rows: 256 x 192 tiles on 8 waves with mfma_i32_32x32x32_i8 ----------------------------
+// ---- wide outputs at 129+ rows: 256 x 192 tiles on 8 waves with mfma_i32_32x32x32_i8 ----------------------------
 // On gfx950 the 16x16x64 int8 instruction issues at half the rate of the 32x32x32 one (measured: 2.4 against
 // 4.4 POP/s with independent accumulators), so the kernel that is bound by the matrix cores uses the latter.
 // The packed tile format serves it unchanged: rows 32 b .. 32 b + 31 of a k-step are two consecutive 1 KiB
@@ -1069,7 +1070,7 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
         p.nt = n >= 16384 ? 5 : 4;
         // very wide outputs: 256 x 192 tiles on 8 waves, one workgroup per CU (one staged activation tile serves
         // more channels, and the 32 x 32 x 32 instruction runs at twice the rate of the 16 x 16 x 64 one)
-        p.wide = x_tiled && n >= 16384 && m > 128 && m <= 256;
+        p.wide = x_tiled && n >= 16384 && m > 128;
         p.m_blocks = (m + 255) / 256;
     } else {
         p.nt = 2;
@@ -1091,11 +1092,13 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
 }
 
 // Many rows, tiled activations: 128 x 256 tiles against the kernels above.  Measured, a 64-wide step of a round of 256
-// workgroups takes 0.32 us in the register-streaming kernel and 0.78 us in the wide one.  37888 x 3584 at 65 / 257 / 1531 rows
-// runs in 32 / 57 / 250 us on tiles against 49 / 86 / 275 (256 rows: 296 tiles, 40 more than units, 52 us against 48 on 198
-// wide tiles), 28672 x 4096 at 256 rows in 40 against 51, 3584 x 18944 at 1531 rows in 120 against 181, 3584 x 3584 at 448
-// rows in 27 against 20.  `fused`: the sum of the register-streaming kernel's parts carries what follows, which is a kernel of
-// its own behind tiles.
+// workgroups takes 0.32 us in the register-streaming kernel, 0.78 us in the wide one and 0.38 to 0.50 us in the LDS-staged one
+// (one workgroup on a compute unit; it starts and ends like a tile).  37888 x 3584 at 65 / 257 / 1531 rows runs in 32 / 56 / 250 us on tiles against 48 / 85 / 275
+// (256 rows: 296 tiles, 40 more than units, 52 us against 48 on 198 wide tiles), 24576 x 1536 at 257 / 640 rows in 27 / 32
+// against 23 / 42 (wide), 28672 x 4096 at 256 rows in 37 against 47, 8192 x 8192 at 128 / 129 / 257 rows in 32 / 37 / 46 against
+// 34 / 34 / 67 (LDS-staged), 3584 x 18944 at 1531 rows in 120 against 181, 3584 x 3584 at 448 rows in 27 against 20.  `fused`: the
+// sum of the register-streaming and the wide kernel's parts carries what follows, which is a kernel of its own behind tiles (the
+// figures of the LDS-staged kernel have it in).
 constexpr int TQ_MT = 4;
 constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f};
 bool plan_q_tiles(int m, int n, int k, bool fused, TileGrid& g) {
@@ -1103,10 +1106,11 @@ bool plan_q_tiles(int m, int n, int k, bool fused, TileGrid& g) {
     float us;
     g = tg_plan((m + 32 * TQ_MT - 1) / (32 * TQ_MT), (n + tq::BN - 1) / tq::BN, (k + Q_KSTEP - 1) / Q_KSTEP, TQ_COST, &us);
     const QPlan p = plan_w8a8(m, n, k, true);
-    if (!p.regs && !p.wide) return true;                      // the LDS-staged kernel on the half-rate instruction
     const int rounds = (p.n_blocks * p.m_blocks * p.split_k + 255) / 256;
-    const float old = (p.wide ? 0.78f : 0.32f) * rounds * p.steps_per_split + 5.f + (p.split_k > 1 ? TQ_COST.reduce : 0.f);
-    return us + (fused && p.split_k > 1 ? 6.f : 0.f) < old;
+    const bool staged = !p.regs && !p.wide;
+    const float step = p.regs ? 0.32f : p.wide ? 0.78f : 0.45f;
+    const float old = step * rounds * p.steps_per_split + (staged ? TQ_COST.fixed : 5.f) + (p.split_k > 1 ? TQ_COST.reduce : 0.f);
+    return us + (fused && p.split_k > 1 && !staged ? 6.f : 0.f) < old;
 }
 
 template <typename T>
@@ -1233,6 +1237,22 @@ extern "C" size_t mf_w8a8_workspace_bytes(int m, int n, int k) {
         need = b > need ? b : need;
     }
     return need;
+}
+
+extern "C" int mf_w8a8_plan(int m, int n, int k, int fused, int* whole, int* cut, int* split) {
+    if (m <= 0 || n <= 0 || k <= 0 || !whole || !cut || !split) return -1;
+    TileGrid g;
+    if (plan_q_tiles(m, n, k, fused != 0, g)) {
+        *split = g.split;
+        *whole = g.split > 1 ? g.full : g.m_blocks * g.n_blocks;
+        *cut = g.m_blocks * g.n_blocks - *whole;
+        return 3;
+    }
+    const QPlan p = plan_w8a8(m, n, k, true);
+    *split = p.split_k;
+    *whole = p.split_k > 1 ? 0 : p.n_blocks * p.m_blocks;
+    *cut = p.split_k > 1 ? p.n_blocks * p.m_blocks : 0;
+    return p.wide ? 2 : p.regs ? 1 : 0;
 }
 
 extern "C" int mf_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale, const void* w_packed,

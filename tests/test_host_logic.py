@@ -55,6 +55,25 @@ def test_argument_errors_are_reported_without_a_gpu():
         _lib.check(rc, "mf_w8a16_gemm")
 
 
+def _plan(query, *sizes):
+    """(kernel, whole output blocks, blocks cut along K, parts of each) of a host plan query."""
+    out = [ctypes.c_int() for _ in range(3)]
+    return (query(*sizes, *[ctypes.addressof(v) for v in out]), *[v.value for v in out])
+
+
+def test_w8a8_plans_take_the_faster_kernel_at_the_measured_lines():
+    """One round of wide tiles against a round and a part of 128 x 256 ones, the LDS-staged kernel where the tiles leave half the
+    device idle, and the wide kernel above 256 rows where the tiles cannot serve the width."""
+    from mindformers_amd import _lib
+    kind = lambda *a: _plan(_lib.load().mf_w8a8_plan, *a)[0]
+    staged, regs, wide, tiles = range(4)
+    assert [kind(m, 24576, 1536, 0) for m in (200, 257, 512, 640)] == [tiles, wide, wide, tiles]
+    assert [kind(m, 37888, 3584, 0) for m in (128, 256, 257, 1531)] == [tiles, wide, tiles, tiles]
+    assert [kind(m, 8192, 8192, 1) for m in (65, 128, 129, 256, 257)] == [tiles, tiles, staged, staged, tiles]
+    assert [kind(m, 16392, 512, 0) for m in (129, 257, 4000)] == [wide] * 3
+    assert kind(64, 28672, 4096, 0) == staged and kind(448, 3584, 3584, 0) == regs
+
+
 def test_ops_refuse_cpu_tensors():
     from mindformers_amd import ops
     x = torch.zeros(4, 64, dtype=torch.bfloat16)

@@ -1375,6 +1375,14 @@ def test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, bias, residua
     assert bool(((y.double() - ref).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(290, 24192, 1472), (300, 16392, 528)])
+def test_w8a8_wide_kernel_past_256_rows(m, n, k):
+    """Several row blocks of the wide kernel, with and without a ragged last piece of channels, at the same bounds."""
+    out = [torch.zeros(1, dtype=torch.int32) for _ in range(3)]
+    assert ops._lib.load().mf_w8a8_plan(m, n, k, 0, *[o.data_ptr() for o in out]) == 2
+    test_w8a8_many_rows_equal_the_row_major_kernel(torch.bfloat16, m, n, k, False, False)
+
+
 @pytest.mark.parametrize("m,k", [(256, 3584), (37, 1376), (1, 64), (130, 208)])
 def test_dynamic_quant_tiled_layout_bit_exact(m, k):
     """The tiled output holds exactly the row-major result, at the positions the int8 GEMM reads."""
