@@ -58,7 +58,7 @@ __device__ __forceinline__ float dequant_bias(float acc, float scale, const uint
 template <typename T>
 __device__ __forceinline__ void store4(uint16_t* y, const uint16_t* bias, const uint16_t* residual,
                                        const float* scale, int64_t row_off, int n, int N, f32x4 acc) {
-    if (n + 3 < N && ((row_off + n) & 3) == 0) {              // residual and result as one 8-byte access each
+    if (n + 3 < N && ((row_off + n) & 3) == 0 && (((uintptr_t)y | (uintptr_t)residual) & 7) == 0) {   // 8-byte accesses
         u32x2 r = {0u, 0u};
         if (residual) r = *(const u32x2*)(residual + row_off + n);
         float o[4];

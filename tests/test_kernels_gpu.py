@@ -1292,6 +1292,21 @@ def test_column_parallel_linear_reference_vectors(golden_dir):
     assert np.abs(to_np(y) - z["legacy_output_with_bias"]).max() < 2e-4
 
 
+@pytest.mark.parametrize("m,n,k", [(5, 96, 328), (40, 256, 4096), (200, 2112, 4096), (130, 4096, 512)])
+def test_w8a16_gemm_residual_at_any_element(m, n, k):
+    """A residual that begins between 8-byte boundaries (single pass, K cut, several row blocks, tiles): the bits of the same
+    residual at an aligned address."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16)
+    w = ops.pack_w8a16(torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8),
+                       torch.rand(n, generator=g, device="cuda") * 1e-3)
+    buf = torch.randn(m * n + 3, generator=g, device="cuda").to(torch.bfloat16)
+    for at in (1, 2, 3):
+        r = buf[at:at + m * n].view(m, n)
+        assert torch.equal(ops.w8a16_linear(x, w, residual=r), ops.w8a16_linear(x, w, residual=r.clone()))
+
+
 # ------------------------------------------------------------------------------------------- W8A8
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,k,smooth", [(256, 3584, True), (5, 512, False), (64, 18944, True), (1, 64, True)])
