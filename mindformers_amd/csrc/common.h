@@ -188,6 +188,17 @@ __device__ __forceinline__ float block_max(float v, float* red) {
     return t;
 }
 
+// acc * a (* b) (+ bias), every operation rounded by itself: kernels of one projection meet bit for bit whichever of them a shape
+// takes, and left to itself the compiler contracts the last product and the sum in some of the epilogues, or (without a bias)
+// rounds the last product to fp16 at once (v_fma_mixlo_f16)
+__device__ __forceinline__ float scaled_bias(float acc, float a, float b, bool two, float bias, bool with_bias) {
+#pragma clang fp contract(off)
+    float v = acc * a;
+    if (two) v = v * b;
+    if (with_bias) v = v + bias;
+    asm("" : "+v"(v));                                        // a float32 value of its own
+    return v;
+}
 
 // Division by a row's scale.  The grid point that is chosen has to equal the CPU statement's, rint(v / s) with a true IEEE
 // division, at five instructions a value where the compiler's division takes about ten and a quarter-rate reciprocal.

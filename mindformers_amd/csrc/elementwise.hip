@@ -285,17 +285,12 @@ __global__ __launch_bounds__(NORM_THREADS) void rmsnorm_quant_kernel(
                 }
                 const float xs = pr.row_scale[m];
                 const f32x4 w_lo = *(const f32x4*)(pr.col_scale + 8 * c), w_hi = *(const f32x4*)(pr.col_scale + 8 * c + 4);
-                float t[8];
+                float t[8], bb[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                if (pr.bias) unpack8<T>(*(const u32x4*)(pr.bias + 8 * c), bb);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    t[i] = (float)lo[i] * xs * w_lo[i];
-                    t[4 + i] = (float)hi[i] * xs * w_hi[i];
-                }
-                if (pr.bias) {
-                    float bb[8];
-                    unpack8<T>(*(const u32x4*)(pr.bias + 8 * c), bb);
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) t[i] += bb[i];
+                    t[i] = scaled_bias((float)lo[i], xs, w_lo[i], true, bb[i], pr.bias != nullptr);
+                    t[4 + i] = scaled_bias((float)hi[i], xs, w_hi[i], true, bb[4 + i], pr.bias != nullptr);
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) raw[i] = pack2<T>(t[2 * i], t[2 * i + 1]);

@@ -123,18 +123,6 @@ __device__ __forceinline__ bool tg_group_locate(const int32_t* __restrict__ offs
     return false;
 }
 
-// acc * a (* b) (+ bias), every operation rounded by itself: the epilogues of the many-row kernels are straight-line code in
-// which the compiler would contract the last product and the sum, or (without a bias) round the last product to fp16 at once
-// (v_fma_mixlo_f16), and the other kernels' results are to be met bit for bit
-__device__ __forceinline__ float scaled_bias(float acc, float a, float b, bool two, float bias, bool with_bias) {
-#pragma clang fp contract(off)
-    float v = acc * a;
-    if (two) v = v * b;
-    if (with_bias) v = v + bias;
-    asm("" : "+v"(v));                                        // a float32 value of its own
-    return v;
-}
-
 // the lanes of a wave exchange values through LDS: its own instructions stay in order
 __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -450,10 +450,9 @@ __global__ __launch_bounds__(QW::WAVES * 64, 1) void w8a8_wide_kernel(
                     const f32x4 ws4 = *(const f32x4*)(w_scale + nw + nl);
                     float v[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        v[i] = (float)acc[nb][mb][4 * q + i] * xs * ws4[i];
-                        if (bias) v[i] += T::to_float(bias[nw + nl + i]);
-                    }
+                    for (int i = 0; i < 4; ++i)
+                        v[i] = scaled_bias((float)acc[nb][mb][4 * q + i], xs, ws4[i], true,
+                                           bias ? T::to_float(bias[nw + nl + i]) : 0.f, bias != nullptr);
                     *(u32x2*)(ep + (32 * mb + rho) * EP_STRIDE + nl * 2) =
                         (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
                 }
@@ -674,11 +673,8 @@ __device__ __forceinline__ void q_reduce8(const int32_t* __restrict__ p, int64_t
     const f32x4 w_lo = *(const f32x4*)(w_scale + n), w_hi = *(const f32x4*)(w_scale + n + 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        float a = (float)lo[i] * xs * w_lo[i], b = (float)hi[i] * xs * w_hi[i];
-        if (bias) {
-            a += T::to_float(bias[n + i]);
-            b += T::to_float(bias[n + 4 + i]);
-        }
+        const float a = scaled_bias((float)lo[i], xs, w_lo[i], true, bias ? T::to_float(bias[n + i]) : 0.f, bias != nullptr);
+        const float b = scaled_bias((float)hi[i], xs, w_hi[i], true, bias ? T::to_float(bias[n + 4 + i]) : 0.f, bias != nullptr);
         out[i] = T::to_float(T::from_float(a));
         out[4 + i] = T::to_float(T::from_float(b));
     }

@@ -1393,8 +1393,7 @@ def test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, bias, residua
 @pytest.mark.parametrize("m,n,k", [(290, 24192, 1472), (300, 16392, 528)])
 def test_w8a8_wide_kernel_past_256_rows(m, n, k):
     """Several row blocks of the wide kernel, with and without a ragged last piece of channels, at the same bounds."""
-    out = [torch.zeros(1, dtype=torch.int32) for _ in range(3)]
-    assert ops._lib.load().mf_w8a8_plan(m, n, k, 0, *[o.data_ptr() for o in out]) == 2
+    assert _w8a8_plan(m, n, k, False)[0] == "wide"
     test_w8a8_many_rows_equal_the_row_major_kernel(torch.bfloat16, m, n, k, False, False)
 
 
@@ -1608,6 +1607,26 @@ def test_w8a8_qkv_rope_and_cache_equals_unfused(dtype, t, n_head, n_kv, d, k, bi
     ops.rope_and_cache(qkv[:, :nq], qkv[:, nq:nq + nkv], qkv[:, nq + nkv:], cos, sin, kc2, vc2, slots_t, n_head)
     assert torch.equal(q1, qkv[:, :nq])
     assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+
+
+def _w8a8_plan(m, n, k, fused):
+    """(kernel, whole output blocks, blocks cut along K, parts of each) that tiled activations take."""
+    out = [torch.zeros(1, dtype=torch.int32) for _ in range(3)]
+    kind = ops._lib.load().mf_w8a8_plan(m, n, k, int(fused), *[o.data_ptr() for o in out])
+    return (("staged", "regs", "wide", "tiles")[kind], *[int(o) for o in out])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_w8a8_biased_kernels_meet(dtype):
+    """With a bias, whose sum must not be contracted with the last product: the wide kernel against the row-major one, and the
+    fused forms, which run the register-streaming kernel and its partial sums here, against the separate calls, whose
+    projection runs on tiles."""
+    assert _w8a8_plan(200, 16392, 528, False)[0] == "wide"
+    test_w8a8_many_rows_equal_the_row_major_kernel(dtype, 200, 16392, 528, True, True)
+    assert _w8a8_plan(65, 1536, 2560, False)[0] == "tiles" and _w8a8_plan(65, 1536, 2560, True)[0] == "regs"
+    test_w8a8_linear_add_rmsnorm_quant_equals_unfused(dtype, 65, 1536, 2560, True, True, True, True)
+    assert _w8a8_plan(257, 4608, 2048, False)[0] == "tiles" and _w8a8_plan(257, 4608, 2048, True)[0] == "regs"
+    test_w8a8_qkv_rope_and_cache_equals_unfused(dtype, 257, 28, 4, 128, 2048, True, True)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
