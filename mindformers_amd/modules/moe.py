@@ -199,6 +199,15 @@ class QuantGroupedMLP(nn.Module):
 
     construct = forward
 
+    def takes_quantized_rows(self):
+        """Whether the rows may arrive as the integers of ``quantize_tokens``: not where a subclass or an instance brings its own
+        ``forward`` or quantisation (it expects the tokens' type and the three arguments that it names), nor under forward
+        hooks, which are shown the rows."""
+        own = type(self).forward is QuantGroupedMLP.forward and type(self)._quant is QuantGroupedMLP._quant
+        hooks = torch.nn.modules.module
+        return own and "forward" not in self.__dict__ and not (
+            self._forward_hooks or self._forward_pre_hooks or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
+
 
 class SharedExpertMLP(MLP):
     """shared_experts.py:32-75: a gated MLP of width moe_shared_expert_intermediate_size (no output gate)."""
@@ -235,7 +244,8 @@ class MoELayer(nn.Module):
         shape = hidden_states.shape
         x = hidden_states.reshape(-1, self.config.hidden_size).contiguous()
         expert_weight, routing_map = self.router(x)
-        quantized = self.experts.quantize_tokens(x) if isinstance(self.experts, QuantGroupedMLP) else None
+        early = isinstance(self.experts, QuantGroupedMLP) and self.experts.takes_quantized_rows()
+        quantized = self.experts.quantize_tokens(x) if early else None
         if quantized is not None:
             px, ps, row_map, counts, offsets = ops.moe_permute_int8(*quantized, routing_map, self.num_experts)
             y = self.experts(px, counts, offsets=offsets, row_scale=ps, out_dtype=x.dtype)

@@ -1255,3 +1255,38 @@ def test_mla_self_attention_with_quantized_projections():
     net2.is_prefill = False
     with pytest.raises(NotImplementedError):
         net2(x, None, key_cache=cache.clone(), **args)
+
+
+def test_moe_experts_with_a_forward_or_hooks_of_their_own_see_the_tokens_type():
+    """W8A8 experts get rows that are quantised already only where nothing else looks at them: a subclass with the three-argument
+    ``forward``, a replaced ``forward`` and a hooked module get the 16-bit rows, and all give the same bits."""
+    from mindformers_amd.modules import MoELayer, QuantGroupedMLP
+    from mindformers_amd.transformer_config import TransformerConfig
+    cfg = TransformerConfig(num_layers=1, num_attention_heads=8, hidden_size=64, hidden_act="silu", num_moe_experts=8,
+                            moe_router_topk=2, shared_expert_num=0, moe_shared_expert_intermediate_size=None,
+                            moe_ffn_hidden_size=32, moe_router_group_topk=2, moe_router_num_groups=4, add_bias_linear=False,
+                            gated_linear_unit=True, compute_dtype="bfloat16", params_dtype="bfloat16",
+                            moe_router_dtype="bfloat16", moe_router_enable_expert_bias=True,
+                            moe_router_score_function="sigmoid")
+
+    class Experts(QuantGroupedMLP):
+        def forward(self, hidden_states, group_list=None, offsets=None):
+            seen.append(hidden_states.dtype)
+            return super().forward(hidden_states, group_list, offsets)
+
+    torch.manual_seed(7)
+    net = MoELayer(cfg)
+    net.router.weight.data.normal_(0, 0.3)
+    w1, w2 = torch.randn(8, 64, 64, device="cuda") * 0.2, torch.randn(8, 32, 64, device="cuda") * 0.2
+    x, seen = torch.randn(40, 64, device="cuda").to(BF), []
+    net.experts = QuantGroupedMLP(8, cfg, act_quant="per_token").quantize_from_float(w1, w2)
+    ref = net(x)
+    handle = net.experts.register_forward_pre_hook(lambda m, args: seen.append(args[0].dtype))
+    assert torch.equal(net(x), ref)
+    handle.remove()
+    original = net.experts.forward
+    net.experts.forward = lambda h, group_list=None, offsets=None: (seen.append(h.dtype), original(h, group_list, offsets))[1]
+    assert torch.equal(net(x), ref)
+    net.experts = Experts(8, cfg, act_quant="per_token").quantize_from_float(w1, w2)
+    assert torch.equal(net(x), ref)
+    assert seen == [BF] * 3
