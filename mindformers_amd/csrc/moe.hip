@@ -128,23 +128,26 @@ __global__ __launch_bounds__(64) void moe_route_kernel(uint16_t* __restrict__ we
     }
 }
 
-// Stable counting sort of the pairs p = t*k + j by expert; a workgroup of 1024 threads places SORT_CHUNK pairs.  Every
+// Stable counting sort of the pairs p = t*k + j by expert; a workgroup of 1024 threads places SORT_CHUNK pairs (one chunk only: of
+// as many waves as its pairs and the experts take).  Every
 // workgroup counts all the pairs itself (the indices are at most 256 KB, read from the L2), those in front of its chunk apart
 // from the rest, so that no second launch, workspace or order among workgroups is needed: a pair's row is its expert's first
 // row + the expert's pairs in earlier chunks + those of earlier waves of the chunk + those of lower lanes of its wave.
 // What bounds it: the latency of a few dependent passes.  16616 pairs on 256 experts: 129 us in one workgroup that
-// walked the pairs 64 at a time, 8 us here.
+// walked the pairs 64 at a time, 8 us here.  (The scan with a run of experts per lane of one wave: 1.6 us more at 1024 experts.)
 constexpr int SORT_CHUNK = 1024;
 __global__ __launch_bounds__(SORT_CHUNK) void moe_sort_kernel(int32_t* __restrict__ row_map, int64_t* __restrict__ counts,
                                                               int32_t* __restrict__ offsets,
                                                               const int32_t* __restrict__ expert_index, int pairs,
                                                               int E) {
     __shared__ int s_before[RT_MAX_E], s_rest[RT_MAX_E], s_cur[RT_MAX_E];
-    __shared__ uint8_t s_wave[SORT_CHUNK / 64][RT_MAX_E];     // pairs of the wave for the expert: at most 64
+    __shared__ __attribute__((aligned(16))) uint8_t s_wave[SORT_CHUNK / 64][RT_MAX_E];   // pairs of the wave: at most 64
+    __shared__ int s_total[SORT_CHUNK / 64];
+    static_assert(RT_MAX_E <= SORT_CHUNK, "a thread per expert");
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int chunk0 = blockIdx.x * SORT_CHUNK;
-    for (int e = tid; e < E; e += SORT_CHUNK) s_before[e] = s_rest[e] = 0;
-    for (int i = tid; i < (int)sizeof(s_wave) / 16; i += SORT_CHUNK) ((u32x4*)s_wave)[i] = (u32x4){0u, 0u, 0u, 0u};
+    if (tid < E) s_before[tid] = s_rest[tid] = 0;
+    for (int i = tid; i < (int)blockDim.x / 64 * RT_MAX_E / 16; i += blockDim.x) ((u32x4*)s_wave)[i] = (u32x4){0u, 0u, 0u, 0u};
     __syncthreads();
     const int p = chunk0 + tid;
     int e = p < pairs ? expert_index[p] : -1;
@@ -170,32 +173,27 @@ __global__ __launch_bounds__(SORT_CHUNK) void moe_sort_kernel(int32_t* __restric
     const int rank = __popcll(same & ((1ull << lane) - 1ull));
     if (e >= 0 && rank == 0) s_wave[wv][e] = (uint8_t)__popcll(same);
     __syncthreads();
-    if (wv == 0) {                                            // exclusive scan: a run of experts per lane of wave 0
-        const int per = (E + 63) / 64;
-        const int e0 = lane * per;
-        int local = 0;
-        for (int i = 0; i < per; ++i)
-            if (e0 + i < E) local += s_before[e0 + i] + s_rest[e0 + i];
-        int incl = local;
+    {                                                         // exclusive scan: an expert per thread
+        const int before = tid < E ? s_before[tid] : 0, c = tid < E ? before + s_rest[tid] : 0;
+        int run = c;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            const int up = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += up;
+            const int up = __shfl_up(run, o, 64);
+            if (lane >= o) run += up;
         }
-        int run = incl - local;
-        for (int i = 0; i < per; ++i) {
-            const int x = e0 + i;
-            if (x < E) {
-                const int c = s_before[x] + s_rest[x];
-                s_cur[x] = run + s_before[x];
-                if (blockIdx.x == 0) {
-                    offsets[x] = run;
-                    counts[x] = c;
-                }
-                run += c;
+        if (lane == 63) s_total[wv] = run;
+        __syncthreads();
+        run -= c;
+#pragma unroll
+        for (int w = 0; w < SORT_CHUNK / 64; ++w) run += w < wv ? s_total[w] : 0;
+        if (tid < E) {
+            s_cur[tid] = run + before;
+            if (blockIdx.x == 0) {
+                offsets[tid] = run;
+                counts[tid] = c;
+                if (tid == E - 1) offsets[E] = run + c;
             }
         }
-        if (blockIdx.x == 0 && lane == 63) offsets[E] = incl;
     }
     __syncthreads();
     if (p >= pairs) return;
@@ -483,7 +481,9 @@ int permute(uint16_t* permuted, float* permuted_scale, int32_t* row_map, int64_t
             const float* x_scale, const int32_t* expert_index, int tokens, int k, int n_experts, int hidden,
             hipStream_t stream) {
     const int pairs = tokens * k, chunks = pairs > SORT_CHUNK ? (pairs + SORT_CHUNK - 1) / SORT_CHUNK : 1;
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(chunks), dim3(SORT_CHUNK), 0, stream, row_map, counts, offsets, expert_index,
+    // one chunk: fewer waves meet at the barriers sooner (1 token on 8 experts: 5.4 us with the gather in 16 waves, 4.7 in one)
+    const int most = pairs > n_experts ? pairs : n_experts, threads = most < SORT_CHUNK ? (most + 63) / 64 * 64 : SORT_CHUNK;
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(chunks), dim3(threads), 0, stream, row_map, counts, offsets, expert_index,
                        pairs, n_experts);
     int rc = MF_LAUNCH_CHECK();
     if (rc || pairs == 0) return rc;

@@ -1775,6 +1775,12 @@ def test_moe_permute_int8_rows(t, h, e, k):
     assert np.array_equal(ps.cpu().numpy()[:order.size], xs[order // k])
 
 
+@pytest.mark.parametrize("t,e,k", [(13, 8, 5), (3, 65, 4), (16, 64, 4), (127, 960, 8), (128, 961, 8)])
+def test_moe_permute_int8_rows_of_one_chunk(t, e, k):
+    """One chunk in as many waves as its pairs or the experts take, on both sides of a wave's edge."""
+    test_moe_permute_int8_rows(t, 16, e, k)
+
+
 def test_moe_permute_grouped_unpermute():
     rng = np.random.default_rng(14)
     dtype = torch.bfloat16
