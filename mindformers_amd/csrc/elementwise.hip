@@ -29,7 +29,7 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // behind branches) | as here: SiLU * up + quantise 1531 x 18944 54.5 | 45.3 us, 16616 x 2048 60.7 | 48.3, quantise
 // 2077 x 7168 29.9 | 16.0, 1531 x 3584 10.5 | 8.0, norm + quantise 1531 x 3584 14.4 | 13.1, norm 4137 x 4096 18.4 | 15.7.
 // One branch on the type in front of all the loads: behind a branch each, the later pieces would wait for the row (norm +
-// quantise, 1 x 7168: 5.0 us there, 4.5 here).
+// quantise, 1 x 4096: 4.3 us there, 4.1 here).
 template <int NV>
 __device__ __forceinline__ void load_gamma(const void* __restrict__ gamma, int dtype, int nvec, float (*gm)[8]) {
     auto piece = [&](int it) { return 8 * min((int)threadIdx.x + it * NORM_THREADS, nvec - 1); };

@@ -201,15 +201,13 @@ class MLASelfAttention(nn.Module):
             t = q.shape[0]
             kv = self.linear_kv_up_proj(kv_c).reshape(t, -1)
             k_no_pe = kv[:, : n * nope].reshape(t, n, nope)
-            value = kv[:, n * nope:].reshape(t, n, vd)
-            k_rep = k_pe[:, None, :].expand(t, n, rope)
+            val = kv[:, n * nope:]
+            k_rep = k_pe.unsqueeze(1).expand(t, n, rope)
             key = torch.cat((k_no_pe, k_rep), dim=-1).reshape(t, n * self.q_head_dim)
-            if self.q_head_dim == 192 and vd == 128:
-                # the attention takes the 128-wide values as they are (the reference pads them to the key width with
-                # the rotary part and keeps the first 128 output columns: the same numbers)
-                val = value.reshape(t, n * vd)
-            else:
-                val = torch.cat((value, k_rep), dim=-1)
+            # 128-wide values under 192-wide keys: the attention takes them as they are (the reference pads them to the key
+            # width with the rotary part and keeps the first 128 output columns: the same numbers)
+            if self.q_head_dim != 192 or vd != 128:
+                val = torch.cat((val.reshape(t, n, vd), k_rep), dim=-1)
                 if vd + rope != self.q_head_dim:
                     val = torch.nn.functional.pad(val, (0, self.q_head_dim - vd - rope))
                 val = val.reshape(t, n * self.q_head_dim)

@@ -466,9 +466,13 @@ def q_starts_from_actual_seq_len(actual_seq_len, total_rows):
     per-sequence lengths (infer_attention.py:459-461, run_infer_flash_attention.py:110,137-142).  The two readings
     never disagree when both are valid (then all entries but the last are zero), so the list is taken as ends when
     it is non-decreasing and ends at T, and as lengths otherwise.  Decided on the device: no host synchronisation."""
-    a = torch.as_tensor(actual_seq_len).reshape(-1).to(torch.int64)
+    a = torch.as_tensor(actual_seq_len).reshape(-1)
+    if a.dtype not in (torch.int32, torch.int64):
+        a = a.to(torch.int64)
     is_ends = (a[-1] == total_rows) & torch.all(a[1:] >= a[:-1])
-    return q_starts_from_ends(torch.where(is_ends, a, torch.cumsum(a, 0)))
+    starts = torch.zeros(a.numel() + 1, dtype=torch.int32, device=a.device)
+    starts[1:].copy_(torch.where(is_ends, a, torch.cumsum(a, 0)))              # the sums of int32 values are int64
+    return starts
 
 
 def q_starts_from_lens(q_seq_lens):
