@@ -84,6 +84,12 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     int64_t v_stride, const float* __restrict__ kv_scale, const float* __restrict__ kv_offset) {
     using vec8 = typename T::vec8;
     using S = PfSmem<D>;
+    // Type of the probabilities and of the widened values in the PV product.  int8 values are exact in either type and fp16 rounds
+    // the probabilities eight times finer than bf16, in the same time.  RMS error against float64, bf16, 512 rows over 4096 tokens,
+    // 32/8 heads of 128: 2.68e-3 in the 16-column kernel, which serves the same caches, 2.85e-3 here with bf16 probabilities
+    // (whose reference point, see below, leaves more of them to round), 2.33e-3 with fp16 ones.
+    using PT = std::conditional_t<KVQ == 1, FP16, T>;
+    using pvec8 = typename PT::vec8;
     static_assert(KVQ == 0 || (KVQ == 1 && DV == D && S::W1 == 0), "int8 caches: per-channel scales, power-of-two heads");
     static_assert(DV == D || DV == S::W0, "value heads as wide as the key heads, or as their first sub-tile");
     constexpr int KS = D / 16;                                // k-steps of the score product
@@ -326,7 +332,7 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
         for (int i = 0; i < 2; ++i) {
             const int c = 2 * pc + i;
             *(vec8*)(kdst + 16 * (c ^ key)) = dequant8<T>(kraw[2 * i], kraw[2 * i + 1]);
-            *(vec8*)(vdst + 16 * ((c + 4 * key4) & (S0::CPR - 1))) = dequant8<T>(vraw[2 * i], vraw[2 * i + 1]);
+            *(pvec8*)(vdst + 16 * ((c + 4 * key4) & (S0::CPR - 1))) = dequant8<PT>(vraw[2 * i], vraw[2 * i + 1]);
         }
     };
 
@@ -361,8 +367,14 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     // m_run follows the running maximum lazily: it moves only when the maximum exceeds it by more than 2^8 in
     // probability (moving it means rescaling the accumulators); probabilities then lie in (0, 256], which bf16 and
     // fp16 hold with the same relative precision, and the result does not depend on the reference point.
+    // fp16 over int8 caches: the reference point is each tile's own maximum (but no more than 2^32 in probability under the largest
+    // seen).  The token at the reference point has probability 1, which needs no rounding, and the 16-column kernel has more such
+    // tokens than a lazy or a running maximum would give here (four waves with a maximum each): RMS error as above 3.37e-4 there,
+    // 3.52e-4 lazily, 3.45e-4 with the running maximum, 3.27e-4 here, for 2 % (1024 tokens) to 10 % (16384) of the time.
     float m_run = 0.5f * PA_NEG, l_run = 0.f;
-    const float lazy = 8.0f / scale_log2;
+    [[maybe_unused]] float m_peak = m_run;
+    constexpr bool TILE_REF = KVQ == 1 && std::is_same<T, FP16>::value;
+    const float lazy = (TILE_REF ? 32.0f : 8.0f) / scale_log2;
 
     // One tile, living in ring buffer R = t mod 3 (a compile-time constant of the step): scores, softmax, PV product,
     // one phase after the other.  A wave does not overlap its own MFMAs with its own vector instructions, so nothing
@@ -410,7 +422,13 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
 #pragma unroll
         for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, sc[i]);
         tmax = max_xor32(tmax);
-        const float m_new = tmax > m_run + lazy ? tmax : m_run;
+        float m_new;
+        if constexpr (TILE_REF) {
+            m_peak = fmaxf(m_peak, tmax);
+            m_new = fmaxf(tmax, m_peak - lazy);
+        } else {
+            m_new = tmax > m_run + lazy ? tmax : m_run;
+        }
         if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {      // the reference point moves: rare
             const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2);
             l_run *= alpha;
@@ -425,11 +443,11 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
         for (int k = 0; k < 8; ++k) {
             const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[2 * k], scale_log2, nm));
             const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[2 * k + 1], scale_log2, nm));
-            pp[k] = pack2<T>(p0, p1);
-            l_run = T::sum2(pp[k], l_run);
+            pp[k] = pack2<PT>(p0, p1);
+            l_run = PT::sum2(pp[k], l_run);
         }
-        const vec8 pf0 = bitcast<vec8>((u32x4){pp[0], pp[1], pp[2], pp[3]});
-        const vec8 pf1 = bitcast<vec8>((u32x4){pp[4], pp[5], pp[6], pp[7]});
+        const pvec8 pf0 = bitcast<pvec8>((u32x4){pp[0], pp[1], pp[2], pp[3]});
+        const pvec8 pf1 = bitcast<pvec8>((u32x4){pp[4], pp[5], pp[6], pp[7]});
 
         // ---- O^T[d, col] += V^T[d, token] . P^T[token, col]: MFMA v = DB th + db (token half th, d block db), two
         // transposing reads each
@@ -451,7 +469,7 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
                 constexpr int th = v / DB, db = v % DB;
                 constexpr int left = NV - 1 - v;
                 wait_lds_reads<2 * (left < P - 1 ? left : P - 1)>();
-                acc[db] = T::mfma32(bitcast<vec8>((u32x4){lo[v % P][0], lo[v % P][1], hi[v % P][0], hi[v % P][1]}),
+                acc[db] = PT::mfma32(bitcast<pvec8>((u32x4){lo[v % P][0], lo[v % P][1], hi[v % P][0], hi[v % P][1]}),
                                     th ? pf1 : pf0, acc[db]);
                 __builtin_amdgcn_sched_barrier(0);
                 fetch(std::integral_constant<int, v + P>{});
@@ -582,16 +600,16 @@ static inline PfPlan pf_plan(int batch, int64_t total_q, int n_heads, int n_kv, 
 // int8 caches with per-channel scales: the 16-column kernel or the 128-column one.  The 128-column kernel widens a tile for
 // 128 columns at once, but its workgroup walks the partition as one chain of tiles (four waves share them in the other) and a
 // group that one query row fills costs it more.  Measured over 0 to 48 decoding sequences beside a chunk of 0 to 1024 rows,
-// contexts up to 1024, 4096 and 16384, 32/8 and 28/4 heads of 128 and 8/2 of 64, both kernels' times follow 12 us + 8.6 ns
-// and 14 us + 13 ns for every token of a group's context (per compute unit, heads of 128), the latter + 22 ns for every token of a
-// partition; a sequence is taken to fill 0.6 of its table on average, a single one all of it.  The line below is chosen from those times: it
-// loses 0.5 % on average to the better kernel.  8 decoding sequences of up to 4096 tokens without | with a chunk of 64 and of 200
-// rows: 16 columns 21 | 45 and 77 us, 128 columns 40 | 49 and 55 us.
+// contexts up to 1024, 4096 and 16384, 32/8 and 28/4 heads of 128 and 8/2 of 64, the kernels' times follow 12 us + 8.6 ns
+// and 14 us + 13 ns for every token of a group's context (per compute unit, heads of 128), the latter + 23 ns for every token of
+// a partition; a sequence is taken to fill 0.6 of its table on average, a single one all of it.  The constants are those of
+// the line that loses least to the better kernel over all of them (0.6 % on average).  8 decoding sequences of up to 4096 tokens
+// without | with a chunk of 64 and of 200 rows: 16 columns 21 | 45 and 77 us, 128 columns 40 | 51 and 57 us.
 static inline bool pf_cols16(const PfPlan& p, int batch, int n_kv, int head_dim, int64_t max_ctx) {
     const float width = head_dim / 128.f;
     const float per_group = n_kv * (max_ctx / 256.f) * width * (0.6f + 0.4f / batch);
-    return per_group * (p.col_groups16 - 1.4f * p.col_groups128) <=
-           200.f + 1.5f * std::min<int64_t>(p.part_tokens, max_ctx) * width;
+    return per_group * (p.col_groups16 - 2.f * p.col_groups128) <=
+           200.f + std::min<int64_t>(p.part_tokens, max_ctx) * width;
 }
 
 // Zero the rows the single-partition prefill path never writes (rows of no sequence): one workgroup per sequence
