@@ -61,6 +61,22 @@ def _plan(query, *sizes):
     return (query(*sizes, *[ctypes.addressof(v) for v in out]), *[v.value for v in out])
 
 
+def test_plans_of_the_shapes_that_the_tile_kernels_are_tested_at():
+    """The GPU tests of the many-row GEMMs name the plan that each shape stands for: (whole tiles, cut tiles, parts of each)."""
+    from mindformers_amd import _lib
+    lib, tiles8, tiles16 = _lib.load(), 3, 1
+    for (m, n, k), plan in {(129, 8208, 208): (66, 0, 1), (65, 16384, 4160): (64, 0, 1), (513, 3584, 9472): (0, 70, 2),
+                            (1100, 9216, 1088): (324, 0, 1), (2100, 8448, 320): (561, 0, 1), (1300, 6144, 1600): (256, 8, 4),
+                            (1675, 9232, 1600): (512, 6, 4)}.items():
+        assert _plan(lib.mf_w8a8_plan, m, n, k, 0) == (tiles8, *plan), (m, n, k)
+    for (m, n, k), plan in {(1300, 6144, 1600): (256, 8, 4), (257, 4608, 9472): (0, 54, 4)}.items():      # fused forms
+        assert _plan(lib.mf_w8a8_plan, m, n, k, 1) == (tiles8, *plan), (m, n, k)
+    for (m, n, k), plan in {(513, 8208, 704): (165, 0, 1), (129, 28672, 4096): (224, 0, 1), (65, 12304, 8192): (0, 49, 4),
+                            (1100, 2064, 4096): (0, 81, 2), (1285, 6160, 1024): (256, 19, 4),
+                            (2305, 4096, 4160): (256, 48, 4)}.items():
+        assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, *plan), (m, n, k)
+
+
 def test_w8a8_plans_take_the_faster_kernel_at_the_measured_lines():
     """One round of wide tiles against a round and a part of 128 x 256 ones, the LDS-staged kernel where the tiles leave half the
     device idle, and the wide kernel above 256 rows where the tiles cannot serve the width."""

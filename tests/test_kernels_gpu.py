@@ -1148,7 +1148,8 @@ def test_w8a16_qkv_rope_and_quant_cache_equals_unfused(dtype, t, n_head, n_kv, d
     (513, 8208, 704, True, True),          # one row and one 16-channel piece past whole tiles, an odd number of k-steps
     (129, 28672, 4096, False, False),      # whole channel blocks, no cut along K
     (65, 12304, 8192, True, False),        # every tile cut along K
-    (1100, 2064, 4096, False, True),       # whole tiles and cut ones
+    (1100, 2064, 4096, False, True),       # every tile cut in two
+    (1285, 6160, 1024, False, True),       # a round of whole tiles and 19 cut in four
     (2305, 4096, 4160, True, True)])       # a full round, the tiles left over in parts of unequal length
 def test_w8a16_many_rows(dtype, m, n, k, bias, residual):
     """The tile kernel against float64 on the device.  Both roundings (the projection, then the sum with the residual) are
@@ -1328,6 +1329,14 @@ def test_w8a16_gemm_residual_at_any_element(m, n, k):
         assert torch.equal(ops.w8a16_linear(x, w, residual=r), ops.w8a16_linear(x, w, residual=r.clone()))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_w8a16_fused_forms_behind_cut_tiles(dtype):
+    """What follows a projection in the same call where its tiles are partly (256 whole, 19 cut in four) or all cut along K."""
+    test_w8a16_linear_add_rmsnorm_equals_unfused(dtype, 1285, 6160, 1024, True)
+    test_w8a16_linear_rmsnorm_leading_equals_unfused(dtype, 1100, 2064, 4096, 1536, False)
+    test_w8a16_qkv_rope_and_cache_equals_unfused(dtype, 1285, 40, 4, 128, 1024, True)
+
+
 # ------------------------------------------------------------------------------------------- W8A8
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,k,smooth", [(256, 3584, True), (5, 512, False), (64, 18944, True), (1, 64, True)])
@@ -1385,8 +1394,10 @@ def test_w8a8_gemm_int32_bit_exact(m, n, k):
     (129, 8208, 208, True, True),          # one row and one 16-channel piece past whole tiles, a short last k-step
     (65, 16384, 4160, False, False),       # one row block, an odd number of k-steps
     (513, 3584, 9472, True, True),         # every tile cut along K
-    (1100, 9216, 1088, True, False),       # whole tiles and cut ones
-    (2100, 4608, 320, False, True)])       # more than a round of whole tiles, few k-steps
+    (1100, 9216, 1088, True, False),       # a round of whole tiles and a part of one, none cut
+    (2100, 8448, 320, False, True),        # two rounds of whole tiles and a part of one, few k-steps
+    (1300, 6144, 1600, True, False),       # a round of whole tiles and eight cut in four
+    (1675, 9232, 1600, True, True)])       # two rounds and six cut in four, a ragged last channel block
 def test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, bias, residual):
     """The tile kernel (tiled activations) gives the bits of the row-major kernel on the same integers, whose int32
     accumulators are exact; the dequantisation against float64: three roundings to fp32, one to the output type and one of
@@ -1635,6 +1646,14 @@ def _w8a8_plan(m, n, k, fused):
     out = [torch.zeros(1, dtype=torch.int32) for _ in range(3)]
     kind = ops._lib.load().mf_w8a8_plan(m, n, k, int(fused), *[o.data_ptr() for o in out])
     return (("staged", "regs", "wide", "tiles")[kind], *[int(o) for o in out])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_w8a8_fused_forms_behind_cut_tiles(dtype):
+    """The norm + quantisation and the RoPE + cache scatter that follow a projection whose tiles are partly or all cut along K."""
+    test_w8a8_linear_add_rmsnorm_quant_equals_unfused(dtype, 1300, 6144, 1600, True, True, True, True)
+    test_w8a8_linear_add_rmsnorm_quant_equals_unfused(dtype, 257, 4608, 9472, False, True, True, True)
+    test_w8a8_qkv_rope_and_cache_equals_unfused(dtype, 1300, 40, 4, 128, 1600, True, True)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
