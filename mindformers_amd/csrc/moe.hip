@@ -369,14 +369,14 @@ __global__ __launch_bounds__(256) void router_gate_kernel(float* __restrict__ ou
 // What bounds it: the fp32 matrix instruction, half the rate of which is reached: at 2077 x 256 x 7168 (85 TFLOP/s of 157
 // nominal) the matrix pipes are busy 70 % of the time that a compute unit has work and LDS 18 % (no bank conflicts), and a
 // compute unit has work 77 % of the time (924 workgroups on 1024 places).  236 us there with operands fetched into registers 16
-// rows at a time, where every 16 experts fetched the tokens anew, 89 us here.  Rounding: four chains a slice as in that
-// kernel, and as many slices or more: RMS error against float64 2.9e-7 there (7 slices; 7.6e-7 in the kernel above, with one),
-// 7.6e-7 in both at 512 experts and 4200 tokens (one slice); two chains a slice would give 4.1e-7 and 10.7e-7.  Offsets of 32 bits from the tile's
-// rows keep it at 126 registers, four workgroups a compute unit (with three, 2077 x 256 x 7168 takes 102 us).  When it is
-// taken: plan_router_gate.
+// rows at a time, where every 16 experts fetched the tokens anew, 89 us here.  Rounding: CHAINS fp32 chains a slice, four as in that
+// kernel, or two where there are slices enough to have as many chains in all (plan_router_gate): RMS error against float64 7.6e-7 in
+// the kernel above and 4.1e-7 here at 2077 x 256 x 7168 (1 and 7 slices), 7.6e-7 in both at 512 experts and 4200 tokens (one slice;
+// two chains would give 10.7e-7).  Offsets of 32 bits from the tile's rows keep it at four workgroups a compute unit (with three,
+// 2077 x 256 x 7168 takes 102 us).
 constexpr int RGT = 64;                                       // tokens, experts and columns of a step
 constexpr int RGT_ROW = RGT + 4;                              // floats of a staged row: 16-byte pieces of 8 rows meet all banks
-template <typename T, typename WT>
+template <typename T, typename WT, int CHAINS>
 __global__ __launch_bounds__(256, 4) void router_gate_tile_kernel(float* __restrict__ out, float* __restrict__ partial,
                                                                const uint16_t* __restrict__ x, const void* __restrict__ w,
                                                                int tokens, int E, int H, int k_per_split) {
@@ -408,9 +408,9 @@ __global__ __launch_bounds__(256, 4) void router_gate_tile_kernel(float* __restr
             if (!in) wr[i] = xr[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
         }
     };
-    // four chains a slice, as the four waves of the kernel above make: the rounding error of a sum grows with the length of
-    // its chain, and there is one slice where the tiles alone fill the device
-    f32x16 acc[4] = {(f32x16)(0.f), (f32x16)(0.f), (f32x16)(0.f), (f32x16)(0.f)};
+    f32x16 acc[CHAINS];
+#pragma unroll
+    for (int i = 0; i < CHAINS; ++i) acc[i] = (f32x16)(0.f);
     const float* pw = sw + (32 * (wv & 1) + r) * RGT_ROW + 32 * h;
     const float* px = sx + (32 * (wv >> 1) + r) * RGT_ROW + 32 * h;
     load(k_begin);
@@ -427,10 +427,11 @@ __global__ __launch_bounds__(256, 4) void router_gate_tile_kernel(float* __restr
         for (int j = 0; j < 8; ++j) {
             const f32x4 a = *(const f32x4*)(pw + 4 * j), b = *(const f32x4*)(px + 4 * j);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], acc[i], 0, 0, 0);
+            for (int i = 0; i < 4; ++i) acc[i % CHAINS] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], acc[i % CHAINS], 0, 0, 0);
         }
     }
-    acc[0] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    acc[0] += acc[1];
+    if constexpr (CHAINS == 4) acc[0] = acc[0] + (acc[2] + acc[3]);
     // lane (r, h) holds token r, experts 8 q + 4 h .. + 3 in elements 4 q .. 4 q + 3
     const int t = t0 + 32 * (wv >> 1) + r;
     if (t >= tokens) return;
@@ -455,10 +456,20 @@ __global__ void router_gate_reduce_kernel(float* __restrict__ out, const float* 
 }
 
 struct GatePlan {
-    int tile, splits, k_per_split;
+    int tile, chains, splits, k_per_split;                    // chains: of a tile's slice
 };
+// slices of H for workgroups of te experts x 64 tokens, `target` of them wanted
+GatePlan slice_router_gate(int tokens, int E, int H, int te, int target) {
+    GatePlan p = {te == RGT, 4, 1, H};
+    const int wgs = ((E + te - 1) / te) * ((tokens + 16 * RG_TT - 1) / (16 * RG_TT));
+    int s = target / wgs;
+    const int max_s = H / 256 < 1 ? 1 : H / 256;              // at least one chunk per wave, or four steps of a tile
+    s = s < 1 ? 1 : (s > max_s ? max_s : s);
+    p.k_per_split = ((H + s - 1) / s + 63) / 64 * 64;
+    p.splits = (H + p.k_per_split - 1) / p.k_per_split;
+    return p;
+}
 GatePlan plan_router_gate(int tokens, int E, int H) {
-    GatePlan p;
     // Tiles take over where there are enough of them, each with enough of H, to pay for their start and end; experts that fill
     // less than three quarters of a tile of 64 need twice as many.  Measured on either side of the line, experts x H: tokens,
     // us without | with tiles: 64 x 2048: 1024 12.5 | 14.4, 2077 21.5 | 18.9; 128 x 2048: 512 12.5 | 14.5,
@@ -466,14 +477,10 @@ GatePlan plan_router_gate(int tokens, int E, int H) {
     // 256 x 256: 1024 5.7 | 10.3, 2077 11.2 | 10.5; 32 x 7168: 2077 29.2 | 33.3, 4200 57.8 | 48.8; 16 x 4096: 8192 28.8 | 45.0.
     // Up to 256 tokens and with up to 16 experts the others always win: they read the weight once, at most 16 rows in vain.
     // (H: 64 rows stay within 32-bit offsets.)
-    p.tile = tokens > 256 && E > 16 && H < (1 << 24) && (float)E * tokens > (E < 48 ? 2.f : 1.f) * (48e3f + 120e6f / H);
-    const int te = p.tile ? RGT : 16;
-    const int wgs = ((E + te - 1) / te) * ((tokens + 16 * RG_TT - 1) / (16 * RG_TT));
-    int s = p.tile ? 1024 / wgs : 512 / wgs;
-    const int max_s = H / 256 < 1 ? 1 : H / 256;              // at least one chunk per wave, or four steps of a tile
-    s = s < 1 ? 1 : (s > max_s ? max_s : s);
-    p.k_per_split = ((H + s - 1) / s + 63) / 64 * 64;
-    p.splits = (H + p.k_per_split - 1) / p.k_per_split;
+    const GatePlan few = slice_router_gate(tokens, E, H, 16, 512);
+    if (tokens <= 256 || E <= 16 || H >= (1 << 24) || (float)E * tokens <= (E < 48 ? 2.f : 1.f) * (48e3f + 120e6f / H)) return few;
+    GatePlan p = slice_router_gate(tokens, E, H, RGT, 1024);
+    p.chains = 2 * p.splits >= 4 * few.splits ? 2 : 4;        // never fewer chains in all than the kernel for fewer tokens makes
     return p;
 }
 
@@ -543,9 +550,10 @@ extern "C" int mf_router_gate_gemm(float* logits, const void* x, const void* w, 
     const dim3 rgrid((unsigned)((n + 255) / 256));
 #define RG_LAUNCH(TT_, WT_)                                                                                      \
     {                                                                                                            \
-        hipLaunchKernelGGL((p.tile ? router_gate_tile_kernel<TT_, WT_> : router_gate_kernel<TT_, WT_>), grid, dim3(256), 0, \
-                           (hipStream_t)stream, logits, partial, (const uint16_t*)x, w, tokens, n_experts, hidden,   \
-                           p.k_per_split);                                                                       \
+        auto kern = !p.tile ? router_gate_kernel<TT_, WT_>                                                       \
+                    : p.chains == 2 ? router_gate_tile_kernel<TT_, WT_, 2> : router_gate_tile_kernel<TT_, WT_, 4>; \
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, logits, partial, (const uint16_t*)x, w, tokens, \
+                           n_experts, hidden, p.k_per_split);                                                    \
         if (partial) {                                                                                           \
             int rc = MF_LAUNCH_CHECK();                                                                          \
             if (rc) return rc;                                                                                   \

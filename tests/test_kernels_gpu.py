@@ -1717,10 +1717,10 @@ def test_router_gate_projection_tiles_past_the_line(dtype, t, e, h, wdt):
     test_router_gate_projection(dtype, t, e, h, wdt)
 
 
-@pytest.mark.parametrize("t,e,h", [(4200, 512, 2048), (2100, 256, 256), (1100, 100, 5120)])
+@pytest.mark.parametrize("t,e,h", [(4200, 512, 2048), (2100, 256, 256), (1100, 100, 5120), (2100, 256, 512)])
 def test_router_gate_tiles_round_no_more_than_four_chains(t, e, h):
-    """RMS error of the tile kernel against float64 (one slice of H, one slice of a short H, several slices): no more than
-    that of a sum in four fp32 chains of a quarter of H each, which is how the kernel for fewer tokens sums a slice.  Two
+    """RMS error of the tile kernel against float64 (one slice of H, one slice of a short H, several slices, two of a short H):
+    no more than that of a sum in four fp32 chains of a quarter of H each, which is how the kernel for fewer tokens sums a slice.  Two
     chains would show sqrt(2) of it; 1.15 leaves room for the sample of 48 rows."""
     g = torch.Generator(device="cuda")
     g.manual_seed(t + e + h)
