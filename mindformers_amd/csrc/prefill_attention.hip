@@ -32,7 +32,7 @@ namespace {
 // one tile ahead into registers and writes them, widened to T (exactly), to the same places of the ring; the matrix
 // path is the same.  The key scale is folded into the query, the key offset drops out of the softmax, value scale and
 // offset are applied once to the (accumulator, sum) pair.  Two 512-row chunks beside 24 decoding sequences of 512 to 4096
-// tokens (32 heads on 8): 235 us on the 16-column kernel, which widens a tile for 16 columns, 140 us here.
+// tokens (32 heads on 8): 235 us on the 16-column kernel, which widens a tile for 16 columns, 140 us here (few rows: pf_cols16).
 // A wave owns its columns over the whole partition, so there is no merge: it writes final rows (single partition) or
 // fp32 partials for the reduce kernel.
 constexpr int PF_COLS = 128;                                  // columns per workgroup
@@ -72,6 +72,7 @@ struct PfSmem {
 };
 
 // Three workgroups per compute unit; two at 192-wide heads (72 KB of LDS and 96 accumulator registers each).
+// (int8 caches at heads of 128: the tile in registers takes them past 168, and 144 bytes a lane are spilled.)
 // DV: width of a value head and of an output head.  DV < D (the prefill of multi-latent attention: 192-wide queries
 // and keys, 128-wide values, packed rows only) loads and multiplies the first sub-tile of the value rows only.
 template <typename T, int D, bool TIB, int DV = D, int KVQ = 0>

@@ -681,6 +681,8 @@ __global__ __launch_bounds__(GW_WAVES * 64, 2) void w8a16_grouped_kernel(
 // expert's rows end), the row blocks of all experts dealt to the XCDs as tg_group_locate says.  Bound by the stream of the
 // expert weights: 256 experts of 65 rows, 4096 x 7168 (gated): 2644 us in passes of 64 rows, 1439 here (5.2 TB/s of weights);
 // 7168 x 2048: 1564 / 804.
+// The four tile heights share 256 registers and spill 16 (68 bytes of scratch a lane), nearly all at the start and the end of a
+// workgroup; one pair is reloaded inside a k-loop.
 template <typename T, int MT>
 __device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* xe, const uint8_t* we, const float* se, int rows,
                                                  int m0, int nb, int N, int K, int gated, int aligned, uint8_t* smem) {
@@ -1063,7 +1065,10 @@ GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
 
 // Tiles against passes of 64 rows of the skinny kernel (more than 64 rows, K of whole steps, N of whole 16-byte pieces, gated
 // too).  Measured, a k-step of a round of 256 skinny workgroups takes 0.40 us: 28672 x 4096 at 65 / 256 / 4137 rows runs in
-// 41 / 65 / 787 us on tiles against 51 / 103 / 1447 us, 4096 x 4096 at 128 / 256 / 700 rows in 18 / 26 / 48 against 17 / 20 / 47.
+// 41 / 65 / 787 us on tiles against 51 / 103 / 1447 us, 4096 x 4096 at 128 / 256 / 700 rows in 18 / 26 / 48 against 17 / 20 / 47,
+// 7168 x 16384 at 112 / 129 / 256 rows in 40 / 64 / 67 against 51 / 78 / 88 (168 skinny workgroups there at 129 rows).  The line is
+// the same whatever follows in the call: the fused forms have the bits of the separate calls, and sums of two kernels differ; with
+// the norm behind it, 7168 x 16384 at 129 rows takes 68 against 82 us.
 bool use_tiles(int m, int n, int k) {
     if (m <= 64 || k % tg::KSTEP != 0 || n % 16 != 0) return false;
     float us;

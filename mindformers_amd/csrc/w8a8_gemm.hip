@@ -978,6 +978,7 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
 // (each fetching the rows anew, a second pass for every second expert), 1435 here (5.2 TB/s of weights); 7168 x 2048: 1280 / 817.
 // With 128-row tiles for every expert of more than 64 rows the padding's matrix instructions counted: the two GEMMs of 256
 // experts of 65 rows on average 2323 us, 2167 with tiles of 96 rows for those up to 96.
+// The three tile heights share 256 registers and spill 46 (188 bytes of scratch a lane), outside the k-loops.
 template <typename T, int MT>
 __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, const float* xs, const uint8_t* we,
                                                 const float* ws, int rows, int m0, int nb, int N, int K, int aligned,
