@@ -59,6 +59,9 @@ struct BF16 {
     static __device__ __forceinline__ void mfma32_acc(f32x16& c, vec8 a, vec8 b) {
         asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     }
+    static __device__ __forceinline__ void mfma16_acc(f32x4& c, vec8 a, vec8 b) {
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
     // likewise with the accumulator in ordinary registers: c = a b, then c += a b
     static __device__ __forceinline__ void mfma32_first(f32x16& c, vec8 a, vec8 b) {
         asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
@@ -91,6 +94,9 @@ struct FP16 {
     }
     static __device__ __forceinline__ void mfma32_acc(f32x16& c, vec8 a, vec8 b) {
         asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
+    static __device__ __forceinline__ void mfma16_acc(f32x4& c, vec8 a, vec8 b) {
+        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     }
     static __device__ __forceinline__ void mfma32_first(f32x16& c, vec8 a, vec8 b) {
         asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
@@ -330,6 +336,13 @@ __device__ __forceinline__ f16x8 dequant8<FP16>(uint32_t lo, uint32_t hi) {
         v[4 + i] = (_Float16)(float)(int)(int8_t)(hi >> (8 * i));
     }
     return v;
+}
+
+// bytes shift / 8 and shift / 8 + 1 of w as a pair of T, exact
+template <typename T>
+__device__ __forceinline__ uint32_t i8x2_to(uint32_t w, int shift) {
+    if constexpr (std::is_same_v<T, BF16>) return i8x2_to_bf16x2(w, shift);
+    else return bitcast<uint32_t>(__builtin_amdgcn_cvt_pkrtz((float)(int)(int8_t)(w >> shift), (float)(int)(int8_t)(w >> (shift + 8))));
 }
 
 // 8 unsigned nibbles holding q + 8 (q in -8 .. 7; nibble i = element i) -> 8 elements of T, exact.

@@ -97,6 +97,7 @@ __device__ __forceinline__ bool tg_group_locate(const int32_t* __restrict__ offs
     for (int e = lane; e < n_experts; e += 64) total += (span(e, r0) + TG_GROUP_ROWS - 1) / TG_GROUP_ROWS;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+    total = __builtin_amdgcn_readfirstlane(total);
     const int id = blockIdx.x, per_xcd = (total + 7) / 8, at = (id >> 3) / n_blocks;
     nb = (id >> 3) - at * n_blocks;
     int want = (id & 7) * per_xcd + at;
@@ -121,6 +122,17 @@ __device__ __forceinline__ bool tg_group_locate(const int32_t* __restrict__ offs
         want -= __builtin_amdgcn_readfirstlane(__shfl(upto, 63, 64));
     }
     return false;
+}
+
+// 16 bytes at an address that is the same in every lane plus the lane's 32-bit offset: the address stays in scalar registers
+template <bool NT = false>
+__device__ __forceinline__ u32x4 load16_at(const uint8_t* base, uint32_t offset) {
+    typedef const __attribute__((address_space(1))) uint8_t* gptr;
+    gptr p = (gptr)base;
+    asm("" : "+s"(p), "+v"(offset));
+    const auto at = (const __attribute__((address_space(1))) u32x4*)(p + offset);
+    if constexpr (NT) return __builtin_nontemporal_load(at);
+    else return *at;
 }
 
 // the lanes of a wave exchange values through LDS: its own instructions stay in order

@@ -528,18 +528,18 @@ struct TileOut {
     const uint16_t *bias, *residual;
     int M, N, gated, aligned;
 
-    // scale and bias of channels 8q + 4h .. + 3 of 32-channel block nt
-    __device__ __forceinline__ void load(const float* scale, int n0, int nt, int q, f32x4& sc, f32x4& bi) const {
-        const int n = min(n0 + 32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1), N - 4);
+    // scale and bias of the lane's four channels of 16-channel tile nt
+    __device__ __forceinline__ void load(const float* scale, int n0, int nt, f32x4& sc, f32x4& bi) const {
+        const int n = min(n0 + 16 * nt + 4 * ((threadIdx.x >> 4) & 3), N - 4);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             sc[i] = scale[n + i];
             bi[i] = bias ? T::to_float(bias[n + i]) : 0.f;
         }
     }
-    // these channels of a row into the stage
-    __device__ __forceinline__ void put(f32x4 v, f32x4 sc, f32x4 bi, int nt, int q, uint8_t* stage) const {
-        const int r = threadIdx.x & 31, c = 32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1);
+    // these channels of the lane's row of 16-row tile j into the stage
+    __device__ __forceinline__ void put(f32x4 v, f32x4 sc, f32x4 bi, int j, int nt, uint8_t* stage) const {
+        const int r = 16 * j + (threadIdx.x & 15), c = 16 * nt + 4 * ((threadIdx.x >> 4) & 3);
         float o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = scaled_bias(v[i], sc[i], 1.f, false, bi[i], bias != nullptr);
@@ -573,32 +573,29 @@ __global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
     const bool whole = blockIdx.x < g.full || g.split == 1;
     const int KS = K / tg::KSTEP, s0 = part * g.steps_per_split;
     const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = mb * 32 * MT, n0 = nb * tg::BN + 64 * wv;
     float* pt = partial + (int64_t)slot * (32 * MT * tg::BN) + (wv * MT * 8 * 64 + lane) * 4;
     const TileOut<T> out{y, bias, residual, M, N, gated, aligned};
-    f32x4 sc[8], bi[8];
+    f32x4 sc[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TileOut<T>::ROW;
-    tg::tile<T, MT>(x, wp, M, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const f32x16 (&acc)[2]) {
+    tg::tile<T, MT, 0, false>(x, wp, M, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const f32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
         if (whole) {
             if (mt == 0) {
                 __syncthreads();                              // every wave has read its last operands
 #pragma unroll
-                for (int e = 0; e < 8; ++e) out.load(scale, n0, e >> 2, e & 3, sc[e], bi[e]);
+                for (int nt = 0; nt < 4; ++nt) out.load(scale, n0, nt, sc[nt], bi[nt]);
             }
             wave_lds_order();
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                out.put((f32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
-                                acc[e >> 2][4 * (e & 3) + 3]}, sc[e], bi[e], e >> 2, e & 3, stage);
+                out.put(acc[e >> 2][e & 3], sc[e & 3], bi[e & 3], e >> 2, e & 3, stage);
             wave_lds_order();
             out.flush(m0 + 32 * mt, n0, stage, lane, 64);
         } else {                                              // accumulator order: whole cache lines
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                *(f32x4*)(pt + (mt * 8 + e) * 256) = (f32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1],
-                                                             acc[e >> 2][4 * (e & 3) + 2], acc[e >> 2][4 * (e & 3) + 3]};
+            for (int e = 0; e < 8; ++e) *(f32x4*)(pt + (mt * 8 + e) * 256) = acc[e >> 2][e & 3];
         }
     });
 }
@@ -622,7 +619,7 @@ __global__ __launch_bounds__(256) void w8a16_tile_reduce_kernel(
     const TileOut<T> out{y, bias, residual, M, N, gated, aligned};
     f32x4 sc[2], bi[2], v[2] = {(f32x4)(0.f), (f32x4)(0.f)};
 #pragma unroll
-    for (int e = 0; e < 2; ++e) out.load(scale, n0, (e0 + e) >> 2, (e0 + e) & 3, sc[e], bi[e]);
+    for (int e = 0; e < 2; ++e) out.load(scale, n0, (e0 + e) & 3, sc[e], bi[e]);
 #pragma unroll 8
     for (int s = 0; s < g.split; ++s)
 #pragma unroll
@@ -681,29 +678,30 @@ __global__ __launch_bounds__(GW_WAVES * 64, 2) void w8a16_grouped_kernel(
 // expert's rows end), the row blocks of all experts dealt to the XCDs as tg_group_locate says.  Bound by the stream of the
 // expert weights: 256 experts of 65 rows, 4096 x 7168 (gated): 2644 us in passes of 64 rows, 1439 here (5.2 TB/s of weights);
 // 7168 x 2048: 1564 / 804.
-// The four tile heights share 256 registers and spill 16 (68 bytes of scratch a lane), nearly all at the start and the end of a
-// workgroup; one pair is reloaded inside a k-loop.
-template <typename T, int MT>
+// Weights of an expert with one block of up to 64 rows are read past the caches, where they would push out the rows that all
+// channel blocks read: 109 experts of 4096 x 7168 at 33 rows 551 us cached, 511 so, 8 of 28672 x 4096 at 33 rows 178 / 163; blocks of
+// more rows gain nothing (7168 x 2048 at 65 rows 679 / 704), and an expert's further blocks share the weights through L2 (200 rows:
+// 1257 / 1420).  Up to 16 bytes of scratch a lane, outside the k-loops.
+template <typename T, int MT, bool NT>
 __device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* xe, const uint8_t* we, const float* se, int rows,
                                                  int m0, int nb, int N, int K, int gated, int aligned, uint8_t* smem) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = nb * tg::BN + 64 * wv;
     const TileOut<T> out{y, nullptr, nullptr, rows, N, gated, aligned};
-    f32x4 sc[8], bi[8];
+    f32x4 sc[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TileOut<T>::ROW;
-    tg::tile<T, MT>(xe, we, rows, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, 0, K / tg::KSTEP, smem,
-                    [&](auto mtc, const f32x16 (&acc)[2]) {
+    tg::tile<T, MT, MT == 4 ? 2 : MT == 3 ? 0 : 2 * MT, NT>(xe, we, rows, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, 0, K / tg::KSTEP, smem,
+                    [&](auto mtc, const f32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
         if (mt == 0) {
             __syncthreads();                                  // every wave has read its last operands
 #pragma unroll
-            for (int e = 0; e < 8; ++e) out.load(se, n0, e >> 2, e & 3, sc[e], bi[e]);
+            for (int nt = 0; nt < 4; ++nt) out.load(se, n0, nt, sc[nt], bi[nt]);
         }
         wave_lds_order();
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-            out.put((f32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
-                            acc[e >> 2][4 * (e & 3) + 3]}, sc[e], bi[e], e >> 2, e & 3, stage);
+            out.put(acc[e >> 2][e & 3], sc[e & 3], bi[e & 3], e >> 2, e & 3, stage);
         wave_lds_order();
         out.flush(m0 + 32 * mt, n0, stage, lane, 64);
     });
@@ -723,10 +721,19 @@ __global__ __launch_bounds__(256, 2) void w8a16_group_tile_kernel(
     const uint8_t* we = wp + (int64_t)e * expert_bytes;
     const float* se = scale + (int64_t)e * N;
     const int left = rows - m0;
-    if (left <= 32) w8a16_group_tile<T, 1>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
-    else if (left <= 64) w8a16_group_tile<T, 2>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
-    else if (left <= 96) w8a16_group_tile<T, 3>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
-    else w8a16_group_tile<T, 4>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem);
+#define GT(MT, NT) w8a16_group_tile<T, MT, NT>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem)
+    if (left <= 32) {
+        if (m0 == 0) GT(1, true);                             // nobody else reads these weights
+        else GT(1, false);
+    } else if (left <= 64) {
+        if (m0 == 0) GT(2, true);
+        else GT(2, false);
+    } else if (left <= 96) {
+        GT(3, false);
+    } else {
+        GT(4, false);
+    }
+#undef GT
 }
 
 template <typename T>
@@ -1032,7 +1039,7 @@ struct GemmPlan {
 // Tile plan of the many-row kernel (4137 x 4096 x 14336: 16 of 528 tiles left over by whole rounds, 531 us uncut, 423 us in
 // 8 parts).
 constexpr int TG_MT = 4;
-constexpr TileCost TG_COST = {0.75f, 1.72f, 6.f, 5.f, 0.065f};
+constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f};
 TileGrid plan_tiles(int m, int n, int k, float* us) {
     return tg_plan((m + 32 * TG_MT - 1) / (32 * TG_MT), (n + tg::BN - 1) / tg::BN, k / tg::KSTEP, TG_COST, us);
 }

@@ -1,38 +1,48 @@
 // W8A16 GEMM for many rows (prompts, chunked prefill): the matrix cores are the bound, not the weights.
 #pragma once
 #include "common.h"
+#include "tile_grid.h"
 
 // A workgroup of 4 waves (one per SIMD, two workgroups per compute unit) owns 32*MT rows x 256 channels; wave w owns channels
 // 64w .. 64w + 63 of all the rows, so that every weight byte of the tile is loaded and converted by exactly one wave and goes
 // from global memory straight into matrix operand registers, while the activation tile of a 64-wide k-step is staged in LDS
-// once and read by all four.  Both operands are fetched two steps ahead by ordinary loads (the compiler counts them), the
-// activations are written to the other of two LDS stages one step ahead, and the operands of a 16-wide sub-step are read and
-// converted behind the matrix instructions of the one before (one instruction group per matrix instruction, pinned by
-// scheduling groups); one barrier per step, in front of the last sub-step, whose operands are in registers by then.
+// once and read by all four.  Weights are fetched two steps ahead by ordinary loads (the compiler counts them); the activations of a
+// step are written to the other of two LDS stages one step ahead.  A step is eight groups, (32 columns, 16 channels) each over all
+// the rows: a group's 2*MT matrix instructions share one weight operand, and behind each of them goes a piece of what is needed
+// next (the conversion of the next group's weights, a row tile of the next 32 columns, a load), in the order written here; one
+// barrier per step, in front of the groups that begin to read the next one.
 //
-// What bounds it: the power budget.  At 4096 x 4096 x 16384 the matrix pipes are busy 72 % of the cycles and the clock stands
-// at 1.6 GHz (2.4 GHz with the conversions, loads and LDS traffic taken out), 1250 TFLOP/s; the library's bf16 GEMM draws the
-// clock down to 1.5 GHz at 86 % (1362).  With MT = 8 (256 rows, one workgroup per unit) half the conversions and weight loads
-// fall away, but nothing overlaps the start and the end of a tile: 1167 TFLOP/s there and 848 against 1100 at K = 4096.
-// 4137 x 28672 x 4096: 1447 us in passes of 64 rows, 787 us here; 4137 x 4096 x 14336: 632 / 383 us.
+// v_mfma_f32_16x16x32: with all operands in registers and two waves a SIMD, 16x16x32 does 2007 TFLOP/s on random data and 2437 on
+// zeros, 32x32x16 1818 and 2484: both fill the matrix pipe, and the smaller one, which reads and writes half the accumulators per
+// operation, leaves the power budget more clock.  The accumulators are held in the accumulation registers by the statements that
+// name them: left to the compiler 32 accumulators of four registers wander through the file and spill.
+//
+// What bounds it: the power budget.  4137 x 28672 x 4096: 782-797 us on 32x32x16, 714-724 here (1360 TFLOP/s); 4137 x 4096 x 14336:
+// 398 / 359; 2025 x 7168 x 16384: 424 / 360.  A lone workgroup on a compute unit (few tiles) is bound by issue: one wave starts a
+// vector instruction every 8 cycles, and a step has 96 beside 64 matrix instructions of 16 (0.7 to 0.9 us a step, two workgroups
+// together 1.55).
 namespace tg {
 
 constexpr int WAVES = 4;
 constexpr int BN = 64 * WAVES;                                // channels per workgroup
 constexpr int KSTEP = 64;
-
+constexpr int DW = 2;                                         // steps of weights in flight
+template <int MT>
+constexpr int DX = MT == 4 ? 1 : 2;                           // steps of activations in flight
 // physical 16-byte chunk of chunk c of a staged activation row (128 bytes): the lanes that share an LDS cycle are those
-// of one half-wave with equal parity of lane bits 2-4; bits 1, 3 and 4 of the row tell the eight rows of equal bit 0
-// among them apart, so the 32-row operand reads and the writes are free of bank conflicts
-__device__ __forceinline__ int key(int row) { return ((row >> 1) & 1) | (((row >> 3) & 3) << 1); }
+// of one half-wave with equal parity of lane bits 2-4.  An operand read has row bits 0-3 in lane bits 0-3 and chunk bit 1 in lane
+// bit 4, a write has the chunk in bits 0-2 and row bits 0-1 above; with this key the sixteen lanes of a cycle meet the sixteen
+// chunks of two rows in both
+__device__ __forceinline__ int key(int row) { return ((row >> 1) & 1) | (((row >> 3) & 1) << 2); }
 
-template <typename T, int MT, typename Epilogue>
+// EARLY: 16-row tiles of a sub-step that are read behind the third channel tile of the one before; the others follow behind the
+// fourth, each into the registers of a tile that has just been used (0: half and half).  NT: weights that nobody else reads (non-temporal loads)
+template <typename T, int MT, int EARLY, bool NT, typename Epilogue>
 __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, int M, int K, int m0,
                                      int tile0, int n_tiles, int s_begin, int s_end, uint8_t* smem, Epilogue&& epilogue) {
     using vec8 = typename T::vec8;
     constexpr int STAGE = 32 * MT * 128;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int h = lane >> 5, r32 = lane & 31;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int s_last = s_end - 1;
 
     // ---- activations: load i of a thread is chunk (t & 7) of row 32i + (t >> 3)
@@ -41,133 +51,109 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
     uint32_t xoff[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) xoff[i] = (uint32_t)min(32 * i + xr, M - 1 - m0) * (uint32_t)K * 2u + 16u * xc;
-    const uint32_t xdst = xr * 128 + ((xc ^ key(xr)) << 4);   // + 4096 per i (the key has no bit above 4)
-    u32x4 xreg[2][MT];
-    auto load_x = [&](auto setc, int s) {
-        const uint32_t k = (uint32_t)min(s, s_last) * (KSTEP * 2);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) xreg[decltype(setc)::value][i] = *(const u32x4*)(xbase + (xoff[i] + k));
+    const uint32_t xdst = xr * 128 + ((xc ^ key(xr)) << 4);   // + 4096 per i (the key has no bit above 3)
+    u32x4 xreg[DX<MT>][MT];
+    auto load_x = [&](auto setc, auto ic, int s) {
+        constexpr int i = decltype(ic)::value;
+        xreg[decltype(setc)::value][i] = load16_at(xbase + (uint32_t)min(s, s_last) * (KSTEP * 2), xoff[i]);
     };
-    auto write_x = [&](auto setc, int stage) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i) *(u32x4*)(smem + stage * STAGE + 4096 * i + xdst) = xreg[decltype(setc)::value][i];
+    auto write_x = [&](auto setc, auto ic, int stage) {
+        constexpr int i = decltype(ic)::value;
+        *(u32x4*)(smem + stage * STAGE + 4096 * i + xdst) = xreg[decltype(setc)::value][i];
     };
-    // ---- weights: of every 32-channel block (two packed tiles) and 64-wide step lane (r, h) holds chunks h and h + 2 of
-    // its channel: columns 16h .. and 32 + 16h ..
-    const uint8_t* wbase[2];
+    // ---- weights: lane (r, g) of a packed 16-channel tile holds columns 16g .. 16g + 15 of channel r
+    const uint8_t* wbase[4];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-        const int t = min(tile0 + 4 * wv + 2 * nt + ((lane >> 4) & 1), n_tiles - 1);
-        wbase[nt] = wp + (int64_t)t * 1024 + h * 256 + (lane & 15) * 16;
-    }
-    u32x4 wreg[2][2][2];
-    auto load_w = [&](auto setc, int s) {
-        const int64_t off = (int64_t)min(s, s_last) * n_tiles * 1024;
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) wreg[decltype(setc)::value][nt][j] = *(const u32x4*)(wbase[nt] + off + 512 * j);
+    for (int nt = 0; nt < 4; ++nt) wbase[nt] = wp + (int64_t)min(tile0 + 4 * wv + nt, n_tiles - 1) * 1024;
+    u32x4 wreg[DW][4];
+    auto load_w = [&](auto setc, auto nc, int s) {
+        constexpr int nt = decltype(nc)::value;
+        wreg[decltype(setc)::value][nt] = load16_at<NT>(wbase[nt] + (int64_t)min(s, s_last) * n_tiles * 1024, lane * 16);
     };
-    // ---- operands of sub-step i (16 columns: 16h + 32(i >> 1) + 8(i & 1) + 0..7 in lane half h)
-    const int frow = r32 * 128, fkey = key(r32);
-    vec8 xf[2][MT], wf[2][2];
-    auto read_x = [&](auto bufc, int stage, auto ic) {
-        constexpr int I = decltype(ic)::value, B = decltype(bufc)::value;
-        const int at = frow + (((2 * h + 4 * (I >> 1) + (I & 1)) ^ fkey) << 4);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) xf[B][mt] = bitcast<vec8>(*(const u32x4*)(smem + stage * STAGE + 4096 * mt + at));
+    // ---- operands: a sub-step u of a step is 32 columns, 16g + 8u .. + 7 in lane (r, g).  The rows of a sub-step stay in registers
+    // while the wave's four channel tiles pass by, converted one ahead
+    const int frow = (lane & 15) * 128, fkey = key(lane & 15);
+    vec8 xf[2][2 * MT], wf;
+    auto read_x = [&](auto mc, int stage, auto uc) {
+        constexpr int m = decltype(mc)::value, U = decltype(uc)::value;
+        const int at = frow + (((2 * (lane >> 4) + U) ^ fkey) << 4);
+        xf[U][m] = bitcast<vec8>(*(const u32x4*)(smem + stage * STAGE + 2048 * m + at));
     };
-    auto cvt_w = [&](auto bufc, auto setc, auto ic) {
-        constexpr int I = decltype(ic)::value, S = decltype(setc)::value, B = decltype(bufc)::value;
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-            wf[B][nt] = dequant8<T>(wreg[S][nt][I >> 1][2 * (I & 1)], wreg[S][nt][I >> 1][2 * (I & 1) + 1]);
-    };
-    f32x16 acc[MT][2];
+    f32x4 acc[MT][2][4];                                      // [32-row block][16-row tile of it][16-channel tile]
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = (f32x16)(0.f);
-    auto mul = [&](auto bufc) {
-        constexpr int B = decltype(bufc)::value;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = T::mfma32(wf[B][nt], xf[B][mt], acc[mt][nt]);
-    };
+        for (int j = 0; j < 8; ++j) acc[mt][j >> 2][j & 3] = (f32x4)(0.f);
     using C0 = std::integral_constant<int, 0>;
     using C1 = std::integral_constant<int, 1>;
-    using C2 = std::integral_constant<int, 2>;
-    using C3 = std::integral_constant<int, 3>;
-    // one matrix instruction, then what hides behind it
-    auto interleave = [&](auto readsc, auto valuc, auto writesc, auto loadsc) {
-        constexpr int NM = 2 * MT;
-        static_for<NM>([&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            constexpr int R = decltype(readsc)::value, V = decltype(valuc)::value, W = decltype(writesc)::value,
-                          L = decltype(loadsc)::value;
-            constexpr int r = (k + 1) * R / NM - k * R / NM, v = (k + 1) * V / NM - k * V / NM,
-                          w = (k + 1) * W / NM - k * W / NM, l = (k + 1) * L / NM - k * L / NM;
-            if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);
-            if constexpr (w > 0) __builtin_amdgcn_sched_group_barrier(0x200, w, 0);
-            if constexpr (l > 0) __builtin_amdgcn_sched_group_barrier(0x020, l, 0);
-            if constexpr (v > 0) __builtin_amdgcn_sched_group_barrier(0x002, v, 0);
-        });
-        __builtin_amdgcn_sched_barrier(0);
-    };
 
-    load_x(C0{}, s_begin);
-    load_w(C0{}, s_begin);
-    load_x(C1{}, s_begin + 1);
-    load_w(C1{}, s_begin + 1);
-    write_x(C0{}, 0);
-    load_x(C0{}, s_begin + 2);
+    // the loop runs pairs of steps; an odd one is made a pair by a step of zeros in front (a copy of a step behind the loop costs
+    // more, in code that every workgroup of a compute unit fetches and in accumulators that move).  The loads go out in the order of
+    // the loop, whose waits the compiler counts for both ways into it
+    const int s_first = s_begin - ((s_end - s_begin) & 1);
+    static_for<MT>([&](auto ic) { load_x(C0{}, ic, max(s_first, s_begin)); });
+    static_for<DW>([&](auto jc) {
+        constexpr int j = decltype(jc)::value, xj = j + 1 + DX<MT> - DW;
+        if constexpr (xj == DX<MT>) {
+            if (s_first < s_begin)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) xreg[0][i] = (u32x4)(0);
+            static_for<MT>([&](auto ic) { write_x(C0{}, ic, 0); });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (xj > 0) static_for<MT>([&](auto ic) { load_x(std::integral_constant<int, xj % DX<MT>>{}, ic, s_first + xj); });
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<4>([&](auto nc) { load_w(jc, nc, max(s_first + j, s_begin)); });
+        __builtin_amdgcn_sched_barrier(0);
+    });
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    read_x(C0{}, 0, C0{});
-    cvt_w(C0{}, C0{}, C0{});
+    static_for<2 * MT>([&](auto mc) { read_x(mc, 0, C0{}); });
+    wf = dequant8<T>(wreg[0][0][0], wreg[0][0][1]);
     __builtin_amdgcn_sched_barrier(0);
 
-    using CX = std::integral_constant<int, MT>;
-    using CZ = std::integral_constant<int, 0>;
-    using CV = std::integral_constant<int, 24>;
-    auto step = [&](auto jc, int s) {
-        constexpr int P = decltype(jc)::value;
-        using CP = std::integral_constant<int, P>;
-        using CQ = std::integral_constant<int, P ^ 1>;
-        read_x(C1{}, P, C1{});
-        cvt_w(C1{}, CP{}, C1{});
-        write_x(CQ{}, P ^ 1);                                 // its readers passed the barrier of the step before
-        mul(C0{});
-        interleave(CX{}, CV{}, CX{}, CZ{});
-        read_x(C0{}, P, C2{});
-        cvt_w(C0{}, CP{}, C2{});
-        load_x(CQ{}, s + 3);
-        mul(C1{});
-        interleave(CX{}, CV{}, CZ{}, CX{});
-        read_x(C1{}, P, C3{});
-        cvt_w(C1{}, CP{}, C3{});
-        load_w(CP{}, s + 2);
-        mul(C0{});
-        interleave(CX{}, CV{}, CZ{}, std::integral_constant<int, 4>{});
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
+    // group (u, nt): every row of sub-step u times channel tile nt, and behind each matrix instruction a piece of what the next
+    // groups need
+    auto group = [&](auto jsc, auto gc, int s) {
+        constexpr int J = decltype(jsc)::value, P = J & 1, G = decltype(gc)::value, U = G >> 2, nt = G & 3, NM = 2 * MT;
+        constexpr int NS = G == 7 ? (J + 1) % DW : J, NU = ((G + 1) >> 2) & 1, NN = (G + 1) & 3;      // the tile converted here
+        using CX = std::integral_constant<int, (J + 1) % DX<MT>>;                               // the next step's activations
+        if constexpr (G == 6) {                               // the other stage is written, this one has been read
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+        }
+        uint32_t w[4];
         __builtin_amdgcn_sched_barrier(0);
-        read_x(C0{}, P ^ 1, C0{});
-        cvt_w(C0{}, CQ{}, C0{});
-        mul(C1{});
-        interleave(CX{}, CV{}, CZ{}, CZ{});
+        asm volatile("s_nop 1");                              // the vector unit's last writes reach the matrix unit
+        static_for<NM>([&](auto mc) {
+            constexpr int m = decltype(mc)::value;
+            T::mfma16_acc(acc[m >> 1][m & 1][nt], wf, xf[U][m]);
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<4>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                if constexpr (j * NM / 4 == m) w[j] = i8x2_to<T>(wreg[NS][NN][2 * NU + (j >> 1)], 16 * (j & 1));
+            });
+            // the next sub-step's rows: two halves behind every other instruction, or EARLY of them first and then one by one
+            constexpr int R = EARLY == 0 ? (m & 1 ? MT * (nt - 2) + m / 2 : NM) : nt == 2 ? (m < NM - EARLY ? NM : m - NM + EARLY) : EARLY + m;
+            if constexpr (nt >= 2 && R < NM)
+                read_x(std::integral_constant<int, R>{}, U == 0 ? P : P ^ 1, std::integral_constant<int, U ^ 1>{});
+            if constexpr (G == 0 && (m & 1) == 0) write_x(CX{}, std::integral_constant<int, m / 2>{}, P ^ 1);   // read before the last barrier
+            if constexpr (G == 0 && (m & 1) == 1) load_x(CX{}, std::integral_constant<int, m / 2>{}, s + 1 + DX<MT>);
+            if constexpr (U == 1 && m == 0) load_w(jsc, std::integral_constant<int, nt>{}, s + DW);    // converted in the group before
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        wf = bitcast<vec8>((u32x4){w[0], w[1], w[2], w[3]});
     };
-    int s = s_begin;
-    for (; s + 2 <= s_end; s += 2) {
-        step(C0{}, s);
-        step(C1{}, s + 1);
-    }
-    if (s < s_end) step(C0{}, s);
-
-    // lane (r, h) holds, of row 32mt + r, channels 8q + 4h .. + 3 of each 32-channel block in elements 4q .. 4q + 3
-    // (compile-time indices: an accumulator indexed by a loop that is not unrolled would live in memory)
+    auto step = [&](auto jsc, int s) {                        // step J of a round over the weights' register sets, LDS stage J & 1
+        static_for<8>([&](auto gc) { group(jsc, gc, s); });
+    };
+    for (int s = s_first; s < s_end; s += DW) static_for<DW>([&](auto jc) { step(jc, s + decltype(jc)::value); });
+    asm volatile("s_nop 15" : "+a"(acc[MT - 1][1][3]));      // the last matrix instructions' results
+    static_for<8 * MT>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        f32x4& a = acc[j >> 3][(j >> 2) & 1][j & 3];
+        asm volatile("" : "+a"(a));
+    });
     static_for<MT>([&](auto mtc) { epilogue(mtc, acc[decltype(mtc)::value]); });
 }
 

@@ -287,8 +287,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(
 constexpr int QR_DEPTH = 3;
 
 // ---- wide outputs at 129+ rows: 256 x 192 tiles on 8 waves with mfma_i32_32x32x32_i8 ----------------------------
-// On gfx950 the 16x16x64 int8 instruction issues at half the rate of the 32x32x32 one (measured: 2.4 against
-// 4.4 POP/s with independent accumulators), so the kernel that is bound by the matrix cores uses the latter.
+// (Both int8 instructions fill the matrix pipe; the 32x32x32 one asks for half as many issue slots.)
 // The packed tile format serves it unchanged: rows 32 b .. 32 b + 31 of a k-step are two consecutive 1 KiB
 // tiles, and lane (rho = lane & 31, h = lane >> 5) finds row rho, bytes 32 u + 16 h .. + 15 of the step at
 // tile (rho >> 4), 16-byte slot 16 (2 u + h) + (rho & 15).  Waves 4 (rows) x 2 (channels): a wave owns 64 rows x 96
@@ -753,19 +752,19 @@ struct QTileOut {
     const float *x_scale, *w_scale;
     const uint16_t* bias;
     int M, N;
-    __device__ __forceinline__ void load(int n0, int nt, int q, f32x4& ws, f32x4& bi) const {
-        const int n = min(n0 + 32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1), N - 4);
+    __device__ __forceinline__ void load(int n0, int nt, f32x4& ws, f32x4& bi) const {
+        const int n = min(n0 + 16 * nt + 4 * ((threadIdx.x >> 4) & 3), N - 4);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             ws[i] = w_scale[n + i];
             bi[i] = bias ? T::to_float(bias[n + i]) : 0.f;
         }
     }
-    __device__ __forceinline__ void put(i32x4 a, float xs, f32x4 ws, f32x4 bi, int nt, int q, uint8_t* stage) const {
+    __device__ __forceinline__ void put(i32x4 a, float xs, f32x4 ws, f32x4 bi, int j, int nt, uint8_t* stage) const {
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = scaled_bias((float)a[i], xs, ws[i], true, bi[i], bias != nullptr);
-        *(u32x2*)(stage + (threadIdx.x & 31) * TG_STAGE_ROW + 2 * (32 * nt + 8 * q + 4 * ((threadIdx.x >> 5) & 1))) =
+        *(u32x2*)(stage + (16 * j + (threadIdx.x & 15)) * TG_STAGE_ROW + 2 * (16 * nt + 4 * ((threadIdx.x >> 4) & 3))) =
             (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
     }
 };
@@ -782,34 +781,33 @@ __global__ __launch_bounds__(256, 2) void w8a8_tile_kernel(
     const bool whole = blockIdx.x < g.full || g.split == 1;
     const int KS = (K + Q_KSTEP - 1) / Q_KSTEP, s0 = part * g.steps_per_split;
     const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = mb * 32 * MT, n0 = nb * tq::BN + 64 * wv;
     int32_t* pt = partial + (int64_t)slot * (32 * MT * tq::BN) + (wv * MT * 8 * 64 + lane) * 4;
     const QTileOut<T> out{x_scale, w_scale, bias, M, N};
-    f32x4 ws[8], bi[8];
+    f32x4 ws[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
-    const tq::TiledRows<tq::XLOADS<MT>> rows((const uint8_t*)xq, m0 >> 4, (M + 15) >> 4);
-    tq::tile<MT>(rows, wp, nb * (tq::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const i32x16 (&acc)[2]) {
+    const tq::TiledRows<tq::XLOADS<MT>> rows((const uint8_t*)xq, m0 >> 4, (M + 15) >> 4, wv);
+    tq::tile<MT, false>(rows, wp, nb * (tq::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const i32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
         if (whole) {
             if (mt == 0) {
                 __syncthreads();                              // every wave has read its last operands
 #pragma unroll
-                for (int e = 0; e < 8; ++e) out.load(n0, e >> 2, e & 3, ws[e], bi[e]);
+                for (int nt = 0; nt < 4; ++nt) out.load(n0, nt, ws[nt], bi[nt]);
             }
-            const float xs = x_scale[min(m0 + 32 * mt + (lane & 31), M - 1)];
             wave_lds_order();
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                out.put((i32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
-                                acc[e >> 2][4 * (e & 3) + 3]}, xs, ws[e], bi[e], e >> 2, e & 3, stage);
+            for (int j = 0; j < 2; ++j) {
+                const float xs = x_scale[min(m0 + 32 * mt + 16 * j + (lane & 15), M - 1)];
+#pragma unroll
+                for (int nt = 0; nt < 4; ++nt) out.put(acc[j][nt], xs, ws[nt], bi[nt], j, nt, stage);
+            }
             wave_lds_order();
             tg_flush<T>(y, residual, stage, m0 + 32 * mt, M, n0, N, 8, aligned, lane, 64);
         } else {                                              // accumulator order: whole cache lines
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                *(i32x4*)(pt + (mt * 8 + e) * 256) = (i32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1],
-                                                             acc[e >> 2][4 * (e & 3) + 2], acc[e >> 2][4 * (e & 3) + 3]};
+            for (int e = 0; e < 8; ++e) *(i32x4*)(pt + (mt * 8 + e) * 256) = acc[e >> 2][e & 3];
         }
     });
 }
@@ -831,11 +829,11 @@ __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
     const int lane = threadIdx.x & 63, e0 = 2 * (threadIdx.x >> 6);
     const int32_t* p = partial + slot * PART + ((wv * MT + mt) * 8 * 64 + lane) * 4;
     const QTileOut<T> out{x_scale, w_scale, bias, M, N};
-    const float xs = x_scale[min(m0 + (lane & 31), M - 1)];
+    const float xs = x_scale[min(m0 + 16 * (e0 >> 2) + (lane & 15), M - 1)];
     f32x4 ws[2], bi[2];
     i32x4 v[2] = {(i32x4)(0), (i32x4)(0)};
 #pragma unroll
-    for (int e = 0; e < 2; ++e) out.load(n0, (e0 + e) >> 2, (e0 + e) & 3, ws[e], bi[e]);
+    for (int e = 0; e < 2; ++e) out.load(n0, (e0 + e) & 3, ws[e], bi[e]);
 #pragma unroll 8
     for (int s = 0; s < g.split; ++s)
 #pragma unroll
@@ -978,31 +976,35 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
 // (each fetching the rows anew, a second pass for every second expert), 1435 here (5.2 TB/s of weights); 7168 x 2048: 1280 / 817.
 // With 128-row tiles for every expert of more than 64 rows the padding's matrix instructions counted: the two GEMMs of 256
 // experts of 65 rows on average 2323 us, 2167 with tiles of 96 rows for those up to 96.
-// The three tile heights share 256 registers and spill 46 (188 bytes of scratch a lane), outside the k-loops.
-template <typename T, int MT>
+// Weights of an expert with one block of up to 64 rows are read past the caches, where they would push out the rows that all
+// channel blocks read: 109 experts of 4096 x 7168 at 33 rows 542 us cached, 513 so, 64 of 2816 x 2048 at 33 rows 77 / 68.  For blocks of
+// more rows it depends on the number of experts (64 of 2816 x 2048 at 100 rows 95 / 83, a layer of 256 experts at 65 rows 2545 / 2632),
+// and an expert's further blocks share the weights through L2 (200 rows: 928 / 1276 us).
+template <typename T, int MT, bool NT>
 __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, const float* xs, const uint8_t* we,
                                                 const float* ws, int rows, int m0, int nb, int N, int K, int aligned,
                                                 uint8_t* smem) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = nb * tq::BN + 64 * wv;
     const QTileOut<T> out{xs, ws, nullptr, rows, N};
-    f32x4 wsv[8], bi[8];
+    f32x4 wsv[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
-    const tq::PlainRows<tq::XLOADS<MT>> src(xe, m0, rows, K);
-    tq::tile<MT>(src, we, nb * (tq::BN / 16), (N + 15) >> 4, 0, (K + Q_KSTEP - 1) / Q_KSTEP, smem,
-                 [&](auto mtc, const i32x16 (&acc)[2]) {
+    const tq::PlainRows<tq::XLOADS<MT>> src(xe, m0, rows, K, wv);
+    tq::tile<MT, NT>(src, we, nb * (tq::BN / 16), (N + 15) >> 4, 0, (K + Q_KSTEP - 1) / Q_KSTEP, smem,
+                 [&](auto mtc, const i32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
         if (mt == 0) {
             __syncthreads();                                  // every wave has read its last operands
 #pragma unroll
-            for (int e = 0; e < 8; ++e) out.load(n0, e >> 2, e & 3, wsv[e], bi[e]);
+            for (int nt = 0; nt < 4; ++nt) out.load(n0, nt, wsv[nt], bi[nt]);
         }
-        const float x1 = xs[min(m0 + 32 * mt + (lane & 31), rows - 1)];
         wave_lds_order();
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            out.put((i32x4){acc[e >> 2][4 * (e & 3)], acc[e >> 2][4 * (e & 3) + 1], acc[e >> 2][4 * (e & 3) + 2],
-                            acc[e >> 2][4 * (e & 3) + 3]}, x1, wsv[e], bi[e], e >> 2, e & 3, stage);
+        for (int j = 0; j < 2; ++j) {
+            const float x1 = xs[min(m0 + 32 * mt + 16 * j + (lane & 15), rows - 1)];
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) out.put(acc[j][nt], x1, wsv[nt], bi[nt], j, nt, stage);
+        }
         wave_lds_order();
         tg_flush<T>(y, nullptr, stage, m0 + 32 * mt, rows, n0, N, 8, aligned, lane, 64);
     });
@@ -1020,9 +1022,17 @@ __global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
     uint16_t* ye = y + (int64_t)row0 * N;
     const uint8_t *xe = (const uint8_t*)xq + (int64_t)row0 * K, *we = wp + (int64_t)e * expert_bytes;
     const float *xs = x_scale + row0, *ws = w_scale + (int64_t)e * N;
-    if (rows - m0 <= 64) w8a8_group_tile<T, 2>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
-    else if (rows - m0 <= 96) w8a8_group_tile<T, 3>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
-    else w8a8_group_tile<T, 4>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem);
+    const int left = rows - m0;
+#define GT(MT, NT) w8a8_group_tile<T, MT, NT>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem)
+    if (left <= 64) {
+        if (m0 == 0) GT(2, true);                             // nobody else reads these weights
+        else GT(2, false);
+    } else if (left <= 96) {
+        GT(3, false);
+    } else {
+        GT(4, false);
+    }
+#undef GT
 }
 
 // What may follow the GEMM in the same call, fused with the split-K reduce where K is split.
@@ -1066,7 +1076,7 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
         // 80-channel tiles, two workgroups per CU: close to 512 tiles balance best; wide N only
         p.nt = n >= 16384 ? 5 : 4;
         // very wide outputs: 256 x 192 tiles on 8 waves, one workgroup per CU (one staged activation tile serves
-        // more channels, and the 32 x 32 x 32 instruction runs at twice the rate of the 16 x 16 x 64 one)
+        // more channels)
         p.wide = x_tiled && n >= 16384 && m > 128;
         p.m_blocks = (m + 255) / 256;
     } else {

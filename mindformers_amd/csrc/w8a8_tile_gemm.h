@@ -1,19 +1,21 @@
 // W8A8 GEMM for many rows, exact int32 sums.
 #pragma once
 #include "common.h"
+#include "tile_grid.h"
 
-// A workgroup of 4 waves owns 32*MT rows x 256 channels, wave w channels 64w .. 64w + 63 of all the rows
-// (v_mfma_i32_32x32x32_i8).  A packed weight tile is the matrix operand, so weights go from global memory into operand
-// registers and nowhere else; the activations of a 64-wide step (tile order too) are staged in LDS once for the four waves.
-// Loads run three steps ahead of their use in three register sets, the LDS stage of a step is written one step ahead, and the
-// operands of a sub-step (32 columns) are read behind the matrix instructions of the one before; one barrier per step.
+// A workgroup of 4 waves owns 32*MT rows x 256 channels, wave w channels 64w .. 64w + 63 of all the rows.  A packed weight tile is
+// the operand of v_mfma_i32_16x16x64_i8 as it lies, so weights go from global memory into operand registers and nowhere else; the
+// activations of a 64-wide step (tile order too) are staged in LDS once for the four waves.  Loads run three steps ahead of their use
+// in three register sets, the LDS stage of a step is written one step ahead, and the rows of half a step are read behind the
+// matrix instructions of the half before; one barrier per step.
 //
-// The 16x16x64 int8 instruction issues at half the rate of the 32x32x32 one here (2.4 against 4.4 POP/s with independent
-// accumulators).  What bounds the kernel is the operand traffic out of L2 (24 KiB per 4.2 M operations a step, 171 op/B, about
-// 12 TB/s) and, with it, the power budget: 2405 TOP/s at 4096 x 4096 x 16384 from warm caches, 2070 at 4137 x 28672 x 4096 with
-// cold weights.  1531 x 37888 x 3584: 275 us on 256 x 192 tiles of 8 waves with both operands through an LDS ring, 250 here;
-// 1531 x 3584 x 18944: 181 us on the register-streaming kernel, 120 here.  Row panels of 8 or 16 blocks instead of 4, or
-// neighbouring tiles paired on one compute unit, change nothing.
+// With all operands in registers 16x16x64 does 4345 TOP/s on random data and 32x32x32 3727 (4866 and 4976 on zeros): both fill the
+// matrix pipe, and the smaller one, which reads and writes half the accumulators per operation, leaves the power budget more clock.
+// What bounds the kernel is the operand traffic out of L2 (24 KiB per 4.2 M operations a step, 171 op/B, about 12 TB/s) and that
+// budget: 4096 x 4096 x 16384 from warm caches 248 us on 32x32x32, 219 here (2515 TOP/s), 1531 x 37888 x 3584 with cold weights
+// 203 / 187, 2077 x 4096 x 7168 73 / 67, 1531 x 3584 x 18944 (168 tiles, one on a compute unit) 118 / 118.  1531 x 37888 x 3584 on 256 x
+// 192 tiles of 8 waves with both operands through an LDS ring: 275.  Row panels of 8 or 16 blocks instead of 4, or neighbouring
+// tiles paired on one compute unit, change nothing.
 namespace tq {
 
 constexpr int WAVES = 4;
@@ -34,36 +36,40 @@ template <int XL>
 struct TiledRows {                                            // tile order: whole KiB, m_tiles of them a step
     const uint8_t* p[XL];
     int64_t step;
-    __device__ __forceinline__ TiledRows(const uint8_t* xq, int m_tile0, int m_tiles) : step((int64_t)m_tiles * 1024) {
+    __device__ __forceinline__ TiledRows(const uint8_t* xq, int m_tile0, int m_tiles, int wv) : step((int64_t)m_tiles * 1024) {
 #pragma unroll
-        for (int i = 0; i < XL; ++i)
-            p[i] = xq + (int64_t)min(m_tile0 + 4 * i + (int)(threadIdx.x >> 6), m_tiles - 1) * 1024 + (threadIdx.x & 63) * 16;
+        for (int i = 0; i < XL; ++i) p[i] = xq + (int64_t)min(m_tile0 + 4 * i + wv, m_tiles - 1) * 1024;
     }
-    __device__ __forceinline__ i32x4 load(int i, int s) const { return *(const i32x4*)(p[i] + s * step); }
+    __device__ __forceinline__ i32x4 load(int i, int s) const {
+        return bitcast<i32x4>(load16_at(p[i] + s * step, (threadIdx.x & 63) * 16));
+    }
 };
 template <int XL>
 struct PlainRows {                                            // rows m0 .. of `rows` rows of K (a multiple of 16) bytes
-    const uint8_t* p[XL];
-    int last;                                                 // columns past K are clamped: their weights are zero
-    __device__ __forceinline__ PlainRows(const uint8_t* xq, int m0, int rows, int K) {
-        const int r = threadIdx.x & 15, c = 16 * ((threadIdx.x >> 4) & 3);
+    const uint8_t* p;
+    uint32_t row[XL];
+    int c, last;                                              // columns past K are clamped: their weights are zero
+    __device__ __forceinline__ PlainRows(const uint8_t* xq, int m0, int rows, int K, int wv) : p(xq + (int64_t)m0 * K) {
+        c = 16 * ((threadIdx.x >> 4) & 3);
+        last = K - 16;
 #pragma unroll
         for (int i = 0; i < XL; ++i)
-            p[i] = xq + (int64_t)min(m0 + 16 * (4 * i + (int)(threadIdx.x >> 6)) + r, rows - 1) * K + c;
-        last = K - 16 - c;
+            row[i] = (uint32_t)min(16 * (4 * i + wv) + (int)(threadIdx.x & 15), rows - 1 - m0) * (uint32_t)K;
     }
-    __device__ __forceinline__ i32x4 load(int i, int s) const { return *(const i32x4*)(p[i] + min(s * KSTEP, last)); }
+    __device__ __forceinline__ i32x4 load(int i, int s) const {
+        return bitcast<i32x4>(load16_at(p, row[i] + (uint32_t)min(s * KSTEP + c, last)));
+    }
 };
 
 // tile0: first 16-channel tile of the weights, n_tiles: tiles of a step
-template <int MT, typename Rows, typename Epilogue>
+// NT: weights that nobody else reads (non-temporal loads)
+template <int MT, bool NT, typename Rows, typename Epilogue>
 __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ wp, int tile0, int n_tiles, int s_begin,
                                      int s_end, uint8_t* smem, Epilogue&& epilogue) {
     constexpr int XL = XLOADS<MT>, STAGE = 64 * XL * KSTEP;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int h = lane >> 5;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int s_last = s_end - 1;
-    i32x4 xreg[D][XL], wreg[D][2][2];
+    i32x4 xreg[D][XL], wreg[D][4];
     auto load_x = [&](auto setc, int s) {
 #pragma unroll
         for (int i = 0; i < XL; ++i) xreg[decltype(setc)::value][i] = x.load(i, min(s, s_last));
@@ -73,43 +79,41 @@ __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ 
         for (int i = 0; i < XL; ++i)
             *(i32x4*)(smem + stage * STAGE + (4 * i + wv) * 1024 + lane * 16) = xreg[decltype(setc)::value][i];
     };
-    // lane (r, h) of a 32-row operand: row r & 15 of tile r >> 4, columns 32u + 16h .. of sub-step u
-    const int lane32 = ((lane >> 4) & 1) * 1024 + h * 256 + (lane & 15) * 16;
-    const uint8_t* wbase[2];
+    // weights: a packed tile is the matrix operand of 16 channels x 64 columns; the tile addresses are the same in every lane
+    const uint8_t* wbase[4];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-        const int t = min(tile0 + 4 * wv + 2 * nt + ((lane >> 4) & 1), n_tiles - 1);
-        wbase[nt] = wp + (int64_t)t * 1024 + h * 256 + (lane & 15) * 16;
-    }
+    for (int nt = 0; nt < 4; ++nt) wbase[nt] = wp + (int64_t)min(tile0 + 4 * wv + nt, n_tiles - 1) * 1024;
+    const uint32_t lane16 = lane * 16;
     auto load_w = [&](auto setc, int s) {
         const int64_t off = (int64_t)min(s, s_last) * n_tiles * 1024;
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) wreg[decltype(setc)::value][nt][u] = *(const i32x4*)(wbase[nt] + off + 512 * u);
+        for (int nt = 0; nt < 4; ++nt) wreg[decltype(setc)::value][nt] = bitcast<i32x4>(load16_at<NT>(wbase[nt] + off, lane16));
     };
+    // activations of 16-row tile t: one KiB in operand order; tiles 0 .. MT - 1 make the first half of a step, the others the second
     i32x4 xf[2][MT];
-    auto read_x = [&](auto bufc, int stage) {                 // buffer = sub-step
+    auto read_x = [&](auto bufc, int stage) {                 // buffer = half
         constexpr int B = decltype(bufc)::value;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) xf[B][mt] = *(const i32x4*)(smem + stage * STAGE + mt * 2048 + 512 * B + lane32);
+        for (int mt = 0; mt < MT; ++mt) xf[B][mt] = *(const i32x4*)(smem + stage * STAGE + (B * MT + mt) * 1024 + lane16);
     };
-    i32x16 acc[MT][2];
+    i32x4 acc[MT][2][4];                                      // [32-row block][16-row tile of it][16-channel tile]
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = (i32x16)(0);
+        for (int j = 0; j < 8; ++j) acc[mt][j >> 2][j & 3] = (i32x4)(0);
     auto mul = [&](auto bufc, auto setc) {
         constexpr int B = decltype(bufc)::value, S = decltype(setc)::value;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wreg[S][nt][B], xf[B][mt], acc[mt][nt], 0, 0, 0);
+            for (int nt = 0; nt < 4; ++nt) {
+                i32x4& a = acc[(B * MT + mt) >> 1][(B * MT + mt) & 1][nt];
+                a = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[S][nt], xf[B][mt], a, 0, 0, 0);
+            }
     };
     // one matrix instruction, then what hides behind it
     auto interleave = [&](auto writesc, auto loadsc) {
-        constexpr int NM = 2 * MT, R = MT, W = decltype(writesc)::value, L = decltype(loadsc)::value;
+        constexpr int NM = 4 * MT, R = MT, W = decltype(writesc)::value, L = decltype(loadsc)::value;
         static_for<NM>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
             constexpr int r = (k + 1) * R / NM - k * R / NM, w = (k + 1) * W / NM - k * W / NM, l = (k + 1) * L / NM - k * L / NM;
@@ -122,12 +126,17 @@ __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ 
     };
     using C0 = std::integral_constant<int, 0>;
     using C1 = std::integral_constant<int, 1>;
+    // (in the order of the loop, whose waits the compiler counts for both ways into it)
+    load_x(C0{}, s_begin);
     static_for<D>([&](auto dc) {
-        load_x(dc, s_begin + decltype(dc)::value);
-        load_w(dc, s_begin + decltype(dc)::value);
+        constexpr int d = decltype(dc)::value;
+        if constexpr (d == D - 1) write_x(C0{}, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_x(std::integral_constant<int, (d + 1) % D>{}, s_begin + d + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(dc, s_begin + d);
+        __builtin_amdgcn_sched_barrier(0);
     });
-    write_x(C0{}, 0);
-    load_x(C0{}, s_begin + D);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     read_x(C0{}, 0);
@@ -156,7 +165,7 @@ __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ 
     static_for<2 * D - 1>([&](auto jc) {
         if (s + decltype(jc)::value < s_end) step(jc, s + decltype(jc)::value);
     });
-    // lane (r, h) holds, of row 32mt + r, channels 8q + 4h .. + 3 of each 32-channel block in elements 4q .. 4q + 3
+    // lane (r, g) holds, of row 32mt + 16j + r, channels 4g .. + 3 of each 16-channel tile
     static_for<MT>([&](auto mtc) { epilogue(mtc, acc[decltype(mtc)::value]); });
 }
 

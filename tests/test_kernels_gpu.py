@@ -1194,6 +1194,25 @@ def test_w8a16_exact_on_integer_grid():
     assert np.array_equal(to_np(y).astype(np.float64), rounded(exact, torch.float16).astype(np.float64))
 
 
+@pytest.mark.parametrize("m,n,k", [(129, 28672, 64), (131, 28672, 128), (257, 28672, 192), (300, 4096, 14336 + 64), (1048, 4096, 4160)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_w8a16_tiles_exact_on_integer_grid(dtype, m, n, k):
+    """The same for the kernel of many rows, whose k-loop runs pairs of 64-wide steps: one step, a pair, odd numbers of them, in whole
+    tiles and in parts, with an infinity in a row's last column, which belongs to that row alone."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + k)
+    w = torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+    x = torch.randint(-3, 4, (m, k), generator=g, device="cuda").to(dtype)
+    s = torch.full((n,), 2.0 ** -12, device="cuda")
+    bad = m // 2
+    x[bad, k - 1] = float("inf")
+    y = ops.w8a16_linear(x, w, s)
+    keep = torch.arange(m, device="cuda") != bad
+    exact = (x[keep].double() @ w.double().t() * 2.0 ** -12).to(dtype)      # |sum| < 2^24: every fp32 partial sum is exact
+    assert torch.equal(y[keep], exact)
+    assert not bool(torch.isfinite(y[bad]).any())
+
+
 @pytest.mark.parametrize("m,n,k", [(37, 200, 1376), (64, 256, 1032), (5, 80, 72)])
 def test_w8a16_inf_in_the_last_columns_of_a_row_stays_in_that_row(m, n, k):
     """K is not a multiple of 64, so the last k-step is short and its padding columns carry zero weights.  An Inf
