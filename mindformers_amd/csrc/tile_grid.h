@@ -7,6 +7,7 @@
 // channel blocks in its L2.  The tiles left over are cut into `split` parts of K each.
 struct TileGrid {
     int m_blocks, n_blocks, full, split, steps_per_split;
+    int mt;                                                   // rows of a block / 32
 };
 constexpr int TG_PANEL = 4;                                   // row blocks walked together along the channels
 __device__ __forceinline__ void tg_locate(const TileGrid& g, int id, int& mb, int& nb, int& part, int& slot) {
@@ -31,11 +32,14 @@ inline int tg_workgroups(const TileGrid& g) { return g.full + (g.m_blocks * g.n_
 // writing and summing the parts.
 struct TileCost {
     float alone, pair, fixed, reduce, part;
+    float alone3;                                             // a k-step of a 96-row tile on a compute unit of its own
 };
 // Whole tiles fill whole multiples of the 256 compute units; what is left over would hold a few of them for a whole tile's
 // time, so it is cut along K where the shorter tail pays for its parts.
-inline TileGrid tg_plan(int m_blocks, int n_blocks, int steps, const TileCost& c, float* us) {
+inline TileGrid tg_plan_rows(int m, int mt, int n_blocks, int steps, const TileCost& c, float* us) {
     TileGrid g;
+    const int m_blocks = (m + 32 * mt - 1) / (32 * mt);
+    g.mt = mt;
     g.m_blocks = m_blocks;
     g.n_blocks = n_blocks;
     const int tiles = m_blocks * n_blocks, rounds = tiles / 256, rem = tiles % 256;
@@ -64,6 +68,21 @@ inline TileGrid tg_plan(int m_blocks, int n_blocks, int steps, const TileCost& c
     g.full = g.split > 1 ? tiles - rem : tiles / 8 * 8;       // a multiple of 8 (see tg_locate)
     *us = best + c.fixed;
     return g;
+}
+
+// 128-row tiles, or 96-row ones where those are all resident at once, each on a compute unit of its own: more units then share the
+// work, and fewer rows are padding.  A plan that is cut along K gives way only to a clearly shorter one (the model is good to some
+// 10 %), one of few k-steps not at all, nor a single row block, which has no more tiles then.  W8A16, us, 128 | 96 rows: 1048 x
+// 4096 x 14336 157 | 135, 1300 x 4096 x 4096 53 | 46, 2025 x 2112 x 7168 (cut in parts) 83 | 71, 129 x 28672 x 4096 62 | 50, but 65 x 28672 x 4096
+// 42 | 46; W8A8: 1531 x 3584 x 18944 120 | 111, 1531 x 3584 x 3584 30.7 | 26.4, 1300 x 4608 x 3584 32.7 | 27.8.
+inline TileGrid tg_plan(int m, int n_blocks, int steps, const TileCost& c, float* us) {
+    const TileGrid g = tg_plan_rows(m, 4, n_blocks, steps, c, us);
+    const int m_blocks = (m + 95) / 96;
+    const int64_t tiles = (int64_t)m_blocks * n_blocks;
+    const float us3 = steps * c.alone3 + c.fixed;
+    if (m <= 128 || steps < 16 || tiles > 256 || us3 >= (g.split > 1 ? 0.85f : 1.f) * *us) return g;
+    *us = us3;
+    return {m_blocks, n_blocks, (int)tiles / 8 * 8, 1, steps, 3};
 }
 
 // Grouped rows (experts): rows a group must average for tiles of 256 channels to replace 64-channel workgroups.  `least` is where

@@ -1038,10 +1038,9 @@ struct GemmPlan {
 
 // Tile plan of the many-row kernel (4137 x 4096 x 14336: 16 of 528 tiles left over by whole rounds, 531 us uncut, 423 us in
 // 8 parts).
-constexpr int TG_MT = 4;
-constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f};
+constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f, 0.56f};
 TileGrid plan_tiles(int m, int n, int k, float* us) {
-    return tg_plan((m + 32 * TG_MT - 1) / (32 * TG_MT), (n + tg::BN - 1) / tg::BN, k / tg::KSTEP, TG_COST, us);
+    return tg_plan(m, (n + tg::BN - 1) / tg::BN, k / tg::KSTEP, TG_COST, us);
 }
 
 GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
@@ -1091,11 +1090,14 @@ void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale,
     float us;
     const TileGrid g = plan_tiles(m, n, k, &us);
     const int aligned = (((uintptr_t)y | (uintptr_t)residual) & 15) == 0;
-    hipLaunchKernelGGL((w8a16_tile_kernel<T, TG_MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y,
-                       (float*)workspace, (const uint16_t*)x, wp, scale, (const uint16_t*)bias, (const uint16_t*)residual, m,
-                       n, k, gated, aligned, g);
-    if (g.split > 1)
-        hipLaunchKernelGGL((w8a16_tile_reduce_kernel<T, TG_MT>), dim3((g.m_blocks * g.n_blocks - g.full) * tg::WAVES * TG_MT), dim3(256), 0, st,
+#define TG_LAUNCH(MT)                                                                                              \
+    hipLaunchKernelGGL((w8a16_tile_kernel<T, MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y, (float*)workspace, \
+                       (const uint16_t*)x, wp, scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, gated, aligned, g)
+    if (g.mt == 3) TG_LAUNCH(3);
+    else TG_LAUNCH(4);
+#undef TG_LAUNCH
+    if (g.split > 1)                                          // 128-row tiles
+        hipLaunchKernelGGL((w8a16_tile_reduce_kernel<T, 4>), dim3((g.m_blocks * g.n_blocks - g.full) * tg::WAVES * 4), dim3(256), 0, st,
                            (uint16_t*)y, (const float*)workspace, scale, (const uint16_t*)bias, (const uint16_t*)residual, m,
                            n, gated, aligned, g);
 }
@@ -1222,7 +1224,7 @@ extern "C" size_t mf_w8a16_workspace_bytes(int m, int n, int k) {
     if (use_tiles(m, n, k)) {
         float us;
         const TileGrid g = plan_tiles(m, n, k, &us);
-        return g.split > 1 ? (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * TG_MT * tg::BN) * sizeof(float) : 0;
+        return g.split > 1 ? (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * g.mt * tg::BN) * sizeof(float) : 0;
     }
     const GemmPlan p = plan_w8a16(m, n, k);
     return p.split_k > 1 ? (size_t)p.split_k * m * n * sizeof(float) : 0;

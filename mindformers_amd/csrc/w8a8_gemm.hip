@@ -1106,12 +1106,11 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
 // 34 / 34 / 67 (LDS-staged), 3584 x 18944 at 1531 rows in 120 against 181, 3584 x 3584 at 448 rows in 27 against 20.  `fused`: the
 // sum of the register-streaming and the wide kernel's parts carries what follows, which is a kernel of its own behind tiles (the
 // figures of the LDS-staged kernel have it in).
-constexpr int TQ_MT = 4;
-constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f};
+constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f, 0.31f};
 bool plan_q_tiles(int m, int n, int k, bool fused, TileGrid& g) {
     if (m <= 64 || n % 16 != 0) return false;
     float us;
-    g = tg_plan((m + 32 * TQ_MT - 1) / (32 * TQ_MT), (n + tq::BN - 1) / tq::BN, (k + Q_KSTEP - 1) / Q_KSTEP, TQ_COST, &us);
+    g = tg_plan(m, (n + tq::BN - 1) / tq::BN, (k + Q_KSTEP - 1) / Q_KSTEP, TQ_COST, &us);
     const QPlan p = plan_w8a8(m, n, k, true);
     const int rounds = (p.n_blocks * p.m_blocks * p.split_k + 255) / 256;
     const bool staged = !p.regs && !p.wide;
@@ -1125,11 +1124,14 @@ void launch_q_tiles(const TileGrid& g, void* y, const int8_t* xq, const float* x
                     const float* w_scale, const void* bias, const void* residual, int m, int n, int k, void* workspace,
                     hipStream_t st) {
     const int aligned = (((uintptr_t)y | (uintptr_t)residual) & 15) == 0;
-    hipLaunchKernelGGL((w8a8_tile_kernel<T, TQ_MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y,
-                       (int32_t*)workspace, xq, x_scale, wp, w_scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n,
-                       k, aligned, g);
-    if (g.split > 1)
-        hipLaunchKernelGGL((w8a8_tile_reduce_kernel<T, TQ_MT>), dim3((g.m_blocks * g.n_blocks - g.full) * tq::WAVES * TQ_MT),
+#define TQ_LAUNCH(MT)                                                                                              \
+    hipLaunchKernelGGL((w8a8_tile_kernel<T, MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y, (int32_t*)workspace, xq, \
+                       x_scale, wp, w_scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, aligned, g)
+    if (g.mt == 3) TQ_LAUNCH(3);
+    else TQ_LAUNCH(4);
+#undef TQ_LAUNCH
+    if (g.split > 1)                                          // 128-row tiles
+        hipLaunchKernelGGL((w8a8_tile_reduce_kernel<T, 4>), dim3((g.m_blocks * g.n_blocks - g.full) * tq::WAVES * 4),
                            dim3(256), 0, st, (uint16_t*)y, (const int32_t*)workspace, x_scale, w_scale,
                            (const uint16_t*)bias, (const uint16_t*)residual, m, n, aligned, g);
 }
@@ -1240,7 +1242,7 @@ extern "C" size_t mf_w8a8_workspace_bytes(int m, int n, int k) {
     }
     TileGrid g;
     if (plan_q_tiles(m, n, k, false, g) && g.split > 1) {     // enough for either kernel
-        const size_t b = (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * TQ_MT * tq::BN) * sizeof(int32_t);
+        const size_t b = (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * g.mt * tq::BN) * sizeof(int32_t);
         need = b > need ? b : need;
     }
     return need;

@@ -77,6 +77,16 @@ def test_plans_of_the_shapes_that_the_tile_kernels_are_tested_at():
         assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, *plan), (m, n, k)
 
 
+def test_plans_of_the_shapes_that_the_96_row_tiles_are_tested_at():
+    """Tiles of 96 rows where they fit the device at once: their number is not that of 128-row tiles, and nothing is cut along K."""
+    from mindformers_amd import _lib
+    lib, tiles8, tiles16 = _lib.load(), 3, 1
+    for (m, n, k), whole in {(1153, 4112, 1216): 221, (1048, 4096, 1088): 176, (2025, 2112, 7168): 198}.items():
+        assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, whole, 0, 1), (m, n, k)
+    for (m, n, k), whole in {(1531, 3584, 3600): 224, (1300, 4608, 1040): 252, (1153, 4624, 1040): 247}.items():
+        assert _plan(lib.mf_w8a8_plan, m, n, k, 0) == (tiles8, whole, 0, 1), (m, n, k)
+
+
 def test_w8a8_plans_take_the_faster_kernel_at_the_measured_lines():
     """One round of wide tiles against a round and a part of 128 x 256 ones, the LDS-staged kernel where the tiles leave half the
     device idle, and the wide kernel above 256 rows where the tiles cannot serve the width."""

@@ -1181,6 +1181,16 @@ def test_w8a16_many_rows(dtype, m, n, k, bias, residual):
         assert torch.equal(fused, ops.silu_mul(y))
 
 
+@pytest.mark.parametrize("dtype,m,n,k", [
+    (torch.bfloat16, 1153, 4112, 1216),    # 96-row tiles: one row and one 16-channel piece past whole ones, an odd number of k-steps
+    (torch.float16, 1048, 4096, 1088),
+    (torch.bfloat16, 2025, 2112, 7168)])   # in place of tiles that are cut along K
+def test_w8a16_many_rows_on_96_row_tiles(dtype, m, n, k):
+    """The same at shapes that take the lower tiles."""
+    test_w8a16_many_rows(dtype, m, n, k, True, False)
+    test_w8a16_many_rows(dtype, m, n, k, False, True)
+
+
 def test_w8a16_exact_on_integer_grid():
     """Power-of-two scales and small-integer activations make every product and sum exact: the kernel must
     return exactly the integer matmul (catches a dropped k-step, a wrong row/column or a transposed operand)."""
@@ -1439,6 +1449,12 @@ def test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, bias, residua
     ref = v + r.double() if residual else v
     tol = EPS[dtype] * (ref.abs() + (v.abs() if residual else 0)) * 1.01 + 4 * 2.0 ** -24 * (v.abs() + 1) + 1e-7
     assert bool(((y.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.bfloat16, 1153, 4624, 1040), (torch.float16, 1531, 3584, 3600)])
+def test_w8a8_many_rows_on_96_row_tiles(dtype, m, n, k):
+    """The same at shapes that take the lower tiles: one row and one channel piece past whole ones, a short last k-step."""
+    test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, True, True)
 
 
 @pytest.mark.parametrize("m,n,k", [(290, 24192, 1472), (300, 16392, 528)])
