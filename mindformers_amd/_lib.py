@@ -136,4 +136,7 @@ def ptr(t):
 
 
 def stream_ptr(device=None):
-    return torch.cuda.current_stream(device).cuda_stream
+    """Handle of the current stream of ``device``.  (By itself: a ``torch.cuda.Stream`` around it costs more than the rest of a
+    small call's checks.)"""
+    index = device.index if device is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

@@ -79,9 +79,13 @@ class QuantDecodeLayer(nn.Module):
         return self
 
     def __getattr__(self, name):
-        raw = self.__dict__.get("raw_weights")
-        if raw is not None and name in raw:
+        d = self.__dict__
+        raw = d.get("raw_weights")
+        if raw and name in raw:
             return raw[name]
+        buffers = d.get("_buffers")                            # nearly all that a step asks for
+        if buffers is not None and name in buffers:
+            return buffers[name]
         return super().__getattr__(name)
 
     def _load_from_state_dict(self, state_dict, prefix, *args, **kwargs):

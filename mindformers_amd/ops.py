@@ -26,10 +26,14 @@ def _dev_ok(*tensors):
     for t in tensors:
         if t is None:
             continue
-        _need(isinstance(t, torch.Tensor) and t.is_cuda, "all tensors must live on the GPU")
-        _need(t.is_contiguous(), "all tensors must be contiguous")
-        dev = dev or t.device
-        _need(t.device == dev, "all tensors must be on the same device")
+        if not (isinstance(t, torch.Tensor) and t.is_cuda):
+            raise ValueError("all tensors must live on the GPU")
+        if not t.is_contiguous():
+            raise ValueError("all tensors must be contiguous")
+        if dev is None:
+            dev = t.device
+        elif t.device != dev:
+            raise ValueError("all tensors must be on the same device")
     return dev
 
 
@@ -38,10 +42,11 @@ def _rows(t, width, what):
     contiguous tensor whose element count is a multiple of width, or a 2-D tensor with unit column stride (a
     column slice of a wider buffer, e.g. q/k/v inside a fused projection output)."""
     if t.is_contiguous():
-        _need(t.numel() % width == 0, f"{what}: {t.numel()} elements is not a multiple of the row width {width}")
+        if t.numel() % width != 0:
+            raise ValueError(f"{what}: {t.numel()} elements is not a multiple of the row width {width}")
         return t, width
-    _need(t.dim() == 2 and t.stride(1) == 1 and t.shape[1] == width and t.stride(0) >= width,
-          f"{what}: must be contiguous or a [rows, {width}] column slice with unit column stride")
+    if not (t.dim() == 2 and t.stride(1) == 1 and t.shape[1] == width and t.stride(0) >= width):
+        raise ValueError(f"{what}: must be contiguous or a [rows, {width}] column slice with unit column stride")
     return t, t.stride(0)
 
 
@@ -50,9 +55,12 @@ def _dev_of(*tensors):
     for t in tensors:
         if t is None:
             continue
-        _need(isinstance(t, torch.Tensor) and t.is_cuda, "all tensors must live on the GPU")
-        dev = dev or t.device
-        _need(t.device == dev, "all tensors must be on the same device")
+        if not (isinstance(t, torch.Tensor) and t.is_cuda):
+            raise ValueError("all tensors must live on the GPU")
+        if dev is None:
+            dev = t.device
+        elif t.device != dev:
+            raise ValueError("all tensors must be on the same device")
     return dev
 
 
@@ -60,7 +68,7 @@ def workspace(nbytes, device, tag="default"):
     """A cached scratch buffer per (device, stream, purpose), grown on demand and never shrunk.  Two streams never
     share one (their kernels would race on the partial sums), and a buffer that is outgrown is kept alive rather than
     freed: a captured HIP graph may still replay into its address."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream, tag)
+    key = (device, stream_ptr(device), tag)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         if buf is not None:
@@ -87,7 +95,8 @@ def reshape_and_cache(key, value, key_cache, value_cache, slot_mapping):
     _need(key.dtype in _ACT and key_cache.dtype == key.dtype, "key and key_cache must share a bf16/fp16 dtype")
     _need(slot_mapping.dtype == torch.int32 and slot_mapping.dim() == 1, "slot_mapping must be int32 [T]")
     t = slot_mapping.numel()
-    _need(key.numel() == t * n_kv * d, f"key has {key.numel()} elements, expected {t}*{n_kv}*{d}")
+    if key.numel() != t * n_kv * d:
+        raise ValueError(f"key has {key.numel()} elements, expected {t}*{n_kv}*{d}")
     if value is not None:
         _need(value_cache is not None and value_cache.shape == key_cache.shape and value.dtype == key.dtype
               and value_cache.dtype == key.dtype and value.numel() == key.numel(), "value / value_cache mismatch")
@@ -167,13 +176,15 @@ def paged_attention(query, key_cache, value_cache, block_tables, context_lens, n
     _need(key_cache.dim() == 4 and value_cache.shape == key_cache.shape, "caches must be [blocks, block_size, n_kv, D]")
     nb, bs, n_kv, d = key_cache.shape
     query, qs = _rows(query, n_heads * d, "query")
-    _need(n_kv == n_kv_heads, f"cache has {n_kv} kv heads, module says {n_kv_heads}")
+    if n_kv != n_kv_heads:
+        raise ValueError(f"cache has {n_kv} kv heads, module says {n_kv_heads}")
     _need(query.dtype in _ACT and key_cache.dtype == query.dtype and value_cache.dtype == query.dtype, "dtype mismatch")
     _need(block_tables.dtype == torch.int32 and block_tables.dim() == 2, "block_tables must be int32 [B, max_blocks]")
     _need(context_lens.dtype == torch.int32 and context_lens.dim() == 1, "context_lens must be int32 [B]")
     b = context_lens.numel()
     _need(block_tables.shape[0] == b, "block_tables rows != batch")
-    _need(query.numel() == b * n_heads * d, f"query has {query.numel()} elements, expected {b}*{n_heads}*{d}")
+    if query.numel() != b * n_heads * d:
+        raise ValueError(f"query has {query.numel()} elements, expected {b}*{n_heads}*{d}")
     max_blocks = block_tables.shape[1]
     if out is None:
         out = torch.empty(query.shape, dtype=query.dtype, device=dev)
@@ -243,7 +254,8 @@ def mla_paged_attention(query, latent_cache, block_tables, context_lens, n_heads
     b = context_lens.numel()
     _need(block_tables.shape[0] == b, "block_tables rows != batch")
     rows = query.numel() // (n_heads * dk) if query.is_contiguous() else query.shape[0]
-    _need(rows == b, f"query has {rows} rows for {b} sequences")
+    if rows != b:
+        raise ValueError(f"query has {rows} rows for {b} sequences")
     max_blocks = block_tables.shape[1]
     if out is None:
         out = torch.empty((b, n_heads * kv_lora_rank), dtype=query.dtype, device=dev)
@@ -267,7 +279,8 @@ def mla_absorb_bmm(x, w, out=None):
     dev = _dev_of(x, w, out)
     _need(x.dim() == 3 and w.dim() == 3 and w.is_contiguous(), "x must be [T, H, K], w a contiguous [H, N, K]")
     t, h, k = x.shape
-    _need(w.shape[0] == h and w.shape[2] == k, f"w is {tuple(w.shape)}, x has {h} heads of {k}")
+    if not (w.shape[0] == h and w.shape[2] == k):
+        raise ValueError(f"w is {tuple(w.shape)}, x has {h} heads of {k}")
     n = w.shape[1]
     _need(x.dtype in _ACT and w.dtype == x.dtype, "x and w must be bf16/fp16 and agree")
     _need(x.stride(2) == 1, "x needs a unit last stride")
@@ -303,8 +316,8 @@ def mla_norm_rope_cache(q, nope, kv, gamma, eps, cos, sin, latent_cache=None, sl
     out = q_rope if q_rope_out is None else q_rope_out
     _need(tuple(out.shape) == (t, n, rope) and out.stride(2) == 1 and out.dtype == q.dtype, "q_rope_out must be a [T, n, rope] view")
     for buf, width, name in ((kv_norm_out, rank, "kv_norm_out"), (k_pe_out, rope, "k_pe_out")):
-        _need(buf is None or (tuple(buf.shape) == (t, width) and buf.is_contiguous() and buf.dtype == q.dtype),
-              f"{name} must be a contiguous [T, {width}]")
+        if not (buf is None or (tuple(buf.shape) == (t, width) and buf.is_contiguous() and buf.dtype == q.dtype)):
+            raise ValueError(f"{name} must be a contiguous [T, {width}]")
     slots = 0
     if latent_cache is not None:
         _need(latent_cache.is_contiguous() and latent_cache.shape[-1] == rank + rope and latent_cache.dtype == q.dtype,
@@ -325,10 +338,12 @@ def mla_norm_rope_cache(q, nope, kv, gamma, eps, cos, sin, latent_cache=None, sl
 
 # --------------------------------------------------------------------------------------------- int8 KV cache
 def _kv_quant_params(scale, offset, row, dev):
-    _need(isinstance(scale, torch.Tensor) and scale.dtype == torch.float32 and scale.numel() == 2 * row and
-          scale.is_contiguous() and scale.device == dev, f"antiquant scale must be float32 [2, {row}] on the GPU")
-    _need(offset is None or (offset.dtype == torch.float32 and offset.numel() == 2 * row and offset.is_contiguous()
-                             and offset.device == dev), f"antiquant offset must be float32 [2, {row}] on the GPU")
+    if not (isinstance(scale, torch.Tensor) and scale.dtype == torch.float32 and scale.numel() == 2 * row and
+          scale.is_contiguous() and scale.device == dev):
+        raise ValueError(f"antiquant scale must be float32 [2, {row}] on the GPU")
+    if not (offset is None or (offset.dtype == torch.float32 and offset.numel() == 2 * row and offset.is_contiguous()
+                             and offset.device == dev)):
+        raise ValueError(f"antiquant offset must be float32 [2, {row}] on the GPU")
 
 
 def quant_reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, scale, offset=None):
@@ -417,7 +432,8 @@ def paged_attention_int8kv(query, key_cache, value_cache, block_tables, context_
     else:
         _need(out.numel() == rows * n_heads * d and out.dtype == query.dtype, "out mismatch")
     if q_starts is None:
-        _need(rows == b, f"query has {rows} rows for {b} sequences")
+        if rows != b:
+            raise ValueError(f"query has {rows} rows for {b} sequences")
         need = lib.mf_paged_attention_workspace_bytes(b, n_heads, d, max_blocks * bs)
         ws = workspace(need, dev, "pa") if need else None
         if token_scales is not None:
@@ -491,7 +507,8 @@ def paged_attention_prefill(query, key_cache, value_cache, block_tables, context
     _need(key_cache.dim() == 4 and value_cache.shape == key_cache.shape, "caches must be [blocks, block_size, n_kv, D]")
     nb, bs, n_kv, d = key_cache.shape
     query, qs = _rows(query, n_heads * d, "query")
-    _need(n_kv == n_kv_heads, f"cache has {n_kv} kv heads, module says {n_kv_heads}")
+    if n_kv != n_kv_heads:
+        raise ValueError(f"cache has {n_kv} kv heads, module says {n_kv_heads}")
     _need(query.dtype in _ACT and key_cache.dtype == query.dtype and value_cache.dtype == query.dtype, "dtype mismatch")
     _need(block_tables.dtype == torch.int32 and block_tables.dim() == 2, "block_tables must be int32 [B, max_blocks]")
     _need(context_lens.dtype == torch.int32 and context_lens.dim() == 1, "context_lens must be int32 [B]")
@@ -688,7 +705,8 @@ def w8a16_linear(x, w, scale=None, bias=None, residual=None):
     dev = _dev_ok(x, bias, residual)
     _need(x.dtype in _ACT, "x must be bf16/fp16")
     n, k = w.n, w.k
-    _need(x.shape[-1] == k, f"x has {x.shape[-1]} input channels, weight expects {k}")
+    if x.shape[-1] != k:
+        raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
     y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=dev)
     _need(bias is None or (bias.dtype == x.dtype and bias.numel() == n), "bias mismatch")
@@ -740,9 +758,11 @@ def pack_w4a16(w_q, scale, group_size=0, qint4x2=False):
     if qint4x2:
         w_q = unpack_qint4x2(w_q)
     n, k = w_q.shape
-    _need(k % 64 == 0 and (group_size == 0 or k % group_size == 0), f"K ({k}) must be a multiple of 64 and of the group size")
+    if not (k % 64 == 0 and (group_size == 0 or k % group_size == 0)):
+        raise ValueError(f"K ({k}) must be a multiple of 64 and of the group size")
     want = (n,) if group_size == 0 else (k // group_size, n)
-    _need(tuple(scale.shape) == want, f"scale must be {want}, got {tuple(scale.shape)}")
+    if tuple(scale.shape) != want:
+        raise ValueError(f"scale must be {want}, got {tuple(scale.shape)}")
     _need(group_size == 0 or n % 4 == 0, "N must be a multiple of 4 with per-group scales")
     packed = torch.empty(lib.mf_w4a16_packed_bytes(n, k), dtype=torch.uint8, device=dev)
     check(lib.mf_w4a16_pack_weight(ptr(packed), ptr(w_q.contiguous()), n, k, stream_ptr(dev)), "mf_w4a16_pack_weight")
@@ -756,7 +776,8 @@ def w4a16_linear(x, w, bias=None, residual=None):
     dev = _dev_ok(x, bias, residual)
     _need(x.dtype in _ACT, "x must be bf16/fp16")
     n, k = w.n, w.k
-    _need(x.shape[-1] == k, f"x has {x.shape[-1]} input channels, weight expects {k}")
+    if x.shape[-1] != k:
+        raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
     y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=dev)
     _need(bias is None or (bias.dtype == x.dtype and bias.numel() == n), "bias mismatch")
@@ -777,7 +798,8 @@ def w8a16_linear_add_rmsnorm(x, w, residual, gamma, eps, bias=None):
     dev = _dev_ok(x, bias, residual, gamma)
     _need(x.dtype in _ACT, "x must be bf16/fp16")
     n, k = w.n, w.k
-    _need(x.shape[-1] == k, f"x has {x.shape[-1]} input channels, weight expects {k}")
+    if x.shape[-1] != k:
+        raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
     h = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=dev)
     y = torch.empty_like(h)
@@ -802,7 +824,8 @@ def w8a16_linear_rmsnorm_leading(x, w, gamma, eps, bias=None):
     dev = _dev_ok(x, bias, gamma)
     _need(x.dtype in _ACT, "x must be bf16/fp16")
     n, k, c = w.n, w.k, gamma.numel()
-    _need(x.shape[-1] == k, f"x has {x.shape[-1]} input channels, weight expects {k}")
+    if x.shape[-1] != k:
+        raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     _need(0 < c <= n and c % 8 == 0 and n % 8 == 0, "the normed columns must be a multiple of 8 within the output")
     m = x.numel() // k
     h = torch.empty(m, n, dtype=x.dtype, device=dev)
@@ -834,7 +857,8 @@ def w8a16_qkv_rope_and_cache(x, w, cos, sin, key_cache, value_cache, slot_mappin
     _need(value_cache.shape == key_cache.shape, "cache shapes differ")
     n, k = w.n, w.k
     _need(n == (n_heads + 2 * n_kv) * d, "weight rows do not match the head geometry")
-    _need(x.shape[-1] == k, f"x has {x.shape[-1]} input channels, weight expects {k}")
+    if x.shape[-1] != k:
+        raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
     _need(slot_mapping.dtype == torch.int32 and slot_mapping.numel() == m, "slot_mapping must be int32 [T]")
     _need(cos.dtype == sin.dtype and cos.numel() == m * d and sin.numel() == m * d, "cos/sin must be [T, head_dim]")
@@ -890,7 +914,8 @@ def w8a16_gated_linear(x, w, bias=None):
     dev = _dev_ok(x, bias)
     _need(x.dtype in _ACT, "x must be bf16/fp16")
     n, k = w.n, w.k
-    _need(x.shape[-1] == k, f"x has {x.shape[-1]} input channels, weight expects {k}")
+    if x.shape[-1] != k:
+        raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
     y = torch.empty(*x.shape[:-1], n // 2, dtype=x.dtype, device=dev)
     _need(bias is None or (bias.dtype == x.dtype and bias.numel() == n), "bias mismatch")
@@ -1046,7 +1071,8 @@ def _w8a8_operands(lib, xq, x_scale, w, what):
     tiled = isinstance(xq, TiledInt8Activations)
     xshape = xq.shape
     xdata = xq.data if tiled else xq
-    _need(xdata.dtype == torch.int8 and x_scale.dtype == torch.float32, f"{what}: xq must be int8, scales fp32")
+    if not (xdata.dtype == torch.int8 and x_scale.dtype == torch.float32):
+        raise ValueError(f"{what}: xq must be int8, scales fp32")
     _need(xshape[-1] == w.k, "shape mismatch")
     m = 1
     for d in xshape[:-1]:

@@ -108,13 +108,15 @@ class DecodeStackRunner:
         launches, 224 us with one copy and one launch.)"""
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("a step's host arrays cannot be captured: a replay would read them from a buffer given back")
-        at = np.concatenate([[0], np.cumsum([(a.size + 15) // 16 * 16 for a in arrays])])   # 64-byte pieces
-        host = torch.empty(int(at[-1]), dtype=torch.int32, pin_memory=True, device="cpu")   # whatever the default device
+        at = [0]
+        for a in arrays:
+            at.append(at[-1] + (a.size + 15) // 16 * 16)       # 64-byte pieces
+        host = torch.empty(at[-1], dtype=torch.int32, pin_memory=True, device="cpu")   # whatever the default device
         flat = host.numpy()
         for a, o in zip(arrays, at):
             flat[o:o + a.size] = a.reshape(-1)
         dev = host.to(self.device, non_blocking=True)
-        return [dev[o:o + a.size].view(a.shape) for a, o in zip(arrays, at)]
+        return [dev[o:o + a.size].view(a.shape) if a.ndim != 1 else dev[o:o + a.size] for a, o in zip(arrays, at)]
 
     def forward(self, hidden_states, valid_length_each_example, block_tables, slot_mapping, prefill=True,
                 position_ids=None, q_seq_lens=None):
