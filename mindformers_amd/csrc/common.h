@@ -369,6 +369,31 @@ __device__ __forceinline__ f16x8 dequant8_u4<FP16>(uint32_t w) {
     return v;
 }
 
+// q / 16 of the two's complement nibble in the low half of byte BYTE, exact (left to itself the compiler shifts the byte down first)
+template <int BYTE>
+__device__ __forceinline__ float i4_16th(uint32_t w) {
+    float f;
+    if constexpr (BYTE == 0) f = __builtin_amdgcn_cvt_off_f32_i4(w);
+    else if constexpr (BYTE == 1) asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f) : "v"(w));
+    else if constexpr (BYTE == 2) asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(f) : "v"(w));
+    else asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(f) : "v"(w));
+    return f;
+}
+// The same nibbles as q / 16, exact too: one instruction looks a two's complement nibble up where the form above takes two.
+template <typename T>
+__device__ __forceinline__ typename T::vec8 dequant8_u4_16th(uint32_t w) {
+    const uint32_t even = w ^ 0x88888888u, odd = even >> 4;    // q in the low nibble of bytes: elements 0 2 4 6 / 1 3 5 7
+    const float f[8] = {i4_16th<0>(even), i4_16th<0>(odd), i4_16th<1>(even), i4_16th<1>(odd),
+                        i4_16th<2>(even), i4_16th<2>(odd), i4_16th<3>(even), i4_16th<3>(odd)};
+    u32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (std::is_same_v<T, BF16>) v[i] = __builtin_amdgcn_perm(__float_as_uint(f[2 * i + 1]), __float_as_uint(f[2 * i]), 0x07060302u);
+        else v[i] = bitcast<uint32_t>(__builtin_amdgcn_cvt_pkrtz(f[2 * i], f[2 * i + 1]));
+    }
+    return bitcast<typename T::vec8>(v);
+}
+
 // Transposing 64-bit LDS read (ds_read_b64_tr_b16).  Within every group of 16 lanes, lane j names four consecutive
 // 16-bit values M[j][0..3]; lane i receives M[(i >> 2) + 4 e][i & 3] for e = 0..3.
 typedef __attribute__((ext_vector_type(4))) short s16x4;

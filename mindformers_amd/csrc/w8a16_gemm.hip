@@ -736,6 +736,101 @@ __global__ __launch_bounds__(256, 2) void w8a16_group_tile_kernel(
 #undef GT
 }
 
+// ---- 4-bit weights, few rows ----------------------------------------------------------------------------------------------------
+// A workgroup owns 16*NT channels of all the (up to 16) rows; its W waves cut K between them and meet in LDS at the end, so that nothing
+// else is shared: no staged activations, no barrier in the k-loop, no partial sums in memory and no second launch.  The 512-byte weight
+// tiles and a lane's own row of the activations (out of the caches; nothing for rows past the last) go from memory straight into operand
+// registers, D steps ahead; a set is loaded again when all of it has been used.  Weights enter as q / 16 (dequant8_u4_16th, 14
+// instructions for 8 weights where the kernel above has 23); the sums are multiplied by 16 at the end, exactly.
+// What bounds it: latency and instructions, at 2.4 to 4.6 TB/s of weights.  One row, groups of 128, cold weights, us, the kernel above with the sum
+// of its K parts | here: 4096 x 4096 10.0 | 6.2, 6144 x 4096 11.9 | 9.3, 28672 x 4096 28.8 | 20.0, 4096 x 14336 17.3 | 12.4, 8192 x 29568 51 |
+// 30; eight rows 10.3 | 7.4, 12.0 | 11.8, 28.8 | 22.2, 17.9 | 14.9, 51 | 33.
+template <typename T, int GROUP, int NT, int W>
+__global__ __launch_bounds__(64 * W) void w4a16_rows_kernel(
+    uint16_t* __restrict__ y, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, const float* __restrict__ scale,
+    const float* __restrict__ gscale, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N,
+    int K, int steps_per_wave) {
+    using vec8 = typename T::vec8;
+    constexpr int D = 4, TB = GW_TILE_BYTES / 2;
+    __shared__ f32x4 red[W][NT][64];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int KS = K / GW_KSTEP, s_begin = wv * steps_per_wave, s_end = min(KS, s_begin + steps_per_wave), s_last = max(s_end - 1, 0);
+    const int n_tiles = (N + 15) >> 4, tile0 = blockIdx.x * NT;
+    const uint8_t* wbase[NT];
+    const float* gbase[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int tile = min(tile0 + t, n_tiles - 1);
+        wbase[t] = wp + (int64_t)tile * TB;
+        gbase[t] = GROUP ? gscale + min(16 * tile + 4 * g, N - 4) : nullptr;   // channels past N: never stored
+    }
+    // rows past the last read as zeros without a fetch: their offsets lie behind the buffer's end
+    const auto xbuf = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00027000);
+    const int xrow = r < M ? r * K * 2 + 32 * g : 0x7ffff000;
+    u32x2 wreg[D][NT];
+    u32x4 xreg[D][2];
+    constexpr int GS = GROUP == 2 * GW_KSTEP ? 2 : 1;          // steps that share group scales
+    f32x4 greg[GROUP ? D / GS : 1][NT];
+    auto load = [&](auto setc, int s) {
+        constexpr int S = decltype(setc)::value;
+        const int sc = min(s, s_last);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) wreg[S][t] = gw_stream_load<u32x2>(wbase[t] + (int64_t)sc * n_tiles * TB + lane * 8);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) xreg[S][u] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, xrow + 16 * u, sc * (2 * GW_KSTEP), 0);
+        if constexpr (GROUP != 0 && S % GS == GS - 1)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) greg[S / GS][t] = *(const f32x4*)(gbase[t] + (int64_t)(sc * GW_KSTEP / GROUP) * N);
+    };
+    f32x4 acc[NT], tot[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = tot[t] = (f32x4)(0.f);
+    auto step = [&](auto jc, int s) {
+        constexpr int J = decltype(jc)::value;
+        vec8 wa[NT][2];
+        const vec8 xa[2] = {bitcast<vec8>(xreg[J][0]), bitcast<vec8>(xreg[J][1])};
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) wa[t][u] = dequant8_u4_16th<T>(wreg[J][t][u]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[t] = T::mfma16(wa[t][u], xa[u], acc[t]);
+        if constexpr (GROUP != 0) {
+            if (GROUP == GW_KSTEP || (J & 1)) {               // a group's last step (a wave begins on a group's border, D is even)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) tot[t][i] = __fmaf_rn(acc[t][i], greg[J / GS][t][i], tot[t][i]);
+                    acc[t] = (f32x4)(0.f);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);                    // the set is free: all of it has been used
+        load(jc, s + D);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (s_begin < s_end) {
+        static_for<D>([&](auto dc) { load(dc, s_begin + decltype(dc)::value); });
+        int s = s_begin;
+        for (; s + D <= s_end; s += D) static_for<D>([&](auto jc) { step(jc, s + decltype(jc)::value); });
+        static_for<D - 1>([&](auto jc) {
+            if (s + decltype(jc)::value < s_end) step(jc, s + decltype(jc)::value);
+        });
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) red[wv][t][lane] = GROUP ? tot[t] : acc[t];
+    __syncthreads();
+    if (wv >= NT) return;
+    f32x4 sum = red[0][wv][lane];                             // wave t: tile t, the waves' parts in order
+#pragma unroll
+    for (int w = 1; w < W; ++w) sum += red[w][wv][lane];
+    const int n = 16 * (tile0 + wv) + 4 * g;
+    if (r < M && n < N) store4<T>(y, bias, residual, scale, (int64_t)r * N, n, N, sum * 16.f);
+}
+
 template <typename T>
 __global__ void w8a16_splitk_reduce_kernel(uint16_t* __restrict__ y, const float* __restrict__ partial,
                                            const float* __restrict__ scale, const uint16_t* __restrict__ bias,
@@ -1100,6 +1195,35 @@ void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale,
         hipLaunchKernelGGL((w8a16_tile_reduce_kernel<T, 4>), dim3((g.m_blocks * g.n_blocks - g.full) * tg::WAVES * 4), dim3(256), 0, st,
                            (uint16_t*)y, (const float*)workspace, scale, (const uint16_t*)bias, (const uint16_t*)residual, m,
                            n, gated, aligned, g);
+}
+
+// Every lane group reads the activations itself, so the rows have to be few: with 16 the other kernel is the faster one on most shapes
+// (4096 x 14336 16.4 us against 20; with eight 17.9 against 14.9).  (K: 32-bit offsets.)
+bool use_w4_rows(int m, int k) { return m <= 8 && k < (1 << 26); }
+// Two channel tiles a workgroup, which share the activations' operands, where that leaves a workgroup for every compute unit (8192 x 29568:
+// 35 us with one, 26 with two; 6144 x 4096, 384 tiles: 8.8 / 8.4).  Waves cut K until the launch has 2048, with at least four steps each
+// (28672 x 4096: 17.4 us on four waves a workgroup, 20.2 on eight).
+template <typename T>
+void launch_w4_rows(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias, const void* residual, int m,
+                    int n, int k, int group, hipStream_t st) {
+    const int steps = k / GW_KSTEP, tiles = (n + 15) / 16, nt = tiles >= 512 ? 2 : 1;
+    int waves = 4;
+    while (waves < 16 && (tiles + nt - 1) / nt * waves < 2048 && steps / (2 * waves) >= 4) waves *= 2;
+    const int per = ((steps + waves - 1) / waves + 1) / 2 * 2;  // groups of 128 columns are two steps
+    const dim3 grid((tiles + nt - 1) / nt);
+    const float *gs = group ? scale : nullptr, *sc = group ? nullptr : scale;
+#define W4R(G, NT, W)                                                                                             \
+    hipLaunchKernelGGL((w4a16_rows_kernel<T, G, NT, W>), grid, dim3(64 * W), 0, st, (uint16_t*)y, (const uint16_t*)x, wp, sc, gs, \
+                       (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, per)
+#define W4R_G(NT, W)                                                                                              \
+    { if (group == 0) W4R(0, NT, W); else if (group == 64) W4R(64, NT, W); else W4R(128, NT, W); }
+#define W4R_W(NT)                                                                                                 \
+    { if (waves == 4) W4R_G(NT, 4) else if (waves == 8) W4R_G(NT, 8) else W4R_G(NT, 16) }
+    if (nt == 2) W4R_W(2)
+    else W4R_W(1)
+#undef W4R_W
+#undef W4R_G
+#undef W4R
 }
 
 template <typename T>
@@ -1469,7 +1593,7 @@ extern "C" int mf_w4a16_pack_weight(void* packed, const int8_t* w, int n, int k,
 }
 
 extern "C" size_t mf_w4a16_workspace_bytes(int m, int n, int k, int group_size) {
-    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    if (m <= 0 || n <= 0 || k <= 0 || use_w4_rows(m, k)) return 0;
     const GemmPlan p = plan_w8a16(m, n, k, group_size == 128 ? 2 : 1);
     return p.split_k > 1 ? (size_t)p.split_k * m * n * sizeof(float) : 0;
 }
@@ -1491,6 +1615,11 @@ extern "C" int mf_w4a16_gemm(void* y, const void* x, const void* w_packed, const
     const size_t need = mf_w4a16_workspace_bytes(m, n, k, group_size);
     MF_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0),
                "w4a16_gemm: 16-byte aligned workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+    if (use_w4_rows(m, k)) {
+        if (dtype == MF_BF16) launch_w4_rows<BF16>(y, x, (const uint8_t*)w_packed, scale, bias, residual, m, n, k, group_size, (hipStream_t)stream);
+        else launch_w4_rows<FP16>(y, x, (const uint8_t*)w_packed, scale, bias, residual, m, n, k, group_size, (hipStream_t)stream);
+        return MF_LAUNCH_CHECK();
+    }
     if (dtype == MF_BF16)
         return launch_w8a16<BF16>(y, x, (const uint8_t*)w_packed, scale, bias, residual, m, n, k, 0, workspace,
                                   (hipStream_t)stream, nullptr, nullptr, 0.f, MF_FP32, nullptr, group_size);

@@ -1296,6 +1296,14 @@ def test_w4a16_exact_on_integer_grid(group, m, n, k):
     assert np.array_equal(to_np(y).astype(np.float64), rounded(exact, torch.float16).astype(np.float64))
 
 
+@pytest.mark.parametrize("group", [0, 64, 128])
+@pytest.mark.parametrize("m,n,k", [(1, 132, 128), (8, 8212, 2176), (9, 132, 640), (7, 64, 8320), (5, 20, 1920), (2, 8192, 8192)])
+def test_w4a16_few_rows_exact_on_integer_grid(group, m, n, k):
+    """The same for the kernel of few rows: one and two channel tiles a workgroup with a ragged last one, waves with more steps than
+    others and with none, every number of waves, and the first row count that it does not serve."""
+    test_w4a16_exact_on_integer_grid(group, m, n, k)
+
+
 def test_w4a16_rejects_bad_operands():
     wq = torch.zeros(64, 128, dtype=torch.int8, device="cuda")
     s = torch.ones(64, device="cuda")
