@@ -82,7 +82,7 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, int n_heads, int n_kv,
     int n_rep, int block_size, int max_blocks, int num_blocks, int max_parts, float scale_log2, int64_t q_stride,
     int batch, const int32_t* __restrict__ q_starts, int part_tokens, int64_t kv_stride, int rows,
-    int64_t v_stride, const float* __restrict__ kv_scale, const float* __restrict__ kv_offset) {
+    int64_t v_stride, const float* __restrict__ kv_scale, const float* __restrict__ kv_offset, float lazy_log2) {
     using vec8 = typename T::vec8;
     using S = PfSmem<D>;
     // Type of the probabilities and of the widened values in the PV product.  int8 values are exact in either type and fp16 rounds
@@ -365,9 +365,9 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     // a column can find a whole tile masked before it has seen any token; starting the running maximum above the
     // mask value makes those probabilities 2^(-huge) = 0 instead of 2^0.  Maxima are kept in raw score units: the
     // (positive) softmax scale is applied inside the exponent.
-    // m_run follows the running maximum lazily: it moves only when the maximum exceeds it by more than 2^8 in
-    // probability (moving it means rescaling the accumulators); probabilities then lie in (0, 256], which bf16 and
-    // fp16 hold with the same relative precision, and the result does not depend on the reference point.
+    // m_run follows the running maximum lazily: it moves only when the maximum exceeds it by more than 2^lazy_log2 (at most 2^8)
+    // in probability (moving it means rescaling the accumulators); probabilities then lie in (0, 256], which bf16 and
+    // fp16 hold with the same relative precision.  Only the rounding depends on the reference point: see pf_plan16.
     // fp16 over int8 caches: the reference point is each tile's own maximum (but no more than 2^32 in probability under the largest
     // seen).  The token at the reference point has probability 1, which needs no rounding, and the 16-column kernel has more such
     // tokens than a lazy or a running maximum would give here (four waves with a maximum each): RMS error as above 3.37e-4 there,
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     float m_run = 0.5f * PA_NEG, l_run = 0.f;
     [[maybe_unused]] float m_peak = m_run;
     constexpr bool TILE_REF = KVQ == 1 && std::is_same<T, FP16>::value;
-    const float lazy = (TILE_REF ? 32.0f : 8.0f) / scale_log2;
+    const float lazy = (TILE_REF ? 32.0f : lazy_log2) / scale_log2;
 
     // One tile, living in ring buffer R = t mod 3 (a compile-time constant of the step): scores, softmax, PV product,
     // one phase after the other.  A wave does not overlap its own MFMAs with its own vector instructions, so nothing
@@ -578,7 +578,16 @@ struct PfPlan {
     int part_tokens;
     int max_parts;
     int64_t col_groups16, col_groups128;                      // upper bounds over the batch, per column-group width
+    float lazy_log2 = 8.f;                                    // how far the maximum may pass the reference point, log2
 };
+
+// the context in `parts` partitions of whole wave tiles, or fewer where rounding leaves some empty
+static inline void pf_cut(PfPlan& p, int64_t max_ctx, int64_t parts) {
+    int64_t pt = (max_ctx + parts - 1) / parts;
+    pt = std::max<int64_t>(PA_WAVE_TOKENS, (pt + PA_WAVE_TOKENS - 1) / PA_WAVE_TOKENS * PA_WAVE_TOKENS);
+    p.part_tokens = (int)pt;
+    p.max_parts = (int)std::max<int64_t>(1, (max_ctx + pt - 1) / pt);
+}
 
 static inline PfPlan pf_plan(int batch, int64_t total_q, int n_heads, int n_kv, int64_t max_ctx) {
     const int n_rep = n_heads / n_kv;
@@ -590,12 +599,40 @@ static inline PfPlan pf_plan(int batch, int64_t total_q, int n_heads, int n_kv, 
     const int64_t wgs = std::max<int64_t>(1, groups) * n_kv;
     int64_t want = (512 + wgs - 1) / wgs;                     // 2 workgroups per CU are resident at a time
     const int64_t most = std::max<int64_t>(1, (max_ctx + 255) / 256);
-    want = std::min(want, most);
-    int64_t pt = (max_ctx + want - 1) / want;
-    pt = std::max<int64_t>(PA_WAVE_TOKENS, (pt + PA_WAVE_TOKENS - 1) / PA_WAVE_TOKENS * PA_WAVE_TOKENS);
-    p.part_tokens = (int)pt;
-    p.max_parts = (int)std::max<int64_t>(1, (max_ctx + pt - 1) / pt);
+    pf_cut(p, max_ctx, std::min(want, most));
     return p;
+}
+
+// 16-bit keys and values: the plan above, or no cut at all where the partials would cost more than the shorter chains give.  A
+// cut pays where a chunk of rows looks back on a long cache; whole prompts have a context no longer than their own rows, and
+// mostly short ones.  Measured over 1/1 to 128/128 heads, 130 to 4096 rows in 1 to 4 prompts: a workgroup takes 8 us + 12 ns +
+// 0.058 ns a dimension for every token of its range (a third more where tiles straddle cache blocks), and a cut adds 0.5 us +
+// 0.33 us for every megabyte of partials written and read back, (1 + tokens / partition) / 2 of them a row of a whole prompt and
+// more of rows that look back.  The longest context is the block table's width; of packed prompts it is taken to lie half-way
+// between their mean and all of the rows (it sets the time, and a batch of one long and many short ones must not lose its cut).
+// us with the plan above | with this one: 28/4 heads, 2 prompts of 1531 rows together 41.5 | 35.1; 32/8, 1024 rows in 4 prompts
+// 26.6 | 15.4, 512 in one 21.6 | 20.2; 16 heads of 192, 300 rows 20.1 | 17.8; 8/1, one prompt of 2048 rows (still cut in four)
+// 33.6 both, uncut 48.1; 16 chunks of 64 rows over 700 tokens, 32/8 35.0 | 28.6.  By a quarter: where the two come closer, a lone chunk
+// beside decoding rows loses (1024 + 16 rows over 1024 tokens, 28/4, blocks of 16, 0.93 of the cut one's price 38.0 | 43.0).
+// The probability at a reference point is 1 and needs no rounding, and a cut row has a reference point in each partition: at 2^8
+// the uncut rows' RMS error against float64 is up to 0.2 % larger (512 rows of 32/8 heads, bf16: 2.0051e-3 cut, 2.0089e-3), so
+// here it moves earlier (2.0025e-3; 2^3: 2.0051e-3, 2^2: 1.9941e-3; 33.3 and 35.3 us for the two prompts above, 32.5 at 2^8).
+// The plan above's workspace serves both; 192-wide heads have one plan whichever value width they come with (the call with
+// 128-wide values has the bits of the one with padded values).
+static inline PfPlan pf_plan16(int batch, int64_t total_q, int n_heads, int n_kv, int head_dim, int64_t max_ctx, bool packed,
+                               bool tile_in_block) {
+    const PfPlan cut = pf_plan(batch, total_q, n_heads, n_kv, max_ctx);
+    if (cut.max_parts == 1) return cut;
+    const float longest = packed ? (0.5f + 0.5f / batch) * total_q : (float)max_ctx;
+    const float us_a_token = (0.012f + 0.000058f * head_dim) * (tile_in_block ? 1.f : 1.35f);
+    const float mb = 8e-6f * (std::min(head_dim, 128) + 2) * total_q * n_heads;   // one partial a row and head, written and read
+    const float cut_us = us_a_token * std::min(longest, (float)cut.part_tokens) + 0.5f +
+                         0.33f * mb * 0.5f * (1.f + longest / cut.part_tokens);
+    if (us_a_token * longest >= 0.75f * cut_us) return cut;
+    PfPlan whole = cut;
+    pf_cut(whole, max_ctx, 1);
+    whole.lazy_log2 = 2.5f;
+    return whole;
 }
 
 // int8 caches with per-channel scales: the 16-column kernel or the 128-column one.  The 128-column kernel widens a tile for
@@ -647,7 +684,9 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
     const int n_rep = n_heads / n_kv;
     const bool contiguous = block_tables == nullptr;
     const int64_t max_ctx = contiguous ? total_q : (int64_t)max_blocks * block_size;
-    const PfPlan plan = pf_plan(batch, total_q, n_heads, n_kv, max_ctx);
+    const bool tib_tok = contiguous || block_size % PF_TOK == 0;       // a staged tile never straddles two blocks
+    const PfPlan plan = KVQ == 0 ? pf_plan16(batch, total_q, n_heads, n_kv, D, max_ctx, contiguous, tib_tok)
+                                 : pf_plan(batch, total_q, n_heads, n_kv, max_ctx);
     float* part_out = plan.max_parts > 1 ? (float*)workspace : nullptr;
     float* part_ml = part_out ? part_out + (int64_t)total_q * n_heads * plan.max_parts * DV : nullptr;
     const float scale_log2 = scale * 1.4426950408889634f;
@@ -677,7 +716,6 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
 #undef PF_LAUNCH
     }
     if constexpr (KVQ != 2) if (!cols16) {
-        const bool tib = contiguous || block_size % PF_TOK == 0;   // a staged tile never straddles two blocks
         static bool lds_set[2][MF_MAX_DEVICES] = {};          // the tile buffers exceed the default dynamic LDS limit
         int dev = 0;
         hipError_t e = hipGetDevice(&dev);
@@ -695,9 +733,9 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
                            part_out, part_ml, (const uint16_t*)query, (const uint16_t*)key_cache,                 \
                            (const uint16_t*)value_cache, block_tables, context_lens, n_heads, n_kv, n_rep,        \
                            block_size, max_blocks, num_blocks, plan.max_parts, scale_log2, q_stride, batch,       \
-                           q_starts, plan.part_tokens, kv_stride, total_q, v_stride, kv_scale, kv_offset);        \
+                           q_starts, plan.part_tokens, kv_stride, total_q, v_stride, kv_scale, kv_offset, plan.lazy_log2); \
     }
-        if (tib) PF_LAUNCH(true)
+        if (tib_tok) PF_LAUNCH(true)
         else PF_LAUNCH(false)
 #undef PF_LAUNCH
     }

@@ -482,6 +482,37 @@ def test_causal_attention_varlen_vs_oracle(dtype, nh, nkv, d, q_lens, fused):
     assert_within(out, ref, mag, dtype, ulps=1.5, what="varlen causal attention")
 
 
+@pytest.mark.parametrize("nh,nkv,d,q_lens,bs", [
+    (32, 8, 128, [130, 127], 32), (28, 4, 128, [981, 550], 16), (16, 16, 64, [300], 8),               # no longer cut
+    (8, 1, 128, [2048], 64), (2, 1, 32, [513], 16), (4, 4, 64, [1, 700, 129], 32),                    # still cut
+])
+def test_whole_prompts_packed_and_paged_and_with_a_wide_table(nh, nkv, d, q_lens, bs):
+    """Whether the context is cut in partitions is decided by the rows and by the longest context there can be: short prompts are
+    not cut, packed or in a cache whose table fits them, but are when the table is wide.  All against the oracle.
+    Probabilities rounded to bf16 and their sum: 0.5 eps each way, the output 0.5 eps, all times (1 + eps) in the second order."""
+    rng = np.random.default_rng(nh + len(q_lens))
+    t, scale, dtype = int(np.sum(q_lens)), 1.0 / np.sqrt(d), torch.bfloat16
+    q, k, v = (rounded(rng.normal(size=(t, n * d)), dtype) for n in (nh, nkv, nkv))
+    starts = dev(_starts(q_lens), torch.int32)
+    ref = O.causal_prefill_attention(q, k, v, q_lens, nh, nkv, scale)
+    mag = O.causal_prefill_attention(q, k, np.abs(v), q_lens, nh, nkv, scale)
+    packed = to_np(ops.causal_attention_varlen(dev(q, dtype), dev(k, dtype), dev(v, dtype), starts, nh, nkv, scale))
+    assert_within(packed, ref, mag, dtype, ulps=1.51, what="packed rows")
+    blocks = [-(-n // bs) for n in q_lens]
+    kc, vc = (np.zeros((sum(blocks), bs, nkv, d), np.float32) for _ in range(2))
+    for width in (max(blocks), 8192 // bs):
+        tables = -np.ones((len(q_lens), width), np.int32)
+        first, row = 0, 0
+        for s, n in enumerate(q_lens):
+            tables[s, :blocks[s]] = np.arange(first, first + blocks[s])
+            for c, x in ((kc, k), (vc, v)):
+                c.reshape(-1, nkv, d)[first * bs:first * bs + n] = x[row:row + n].reshape(n, nkv, d)
+            first, row = first + blocks[s], row + n
+        paged = to_np(ops.paged_attention_prefill(dev(q, dtype), dev(kc, dtype), dev(vc, dtype), dev(tables, torch.int32),
+                                                  dev(np.array(q_lens), torch.int32), starts, nh, nkv, scale))
+        assert_within(paged, ref, mag, dtype, ulps=1.51, what=f"paged rows, table of {width} blocks")
+
+
 @pytest.mark.parametrize("dtype,nh,nkv,q_lens,strided", [
     (torch.bfloat16, 16, 16, [130, 1, 64], False), (torch.float16, 8, 2, [33, 200], True),
     (torch.bfloat16, 2, 2, [1500], False), (torch.bfloat16, 128, 128, [40, 300], True),
