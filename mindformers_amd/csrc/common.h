@@ -50,7 +50,7 @@ struct BF16 {
     static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }
-    // 32x32x16: twice the work of the 16x16x32 instruction in the same issue time
+    // 32x32x16: twice the work of the 16x16x32 instruction in twice the time, from as many operand registers
     static __device__ __forceinline__ f32x16 mfma32(vec8 a, vec8 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }

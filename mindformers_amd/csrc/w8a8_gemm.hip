@@ -20,8 +20,8 @@
 // applied on the global-address side, which makes the operand reads bank-conflict free.
 // Small N cannot fill the chip with output tiles alone: K is then split across workgroups, which write exact
 // int32 partial tiles that a second kernel sums (integer sums do not depend on the order).
-// More kernels serve the shapes where that one is not the best: from 65 rows on with tiled activations 128 x 256 tiles with
-// the full-rate v_mfma_i32_32x32x32_i8 (w8a8_tile_kernel); where those leave a part of a round over, for narrow outputs and
+// More kernels serve the shapes where that one is not the best: from 65 rows on with tiled activations 128 x 256 or 96 x 256
+// tiles with v_mfma_i32_16x16x64_i8 (w8a8_tile_kernel); where those leave a part of a round over, for narrow outputs and
 // few rows, a register-streaming kernel (w8a8_regs_kernel) and, for very wide outputs at 129+ rows (also where the tiles cannot
 // serve the call: accumulators asked for, N not a multiple of 16), 256 x 192 tiles on 8 waves with a coalesced, LDS-turned
 // epilogue (w8a8_wide_kernel).
