@@ -1200,15 +1200,17 @@ void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale,
 // Every lane group reads the activations itself, so the rows have to be few: with 16 the other kernel is the faster one on most shapes
 // (4096 x 14336 16.4 us against 20; with eight 17.9 against 14.9).  (K: 32-bit offsets.)
 bool use_w4_rows(int m, int k) { return m <= 8 && k < (1 << 26); }
-// Two channel tiles a workgroup, which share the activations' operands, where that leaves a workgroup for every compute unit (8192 x 29568:
-// 35 us with one, 26 with two; 6144 x 4096, 384 tiles: 8.8 / 8.4).  Waves cut K until the launch has 2048, with at least four steps each
-// (28672 x 4096: 17.4 us on four waves a workgroup, 20.2 on eight).
+// Two channel tiles a workgroup, which share the activations' operands, where one would leave more workgroups than compute units and
+// with them a second, part-filled round.  Waves cut K until the launch has 2048, with at least four steps each; no more than eight
+// with two tiles, whose accumulators and operands fill the registers of sixteen.  Eight rows, groups of 128, cold weights, us, one tile | two on
+// up to 16 waves | two on up to 8: 6144 x 4096 11.3 | 10.2 | 8.3, 6144 x 8192 17.4 | 14.3 | 12.3, 4112 x 4096 10.8 | 10.1 | 8.3, 8176 x 14336
+// 26.6 | 19.3 | 19.3; one row 9.1 | 8.9 | 7.4, 14.1 | 12.7 | 11.1, 7.9 | 8.8 | 7.3, 22.2 | 17.7 | 17.8.
 template <typename T>
 void launch_w4_rows(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias, const void* residual, int m,
                     int n, int k, int group, hipStream_t st) {
-    const int steps = k / GW_KSTEP, tiles = (n + 15) / 16, nt = tiles >= 512 ? 2 : 1;
+    const int steps = k / GW_KSTEP, tiles = (n + 15) / 16, nt = tiles > 256 ? 2 : 1, most = nt == 2 ? 8 : 16;
     int waves = 4;
-    while (waves < 16 && (tiles + nt - 1) / nt * waves < 2048 && steps / (2 * waves) >= 4) waves *= 2;
+    while (waves < most && (tiles + nt - 1) / nt * waves < 2048 && steps / (2 * waves) >= 4) waves *= 2;
     const int per = ((steps + waves - 1) / waves + 1) / 2 * 2;  // groups of 128 columns are two steps
     const dim3 grid((tiles + nt - 1) / nt);
     const float *gs = group ? scale : nullptr, *sc = group ? nullptr : scale;
@@ -1217,11 +1219,11 @@ void launch_w4_rows(void* y, const void* x, const uint8_t* wp, const float* scal
                        (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, per)
 #define W4R_G(NT, W)                                                                                              \
     { if (group == 0) W4R(0, NT, W); else if (group == 64) W4R(64, NT, W); else W4R(128, NT, W); }
-#define W4R_W(NT)                                                                                                 \
-    { if (waves == 4) W4R_G(NT, 4) else if (waves == 8) W4R_G(NT, 8) else W4R_G(NT, 16) }
-    if (nt == 2) W4R_W(2)
-    else W4R_W(1)
-#undef W4R_W
+    if (nt == 2 && waves == 4) W4R_G(2, 4)
+    else if (nt == 2) W4R_G(2, 8)
+    else if (waves == 4) W4R_G(1, 4)
+    else if (waves == 8) W4R_G(1, 8)
+    else W4R_G(1, 16)
 #undef W4R_G
 #undef W4R
 }
