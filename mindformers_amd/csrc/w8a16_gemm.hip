@@ -1197,9 +1197,26 @@ void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale,
                            n, gated, aligned, g);
 }
 
-// Every lane group reads the activations itself, so the rows have to be few: with 16 the other kernel is the faster one on most shapes
-// (4096 x 14336 16.4 us against 20; with eight 17.9 against 14.9).  (K: 32-bit offsets.)
-bool use_w4_rows(int m, int k) { return m <= 8 && k < (1 << 26); }
+// Every lane group reads the activations itself, so the rows have to be few.  The other kernel cuts K between workgroups, so it wins where
+// the channel tiles are too few for the compute units and K is long, and with groups of 64 (twice the scale loads) where the workgroups
+// fill their last round to five eighths at most or the many short workgroups of wide outputs start and end more than they work.
+// Measured at 64 to 65536 channels, K 256 to 29568, 1 to 8 rows, cold weights: 14 of 9954 calls are left more than 3 % slower than on the
+// other kernel, by 8 % at most (64 channels, and 129 to 160 tiles in groups of 64).  us at eight rows, the other kernel | this one: per channel
+// 1024 x 14336 9.3 | 13.5, 65536 x 1024 13.2 | 16.6; groups of 128: 2560 x 18944 21.0 | 19.2; groups of 64: 512 x 8192 10.0 | 11.8, 4112 x
+// 29568 32.0 | 36.6, 10240 x 8192 22.4 | 24.7, 28672 x 1024 9.6 | 11.3, 65536 x 3072 35.9 | 40.0.  At 9 to 16 rows either may be the faster
+// one by half (groups of 128, 12 rows: 8192 x 8192 takes 0.71 of the other kernel's time, 3072 x 8192 1.04, 1024 x 14336 1.61).  (K:
+// 32-bit offsets.)
+bool use_w4_rows(int m, int n, int k, int group) {
+    const int steps = k / GW_KSTEP, tiles = (n + 15) / 16, pairs = (tiles + 1) / 2;
+    const bool g64 = group == 64;
+    if (m > 8 || k >= (1 << 26)) return false;
+    if (tiles <= 128) return steps * (10 + m + 2 * g64) <= 1790;
+    if (steps <= 16) return tiles <= (g64 ? 1536 : 2560);
+    if (!g64 || tiles <= 256) return true;
+    if (pairs <= 160) return steps <= 192;
+    if (pairs > 256 && pairs <= 320) return steps < 64 || m <= 2;
+    return tiles <= 2560 || steps > 48;
+}
 // Two channel tiles a workgroup, which share the activations' operands, where one would leave more workgroups than compute units and
 // with them a second, part-filled round.  Waves cut K until the launch has 2048, with at least four steps each; no more than eight
 // with two tiles, whose accumulators and operands fill the registers of sixteen.  Eight rows, groups of 128, cold weights, us, one tile | two on
@@ -1595,7 +1612,7 @@ extern "C" int mf_w4a16_pack_weight(void* packed, const int8_t* w, int n, int k,
 }
 
 extern "C" size_t mf_w4a16_workspace_bytes(int m, int n, int k, int group_size) {
-    if (m <= 0 || n <= 0 || k <= 0 || use_w4_rows(m, k)) return 0;
+    if (m <= 0 || n <= 0 || k <= 0 || use_w4_rows(m, n, k, group_size)) return 0;
     const GemmPlan p = plan_w8a16(m, n, k, group_size == 128 ? 2 : 1);
     return p.split_k > 1 ? (size_t)p.split_k * m * n * sizeof(float) : 0;
 }
@@ -1617,7 +1634,7 @@ extern "C" int mf_w4a16_gemm(void* y, const void* x, const void* w_packed, const
     const size_t need = mf_w4a16_workspace_bytes(m, n, k, group_size);
     MF_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0),
                "w4a16_gemm: 16-byte aligned workspace of %zu bytes needed, %zu given", need, workspace_bytes);
-    if (use_w4_rows(m, k)) {
+    if (use_w4_rows(m, n, k, group_size)) {
         if (dtype == MF_BF16) launch_w4_rows<BF16>(y, x, (const uint8_t*)w_packed, scale, bias, residual, m, n, k, group_size, (hipStream_t)stream);
         else launch_w4_rows<FP16>(y, x, (const uint8_t*)w_packed, scale, bias, residual, m, n, k, group_size, (hipStream_t)stream);
         return MF_LAUNCH_CHECK();

@@ -77,6 +77,19 @@ def test_plans_of_the_shapes_that_the_tile_kernels_are_tested_at():
         assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, *plan), (m, n, k)
 
 
+def test_few_row_4_bit_products_take_the_kernel_that_cuts_k_where_that_is_the_faster_one():
+    """The few-row kernel needs no workspace, the one that cuts K between workgroups does (at these sizes): narrow outputs with a long
+    K, and groups of 64 where the few-row kernel's workgroups leave most of a round empty, were slower on the former."""
+    from mindformers_amd import _lib
+    lib = _lib.load()
+    for m, n, k, group in [(8, 64, 16384, 0), (1, 1024, 14336, 128), (4, 2048, 14336, 64), (8, 512, 8192, 0), (8, 4112, 29568, 64),
+                           (8, 10240, 8192, 64), (9, 4096, 4096, 128)]:
+        assert lib.mf_w4a16_workspace_bytes(m, n, k, group) > 0, (m, n, k, group)
+    for m, n, k, group in [(8, 64, 2048, 0), (1, 1024, 8192, 128), (8, 4096, 14336, 64), (8, 2560, 18944, 128), (8, 4112, 8192, 64),
+                           (8, 28672, 4096, 128), (1, 6144, 4096, 0)]:
+        assert lib.mf_w4a16_workspace_bytes(m, n, k, group) == 0, (m, n, k, group)
+
+
 def test_plans_of_the_shapes_that_the_96_row_tiles_are_tested_at():
     """Tiles of 96 rows where they fit the device at once: their number is not that of 128-row tiles, and nothing is cut along K."""
     from mindformers_amd import _lib

@@ -1328,10 +1328,15 @@ def test_w4a16_exact_on_integer_grid(group, m, n, k):
 
 
 @pytest.mark.parametrize("group", [0, 64, 128])
-@pytest.mark.parametrize("m,n,k", [(1, 132, 128), (8, 8212, 2176), (9, 132, 640), (7, 64, 8320), (5, 20, 1920), (2, 8192, 8192)])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 132, 128), (5, 20, 1920), (6, 1040, 2176), (7, 64, 4224),       # one channel tile a workgroup: 4, 4, 8 and 16 waves
+    (3, 8200, 1920), (8, 8212, 2176), (6, 4112, 4224), (2, 8192, 8192),  # two: 4 and 8 waves, also with an odd number of tiles
+    (9, 132, 640), (7, 64, 8320)])                                      # the other kernel: more rows, a long K of few channels
 def test_w4a16_few_rows_exact_on_integer_grid(group, m, n, k):
-    """The same for the kernel of few rows: one and two channel tiles a workgroup with a ragged last one, waves with more steps than
-    others and with none, every number of waves, and the first row count that it does not serve."""
+    """The same for the kernel of few rows in each of its forms, with ragged last tiles, waves with more steps than others and with
+    none, and on both sides of the lines where it ends."""
+    few = m <= 8 and k != 8320
+    assert not few or ops._lib.load().mf_w4a16_workspace_bytes(m, n, k, group) == 0       # the other one cuts K in most of these
     test_w4a16_exact_on_integer_grid(group, m, n, k)
 
 
