@@ -71,10 +71,13 @@ inline TileGrid tg_plan_rows(int m, int mt, int n_blocks, int steps, const TileC
 }
 
 // 128-row tiles, or 96-row ones where those are all resident at once, each on a compute unit of its own: more units then share the
-// work, and fewer rows are padding.  A plan that is cut along K gives way only to a clearly shorter one (the model is good to some
-// 10 %), one of few k-steps not at all, nor a single row block, which has no more tiles then.  W8A16, us, 128 | 96 rows: 1048 x
-// 4096 x 14336 157 | 135, 1300 x 4096 x 4096 53 | 46, 2025 x 2112 x 7168 (cut in parts) 83 | 71, 129 x 28672 x 4096 62 | 50, but 65 x 28672 x 4096
-// 42 | 46; W8A8: 1531 x 3584 x 18944 120 | 111, 1531 x 3584 x 3584 30.7 | 26.4, 1300 x 4608 x 3584 32.7 | 27.8.
+// work, and fewer rows are padding.  One of few k-steps does not change, nor a single row block, which has no more tiles then.  W8A16, us,
+// 128 | 96 rows: 1048 x 4096 x 14336 157 | 135, 1300 x 4096 x 4096 53 | 46, 2025 x 2112 x 7168 83 | 71, 129 x 28672 x 4096 62 | 50, but
+// 65 x 28672 x 4096 42 | 46; W8A8: 1531 x 3584 x 18944 120 | 111, 1531 x 3584 x 3584 30.7 | 26.4, 1300 x 4608 x 3584 32.7 | 27.8.
+// Nor does a plan that is cut along K: with so few tiles its parts are all resident too, and they share the units better than 96-row
+// tiles do (23 of 23 shapes measured; W8A16 777 x 4096 x 4096 37.6 | 44.0, 513 x 6144 x 4096 38.5 | 44.5, 864 x 3584 x 3584 34.0 | 40.1; W8A8
+// 1632 x 2112 x 7168 35.8 | 39.3, 448 x 5120 x 5120 27.4 | 29.8).  The model prices parts that run at once too high (0.015 us each there,
+// not c.part), so against other kernels such a plan counts no more than the 96-row tiles would.
 inline TileGrid tg_plan(int m, int n_blocks, int steps, const TileCost& c, float* us) {
     const TileGrid g = tg_plan_rows(m, 4, n_blocks, steps, c, us);
     const int m_blocks = (m + 95) / 96;
@@ -82,6 +85,7 @@ inline TileGrid tg_plan(int m, int n_blocks, int steps, const TileCost& c, float
     const float us3 = steps * c.alone3 + c.fixed;
     if (m <= 128 || steps < 16 || tiles > 256 || us3 >= (g.split > 1 ? 0.85f : 1.f) * *us) return g;
     *us = us3;
+    if (g.split > 1) return g;
     return {m_blocks, n_blocks, (int)tiles / 8 * 8, 1, steps, 3};
 }
 

@@ -100,6 +100,16 @@ def test_plans_of_the_shapes_that_the_96_row_tiles_are_tested_at():
         assert _plan(lib.mf_w8a8_plan, m, n, k, 0) == (tiles8, whole, 0, 1), (m, n, k)
 
 
+def test_a_plan_that_is_cut_along_k_keeps_its_128_row_tiles():
+    """Its parts share the compute units better than whole tiles of 96 rows do."""
+    from mindformers_amd import _lib
+    lib, tiles8, tiles16 = _lib.load(), 3, 1
+    for (m, n, k), cut in {(777, 4096, 4096): 112, (513, 6144, 4096): 120, (960, 4096, 4096): 128, (864, 3584, 3584): 98}.items():
+        assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, 0, cut, 2), (m, n, k)
+    for (m, n, k), cut in {(1632, 2112, 7168): 117, (448, 5120, 5120): 80}.items():
+        assert _plan(lib.mf_w8a8_plan, m, n, k, 0) == (tiles8, 0, cut, 2), (m, n, k)
+
+
 def test_w8a8_plans_take_the_faster_kernel_at_the_measured_lines():
     """One round of wide tiles against a round and a part of 128 x 256 ones, the LDS-staged kernel where the tiles leave half the
     device idle, and the wide kernel above 256 rows where the tiles cannot serve the width."""
