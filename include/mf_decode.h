@@ -164,6 +164,10 @@ int mf_paged_attention_decode_int8kv(void* out, const void* query, const void* k
                                      int n_heads, int n_kv_heads, int head_dim, int block_size,
                                      int max_blocks_per_seq, int num_blocks, float scale, int64_t q_row_stride,
                                      int dtype, void* workspace, size_t workspace_bytes, void* stream);
+/* Partitions that mf_paged_attention_prefill (16-bit caches) cuts the longest context in for these sizes, 1 = none; block_size 0 =
+ * packed rows, else max_context = block_size * max_blocks_per_seq.  Host arithmetic only, for tests and tools. */
+int mf_paged_attention_prefill_partitions(int batch, int total_q, int n_heads, int n_kv_heads, int head_dim, int block_size,
+                                          int max_context);
 int mf_paged_attention_prefill_int8kv(void* out, const void* query, const void* key_cache, const void* value_cache,
                                       const int32_t* block_tables, const int32_t* context_lens,
                                       const int32_t* q_starts, const float* antiquant_scale,

@@ -605,30 +605,33 @@ static inline PfPlan pf_plan(int batch, int64_t total_q, int n_heads, int n_kv, 
 
 // 16-bit keys and values: the plan above, or no cut at all where the partials would cost more than the shorter chains give.  A
 // cut pays where a chunk of rows looks back on a long cache; whole prompts have a context no longer than their own rows, and
-// mostly short ones.  Measured over 1/1 to 128/128 heads, 130 to 4096 rows in 1 to 4 prompts: a workgroup takes 8 us + 12 ns +
+// mostly short ones.  Measured over 1/1 to 128/128 heads, 80 to 4096 rows in 1 to 16 prompts: a workgroup takes 8 us + 12 ns +
 // 0.058 ns a dimension for every token of its range (a third more where tiles straddle cache blocks), and a cut adds 0.5 us +
 // 0.33 us for every megabyte of partials written and read back, (1 + tokens / partition) / 2 of them a row of a whole prompt and
-// more of rows that look back.  The longest context is the block table's width; of packed prompts it is taken to lie half-way
-// between their mean and all of the rows (it sets the time, and a batch of one long and many short ones must not lose its cut).
-// us with the plan above | with this one: 28/4 heads, 2 prompts of 1531 rows together 41.5 | 35.1; 32/8, 1024 rows in 4 prompts
-// 26.6 | 15.4, 512 in one 21.6 | 20.2; 16 heads of 192, 300 rows 20.1 | 17.8; 8/1, one prompt of 2048 rows (still cut in four)
-// 33.6 both, uncut 48.1; 16 chunks of 64 rows over 700 tokens, 32/8 35.0 | 28.6.  By a quarter: where the two come closer, a lone chunk
-// beside decoding rows loses (1024 + 16 rows over 1024 tokens, 28/4, blocks of 16, 0.93 of the cut one's price 38.0 | 43.0).
-// The probability at a reference point is 1 and needs no rounding, and a cut row has a reference point in each partition: at 2^8
-// the uncut rows' RMS error against float64 is up to 0.2 % larger (512 rows of 32/8 heads, bf16: 2.0051e-3 cut, 2.0089e-3), so
-// here it moves earlier (2.0025e-3; 2^3: 2.0051e-3, 2^2: 1.9941e-3; 33.3 and 35.3 us for the two prompts above, 32.5 at 2^8).
+// more of rows that look back.  The longest context is taken to be the most there can be, the block table's width (a table wider than
+// any context counts in full) or all of the packed rows: it sets the time, and a batch of one long and many short ones must not lose
+// its cut.  us with the plan above | uncut: 28/4 heads, 2 prompts of 1531 rows together 43.3 | 33.5; 32/8, 1024 rows in 4 prompts 29.1 |
+// 18.0, 512 in one 23.7 | 22.6; 16 heads of 192, 300 rows 22.2 | 20.5; 16 chunks of 64 rows over 700 tokens, 32/8 38.7 | 32.8; still
+// cut: 8/1, one prompt of 2048 rows 36.1 | 53.4, and beside 15 prompts of one row 16 heads of 64, 1009 rows, 21.9 | 27.0, 16 of 192 35.5 |
+// 42.1 (so are 16 even prompts of 1531 rows together, 24/8 heads, 27.5 | 16.3: the sizes are the same).  By 15 % for packed rows
+// (at the same price 400 rows of 16/2 heads 18.2 | 20.0) and by a quarter in a cache, where a lone chunk beside decoding rows loses
+// when the two come closer (1024 + 16 rows over 1024 tokens, 28/4, blocks of 16, 0.93 of the cut one's price 38.0 | 43.0).
+// The probability at a reference point is 1 and needs no rounding, and a cut row has a reference point in each partition: where it
+// moves at 2^8 the uncut rows' RMS error against float64 is up to 0.6 % larger, so here it moves at 2^2.5.  512 rows of 32/8 heads in
+// bf16, error and us: cut 2.0052e-3 23.7, uncut at 2^8 2.0091e-3 21.6, 2^3 2.0053e-3 22.0, 2^2.5 2.0027e-3 22.6, 2^2 1.9942e-3 22.9; the two
+// prompts above 2.0357e-3 43.3, 2.0357e-3 32.0, 2.0308e-3 32.7, 2.0280e-3 33.5, 2.0182e-3 33.9; the 16 chunks 2.3085e-3 38.7, 2.3229e-3 31.8,
+// 2.3078e-3 32.4, 2.3013e-3 32.8, 2.2824e-3 33.5.
 // The plan above's workspace serves both; 192-wide heads have one plan whichever value width they come with (the call with
 // 128-wide values has the bits of the one with padded values).
 static inline PfPlan pf_plan16(int batch, int64_t total_q, int n_heads, int n_kv, int head_dim, int64_t max_ctx, bool packed,
                                bool tile_in_block) {
     const PfPlan cut = pf_plan(batch, total_q, n_heads, n_kv, max_ctx);
     if (cut.max_parts == 1) return cut;
-    const float longest = packed ? (0.5f + 0.5f / batch) * total_q : (float)max_ctx;
     const float us_a_token = (0.012f + 0.000058f * head_dim) * (tile_in_block ? 1.f : 1.35f);
     const float mb = 8e-6f * (std::min(head_dim, 128) + 2) * total_q * n_heads;   // one partial a row and head, written and read
-    const float cut_us = us_a_token * std::min(longest, (float)cut.part_tokens) + 0.5f +
-                         0.33f * mb * 0.5f * (1.f + longest / cut.part_tokens);
-    if (us_a_token * longest >= 0.75f * cut_us) return cut;
+    const float cut_us = us_a_token * std::min((float)max_ctx, (float)cut.part_tokens) + 0.5f +
+                         0.33f * mb * 0.5f * (1.f + (float)max_ctx / cut.part_tokens);
+    if (us_a_token * max_ctx >= (packed ? 0.85f : 0.75f) * cut_us) return cut;
     PfPlan whole = cut;
     pf_cut(whole, max_ctx, 1);
     whole.lazy_log2 = 2.5f;
@@ -772,6 +775,14 @@ extern "C" size_t mf_paged_attention_prefill_workspace_bytes(int batch, int tota
     const PfPlan plan = pf_plan(batch, total_q, n_heads, n_kv_heads, max_context);
     if (plan.max_parts <= 1) return 0;
     return (size_t)total_q * n_heads * plan.max_parts * (head_dim + 2) * sizeof(float);
+}
+
+extern "C" int mf_paged_attention_prefill_partitions(int batch, int total_q, int n_heads, int n_kv_heads, int head_dim,
+                                                     int block_size, int max_context) {
+    if (batch <= 0 || total_q <= 0 || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || block_size < 0) return 0;
+    const bool packed = block_size == 0;
+    return pf_plan16(batch, total_q, n_heads, n_kv_heads, head_dim, packed ? total_q : max_context, packed,
+                     block_size % PF_TOK == 0).max_parts;
 }
 
 extern "C" int mf_paged_attention_prefill_int8kv_columns(int batch, int total_q, int n_heads, int n_kv_heads, int head_dim,

@@ -77,6 +77,19 @@ def test_plans_of_the_shapes_that_the_tile_kernels_are_tested_at():
         assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, *plan), (m, n, k)
 
 
+def test_prompt_attention_is_cut_by_the_longest_context_there_can_be():
+    """Packed rows may all belong to one prompt, whatever the number of prompts: the sizes decide, so one long prompt among many short
+    ones keeps its partitions.  Rows in a cache go by the width of its table."""
+    from mindformers_amd import _lib
+    parts = _lib.load().mf_paged_attention_prefill_partitions
+    for nh, nkv, d, rows in [(16, 16, 64, 1024), (16, 16, 192, 1024), (12, 2, 128, 512), (8, 1, 128, 2048)]:
+        assert all(parts(batch, rows, nh, nkv, d, 0, 0) > 1 for batch in (1, 2, 16)), (nh, nkv, d, rows)
+    for nh, nkv, d, rows in [(28, 4, 128, 1531), (32, 8, 128, 1024), (32, 8, 128, 512), (128, 128, 192, 300), (32, 8, 128, 4137)]:
+        assert all(parts(batch, rows, nh, nkv, d, 0, 0) == 1 for batch in (1, 2, 16)), (nh, nkv, d, rows)
+    assert parts(2, 1531, 28, 4, 128, 16, 992) == 1 and parts(2, 1531, 28, 4, 128, 16, 8192) > 1
+    assert parts(17, 1040, 28, 4, 128, 16, 1024) > 1                       # a chunk beside decoding rows
+
+
 def test_few_row_4_bit_products_take_the_kernel_that_cuts_k_where_that_is_the_faster_one():
     """The few-row kernel needs no workspace, the one that cuts K between workgroups does (at these sizes): narrow outputs with a long
     K, and groups of 64 where the few-row kernel's workgroups leave most of a round empty, were slower on the former."""

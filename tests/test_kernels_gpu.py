@@ -482,14 +482,18 @@ def test_causal_attention_varlen_vs_oracle(dtype, nh, nkv, d, q_lens, fused):
     assert_within(out, ref, mag, dtype, ulps=1.5, what="varlen causal attention")
 
 
-@pytest.mark.parametrize("nh,nkv,d,q_lens,bs", [
-    (32, 8, 128, [130, 127], 32), (28, 4, 128, [981, 550], 16), (16, 16, 64, [300], 8),               # no longer cut
-    (8, 1, 128, [2048], 64), (2, 1, 32, [513], 16), (4, 4, 64, [1, 700, 129], 32),                    # still cut
-])
-def test_whole_prompts_packed_and_paged_and_with_a_wide_table(nh, nkv, d, q_lens, bs):
+@pytest.mark.parametrize("nh,nkv,d,q_lens,bs,parts", [
+    (32, 8, 128, [130, 127], 32, (1, 1, 8)), (28, 4, 128, [981, 550], 16, (1, 1, 2)), (16, 16, 192, [300], 0, (1,)),
+    (32, 8, 128, [512], 8, (1, 2, 4)), (16, 16, 64, [300], 8, (2, 2, 11)), (8, 1, 128, [2048], 64, (4, 4, 4)),
+    (2, 1, 32, [513], 16, (3, 3, 32)), (4, 4, 64, [1, 700, 129], 32, (4, 3, 16)),
+    (12, 2, 128, [497] + [1] * 15, 16, (2, 2, 11))])                       # one long prompt among short ones: cut, whatever their number
+def test_whole_prompts_packed_and_paged_and_with_a_wide_table(nh, nkv, d, q_lens, bs, parts):
     """Whether the context is cut in partitions is decided by the rows and by the longest context there can be: short prompts are
-    not cut, packed or in a cache whose table fits them, but are when the table is wide.  All against the oracle.
+    not cut, packed or in a cache whose table fits them, but are when the table is wide.  ``parts``: partitions of the packed rows, of
+    the fitting table and of the wide one.  All against the oracle.
     Probabilities rounded to bf16 and their sum: 0.5 eps each way, the output 0.5 eps, all times (1 + eps) in the second order."""
+    plan = lambda width: ops._lib.load().mf_paged_attention_prefill_partitions(len(q_lens), sum(q_lens), nh, nkv, d, bs if width else 0,
+                                                                               width)
     rng = np.random.default_rng(nh + len(q_lens))
     t, scale, dtype = int(np.sum(q_lens)), 1.0 / np.sqrt(d), torch.bfloat16
     q, k, v = (rounded(rng.normal(size=(t, n * d)), dtype) for n in (nh, nkv, nkv))
@@ -498,7 +502,11 @@ def test_whole_prompts_packed_and_paged_and_with_a_wide_table(nh, nkv, d, q_lens
     mag = O.causal_prefill_attention(q, k, np.abs(v), q_lens, nh, nkv, scale)
     packed = to_np(ops.causal_attention_varlen(dev(q, dtype), dev(k, dtype), dev(v, dtype), starts, nh, nkv, scale))
     assert_within(packed, ref, mag, dtype, ulps=1.51, what="packed rows")
+    assert plan(0) == parts[0]
+    if bs == 0:
+        return
     blocks = [-(-n // bs) for n in q_lens]
+    assert (plan(max(blocks) * bs), plan(8192)) == parts[1:]
     kc, vc = (np.zeros((sum(blocks), bs, nkv, d), np.float32) for _ in range(2))
     for width in (max(blocks), 8192 // bs):
         tables = -np.ones((len(q_lens), width), np.int32)
