@@ -136,8 +136,14 @@ def ptr(t):
     return None if t is None else t.data_ptr()
 
 
+# by itself: a torch.cuda.Stream around the handle costs more than the rest of a small call's checks
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(device=None):
-    """Handle of the current stream of ``device``.  (By itself: a ``torch.cuda.Stream`` around it costs more than the rest of a
-    small call's checks.)"""
-    index = device.index if device is not None else None
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    """Handle of the current stream of ``device``: what ``torch.cuda.current_stream`` takes, and refused where it refuses (a device that
+    is not a GPU)."""
+    if _raw_stream is None or not isinstance(device, torch.device) or device.type != "cuda":
+        return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    return _raw_stream(torch.cuda.current_device() if index is None else index)

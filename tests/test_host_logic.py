@@ -55,6 +55,18 @@ def test_argument_errors_are_reported_without_a_gpu():
         _lib.check(rc, "mf_w8a16_gemm")
 
 
+@pytest.mark.parametrize("device", [torch.device("cpu"), "cpu", torch.device("meta")])
+def test_no_stream_of_a_device_that_is_not_a_gpu(device, monkeypatch):
+    """A CPU device has no stream: it is refused, and not answered with the current GPU's."""
+    from mindformers_amd import _lib
+    monkeypatch.setattr(torch.cuda, "_lazy_init", lambda: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    monkeypatch.setattr(_lib, "_raw_stream", lambda index: 0, raising=False)
+    with pytest.raises(ValueError):
+        _lib.stream_ptr(device)
+
+
 def _plan(query, *sizes):
     """(kernel, whole output blocks, blocks cut along K, parts of each) of a host plan query."""
     out = [ctypes.c_int() for _ in range(3)]

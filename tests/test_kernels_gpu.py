@@ -27,6 +27,14 @@ def _load_ops():
     yield
 
 
+def test_stream_handles_are_those_of_the_current_stream():
+    """However the device is named, and after a change of streams."""
+    from mindformers_amd._lib import stream_ptr
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            assert {stream_ptr(d) for d in (None, 0, "cuda:0", torch.device("cuda"), torch.device("cuda", 0))} == {stream.cuda_stream}
+
+
 # ------------------------------------------------------------------------------------------- KV scatter
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("t,n_kv,d,bs,nb", [(64, 8, 128, 128, 40), (4, 2, 64, 16, 64), (7, 1, 32, 16, 9), (3, 3, 20, 4, 11)])
