@@ -1362,7 +1362,8 @@ extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq,
                "grouped_w8a8_gemm: xq and w_packed must be 16-byte aligned");
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
     dim3 grid((n + QG_BN - 1) / QG_BN, n_experts);
-    if (y && !acc_out && n % 16 == 0 &&
+    // (K: the tiles' 32-bit offsets reach over 128 rows)
+    if (y && !acc_out && n % 16 == 0 && k <= (1 << 25) &&
         total_rows > tg_group_min_rows(n_experts, (n + tq::BN - 1) / tq::BN, k, QG_TILE_ROWS) * (int64_t)n_experts) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tq::BN - 1) / tq::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;

@@ -2004,6 +2004,19 @@ def test_grouped_w8a8_accumulators_bit_exact(counts, n, k):
         assert np.all(np.abs(got_y[r0:r1] - yref) <= 1.01 * EPS[torch.bfloat16] * np.abs(yref) + 1e-6), ex
 
 
+def test_grouped_w8a8_rows_of_more_than_32_mib():
+    """128 rows of 2^25 + 64 columns reach past 4 GiB: the last row's last columns are its own, not the first row's first ones."""
+    rows, n, k = 128, 16, 2 ** 25 + 64
+    xq = torch.zeros(rows, k, dtype=torch.int8, device="cuda")
+    xq[0, :64], xq[rows - 1, k - 64:] = 5, 1
+    wq = torch.zeros(1, n, k, dtype=torch.int8, device="cuda")
+    wq[0, :, k - 64:] = torch.arange(n, dtype=torch.int8, device="cuda")[:, None]
+    one = torch.ones(rows, device="cuda")
+    w = ops.pack_w8a16(wq, one[:n].reshape(1, n).contiguous())
+    y = ops.grouped_w8a8_linear(xq, one, w, torch.tensor([0, rows], dtype=torch.int32, device="cuda"))
+    assert torch.equal(y[rows - 1].float(), 64.0 * torch.arange(n, device="cuda")) and not bool(y[:rows - 1].any())
+
+
 @pytest.mark.parametrize("counts,n,k", [
     ([0, 1, 32, 33, 64, 65, 96, 97, 128, 129, 0, 300], 272, 192),   # both sides of every row-tile edge, a ragged last tile
     ([20] * 70 + [0] * 3 + [17], 48, 64),                       # more experts than lanes, one step of K
