@@ -1231,7 +1231,7 @@ def test_w8a16_many_rows(dtype, m, n, k, bias, residual):
 @pytest.mark.parametrize("dtype,m,n,k", [
     (torch.bfloat16, 1153, 4112, 1216),    # 96-row tiles: one row and one 16-channel piece past whole ones, an odd number of k-steps
     (torch.float16, 1048, 4096, 1088),
-    (torch.bfloat16, 2025, 2112, 7168)])   # in place of tiles that are cut along K
+    (torch.bfloat16, 2025, 2112, 7168)])
 def test_w8a16_many_rows_on_96_row_tiles(dtype, m, n, k):
     """The same at shapes that take the lower tiles."""
     test_w8a16_many_rows(dtype, m, n, k, True, False)
@@ -1251,11 +1251,11 @@ def test_w8a16_exact_on_integer_grid():
     assert np.array_equal(to_np(y).astype(np.float64), rounded(exact, torch.float16).astype(np.float64))
 
 
-@pytest.mark.parametrize("m,n,k", [(129, 28672, 64), (131, 28672, 128), (257, 28672, 192), (300, 4096, 14336 + 64), (1048, 4096, 4160)])
+@pytest.mark.parametrize("m,n,k", [(1537, 14336, 64), (1537, 8192, 128), (1537, 4096, 192), (300, 4096, 14336 + 64), (1048, 4096, 4160)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_w8a16_tiles_exact_on_integer_grid(dtype, m, n, k):
     """The same for the kernel of many rows, whose k-loop runs pairs of 64-wide steps: one step, a pair, odd numbers of them, in whole
-    tiles and in parts, with an infinity in a row's last column, which belongs to that row alone."""
+    tiles and in parts, with an infinity in a row's last column, which belongs to that row alone.  (The host tests name these plans.)"""
     g = torch.Generator(device="cuda")
     g.manual_seed(m + k)
     w = torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
@@ -1300,10 +1300,13 @@ def test_w8a16_inf_in_the_last_columns_of_a_row_stays_in_that_row(m, n, k):
     (1, 4096, 4096, False, False), (16, 704, 512, True, False), (32, 512, 1408, True, True),
     (64, 6144, 4096, False, True), (65, 132, 2048, False, False), (130, 256, 512, True, True),
     (33, 64, 128, False, False), (4, 3584, 18944, False, False),
+    (2, 1040, 640, True, True), (8, 1044, 2176, False, True), (5, 528, 4224, True, True),     # few rows, a channel tile a workgroup
+    (1, 28672, 512, True, True), (3, 8208, 2176, True, True),                                 # few rows, two of them
 ])
 def test_w4a16_gemm(dtype, group, m, n, k, bias, residual):
     """4-bit weight-only GEMM against the oracle: per-channel and per-group scales, row counts on both sides of every
-    tile height, shapes that split K and shapes that do not, from the two-per-byte and the one-per-byte weight forms."""
+    tile height, shapes that split K and shapes that do not, every form of the few-row kernel with bias and residual, from the
+    two-per-byte and the one-per-byte weight forms."""
     rng = np.random.default_rng(m * 7 + n + group)
     w = rng.normal(0, 0.02, (n, k)).astype(np.float32)
     wq, s = O.quantize_weight_int4(w, group)
