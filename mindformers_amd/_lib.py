@@ -138,12 +138,16 @@ def ptr(t):
 
 # by itself: a torch.cuda.Stream around the handle costs more than the rest of a small call's checks
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_gpus = {}                                                    # devices that have been checked -> index (the type alone costs 0.25 us a call)
 
 
 def stream_ptr(device=None):
     """Handle of the current stream of ``device``: what ``torch.cuda.current_stream`` takes, and refused where it refuses (a device that
     is not a GPU)."""
-    if _raw_stream is None or not isinstance(device, torch.device) or device.type != "cuda":
-        return torch.cuda.current_stream(device).cuda_stream
-    index = device.index
-    return _raw_stream(torch.cuda.current_device() if index is None else index)
+    index = _gpus.get(device)
+    if index is not None:
+        return _raw_stream(index)
+    stream = torch.cuda.current_stream(device)
+    if _raw_stream is not None and isinstance(device, torch.device) and device.index is not None:
+        _gpus[device] = device.index
+    return stream.cuda_stream
