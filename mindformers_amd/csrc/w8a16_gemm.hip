@@ -515,12 +515,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 3 : 1) void w8a16_gemm4_ke
 }
 
 // ---- many rows ---------------------------------------------------------------------------------------------------------
-// More rows than two or three passes of the skinny kernel: tiles of 128 rows x 256 channels (w8a16_tile_gemm.h).
+// More rows than two or three passes of the skinny kernel: tiles of 128 or 96 rows x 256 channels (w8a16_tile_gemm.h).
 // Output of one wave: 64 channels from n0 on, 32 rows at a time.  The channels of a row lie spread over the accumulators of
-// two lanes, so the values (dequantised, with bias, gated where asked, rounded to T) go through LDS and leave as whole
+// four lanes, so the values (dequantised, with bias, gated where asked, rounded to T) go through LDS and leave as whole
 // 128-byte (gated: 64-byte) pieces of rows; the residual is read the same way.  Rounding points as in store4 / store_gated.
-// (8-byte stores straight from the accumulators, each waiting for its own scales: 4096 x 4096 at 1536 rows 69.8 us against
-// 54.3, 24576 x 1536 at 129 rows 42.3 against 25.6.)  N is a multiple of 16.
+// (8-byte stores straight from the accumulators, each waiting for its own scales, on an earlier form of the tiles: 4096 x 4096 at 1536
+// rows 69.8 us against 54.3, 24576 x 1536 at 129 rows 42.3 against 25.6.)  N is a multiple of 16.
 template <typename T>
 struct TileOut {
     static constexpr int ROW = TG_STAGE_ROW;
@@ -742,9 +742,10 @@ __global__ __launch_bounds__(256, 2) void w8a16_group_tile_kernel(
 // tiles and a lane's own row of the activations (out of the caches; nothing for rows past the last) go from memory straight into operand
 // registers, D steps ahead; a set is loaded again when all of it has been used.  Weights enter as q / 16 (dequant8_u4_16th, 14
 // instructions for 8 weights where the kernel above has 23); the sums are multiplied by 16 at the end, exactly.
-// What bounds it: latency and instructions, at 2.4 to 4.6 TB/s of weights.  One row, groups of 128, cold weights, us, the kernel above with the sum
-// of its K parts | here: 4096 x 4096 10.0 | 6.2, 6144 x 4096 11.9 | 9.3, 28672 x 4096 28.8 | 20.0, 4096 x 14336 17.3 | 12.4, 8192 x 29568 51 |
-// 30; eight rows 10.3 | 7.4, 12.0 | 11.8, 28.8 | 22.2, 17.9 | 14.9, 51 | 33.
+// What bounds it: latency and instructions, at 1.5 TB/s of weights and scales (4096 x 4096) to 4.2 (8192 x 29568).  One row, groups of 128,
+// 0.8 GB of weights in turn (nothing cached), us, the kernel above with the sum of its K parts | here: 4096 x 4096 9.9 | 5.8, 6144 x 4096
+// 11.5 | 7.5, 28672 x 4096 29.8 | 20.2, 4096 x 14336 17.2 | 12.3, 8192 x 29568 51.6 | 30.8; eight rows 10.1 | 7.0, 11.9 | 8.4, 29.1 |
+// 22.3, 17.8 | 14.6, 51.6 | 33.6.
 template <typename T, int GROUP, int NT, int W>
 __global__ __launch_bounds__(64 * W) void w4a16_rows_kernel(
     uint16_t* __restrict__ y, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, const float* __restrict__ scale,
@@ -1131,7 +1132,7 @@ struct GemmPlan {
     int steps_per_split;
 };
 
-// Tile plan of the many-row kernel (4137 x 4096 x 14336: 16 of 528 tiles left over by whole rounds, 531 us uncut, 423 us in
+// Tile plan of the many-row kernel (4137 x 4096 x 14336: 16 of 528 tiles left over by whole rounds, 455 us uncut, 351 us in
 // 8 parts).
 constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f, 0.56f};
 TileGrid plan_tiles(int m, int n, int k, float* us) {
@@ -1166,10 +1167,10 @@ GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
 
 // Tiles against passes of 64 rows of the skinny kernel (more than 64 rows, K of whole steps, N of whole 16-byte pieces, gated
 // too).  Measured, a k-step of a round of 256 skinny workgroups takes 0.40 us: 28672 x 4096 at 65 / 256 / 4137 rows runs in
-// 41 / 65 / 787 us on tiles against 51 / 103 / 1447 us, 4096 x 4096 at 128 / 256 / 700 rows in 18 / 26 / 48 against 17 / 20 / 47,
-// 7168 x 16384 at 112 / 129 / 256 rows in 40 / 64 / 67 against 51 / 78 / 88 (168 skinny workgroups there at 129 rows).  The line is
+// 41 / 59 / 714 us on tiles against 52 / 106 / 1431 us, 4096 x 4096 at 128 / 256 / 700 rows in 21 / 22 / 36 against 17 / 21 / 47,
+// 7168 x 16384 at 112 / 129 / 256 rows in 42 / 62 / 65 against 53 / 84 / 88 (168 skinny workgroups there at 129 rows).  The line is
 // the same whatever follows in the call: the fused forms have the bits of the separate calls, and sums of two kernels differ; with
-// the norm behind it, 7168 x 16384 at 129 rows takes 68 against 82 us.
+// the norm behind it, 7168 x 16384 at 129 rows takes 65 against 84 us.
 bool use_tiles(int m, int n, int k) {
     if (m <= 64 || k % tg::KSTEP != 0 || n % 16 != 0) return false;
     float us;

@@ -18,7 +18,7 @@
 // name them: left to the compiler 32 accumulators of four registers wander through the file and spill.
 //
 // What bounds it: the power budget.  4137 x 28672 x 4096: 782-797 us on 32x32x16, 714-724 here (1360 TFLOP/s); 4137 x 4096 x 14336:
-// 398 / 359; 2025 x 7168 x 16384: 424 / 360.  A lone workgroup on a compute unit (few tiles) is bound by issue: one wave starts a
+// 398 / 351-359; 2025 x 7168 x 16384: 424 / 350-360.  A lone workgroup on a compute unit (few tiles) is bound by issue: one wave starts a
 // vector instruction every 8 cycles, and a step has 96 beside 64 matrix instructions of 16 (0.7 to 0.9 us a step, two workgroups
 // together 1.55).
 namespace tg {

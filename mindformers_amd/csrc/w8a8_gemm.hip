@@ -1100,10 +1100,10 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
 
 // Many rows, tiled activations: 128 x 256 tiles against the kernels above.  Measured, a 64-wide step of a round of 256
 // workgroups takes 0.32 us in the register-streaming kernel, 0.78 us in the wide one and 0.38 to 0.50 us in the LDS-staged one
-// (one workgroup on a compute unit; it starts and ends like a tile).  37888 x 3584 at 65 / 257 / 1531 rows runs in 32 / 56 / 250 us on tiles against 48 / 85 / 275
-// (256 rows: 296 tiles, 40 more than units, 52 us against 48 on 198 wide tiles), 24576 x 1536 at 257 / 640 rows in 27 / 32
-// against 23 / 42 (wide), 28672 x 4096 at 256 rows in 37 against 47, 8192 x 8192 at 128 / 129 / 257 rows in 32 / 37 / 46 against
-// 34 / 34 / 67 (LDS-staged), 3584 x 18944 at 1531 rows in 120 against 181, 3584 x 3584 at 448 rows in 27 against 20.  `fused`: the
+// (one workgroup on a compute unit; it starts and ends like a tile).  37888 x 3584 at 65 / 257 / 1531 rows runs in 35 / 54 / 182 us on
+// tiles against 51 / 86 / 232 (256 rows: 296 tiles, 40 more than units, 50 us against 48 on 198 wide tiles), 24576 x 1536 at 257 / 640
+// rows in 26 / 31 against 24 / 46 (wide), 28672 x 4096 at 256 rows in 38 against 48, 8192 x 8192 at 128 / 129 / 257 rows in 27 / 32 / 41
+// against 33 / 33 / 55 (LDS-staged), 3584 x 18944 at 1531 rows in 113 against 172, 3584 x 3584 at 448 rows in 26 against 22.  `fused`: the
 // sum of the register-streaming and the wide kernel's parts carries what follows, which is a kernel of its own behind tiles (the
 // figures of the LDS-staged kernel have it in).
 constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f, 0.31f};

@@ -13,8 +13,8 @@
 // matrix pipe, and the smaller one, which reads and writes half the accumulators per operation, leaves the power budget more clock.
 // What bounds the kernel is the operand traffic out of L2 (24 KiB per 4.2 M operations a step, 171 op/B, about 12 TB/s) and that
 // budget: 4096 x 4096 x 16384 from warm caches 248 us on 32x32x32, 219 here (2515 TOP/s), 1531 x 37888 x 3584 with cold weights
-// 203 / 187, 2077 x 4096 x 7168 73 / 67, 1531 x 3584 x 18944 (168 tiles, one on a compute unit) 118 / 118.  1531 x 37888 x 3584 on 256 x
-// 192 tiles of 8 waves with both operands through an LDS ring: 275.  Row panels of 8 or 16 blocks instead of 4, or neighbouring
+// 203 / 187, 2077 x 4096 x 7168 73 / 67, 1531 x 3584 x 18944 118 / 118 on 168 tiles of 128 rows, one on a compute unit (on the 224 of 96
+// rows that it runs on 113).  1531 x 37888 x 3584 on 256 x 192 tiles of 8 waves with both operands through an LDS ring: 232 to 275.  Row panels of 8 or 16 blocks instead of 4, or neighbouring
 // tiles paired on one compute unit, change nothing.
 namespace tq {
 
