@@ -1172,7 +1172,7 @@ GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
 // the same whatever follows in the call: the fused forms have the bits of the separate calls, and sums of two kernels differ; with
 // the norm behind it, 7168 x 16384 at 129 rows takes 65 against 84 us.
 bool use_tiles(int m, int n, int k) {
-    if (m <= 64 || k % tg::KSTEP != 0 || n % 16 != 0) return false;
+    if (m <= 64 || k % tg::KSTEP != 0 || n % 16 != 0 || k > (1 << 24)) return false;   // K: 32-bit offsets over 128 rows
     float us;
     plan_tiles(m, n, k, &us);
     const GemmPlan p = plan_w8a16(m, n, k);
@@ -1557,7 +1557,7 @@ static int grouped_w8a16_entry(const char* who, void* y, const void* x, const vo
     MF_REQUIRE(!gated || n % 4 == 0, "%s: N (%d) must be a multiple of 4 (gate / up pairs)", who, n);
     MF_REQUIRE((((uintptr_t)x | (uintptr_t)w_packed) & 15) == 0, "%s: x and w_packed must be 16-byte aligned", who);
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
-    if (n % 16 == 0 && k % tg::KSTEP == 0 &&
+    if (n % 16 == 0 && k % tg::KSTEP == 0 && k <= (1 << 24) &&   // K: the tiles' 32-bit offsets reach over 128 rows
         total_rows > gw_group_tile_rows(n_experts, n, k) * (int64_t)n_experts) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tg::BN - 1) / tg::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;

@@ -86,8 +86,10 @@ def test_plans_of_the_shapes_that_the_tile_kernels_are_tested_at():
     for (m, n, k), plan in {(513, 8208, 704): (165, 0, 1), (129, 28672, 4096): (224, 0, 1), (65, 12304, 8192): (0, 49, 4),
                             (1100, 2064, 4096): (0, 81, 2), (1285, 6160, 1024): (256, 19, 4),
                             (2305, 4096, 4160): (256, 48, 4), (1537, 14336, 64): (728, 0, 1), (1537, 8192, 128): (416, 0, 1),
-                            (1537, 4096, 192): (208, 0, 1), (300, 4096, 14400): (0, 48, 4)}.items():
+                            (1537, 4096, 192): (208, 0, 1), (300, 4096, 14400): (0, 48, 4),
+                            (129, 4096, 1 << 24): (0, 32, 8)}.items():
         assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, *plan), (m, n, k)
+    assert _plan(lib.mf_w8a16_plan, 129, 4096, 17_000_000)[0] != tiles16         # 128 rows are more than 4 GiB
 
 
 def test_prompt_attention_is_cut_by_the_longest_context_there_can_be():

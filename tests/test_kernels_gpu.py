@@ -2020,6 +2020,18 @@ def test_grouped_w8a8_rows_of_more_than_32_mib():
     assert torch.equal(y[rows - 1].float(), 64.0 * torch.arange(n, device="cuda")) and not bool(y[:rows - 1].any())
 
 
+def test_grouped_w8a16_rows_of_more_than_32_mib():
+    """The same with 16-bit rows of 17 million columns."""
+    rows, n, k = 128, 16, 17_000_000
+    x = torch.zeros(rows, k, dtype=torch.bfloat16, device="cuda")
+    x[0, :64], x[rows - 1, k - 64:] = 5, 1
+    wq = torch.zeros(1, n, k, dtype=torch.int8, device="cuda")
+    wq[0, :, k - 64:] = torch.arange(n, dtype=torch.int8, device="cuda")[:, None]
+    w = ops.pack_w8a16(wq, torch.ones(1, n, device="cuda"))
+    y = ops.grouped_w8a16_linear(x, w, torch.tensor([0, rows], dtype=torch.int32, device="cuda"))
+    assert torch.equal(y[rows - 1].float(), 64.0 * torch.arange(n, device="cuda")) and not bool(y[:rows - 1].any())
+
+
 @pytest.mark.parametrize("counts,n,k", [
     ([0, 1, 32, 33, 64, 65, 96, 97, 128, 129, 0, 300], 272, 192),   # both sides of every row-tile edge, a ragged last tile
     ([20] * 70 + [0] * 3 + [17], 48, 64),                       # more experts than lanes, one step of K
