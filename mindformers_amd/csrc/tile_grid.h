@@ -98,6 +98,14 @@ inline int tg_group_min_rows(int n_experts, int n_blocks, int k, int least) {
     return k > 2048 && (int64_t)n_experts * n_blocks < 256 ? 64 : least;
 }
 
+// Output of a kernel that streams the weights of many experts: written past the caches.  Lines that wait in L2 leave it one by one
+// between the loads of the stream, and each costs the stream more than its own time; behind a short stream they stay in the caches for
+// the next kernel.  256 experts of 65 rows on average (11.3 GB), W8A8, us without stores | past the caches | cached: 4096 x 7168 1098 |
+// 1252 | 1320 (136 MB written), 7168 x 2048 565 | 762 | 800 (238 MB).  Both projections with what lies between them, W8A16, past the
+// caches | cached: 24 rows an expert 1751 | 1803, 48: 1920 | 2070, 65: 2116 | 2152; 8 experts of 28672 x 4096 (0.94 GB), 65 rows 367 |
+// 364; 64 of 2816 x 2048 (0.37 GB), 33 rows 114 | 107.
+inline bool tg_group_stream(int n_experts, int64_t expert_bytes) { return n_experts * expert_bytes > (1LL << 30); }
+
 // Grouped rows (experts): the row blocks of all experts, in order, times the channel blocks.  Their number is known on the
 // device only (offsets [n_experts + 1]), so the launch covers what the total allows and each workgroup finds its own by a
 // scan of the offsets.  Ids go to the XCDs in turn; XCD j is given the j-th eighth of the row blocks, all channel blocks of
@@ -167,8 +175,9 @@ __device__ __forceinline__ void wave_lds_order() {
 // 32 staged rows of up to 64 channels (144 bytes a row: 16-byte slots spread over the banks) to memory as whole 16-byte pieces
 // of rows, by `threads` threads of which this is number t; the residual, read the same way, is added to the rounded values.
 // cols = row length of y, c0 = first channel, per = 16-byte pieces of a staged row.
+// STREAM: stores past the caches, see tg_group_stream.
 constexpr int TG_STAGE_ROW = 144;
-template <typename T>
+template <typename T, bool STREAM = false>
 __device__ __forceinline__ void tg_flush(uint16_t* y, const uint16_t* residual, const uint8_t* stage, int m0, int M, int c0,
                                          int cols, int per, bool aligned, int t, int threads) {
     const int row = t / per, c = c0 + 8 * (t - row * per), step = threads / per;
@@ -188,8 +197,10 @@ __device__ __forceinline__ void tg_flush(uint16_t* y, const uint16_t* residual, 
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = pack2<T>(__fadd_rn(f[2 * i], g[2 * i]), __fadd_rn(f[2 * i + 1], g[2 * i + 1]));
         }
-        if (aligned) *(u32x4*)(y + at) = v;
-        else
+        if (aligned) {
+            if constexpr (STREAM) __builtin_nontemporal_store(v, (u32x4*)(y + at));
+            else *(u32x4*)(y + at) = v;
+        } else
             for (int i = 0; i < 8; ++i) y[at + i] = (uint16_t)(v[i >> 1] >> (16 * (i & 1)));
     }
 }

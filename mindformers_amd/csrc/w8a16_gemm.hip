@@ -556,8 +556,9 @@ struct TileOut {
         }
     }
     // the 32 staged rows to memory, by `threads` threads of which this is number t
+    template <bool STREAM = false>
     __device__ __forceinline__ void flush(int m0, int n0, const uint8_t* stage, int t, int threads) const {
-        tg_flush<T>(y, residual, stage, m0, M, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? 4 : 8, aligned, t, threads);
+        tg_flush<T, STREAM>(y, residual, stage, m0, M, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? 4 : 8, aligned, t, threads);
     }
 };
 
@@ -682,7 +683,7 @@ __global__ __launch_bounds__(GW_WAVES * 64, 2) void w8a16_grouped_kernel(
 // channel blocks read: 109 experts of 4096 x 7168 at 33 rows 551 us cached, 511 so, 8 of 28672 x 4096 at 33 rows 178 / 163; blocks of
 // more rows gain nothing (7168 x 2048 at 65 rows 679 / 704), and an expert's further blocks share the weights through L2 (200 rows:
 // 1257 / 1420).  Up to 16 bytes of scratch a lane, outside the k-loops.
-template <typename T, int MT, bool NT>
+template <typename T, int MT, bool NT, bool STREAM>
 __device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* xe, const uint8_t* we, const float* se, int rows,
                                                  int m0, int nb, int N, int K, int gated, int aligned, uint8_t* smem) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -703,11 +704,11 @@ __device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* xe
         for (int e = 0; e < 8; ++e)
             out.put(acc[e >> 2][e & 3], sc[e & 3], bi[e & 3], e >> 2, e & 3, stage);
         wave_lds_order();
-        out.flush(m0 + 32 * mt, n0, stage, lane, 64);
+        out.template flush<STREAM>(m0 + 32 * mt, n0, stage, lane, 64);
     });
 }
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(256, 2) void w8a16_group_tile_kernel(
     uint16_t* __restrict__ y, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, const float* __restrict__ scale,
     const int32_t* __restrict__ offsets, int n_experts, int total_rows, int N, int K, int64_t expert_bytes, int gated,
@@ -721,7 +722,7 @@ __global__ __launch_bounds__(256, 2) void w8a16_group_tile_kernel(
     const uint8_t* we = wp + (int64_t)e * expert_bytes;
     const float* se = scale + (int64_t)e * N;
     const int left = rows - m0;
-#define GT(MT, NT) w8a16_group_tile<T, MT, NT>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem)
+#define GT(MT, NT) w8a16_group_tile<T, MT, NT, STREAM>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem)
     if (left <= 32) {
         if (m0 == 0) GT(1, true);                             // nobody else reads these weights
         else GT(1, false);
@@ -1561,12 +1562,13 @@ static int grouped_w8a16_entry(const char* who, void* y, const void* x, const vo
         total_rows > gw_group_tile_rows(n_experts, n, k) * (int64_t)n_experts) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tg::BN - 1) / tg::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;
-#define GGT_LAUNCH(TT)                                                                                            \
-    hipLaunchKernelGGL((w8a16_group_tile_kernel<TT>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y,        \
+        const bool stream_out = tg_group_stream(n_experts, expert_bytes);
+#define GGT_LAUNCH(TT, ST)                                                                                        \
+    hipLaunchKernelGGL((w8a16_group_tile_kernel<TT, ST>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y,        \
                        (const uint16_t*)x, (const uint8_t*)w_packed, scale, offsets, n_experts, total_rows, n, k,    \
                        expert_bytes, gated, aligned)
-        if (dtype == MF_BF16) GGT_LAUNCH(BF16);
-        else GGT_LAUNCH(FP16);
+        if (dtype == MF_BF16) { if (stream_out) GGT_LAUNCH(BF16, true); else GGT_LAUNCH(BF16, false); }
+        else { if (stream_out) GGT_LAUNCH(FP16, true); else GGT_LAUNCH(FP16, false); }
 #undef GGT_LAUNCH
         return MF_LAUNCH_CHECK();
     }

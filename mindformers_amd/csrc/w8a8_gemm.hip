@@ -980,7 +980,7 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
 // channel blocks read: 109 experts of 4096 x 7168 at 33 rows 542 us cached, 513 so, 64 of 2816 x 2048 at 33 rows 77 / 68.  For blocks of
 // more rows it depends on the number of experts (64 of 2816 x 2048 at 100 rows 95 / 83, a layer of 256 experts at 65 rows 2545 / 2632),
 // and an expert's further blocks share the weights through L2 (200 rows: 928 / 1276 us).
-template <typename T, int MT, bool NT>
+template <typename T, int MT, bool NT, bool STREAM>
 __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, const float* xs, const uint8_t* we,
                                                 const float* ws, int rows, int m0, int nb, int N, int K, int aligned,
                                                 uint8_t* smem) {
@@ -1006,11 +1006,11 @@ __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, 
             for (int nt = 0; nt < 4; ++nt) out.put(acc[j][nt], x1, wsv[nt], bi[nt], j, nt, stage);
         }
         wave_lds_order();
-        tg_flush<T>(y, nullptr, stage, m0 + 32 * mt, rows, n0, N, 8, aligned, lane, 64);
+        tg_flush<T, STREAM>(y, nullptr, stage, m0 + 32 * mt, rows, n0, N, 8, aligned, lane, 64);
     });
 }
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
     uint16_t* __restrict__ y, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
     const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const int32_t* __restrict__ offsets, int n_experts,
@@ -1023,7 +1023,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
     const uint8_t *xe = (const uint8_t*)xq + (int64_t)row0 * K, *we = wp + (int64_t)e * expert_bytes;
     const float *xs = x_scale + row0, *ws = w_scale + (int64_t)e * N;
     const int left = rows - m0;
-#define GT(MT, NT) w8a8_group_tile<T, MT, NT>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem)
+#define GT(MT, NT) w8a8_group_tile<T, MT, NT, STREAM>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem)
     if (left <= 64) {
         if (m0 == 0) GT(2, true);                             // nobody else reads these weights
         else GT(2, false);
@@ -1367,11 +1367,12 @@ extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq,
         total_rows > tg_group_min_rows(n_experts, (n + tq::BN - 1) / tq::BN, k, QG_TILE_ROWS) * (int64_t)n_experts) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tq::BN - 1) / tq::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;
-#define QGT_LAUNCH(TT)                                                                                           \
-    hipLaunchKernelGGL((w8a8_group_tile_kernel<TT>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y, xq, x_scale, \
+        const bool stream_out = tg_group_stream(n_experts, expert_bytes);
+#define QGT_LAUNCH(TT, ST)                                                                                       \
+    hipLaunchKernelGGL((w8a8_group_tile_kernel<TT, ST>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y, xq, x_scale, \
                        (const uint8_t*)w_packed, w_scale, offsets, n_experts, total_rows, n, k, expert_bytes, aligned)
-        if (out_dtype == MF_BF16) QGT_LAUNCH(BF16);
-        else QGT_LAUNCH(FP16);
+        if (out_dtype == MF_BF16) { if (stream_out) QGT_LAUNCH(BF16, true); else QGT_LAUNCH(BF16, false); }
+        else { if (stream_out) QGT_LAUNCH(FP16, true); else QGT_LAUNCH(FP16, false); }
 #undef QGT_LAUNCH
         return MF_LAUNCH_CHECK();
     }
