@@ -585,6 +585,13 @@ int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const floa
                          const float* w_scale, const int32_t* offsets, int n_experts, int total_rows, int n, int k,
                          int out_dtype, void* stream);
 
+/* mf_grouped_w8a8_gemm with the experts' activation in its epilogue, as mf_grouped_w8a16_gemm_silu_mul has it: rows of every
+ * expert's weight (and w_scale) interleaved gate / up, y [R, N/2] (4-byte aligned), N % 4 == 0; same bits as
+ * mf_grouped_w8a8_gemm followed by mf_silu_mul(layout 1). */
+int mf_grouped_w8a8_gemm_silu_mul(void* y, const int8_t* xq, const float* x_scale, const void* w_packed,
+                                  const float* w_scale, const int32_t* offsets, int n_experts, int total_rows, int n, int k,
+                                  int out_dtype, void* stream);
+
 /* MoeTokenUnpermute(permuted_tokens, sorted_indices, probs) — moe_layer.py:151-155.
  * out[t,:] = sum_j probs[t,j] * y[row_map[t*k+j],:] accumulated in fp32 in order j = 0..k-1
  * (+ shared[t,:] if shared != NULL, the shared-expert add of moe_layer.py:159-160). */

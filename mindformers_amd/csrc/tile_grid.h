@@ -101,9 +101,11 @@ inline int tg_group_min_rows(int n_experts, int n_blocks, int k, int least) {
 // Output of a kernel that streams the weights of many experts: written past the caches.  Lines that wait in L2 leave it one by one
 // between the loads of the stream, and each costs the stream more than its own time; behind a short stream they stay in the caches for
 // the next kernel.  256 experts of 65 rows on average (11.3 GB), W8A8, us without stores | past the caches | cached: 4096 x 7168 1098 |
-// 1252 | 1320 (136 MB written), 7168 x 2048 565 | 762 | 800 (238 MB).  Both projections with what lies between them, W8A16, past the
-// caches | cached: 24 rows an expert 1751 | 1803, 48: 1920 | 2070, 65: 2116 | 2152; 8 experts of 28672 x 4096 (0.94 GB), 65 rows 367 |
-// 364; 64 of 2816 x 2048 (0.37 GB), 33 rows 114 | 107.
+// 1252 | 1320 (136 MB written), 7168 x 2048 565 | 762 | 800 (238 MB).  Both projections with what lies between them, past the
+// caches | cached: W8A8 24 rows an expert 1768 | 1819, 48: 1910 | 2056, 65: 2036 | 2088, W8A16 24: 1751 | 1803, 48: 1920 | 2070, 65: 2116 |
+// 2152; 8 experts of 28672 x 4096 (0.94 GB), 65 rows 309 | 306, W8A16 367 | 364; 64 of 2816 x 2048 (0.37 GB), 33 rows 114 | 110, W8A16
+// 114 | 107.  The cost lies in the switches of the memory between reads and writes more than in the bytes: with a quarter of the rows
+// written 1213 and 725.
 inline bool tg_group_stream(int n_experts, int64_t expert_bytes) { return n_experts * expert_bytes > (1LL << 30); }
 
 // Grouped rows (experts): the row blocks of all experts, in order, times the channel blocks.  Their number is known on the

@@ -108,6 +108,19 @@ __device__ __forceinline__ void q2_store4(uint16_t* y, int32_t* acc_out, const f
     }
 }
 
+// Four dequantised channels (gate, up, gate, up) of one row to the two activations silu(gate) * up.  Rounding points as the unfused
+// sequence has them: the projection output, silu(gate) and the product are each rounded to T.
+template <typename T>
+__device__ __forceinline__ uint32_t q2_gated4(const float (&v)[4]) {
+    float a[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const float gv = T::to_float(T::from_float(v[2 * e])), uv = T::to_float(T::from_float(v[2 * e + 1]));
+        a[e] = T::to_float(T::from_float(silu_f(gv))) * uv;
+    }
+    return pack2<T>(a[0], a[1]);
+}
+
 // grid = (n_blocks, split_k, m_blocks)
 template <typename T, int NT, int MSPLIT, int ST, bool KTAIL, bool XT>
 __global__ __launch_bounds__(256, 2) void w8a8_gemm_kernel(
@@ -751,7 +764,7 @@ template <typename T>
 struct QTileOut {
     const float *x_scale, *w_scale;
     const uint16_t* bias;
-    int M, N;
+    int M, N, gated;                                          // gated: see q2_gated4
     __device__ __forceinline__ void load(int n0, int nt, f32x4& ws, f32x4& bi) const {
         const int n = min(n0 + 16 * nt + 4 * ((threadIdx.x >> 4) & 3), N - 4);
 #pragma unroll
@@ -764,8 +777,10 @@ struct QTileOut {
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = scaled_bias((float)a[i], xs, ws[i], true, bi[i], bias != nullptr);
-        *(u32x2*)(stage + (16 * j + (threadIdx.x & 15)) * TG_STAGE_ROW + 2 * (16 * nt + 4 * ((threadIdx.x >> 4) & 3))) =
-            (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+        uint8_t* row = stage + (16 * j + (threadIdx.x & 15)) * TG_STAGE_ROW;
+        const int c = 16 * nt + 4 * ((threadIdx.x >> 4) & 3);
+        if (gated) *(uint32_t*)(row + c) = q2_gated4<T>(v);
+        else *(u32x2*)(row + 2 * c) = (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
     }
 };
 
@@ -784,7 +799,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_tile_kernel(
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = mb * 32 * MT, n0 = nb * tq::BN + 64 * wv;
     int32_t* pt = partial + (int64_t)slot * (32 * MT * tq::BN) + (wv * MT * 8 * 64 + lane) * 4;
-    const QTileOut<T> out{x_scale, w_scale, bias, M, N};
+    const QTileOut<T> out{x_scale, w_scale, bias, M, N, 0};
     f32x4 ws[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
     const tq::TiledRows<tq::XLOADS<MT>> rows((const uint8_t*)xq, m0 >> 4, (M + 15) >> 4, wv);
@@ -828,7 +843,7 @@ __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
     if (m0 >= M || n0 >= N) return;
     const int lane = threadIdx.x & 63, e0 = 2 * (threadIdx.x >> 6);
     const int32_t* p = partial + slot * PART + ((wv * MT + mt) * 8 * 64 + lane) * 4;
-    const QTileOut<T> out{x_scale, w_scale, bias, M, N};
+    const QTileOut<T> out{x_scale, w_scale, bias, M, N, 0};
     const float xs = x_scale[min(m0 + 16 * (e0 >> 2) + (lane & 15), M - 1)];
     f32x4 ws[2], bi[2];
     i32x4 v[2] = {(i32x4)(0), (i32x4)(0)};
@@ -867,7 +882,7 @@ template <typename T, int MT>
 __device__ __forceinline__ void w8a8_group_pass(uint16_t* __restrict__ y, int32_t* __restrict__ acc_out,
                                                 const int8_t* __restrict__ x, const float* __restrict__ xs,
                                                 const uint8_t* __restrict__ wp, const float* __restrict__ ws, int rows,
-                                                int N, int K, int n0, int m0, int32_t* red) {
+                                                int N, int K, int n0, int m0, int gated, int32_t* red) {
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
@@ -936,7 +951,14 @@ __device__ __forceinline__ void w8a8_group_pass(uint16_t* __restrict__ y, int32_
         i32x4 sum = *(const i32x4*)(red + ml * QG_BN + sw);
 #pragma unroll
         for (int q = 1; q < QG_WAVES; ++q) sum += *(const i32x4*)(red + (q * XROWS + ml) * QG_BN + sw);
-        q2_store4<T>(y, acc_out, xs, ws, nullptr, nullptr, m, n, N, sum);
+        if (gated) {                                          // N is a multiple of 4
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = scaled_bias((float)sum[i], xs[m], ws[n + i], true, 0.f, false);
+            *(uint32_t*)(y + (int64_t)m * (N >> 1) + (n >> 1)) = q2_gated4<T>(v);
+        } else {
+            q2_store4<T>(y, acc_out, xs, ws, nullptr, nullptr, m, n, N, sum);
+        }
     }
 }
 
@@ -944,7 +966,7 @@ template <typename T, int MTMAX>
 __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
     uint16_t* __restrict__ y, int32_t* __restrict__ acc_out, const int8_t* __restrict__ xq,
     const float* __restrict__ x_scale, const uint8_t* __restrict__ wp, const float* __restrict__ w_scale,
-    const int32_t* __restrict__ offsets, int total_rows, int N, int K, int64_t expert_bytes) {
+    const int32_t* __restrict__ offsets, int total_rows, int N, int K, int64_t expert_bytes, int gated) {
     __shared__ __attribute__((aligned(16))) int32_t red[QG_SMEM<MTMAX> / 4];
     const int e = blockIdx.y;
     int row0 = offsets[e], row1 = offsets[e + 1];
@@ -954,19 +976,19 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
     if (rows == 0) return;
     const uint8_t* we = wp + (int64_t)e * expert_bytes;
     const float* se = w_scale + (int64_t)e * N;
-    uint16_t* ye = y ? y + (int64_t)row0 * N : nullptr;
+    uint16_t* ye = y ? y + (int64_t)row0 * (gated ? N >> 1 : N) : nullptr;
     int32_t* ae = acc_out ? acc_out + (int64_t)row0 * N : nullptr;
     const int8_t* xe = xq + (int64_t)row0 * K;
     const float* xse = x_scale + row0;
     const int n0 = blockIdx.x * QG_BN;
     if (rows <= 16) {
-        w8a8_group_pass<T, 1>(ye, ae, xe, xse, we, se, rows, N, K, n0, 0, red);
+        w8a8_group_pass<T, 1>(ye, ae, xe, xse, we, se, rows, N, K, n0, 0, gated, red);
     } else if (rows <= 32 || MTMAX == 2) {
         for (int m0 = 0; m0 < rows; m0 += 32)
-            w8a8_group_pass<T, 2>(ye, ae, xe, xse, we, se, rows, N, K, n0, m0, red);
+            w8a8_group_pass<T, 2>(ye, ae, xe, xse, we, se, rows, N, K, n0, m0, gated, red);
     } else {
         for (int m0 = 0; m0 < rows; m0 += 16 * MTMAX)
-            w8a8_group_pass<T, MTMAX>(ye, ae, xe, xse, we, se, rows, N, K, n0, m0, red);
+            w8a8_group_pass<T, MTMAX>(ye, ae, xe, xse, we, se, rows, N, K, n0, m0, gated, red);
     }
 }
 
@@ -976,17 +998,19 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
 // (each fetching the rows anew, a second pass for every second expert), 1435 here (5.2 TB/s of weights); 7168 x 2048: 1280 / 817.
 // With 128-row tiles for every expert of more than 64 rows the padding's matrix instructions counted: the two GEMMs of 256
 // experts of 65 rows on average 2323 us, 2167 with tiles of 96 rows for those up to 96.
+// gated: silu(gate) * up in the epilogue, which halves what the first projection writes and the quantisation behind it reads: a layer of
+// 256 experts on 2077 tokens 2500 us, 2464 gated (quantisation of the product 44 / 25).
 // Weights of an expert with one block of up to 64 rows are read past the caches, where they would push out the rows that all
 // channel blocks read: 109 experts of 4096 x 7168 at 33 rows 542 us cached, 513 so, 64 of 2816 x 2048 at 33 rows 77 / 68.  For blocks of
 // more rows it depends on the number of experts (64 of 2816 x 2048 at 100 rows 95 / 83, a layer of 256 experts at 65 rows 2545 / 2632),
 // and an expert's further blocks share the weights through L2 (200 rows: 928 / 1276 us).
 template <typename T, int MT, bool NT, bool STREAM>
 __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, const float* xs, const uint8_t* we,
-                                                const float* ws, int rows, int m0, int nb, int N, int K, int aligned,
-                                                uint8_t* smem) {
+                                                const float* ws, int rows, int m0, int nb, int N, int K, int gated,
+                                                int aligned, uint8_t* smem) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = nb * tq::BN + 64 * wv;
-    const QTileOut<T> out{xs, ws, nullptr, rows, N};
+    const QTileOut<T> out{xs, ws, nullptr, rows, N, gated};
     f32x4 wsv[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
     const tq::PlainRows<tq::XLOADS<MT>> src(xe, m0, rows, K, wv);
@@ -1006,7 +1030,8 @@ __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, 
             for (int nt = 0; nt < 4; ++nt) out.put(acc[j][nt], x1, wsv[nt], bi[nt], j, nt, stage);
         }
         wave_lds_order();
-        tg_flush<T, STREAM>(y, nullptr, stage, m0 + 32 * mt, rows, n0, N, 8, aligned, lane, 64);
+        tg_flush<T, STREAM>(y, nullptr, stage, m0 + 32 * mt, rows, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? 4 : 8, aligned,
+                            lane, 64);
     });
 }
 
@@ -1014,16 +1039,16 @@ template <typename T, bool STREAM>
 __global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
     uint16_t* __restrict__ y, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
     const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const int32_t* __restrict__ offsets, int n_experts,
-    int total_rows, int N, int K, int64_t expert_bytes, int aligned) {
+    int total_rows, int N, int K, int64_t expert_bytes, int gated, int aligned) {
     constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW, OPS = tq::LDS_BYTES<4>;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
     int e, m0, row0, rows, nb;
     if (!tg_group_locate(offsets, n_experts, total_rows, (N + tq::BN - 1) / tq::BN, e, m0, row0, rows, nb)) return;
-    uint16_t* ye = y + (int64_t)row0 * N;
+    uint16_t* ye = y + (int64_t)row0 * (gated ? N >> 1 : N);
     const uint8_t *xe = (const uint8_t*)xq + (int64_t)row0 * K, *we = wp + (int64_t)e * expert_bytes;
     const float *xs = x_scale + row0, *ws = w_scale + (int64_t)e * N;
     const int left = rows - m0;
-#define GT(MT, NT) w8a8_group_tile<T, MT, NT, STREAM>(ye, xe, xs, we, ws, rows, m0, nb, N, K, aligned, smem)
+#define GT(MT, NT) w8a8_group_tile<T, MT, NT, STREAM>(ye, xe, xs, we, ws, rows, m0, nb, N, K, gated, aligned, smem)
     if (left <= 64) {
         if (m0 == 0) GT(2, true);                             // nobody else reads these weights
         else GT(2, false);
@@ -1350,16 +1375,17 @@ extern "C" int mf_w8a8_qkv_rope_and_cache(void* qkv, const int8_t* xq, const flo
                              x_layout == 1, workspace, (hipStream_t)stream, nullptr, &rc);
 }
 
-extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale,
-                                    const void* w_packed, const float* w_scale, const int32_t* offsets, int n_experts,
-                                    int total_rows, int n, int k, int out_dtype, void* stream) {
-    MF_REQUIRE(out_dtype == MF_BF16 || out_dtype == MF_FP16, "grouped_w8a8_gemm: out_dtype must be bf16 or fp16");
+static int grouped_w8a8_entry(const char* who, void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale,
+                              const void* w_packed, const float* w_scale, const int32_t* offsets, int n_experts, int total_rows,
+                              int n, int k, int out_dtype, int gated, void* stream) {
+    MF_REQUIRE(out_dtype == MF_BF16 || out_dtype == MF_FP16, "%s: out_dtype must be bf16 or fp16", who);
     if (total_rows == 0) return 0;
-    MF_REQUIRE((y || acc_out) && xq && x_scale && w_packed && w_scale && offsets, "grouped_w8a8_gemm: null argument");
-    MF_REQUIRE(n_experts > 0 && n_experts <= 65535 && total_rows >= 0 && n > 0 && k > 0, "grouped_w8a8_gemm: bad sizes");
-    MF_REQUIRE(k % 16 == 0, "grouped_w8a8_gemm: K (%d) must be a multiple of 16", k);
-    MF_REQUIRE((((uintptr_t)xq | (uintptr_t)w_packed) & 15) == 0,
-               "grouped_w8a8_gemm: xq and w_packed must be 16-byte aligned");
+    MF_REQUIRE((y || acc_out) && xq && x_scale && w_packed && w_scale && offsets, "%s: null argument", who);
+    MF_REQUIRE(n_experts > 0 && n_experts <= 65535 && total_rows >= 0 && n > 0 && k > 0, "%s: bad sizes", who);
+    MF_REQUIRE(k % 16 == 0, "%s: K (%d) must be a multiple of 16", who, k);
+    MF_REQUIRE(!gated || n % 4 == 0, "%s: N (%d) must be a multiple of 4 (gate / up pairs)", who, n);
+    MF_REQUIRE(!gated || ((uintptr_t)y & 3) == 0, "%s: y must be 4-byte aligned", who);
+    MF_REQUIRE((((uintptr_t)xq | (uintptr_t)w_packed) & 15) == 0, "%s: xq and w_packed must be 16-byte aligned", who);
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
     dim3 grid((n + QG_BN - 1) / QG_BN, n_experts);
     // (K: the tiles' 32-bit offsets reach over 128 rows)
@@ -1370,7 +1396,8 @@ extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq,
         const bool stream_out = tg_group_stream(n_experts, expert_bytes);
 #define QGT_LAUNCH(TT, ST)                                                                                       \
     hipLaunchKernelGGL((w8a8_group_tile_kernel<TT, ST>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y, xq, x_scale, \
-                       (const uint8_t*)w_packed, w_scale, offsets, n_experts, total_rows, n, k, expert_bytes, aligned)
+                       (const uint8_t*)w_packed, w_scale, offsets, n_experts, total_rows, n, k, expert_bytes, gated, \
+                       aligned)
         if (out_dtype == MF_BF16) { if (stream_out) QGT_LAUNCH(BF16, true); else QGT_LAUNCH(BF16, false); }
         else { if (stream_out) QGT_LAUNCH(FP16, true); else QGT_LAUNCH(FP16, false); }
 #undef QGT_LAUNCH
@@ -1381,7 +1408,7 @@ extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq,
 #define QG_LAUNCH(TT, MTV)                                                                                      \
     hipLaunchKernelGGL((w8a8_grouped_kernel<TT, MTV>), grid, dim3(QG_WAVES * 64), 0, (hipStream_t)stream,        \
                        (uint16_t*)y, acc_out, xq, x_scale, (const uint8_t*)w_packed, w_scale, offsets, total_rows, n, \
-                       k, expert_bytes)
+                       k, expert_bytes, gated)
     if (out_dtype == MF_BF16) {
         if (big) QG_LAUNCH(BF16, 4);
         else QG_LAUNCH(BF16, 2);
@@ -1391,4 +1418,18 @@ extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq,
     }
 #undef QG_LAUNCH
     return MF_LAUNCH_CHECK();
+}
+
+extern "C" int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale,
+                                    const void* w_packed, const float* w_scale, const int32_t* offsets, int n_experts,
+                                    int total_rows, int n, int k, int out_dtype, void* stream) {
+    return grouped_w8a8_entry("grouped_w8a8_gemm", y, acc_out, xq, x_scale, w_packed, w_scale, offsets, n_experts, total_rows, n, k,
+                              out_dtype, 0, stream);
+}
+
+extern "C" int mf_grouped_w8a8_gemm_silu_mul(void* y, const int8_t* xq, const float* x_scale, const void* w_packed,
+                                             const float* w_scale, const int32_t* offsets, int n_experts, int total_rows, int n,
+                                             int k, int out_dtype, void* stream) {
+    return grouped_w8a8_entry("grouped_w8a8_gemm_silu_mul", y, nullptr, xq, x_scale, w_packed, w_scale, offsets, n_experts,
+                              total_rows, n, k, out_dtype, 1, stream);
 }

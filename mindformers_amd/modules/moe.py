@@ -107,7 +107,8 @@ class QuantGroupedMLP(nn.Module):
     ``act_quant="per_token"`` / ``"per_tensor"`` (W8A8, the routed experts of a W8A8 checkpoint such as
     research/deepseek3/deepseek_r1_671b/predict_deepseek_r1_671b_w8a8.yaml:89-92): the permuted rows are quantised per
     token, or with one calibrated scale per projection (``act_scale1`` / ``act_scale2``, loaded with the checkpoint),
-    and both projections run on the int8 matrix cores with exact int32 accumulators.  ``smooth`` (per_token only):
+    and both projections run on the int8 matrix cores with exact int32 accumulators, the first with silu(gate) * hidden in
+    its epilogue too.  ``smooth`` (per_token only):
     the rows of expert e are multiplied by ``smooth_scale1[e]`` [H] in front of the first projection and the
     activation product by ``smooth_scale2[e]`` [F] in front of the second (outliers_suppression: smooth; the weight
     side of the pair is folded into the checkpoint's int8 weights)."""
@@ -150,9 +151,8 @@ class QuantGroupedMLP(nn.Module):
         return self
 
     def prepare(self):
-        # W8A16: gate / up rows interleaved, so that the first GEMM's epilogue holds each pair in one lane
-        self._p1 = (ops.pack_w8a16(self.weight1, self.w1_scale) if self.act_quant
-                    else ops.pack_w8a16_gated(self.weight1, self.w1_scale, "halves"))
+        # gate / up rows interleaved, so that the first GEMM's epilogue holds each pair in one lane
+        self._p1 = ops.pack_w8a16_gated(self.weight1, self.w1_scale, "halves")
         self._p2 = ops.pack_w8a16(self.weight2, self.w2_scale)
         return self
 
@@ -188,13 +188,13 @@ class QuantGroupedMLP(nn.Module):
             xq, xs = ops.dynamic_quant(hidden_states.contiguous(), self.smooth_scale1, offsets=offsets)
         else:
             xq, xs = self._quant(hidden_states.contiguous(), self.act_scale1)
-        h = ops.grouped_w8a8_linear(xq, xs, self._p1, offsets, out_dtype=dt)
+        a = ops.grouped_w8a8_linear(xq, xs, self._p1, offsets, out_dtype=dt)      # silu(gate) * hidden included
         if self.act_quant == "per_tensor":
-            aq, a_s = ops.static_quant(ops.silu_mul(h), self.act_scale2)
+            aq, a_s = ops.static_quant(a, self.act_scale2)
         elif self.smooth_scale2 is not None:
-            aq, a_s = ops.silu_mul_dynamic_quant(h, self.smooth_scale2, offsets=offsets)
+            aq, a_s = ops.dynamic_quant(a, self.smooth_scale2, offsets=offsets)
         else:
-            aq, a_s = ops.silu_mul_dynamic_quant(h)
+            aq, a_s = ops.dynamic_quant(a)
         return ops.grouped_w8a8_linear(aq, a_s, self._p2, offsets, out_dtype=dt)
 
     construct = forward

@@ -1230,17 +1230,23 @@ def grouped_w8a16_linear(x, w, offsets, scale=None):
 def grouped_w8a8_linear(xq, x_scale, w, offsets, out_dtype=torch.bfloat16, return_acc=False):
     """GroupedMatmulV4 on int8 operands: xq int8 [R, K] row-major with per-row scales (``dynamic_quant`` of the permuted
     rows), ``w`` a PackedInt8Weight of [E, N, K], offsets int32 [E+1].  Exact int32 accumulators, dequantised to
-    out_dtype; with ``return_acc`` also the int32 [R, N] accumulators."""
+    out_dtype; with ``return_acc`` also the int32 [R, N] accumulators.  A weight packed with ``pack_w8a16_gated`` runs with
+    silu(gate) * up in the epilogue and returns [R, N/2]."""
     lib = _lib.load()
-    _need(isinstance(w, PackedInt8Weight) and w.experts is not None and not w.gated,
-          "grouped_w8a8_linear needs stacked expert weights [E, N, K] (not gated)")
+    _need(isinstance(w, PackedInt8Weight) and w.experts is not None and not (w.gated and return_acc),
+          "grouped_w8a8_linear needs stacked expert weights [E, N, K] (not gated where the accumulators are wanted)")
     dev = _dev_ok(xq, x_scale, offsets)
     e, n, k = w.experts, w.n, w.k
     _need(xq.dtype == torch.int8 and xq.dim() == 2 and xq.shape[1] == k, "xq must be int8 [R, K]")
     _need(x_scale.dtype == torch.float32 and x_scale.numel() == xq.shape[0], "x_scale must be fp32 [R]")
     _need(offsets.dtype == torch.int32 and offsets.numel() == e + 1, "offsets must be int32 [E+1]")
     _need(out_dtype in _ACT, "out_dtype must be bf16/fp16")
-    y = torch.empty(xq.shape[0], n, dtype=out_dtype, device=dev)
+    y = torch.empty(xq.shape[0], n // 2 if w.gated else n, dtype=out_dtype, device=dev)
+    if w.gated:
+        check(lib.mf_grouped_w8a8_gemm_silu_mul(ptr(y), ptr(xq), ptr(x_scale), ptr(w.packed), ptr(w.scale), ptr(offsets), e,
+                                                xq.shape[0], n, k, dtype_code(out_dtype), stream_ptr(dev)),
+              "mf_grouped_w8a8_gemm_silu_mul")
+        return y
     acc = torch.empty(xq.shape[0], n, dtype=torch.int32, device=dev) if return_acc else None
     check(lib.mf_grouped_w8a8_gemm(ptr(y), ptr(acc), ptr(xq), ptr(x_scale), ptr(w.packed), ptr(w.scale), ptr(offsets), e,
                                    xq.shape[0], n, k, dtype_code(out_dtype), stream_ptr(dev)), "mf_grouped_w8a8_gemm")

@@ -2063,6 +2063,29 @@ def test_grouped_gemms_at_prompt_sizes(counts, n, k, dtype):
     assert torch.equal(fused, ops.silu_mul(y))
 
 
+@pytest.mark.parametrize("counts,n,k", [
+    ([0, 1, 32, 33, 64, 65, 96, 97, 128, 129, 0, 300], 272, 192),   # tiles: every row-tile edge, a ragged last tile
+    ([0, 0, 400], 1056, 1040),                                  # tiles, one expert; K ends inside a step
+    ([0, 5, 16, 20, 3, 1, 0, 3], 192, 208),                     # passes of 16 and 32 rows
+    ([14, 40, 65, 3], 100, 64),                                 # passes of 64 rows: N is no multiple of 16
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_grouped_w8a8_gated_equals_unfused(counts, n, k, dtype):
+    """silu(gate) * up in the epilogue of the grouped int8 GEMM: the bits of the plain GEMM followed by silu_mul."""
+    rng = np.random.default_rng(n + k)
+    counts, off = _ragged_groups(rng, counts)
+    e, rows = len(counts), int(counts.sum())
+    od = torch.from_numpy(off).cuda()
+    qd = torch.from_numpy(rng.integers(-127, 128, (e, n, k)).astype(np.int8)).cuda()
+    sd = torch.from_numpy(rng.uniform(1e-4, 5e-4, (e, n)).astype(np.float32)).cuda()
+    xq, xs = ops.dynamic_quant(dev(rounded(rng.normal(size=(rows, k)), dtype), dtype))
+    y = ops.grouped_w8a8_linear(xq, xs, ops.pack_w8a16(qd, sd), od, out_dtype=dtype)
+    fused = ops.grouped_w8a8_linear(xq, xs, ops.pack_w8a16_gated(qd, sd, "halves"), od, out_dtype=dtype)
+    c = n // 16 * 8                                             # silu_mul takes multiples of 8 columns
+    ref = ops.silu_mul(torch.cat((y[:, :c], y[:, n // 2:n // 2 + c]), dim=1))
+    assert fused.shape == (rows, n // 2) and torch.equal(fused[:, :c], ref)
+
+
 @pytest.mark.parametrize("counts,n", [
     ([50, 80, 62], 48), ([65, 64, 66], 48),                     # few tiles: up to 64 rows a group the passes, above it tiles
     ([20] * 255 + [8], 32), ([21] * 200 + [22] * 56, 32),       # tiles enough: 20 rows (16-bit activations; 12 with int8 ones)
