@@ -154,6 +154,18 @@ int mf_causal_attention_qk192_v128(void* out, const void* query, const void* key
                                    float scale, int64_t q_row_stride, int64_t k_row_stride, int64_t v_row_stride,
                                    int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same with the two parts of the keys where the layer has them: key_nope [total_q, n_heads * 128] (a column slice of the
+ * up-projection) and key_rope [total_q, 64], the rotary part that all heads share (:411-416 copies it behind every head's
+ * 128 values).  As many kv heads as heads; the bits of the call with joined keys. */
+int mf_causal_attention_shared_rope(void* out, const void* query, const void* key_nope, const void* key_rope,
+                                    const void* value, const int32_t* q_starts, int batch, int total_q, int n_heads,
+                                    float scale, int64_t q_row_stride, int64_t k_row_stride, int64_t rope_row_stride,
+                                    int64_t v_row_stride, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Row offsets int32 [n + 1] of packed sequences from a list of n > 0 int32 or int64 values on the device: the list itself
+ * where it is one of row ends (it does not fall and ends at total_rows), its running sums otherwise (lengths). */
+int mf_q_starts(int32_t* starts, const void* seq, int seq_is_int64, int n, int64_t total_rows, void* stream);
+
 /* mf_paged_attention_decode / _prefill on int8 caches: same arguments plus antiquant_scale / antiquant_offset
  * (offset may be NULL); workspaces as for the 16-bit entry points; paged keys only.  Scores use the query with
  * the key scale folded in (rounded to dtype); a key offset shifts all scores of a row equally and cancels in the

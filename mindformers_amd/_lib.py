@@ -41,6 +41,8 @@ SIGNATURES = {
                                                         _L, _I, _P, _Z, _P]),
     "mf_paged_attention_prefill_int8kv_per_token": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I,
                                                          _I, _F, _L, _I, _P, _Z, _P]),
+    "mf_causal_attention_shared_rope": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _F, _L, _L, _L, _L, _I, _P, _Z, _P]),
+    "mf_q_starts": (_I, [_P, _P, _I, _I, _L, _P]),
     "mf_causal_attention_qk192_v128": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _L, _L, _L, _I, _P, _Z, _P]),
     "mf_mla_paged_attention_workspace_bytes": (_Z, [_I, _I, _I]),
     "mf_mla_paged_attention_decode": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _L, _I, _P, _Z, _P]),

@@ -71,10 +71,21 @@ struct PfSmem {
     static constexpr int BYTES = PF_RING * BUF;
 };
 
+// Where the second sub-tile of the key rows lies when the values are narrower than the keys: a tensor of its own (the rotary part of
+// multi-latent attention, one row of 64 values for all the heads) or the tail of every head of the key rows.
+struct PfRope {
+    const uint16_t* base;                                     // second sub-tile of head 0 of row 0
+    int64_t stride;                                           // elements from row to row
+    int head, key_head;                                       // elements from head to head, here and in the key rows
+};
+
 // Three workgroups per compute unit; two at 192-wide heads (72 KB of LDS and 96 accumulator registers each).
 // (int8 caches at heads of 128: the tile in registers takes them past 168, and 144 bytes a lane are spilled.)
 // DV: width of a value head and of an output head.  DV < D (the prefill of multi-latent attention: 192-wide queries
-// and keys, 128-wide values, packed rows only) loads and multiplies the first sub-tile of the value rows only.
+// and keys, 128-wide values, packed rows only) loads and multiplies the first sub-tile of the value rows only, and takes the second
+// sub-tile of the keys from where `rope` says.  The rotary part that all heads share is read where it lies: writing it behind
+// every head's 128 up-projected values took 102 us of a layer's 930 (2025 rows, 128 heads: 66 MB read, 100 MB written), and its rows
+// come out of L2 here instead of 128 copies out of memory.
 template <typename T, int D, bool TIB, int DV = D, int KVQ = 0>
 __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_attention_kernel(
     uint16_t* __restrict__ out, float* __restrict__ part_out, float* __restrict__ part_ml,
@@ -82,7 +93,7 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ ctx_lens, int n_heads, int n_kv,
     int n_rep, int block_size, int max_blocks, int num_blocks, int max_parts, float scale_log2, int64_t q_stride,
     int batch, const int32_t* __restrict__ q_starts, int part_tokens, int64_t kv_stride, int rows,
-    int64_t v_stride, const float* __restrict__ kv_scale, const float* __restrict__ kv_offset, float lazy_log2) {
+    int64_t v_stride, const float* __restrict__ kv_scale, const float* __restrict__ kv_offset, float lazy_log2, PfRope rope) {
     using vec8 = typename T::vec8;
     using S = PfSmem<D>;
     // Type of the probabilities and of the widened values in the PV product.  int8 values are exact in either type and fp16 rounds
@@ -211,6 +222,8 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
     const int32_t* table = block_tables + (int64_t)b * max_blocks;
     const int64_t row_bytes = kv_stride * 2;
     const int64_t v_row_bytes = v_stride * 2;
+    constexpr bool SPLIT = DV < D;                            // the keys' second sub-tile has an address of its own
+    const int64_t rope_row_bytes = SPLIT ? rope.stride * 2 : 0;
 
     // ---- tile loads: load i of wave w into a sub-tile brings its rows (LW i + w) RPI .. + RPI - 1; lane = (row in
     // the group, LDS slot).  The loads of the first sub-tile come first in the arrays.
@@ -227,9 +240,9 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
         const int row = (SS::LW * li + w) * SS::RPI + lrow;
         const int key = (row / SS::RPB) & (SS::CPR - 1);
         const int key4 = (row / SS::RPB) & (SS::CPR / 4 - 1);
-        kcol[i] = (uint32_t)(kvh * D * 2 + col0 + 16 * (lslot ^ key));
+        kcol[i] = (uint32_t)(!SPLIT ? kvh * D * 2 + col0 : kvh * 2 * (second ? rope.head : rope.key_head)) + 16 * (lslot ^ key);
         vcol[i] = (uint32_t)(kvh * DV * 2 + col0 + 16 * ((lslot - 4 * key4) & (SS::CPR - 1)));
-        kofs[i] = (uint32_t)(row * (int)(kv_stride * 2)) + kcol[i];      // offsets within a whole tile
+        kofs[i] = (uint32_t)(row * (int)((SPLIT && second ? rope.stride : kv_stride) * 2)) + kcol[i];   // offsets within a whole tile
         vofs[i] = (uint32_t)(row * (int)(v_stride * 2)) + vcol[i];
     });
     const int part_end = min(Lwg, part_start + part_tokens);
@@ -261,7 +274,8 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
                 using SS = std::conditional_t<second, S1, S0>;
                 constexpr int li = i - (second ? S0::NI : 0);
                 uint8_t* dst = kdst + (second ? S::SUB1 : 0) + (SS::LW * li + w) * SS::RPI * SS::ROWB;
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kb + kofs[i]),
+                const uint8_t* kbase = SPLIT && second ? (const uint8_t*)rope.base + slot0 * rope_row_bytes : kb;
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kbase + kofs[i]),
                                                  (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
                 if constexpr (i < NIV)
                     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vb + vofs[i]),
@@ -279,7 +293,8 @@ __global__ __launch_bounds__(PA_WAVES * 64, D == 192 ? 2 : 3) void prefill_atten
             const int rc = min(r0 + lane / SS::CPR, last_row);
             const uint8_t *kp, *vp;
             if constexpr (TIB) {                              // uniform base, 32-bit lane offset
-                kp = (const uint8_t*)kc + slot0 * row_bytes + ((uint32_t)(rc * (int)row_bytes) + kcol[i]);
+                const int64_t krow = SPLIT && second ? rope_row_bytes : row_bytes;
+                kp = (const uint8_t*)(SPLIT && second ? rope.base : kc) + slot0 * krow + ((uint32_t)(rc * (int)krow) + kcol[i]);
                 vp = (const uint8_t*)vc + slot0 * v_row_bytes + ((uint32_t)(rc * (int)v_row_bytes) + vcol[i]);
             } else {
                 const int tok = ts + rc;
@@ -681,7 +696,7 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
               const int32_t* block_tables, const int32_t* context_lens, const int32_t* q_starts, int batch,
               int total_q, int n_heads, int n_kv, int block_size, int max_blocks, int num_blocks, float scale,
               int64_t q_stride, int64_t kv_stride, void* workspace, hipStream_t st, const float* kv_scale,
-              const float* kv_offset, int64_t v_stride = 0) {
+              const float* kv_offset, int64_t v_stride = 0, PfRope rope = {}) {
     static_assert(DV == D || KVQ == 0, "value heads narrower than the key heads: 16-bit packed rows only");
     if (v_stride <= 0) v_stride = kv_stride;
     const int n_rep = n_heads / n_kv;
@@ -736,7 +751,8 @@ int launch_pf(void* out, const void* query, const void* key_cache, const void* v
                            part_out, part_ml, (const uint16_t*)query, (const uint16_t*)key_cache,                 \
                            (const uint16_t*)value_cache, block_tables, context_lens, n_heads, n_kv, n_rep,        \
                            block_size, max_blocks, num_blocks, plan.max_parts, scale_log2, q_stride, batch,       \
-                           q_starts, plan.part_tokens, kv_stride, total_q, v_stride, kv_scale, kv_offset, plan.lazy_log2); \
+                           q_starts, plan.part_tokens, kv_stride, total_q, v_stride, kv_scale, kv_offset, plan.lazy_log2, \
+                           rope);                                                                                  \
     }
         if (tib_tok) PF_LAUNCH(true)
         else PF_LAUNCH(false)
@@ -911,6 +927,38 @@ extern "C" int mf_paged_attention_prefill_int8kv_per_token(void* out, const void
                             value_scale_cache);
 }
 
+// packed rows of 192-wide queries and keys with 128-wide values; key and rope: see PfRope (rope.base == nullptr: joined keys)
+static int qk192_v128_entry(const char* who, void* out, const void* query, const void* key, const void* value,
+                            const int32_t* q_starts, int batch, int total_q, int n_heads, int n_kv_heads, float scale,
+                            int64_t q_row_stride, int64_t k_row_stride, int64_t v_row_stride, PfRope rope, int dtype,
+                            void* workspace, size_t workspace_bytes, void* stream) {
+    MF_REQUIRE(n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0,
+               "%s: n_heads (%d) must be a positive multiple of n_kv_heads (%d)", who, n_heads, n_kv_heads);
+    const int key_width = rope.base ? 128 : 192;
+    if (q_row_stride <= 0) q_row_stride = (int64_t)n_heads * 192;
+    if (k_row_stride <= 0) k_row_stride = (int64_t)n_kv_heads * key_width;
+    if (v_row_stride <= 0) v_row_stride = (int64_t)n_kv_heads * 128;
+    if (!rope.base) rope = {(const uint16_t*)key + 128, k_row_stride, 192, 192};
+    MF_REQUIRE(scale > 0.f, "%s: the softmax scale must be positive", who);
+    MF_REQUIRE(q_row_stride >= (int64_t)n_heads * 192 && k_row_stride >= (int64_t)n_kv_heads * key_width &&
+                   v_row_stride >= (int64_t)n_kv_heads * 128 && rope.stride >= 64 && q_row_stride % 8 == 0 &&
+                   k_row_stride % 8 == 0 && v_row_stride % 8 == 0 && rope.stride % 8 == 0,
+               "%s: row strides must cover a row and be multiples of 8 elements", who);
+    MF_REQUIRE((((uintptr_t)out | (uintptr_t)query | (uintptr_t)key | (uintptr_t)value | (uintptr_t)rope.base) & 15) == 0,
+               "%s: out / query / key / value must be 16-byte aligned", who);
+    const size_t need = mf_paged_attention_prefill_workspace_bytes(batch, total_q, n_heads, n_kv_heads, 128, total_q);
+    MF_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0),
+               "%s: 16-byte aligned workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == MF_BF16)
+        return launch_pf<BF16, 192, 0, 128>(out, query, key, value, nullptr, nullptr, q_starts, batch, total_q, n_heads,
+                                            n_kv_heads, 0, 0, 0, scale, q_row_stride, k_row_stride, workspace, st,
+                                            nullptr, nullptr, v_row_stride, rope);
+    return launch_pf<FP16, 192, 0, 128>(out, query, key, value, nullptr, nullptr, q_starts, batch, total_q, n_heads,
+                                        n_kv_heads, 0, 0, 0, scale, q_row_stride, k_row_stride, workspace, st, nullptr,
+                                        nullptr, v_row_stride, rope);
+}
+
 extern "C" int mf_causal_attention_qk192_v128(void* out, const void* query, const void* key, const void* value,
                                               const int32_t* q_starts, int batch, int total_q, int n_heads,
                                               int n_kv_heads, float scale, int64_t q_row_stride,
@@ -920,29 +968,56 @@ extern "C" int mf_causal_attention_qk192_v128(void* out, const void* query, cons
     MF_REQUIRE(batch >= 0 && total_q >= 0, "causal_attention_qk192_v128: negative batch or row count");
     if (batch == 0 || total_q == 0) return 0;
     MF_REQUIRE(out && query && key && value && q_starts, "causal_attention_qk192_v128: null argument");
-    MF_REQUIRE(scale > 0.f, "causal_attention_qk192_v128: the softmax scale must be positive");
-    MF_REQUIRE(n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0,
-               "causal_attention_qk192_v128: n_heads (%d) must be a positive multiple of n_kv_heads (%d)", n_heads,
-               n_kv_heads);
-    if (q_row_stride <= 0) q_row_stride = (int64_t)n_heads * 192;
-    if (k_row_stride <= 0) k_row_stride = (int64_t)n_kv_heads * 192;
-    if (v_row_stride <= 0) v_row_stride = (int64_t)n_kv_heads * 128;
-    MF_REQUIRE(q_row_stride >= (int64_t)n_heads * 192 && k_row_stride >= (int64_t)n_kv_heads * 192 &&
-                   v_row_stride >= (int64_t)n_kv_heads * 128 && q_row_stride % 8 == 0 && k_row_stride % 8 == 0 &&
-                   v_row_stride % 8 == 0,
-               "causal_attention_qk192_v128: row strides must cover a row and be multiples of 8 elements");
-    MF_REQUIRE((((uintptr_t)out | (uintptr_t)query | (uintptr_t)key | (uintptr_t)value) & 15) == 0,
-               "causal_attention_qk192_v128: out / query / key / value must be 16-byte aligned");
-    const size_t need = mf_paged_attention_prefill_workspace_bytes(batch, total_q, n_heads, n_kv_heads, 128, total_q);
-    MF_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0),
-               "causal_attention_qk192_v128: 16-byte aligned workspace of %zu bytes needed, %zu given", need,
-               workspace_bytes);
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype == MF_BF16)
-        return launch_pf<BF16, 192, 0, 128>(out, query, key, value, nullptr, nullptr, q_starts, batch, total_q, n_heads,
-                                            n_kv_heads, 0, 0, 0, scale, q_row_stride, k_row_stride, workspace, st,
-                                            nullptr, nullptr, v_row_stride);
-    return launch_pf<FP16, 192, 0, 128>(out, query, key, value, nullptr, nullptr, q_starts, batch, total_q, n_heads,
-                                        n_kv_heads, 0, 0, 0, scale, q_row_stride, k_row_stride, workspace, st, nullptr,
-                                        nullptr, v_row_stride);
+    return qk192_v128_entry("causal_attention_qk192_v128", out, query, key, value, q_starts, batch, total_q, n_heads, n_kv_heads,
+                            scale, q_row_stride, k_row_stride, v_row_stride, PfRope{}, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mf_causal_attention_shared_rope(void* out, const void* query, const void* key_nope, const void* key_rope,
+                                               const void* value, const int32_t* q_starts, int batch, int total_q, int n_heads,
+                                               float scale, int64_t q_row_stride, int64_t k_row_stride,
+                                               int64_t rope_row_stride, int64_t v_row_stride, int dtype, void* workspace,
+                                               size_t workspace_bytes, void* stream) {
+    MF_REQUIRE(dtype == MF_BF16 || dtype == MF_FP16, "causal_attention_shared_rope: dtype must be bf16 or fp16");
+    MF_REQUIRE(batch >= 0 && total_q >= 0, "causal_attention_shared_rope: negative batch or row count");
+    if (batch == 0 || total_q == 0) return 0;
+    MF_REQUIRE(out && query && key_nope && key_rope && value && q_starts, "causal_attention_shared_rope: null argument");
+    const PfRope rope = {(const uint16_t*)key_rope, rope_row_stride > 0 ? rope_row_stride : 64, 0, 128};
+    return qk192_v128_entry("causal_attention_shared_rope", out, query, key_nope, value, q_starts, batch, total_q, n_heads, n_heads,
+                            scale, q_row_stride, k_row_stride, v_row_stride, rope, dtype, workspace, workspace_bytes, stream);
+}
+
+// Row offsets of packed sequences: starts[0] = 0, then the running sums of seq, or seq itself where it already is a list of row
+// ends (it does not fall and ends at total_rows).  One wave; sums in 64 bits, as the list may be.
+template <typename I>
+__global__ __launch_bounds__(64) void pf_q_starts_kernel(int32_t* __restrict__ starts, const I* __restrict__ seq, int n,
+                                                         int64_t total_rows) {
+    const int lane = threadIdx.x;
+    bool rising = true;
+    for (int i = lane; i < n; i += 64) rising = rising && (i == 0 || seq[i] >= seq[i - 1]);
+    const bool ends = __ballot(!rising) == 0 && (int64_t)seq[n - 1] == total_rows;
+    if (lane == 0) starts[0] = 0;
+    int64_t base = 0;
+    for (int c0 = 0; c0 < n; c0 += 64) {
+        const int i = c0 + lane;
+        const int64_t v = i < n ? (int64_t)seq[i] : 0;
+        int64_t sum = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const long long up = __shfl_up((long long)sum, o, 64);
+            if (lane >= o) sum += up;
+        }
+        if (i < n) starts[i + 1] = (int32_t)(ends ? v : base + sum);
+        base += __shfl((long long)sum, 63, 64);
+    }
+}
+
+extern "C" int mf_q_starts(int32_t* starts, const void* seq, int seq_is_int64, int n, int64_t total_rows, void* stream) {
+    MF_REQUIRE(starts && seq && n > 0, "q_starts: null argument or empty list");
+    if (seq_is_int64)
+        hipLaunchKernelGGL((pf_q_starts_kernel<int64_t>), dim3(1), dim3(64), 0, (hipStream_t)stream, starts, (const int64_t*)seq, n,
+                           total_rows);
+    else
+        hipLaunchKernelGGL((pf_q_starts_kernel<int32_t>), dim3(1), dim3(64), 0, (hipStream_t)stream, starts, (const int32_t*)seq, n,
+                           total_rows);
+    return MF_LAUNCH_CHECK();
 }

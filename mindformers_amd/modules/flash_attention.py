@@ -66,17 +66,8 @@ class FlashAttention(nn.Module):
         else:
             q2 = query.reshape(-1, shape[-1])
         if self.is_prefill:
-            # FlashAttentionScore over this step's packed rows (flash_attention.py:129-134); keys are the step's own,
-            # so the query and key lists must agree
-            if actual_seq_kvlen is not None and actual_seq_kvlen is not actual_seq_qlen:
-                if not torch.equal(torch.as_tensor(actual_seq_kvlen).cpu(), torch.as_tensor(actual_seq_qlen).cpu()):
-                    raise NotImplementedError("prefill with actual_seq_kvlen != actual_seq_qlen is not built "
-                                              "(use the decode branch with q_seq_lens for chunked prefill)")
-            if actual_seq_qlen is None:
-                starts = torch.tensor([0, q2.shape[0]], dtype=torch.int32, device=query.device)
-            else:
-                starts = ops.q_starts_from_actual_seq_len(torch.as_tensor(actual_seq_qlen, device=query.device),
-                                                          q2.shape[0])
+            # FlashAttentionScore over this step's packed rows (flash_attention.py:129-134)
+            starts = self._starts(q2, actual_seq_qlen, actual_seq_kvlen)
             k2 = key if key.dim() == 2 else key.reshape(q2.shape[0], -1)
             v2 = value if value.dim() == 2 else value.reshape(q2.shape[0], -1)
             # the kv head count of this step's keys: kv_head_num, which for multi-latent attention differs from the
@@ -111,3 +102,28 @@ class FlashAttention(nn.Module):
         return out.reshape(shape)
 
     construct = forward
+
+    @staticmethod
+    def _starts(query, actual_seq_qlen, actual_seq_kvlen):
+        """Row offsets of a prefill's sequences; keys are the step's own, so the query and key lists must agree."""
+        if actual_seq_kvlen is not None and actual_seq_kvlen is not actual_seq_qlen:
+            if not torch.equal(torch.as_tensor(actual_seq_kvlen).cpu(), torch.as_tensor(actual_seq_qlen).cpu()):
+                raise NotImplementedError("prefill with actual_seq_kvlen != actual_seq_qlen is not built "
+                                          "(use the decode branch with q_seq_lens for chunked prefill)")
+        if actual_seq_qlen is None:
+            return torch.tensor([0, query.shape[0]], dtype=torch.int32, device=query.device)
+        return ops.q_starts_from_actual_seq_len(torch.as_tensor(actual_seq_qlen, device=query.device), query.shape[0])
+
+    def takes_key_parts(self):
+        """Whether ``prefill_shared_rope`` stands for ``forward``: not where a subclass or an instance brings its own ``forward``,
+        nor under forward hooks, which are shown the joined keys."""
+        hooks = torch.nn.modules.module
+        return type(self).forward is FlashAttention.forward and "forward" not in self.__dict__ and not (
+            self._forward_hooks or self._forward_pre_hooks or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
+
+    def prefill_shared_rope(self, query, key_nope, key_rope, value, actual_seq_qlen=None, actual_seq_kvlen=None):
+        """The prefill branch of ``forward`` for multi-latent attention, on the two parts of the keys
+        (``ops.causal_attention_shared_rope``): the same bits without the copy that joins them."""
+        return ops.causal_attention_shared_rope(query, key_nope, key_rope, value,
+                                                self._starts(query, actual_seq_qlen, actual_seq_kvlen), self.head_num,
+                                                self.scale_value)

@@ -200,8 +200,14 @@ class MLASelfAttention(nn.Module):
             q, kv_c, k_pe = self._project(hidden_states, rotary_pos_cos, rotary_pos_sin, slot_mapping, key_cache)
             t = q.shape[0]
             kv = self.linear_kv_up_proj(kv_c).reshape(t, -1)
-            k_no_pe = kv[:, : n * nope].reshape(t, n, nope)
             val = kv[:, n * nope:]
+            core = self.core_attention
+            if (nope, rope, vd) == (128, 64, 128) and type(core) is FlashAttention and core.takes_key_parts() \
+                    and core.head_num == n and (key_cache is None or key_cache.dtype == kv.dtype):
+                # the kernel reads the rotary part that all heads share where it lies
+                return self.linear_proj(core.prefill_shared_rope(q.reshape(t, n * self.q_head_dim), kv[:, : n * nope], k_pe, val,
+                                                                 actual_seq_qlen, actual_seq_kvlen))
+            k_no_pe = kv[:, : n * nope].reshape(t, n, nope)
             k_rep = k_pe.unsqueeze(1).expand(t, n, rope)
             key = torch.cat((k_no_pe, k_rep), dim=-1).reshape(t, n * self.q_head_dim)
             # 128-wide values under 192-wide keys: the attention takes them as they are (the reference pads them to the key

@@ -485,6 +485,12 @@ def q_starts_from_actual_seq_len(actual_seq_len, total_rows):
     a = torch.as_tensor(actual_seq_len).reshape(-1)
     if a.dtype not in (torch.int32, torch.int64):
         a = a.to(torch.int64)
+    if a.is_cuda and a.numel():
+        a = a.contiguous()
+        starts = torch.empty(a.numel() + 1, dtype=torch.int32, device=a.device)
+        check(_lib.load().mf_q_starts(ptr(starts), ptr(a), 1 if a.dtype == torch.int64 else 0, a.numel(), total_rows,
+                                      stream_ptr(a.device)), "mf_q_starts")
+        return starts
     is_ends = (a[-1] == total_rows) & torch.all(a[1:] >= a[:-1])
     starts = torch.zeros(a.numel() + 1, dtype=torch.int32, device=a.device)
     starts[1:].copy_(torch.where(is_ends, a, torch.cumsum(a, 0)))              # the sums of int32 values are int64
@@ -576,6 +582,34 @@ def causal_attention_varlen(query, key, value, q_starts, n_heads, n_kv_heads, sc
                                          total_q, n_heads, n_kv_heads, d, 0, 0, 0, float(scale), qs, ks,
                                          dtype_code(query.dtype), ptr(ws), ws.numel() if ws is not None else 0,
                                          stream_ptr(dev)), "mf_paged_attention_prefill")
+    return out
+
+
+def causal_attention_shared_rope(query, key_nope, key_rope, value, q_starts, n_heads, scale):
+    """``causal_attention_varlen`` of multi-latent attention's prefill on the parts of its keys: query [T, n * 192], key_nope and
+    value [T, n * 128] (column slices of the up-projection), key_rope [T, 64], which every head's keys end with.  The bits of
+    the call with the two parts joined."""
+    lib = _lib.load()
+    dev = _dev_of(query, key_nope, key_rope, value)
+    _need(query.dtype in _ACT and key_nope.dtype == query.dtype and key_rope.dtype == query.dtype
+          and value.dtype == query.dtype, "dtype mismatch")
+    _need(query.dim() == 2 and key_nope.dim() == 2 and key_rope.dim() == 2 and value.dim() == 2, "operands must be 2-D")
+    t = query.shape[0]
+    _need(tuple(query.shape) == (t, n_heads * 192) and tuple(key_nope.shape) == (t, n_heads * 128)
+          and tuple(value.shape) == (t, n_heads * 128) and tuple(key_rope.shape) == (t, 64),
+          "query [T, n * 192], key_nope and value [T, n * 128] and key_rope [T, 64] expected")
+    query, qs = _rows(query, n_heads * 192, "query")
+    key_nope, ks = _rows(key_nope, n_heads * 128, "key_nope")
+    key_rope, rs = _rows(key_rope, 64, "key_rope")
+    value, vs = _rows(value, n_heads * 128, "value")
+    b = _q_starts(q_starts, dev)
+    out = torch.empty((t, n_heads * 128), dtype=query.dtype, device=dev)
+    need = lib.mf_paged_attention_prefill_workspace_bytes(b, t, n_heads, n_heads, 128, t)
+    ws = workspace(need, dev, "pa_prefill") if need else None
+    check(lib.mf_causal_attention_shared_rope(ptr(out), ptr(query), ptr(key_nope), ptr(key_rope), ptr(value), ptr(q_starts), b,
+                                              t, n_heads, float(scale), qs, ks, rs, vs, dtype_code(query.dtype), ptr(ws),
+                                              ws.numel() if ws is not None else 0, stream_ptr(dev)),
+          "mf_causal_attention_shared_rope")
     return out
 
 

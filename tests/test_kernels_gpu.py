@@ -561,6 +561,40 @@ def test_causal_attention_with_128_wide_values_under_192_wide_keys(dtype, nh, nk
         ops.causal_attention_varlen(dev(q, dtype), dev(k, dtype), dev(v[:, : nkv * 64].copy(), dtype), starts, nh, nkv, scale)
 
 
+@pytest.mark.parametrize("dtype,nh,q_lens,gap", [
+    (torch.bfloat16, 16, [130, 1, 64], 0), (torch.float16, 3, [33, 200, 31], 8), (torch.bfloat16, 2, [1500], 0),   # the last one cut
+    (torch.bfloat16, 128, [40, 300], 64), (torch.float16, 1, [1], 0),
+])
+def test_causal_attention_on_the_parts_of_the_keys(dtype, nh, q_lens, gap):
+    """Keys whose rotary part is one row for all heads, as column slices with and without space between the rows: the bits of
+    the call on joined keys."""
+    rng = np.random.default_rng(nh + gap)
+    t = int(np.sum(q_lens))
+    q = dev(rounded(rng.normal(size=(t, nh * 192)), dtype), dtype)
+    kv = dev(rounded(rng.normal(size=(t, nh * 256 + gap)), dtype), dtype)
+    pe = dev(rounded(rng.normal(size=(t, 64 + gap)), dtype), dtype)[:, :64]
+    nope, v = kv[:, :nh * 128], kv[:, nh * 128:nh * 256]
+    starts = dev(_starts(q_lens), torch.int32)
+    joined = torch.cat((nope.reshape(t, nh, 128), pe.unsqueeze(1).expand(t, nh, 64)), dim=-1).reshape(t, nh * 192)
+    ref = ops.causal_attention_varlen(q, joined, v, starts, nh, nh, 192 ** -0.5)
+    assert torch.equal(ops.causal_attention_shared_rope(q, nope, pe, v, starts, nh, 192 ** -0.5), ref)
+    with pytest.raises(ValueError):
+        ops.causal_attention_shared_rope(q, nope, kv[:, :32], v, starts, nh, 192 ** -0.5)
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("lens", [[5], [0], [3, 0, 7], [0, 0, 9], [9, 4, 2, 6] * 40, [1] * 64, [2] * 65])
+def test_q_starts_on_the_gpu_equal_the_host_ones(lens, dtype):
+    """Lengths, row ends and lists that are both, also strided: the kernel gives what the torch expressions give on the CPU."""
+    total = sum(lens)
+    for values in (lens, list(np.cumsum(lens)), lens[::-1], [total] * len(lens)):
+        a = torch.tensor(values, dtype=dtype)
+        ref = ops.q_starts_from_actual_seq_len(a, total)
+        got = ops.q_starts_from_actual_seq_len(a.cuda(), total)
+        wide = ops.q_starts_from_actual_seq_len(torch.stack((a, a + 1), 1).cuda()[:, 0], total)
+        assert got.dtype == torch.int32 and torch.equal(got.cpu(), ref) and torch.equal(wide.cpu(), ref)
+
+
 @pytest.mark.parametrize("case,n_kv", [("1", 2), ("2", 1)])
 def test_prefill_reference_vectors(golden_dir, case, n_kv):
     """prefill_output_{1,2} of the reference's flash-attention unit test, from the packed rows and through the cache."""

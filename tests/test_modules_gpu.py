@@ -1257,6 +1257,25 @@ def test_mla_self_attention_with_quantized_projections():
         net2(x, None, key_cache=cache.clone(), **args)
 
 
+def test_mla_prefill_under_hooks_sees_joined_keys():
+    """The prefill attention takes the two parts of the keys only where nothing else looks at them: a hooked core attention and a
+    replaced ``forward`` get 192-wide keys, and all give the same bits."""
+    rng = np.random.default_rng(5)
+    net = _mla_module_and_params(rng, 512, 4, None, rope_type="rope")[0]
+    t, q_lens = 45, torch.tensor([20, 25], dtype=torch.int32, device="cuda")
+    x = dev(rounded(rng.normal(size=(t, 512)), BF), BF)
+    cos, sin = net.rotary_pos_emb.get_cos_sin_for_decode(torch.cat((torch.arange(20), torch.arange(25))).cuda())
+    args, seen = dict(rotary_pos_cos=cos, rotary_pos_sin=sin, actual_seq_qlen=q_lens), []
+    ref = net(x, None, **args)
+    handle = net.core_attention.register_forward_pre_hook(lambda m, a: seen.append(tuple(a[1].shape)))
+    assert torch.equal(net(x, None, **args), ref)
+    handle.remove()
+    original = net.core_attention.forward
+    net.core_attention.forward = lambda q, k, *a, **kw: (seen.append(tuple(k.shape)), original(q, k, *a, **kw))[1]
+    assert torch.equal(net(x, None, **args), ref)
+    assert seen == [(t, 4 * 192)] * 2
+
+
 def test_moe_experts_with_a_forward_or_hooks_of_their_own_see_the_tokens_type():
     """W8A8 experts get rows that are quantised already only where nothing else looks at them: a subclass with the three-argument
     ``forward``, a replaced ``forward`` and a hooked module get the 16-bit rows, and all give the same bits."""
