@@ -502,7 +502,7 @@ int mf_grouped_silu_mul_dynamic_quant(int8_t* xq, float* x_scale, const void* ga
  * bytes (int32 partial sums when K is split across workgroups; 0 for wide N). */
 size_t mf_w8a8_workspace_bytes(int m, int n, int k);
 /* As mf_w8a16_plan, for tiled activations (x_layout 1) and an output y without accumulators: 0 = LDS-staged, 1 =
- * register-streaming, 2 = wide, 3 = 128 x 256 tiles; fused: a norm + quantisation or RoPE + cache form. */
+ * register-streaming, 2 = wide (256 x 192, up to 256 rows also 128 x 320), 3 = tiles; fused: a norm + quantisation or RoPE + cache form. */
 int mf_w8a8_plan(int m, int n, int k, int fused, int* whole, int* cut, int* split);
 int mf_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale, const void* w_packed,
                  const float* w_scale, const void* bias, const void* residual, int m, int n, int k, int dtype,

@@ -7,7 +7,7 @@
 // channel blocks in its L2.  The tiles left over are cut into `split` parts of K each.
 struct TileGrid {
     int m_blocks, n_blocks, full, split, steps_per_split;
-    int mt;                                                   // rows of a block / 32
+    int mt, nt;                                               // rows of a block / 32, channels of a block / 64
 };
 constexpr int TG_PANEL = 4;                                   // row blocks walked together along the channels
 __device__ __forceinline__ void tg_locate(const TileGrid& g, int id, int& mb, int& nb, int& part, int& slot) {
@@ -32,14 +32,15 @@ inline int tg_workgroups(const TileGrid& g) { return g.full + (g.m_blocks * g.n_
 // writing and summing the parts.
 struct TileCost {
     float alone, pair, fixed, reduce, part;
-    float alone3;                                             // a k-step of a 96-row tile on a compute unit of its own
+    // other shapes of tile (32*mt rows, 64*nt channels), each on a compute unit of its own: a launch, a k-step
+    struct { int mt, nt; float fixed, step; } once[4];
 };
 // Whole tiles fill whole multiples of the 256 compute units; what is left over would hold a few of them for a whole tile's
 // time, so it is cut along K where the shorter tail pays for its parts.
-inline TileGrid tg_plan_rows(int m, int mt, int n_blocks, int steps, const TileCost& c, float* us) {
+inline TileGrid tg_plan_rounds(int m, int n, int steps, const TileCost& c, float* us) {
     TileGrid g;
-    const int m_blocks = (m + 32 * mt - 1) / (32 * mt);
-    g.mt = mt;
+    const int m_blocks = (m + 127) / 128, n_blocks = (n + 255) / 256;
+    g.mt = g.nt = 4;
     g.m_blocks = m_blocks;
     g.n_blocks = n_blocks;
     const int tiles = m_blocks * n_blocks, rounds = tiles / 256, rem = tiles % 256;
@@ -70,23 +71,36 @@ inline TileGrid tg_plan_rows(int m, int mt, int n_blocks, int steps, const TileC
     return g;
 }
 
-// 128-row tiles, or 96-row ones where those are all resident at once, each on a compute unit of its own: more units then share the
-// work, and fewer rows are padding.  One of few k-steps does not change, nor a single row block, which has no more tiles then.  W8A16, us,
-// 128 | 96 rows: 1048 x 4096 x 14336 157 | 135, 1300 x 4096 x 4096 53 | 46, 2025 x 2112 x 7168 83 | 71, 129 x 28672 x 4096 62 | 50, but
-// 65 x 28672 x 4096 42 | 46; W8A8: 1531 x 3584 x 18944 120 | 111, 1531 x 3584 x 3584 30.7 | 26.4, 1300 x 4608 x 3584 32.7 | 27.8.
-// Nor does a plan that is cut along K: with so few tiles its parts are all resident too, and they share the units better than 96-row
-// tiles do (23 of 23 shapes measured; W8A16 777 x 4096 x 4096 37.6 | 44.0, 513 x 6144 x 4096 38.5 | 44.5, 864 x 3584 x 3584 34.0 | 40.1; W8A8
-// 1632 x 2112 x 7168 35.8 | 39.3, 448 x 5120 x 5120 27.4 | 29.8).  The model prices parts that run at once too high (0.015 us each there,
-// not c.part), so against other kernels such a plan counts no more than the 96-row tiles would.
-inline TileGrid tg_plan(int m, int n_blocks, int steps, const TileCost& c, float* us) {
-    const TileGrid g = tg_plan_rows(m, 4, n_blocks, steps, c, us);
-    const int m_blocks = (m + 95) / 96;
-    const int64_t tiles = (int64_t)m_blocks * n_blocks;
-    const float us3 = steps * c.alone3 + c.fixed;
-    if (m <= 128 || steps < 16 || tiles > 256 || us3 >= (g.split > 1 ? 0.85f : 1.f) * *us) return g;
-    *us = us3;
-    if (g.split > 1) return g;
-    return {m_blocks, n_blocks, (int)tiles / 8 * 8, 1, steps, 3};
+// Tiles of 128 x 256, or of another shape where those are all resident at once, each on a compute unit of its own, and the shape is
+// the shortest: more units then share the work, or fewer rows and channels are padding.  A tile of fewer channels pays more for its
+// activations a matrix instruction, a wider one needs all the registers of a compute unit, so neither gains where the device is full for
+// several rounds.  us on 128 x 256 or 96 x 256 | with the other shapes: W8A16 1048 x 4096 x 4096 45.5 | 39.2 (96 x 192), 1048 x 4096 x
+// 14336 135 | 122, 2500 x 2112 x 7168 76.0 | 70.4 (128 x 192); W8A8 1531 x 3584 x 18944 114 | 104 (128 x 192), 1048 x 4096 x 7168 47.1 |
+// 40.6 (96 x 192), 700 x 5120 x 5120 33.6 | 29.8, 2025 x 5120 x 5120 62.0 | 53.8 (128 x 320).  On 10 shapes each of 130 to 3000 rows the
+// prices find the fastest one within 1 % on average.
+// A single row block does not change, nor one of fewer than 16 k-steps (24 for the shapes that are not 256 channels wide, which were
+// measured from there on and have to be 6 % shorter, about what the prices err by).  Nor does a plan all of whose tiles are cut along K: its parts are all resident too, and the model prices
+// parts that run at once too high (0.015 us each there, not c.part); against other kernels it counts a tenth less than 96 x 256 tiles would.
+// 96 x 256 | 128 x 256 in two parts: W8A16 777 x 4096 x 4096 44.0 | 37.6, 513 x 6144 x 4096 44.5 | 38.5, W8A8 448 x 5120 x 5120 29.8 |
+// 27.4.  Where only what is left over by whole rounds is cut, another shape has to be a fifth shorter.  96 x 192 where 96 x 256 would
+// leave a quarter of the units idle, and more of them are wanted (2025 x 2112 x 7168, 198 tiles of 96 x 256, would gain a seventh as well).
+inline TileGrid tg_plan(int m, int n, int steps, const TileCost& c, float* us) {
+    const TileGrid g = tg_plan_rounds(m, n, steps, c, us);
+    if (m <= 128 || steps < 16) return g;
+    const bool all_cut = g.split > 1 && g.full == 0;
+    const auto tiles_of = [&](int mt, int nt) { return (int64_t)((m + 32 * mt - 1) / (32 * mt)) * ((n + 64 * nt - 1) / (64 * nt)); };
+    TileGrid best = g;
+    float least = (g.split == 1 ? 1.f : all_cut ? 0.85f : 0.8f) * *us;
+    for (const auto& s : c.once) {
+        const int64_t tiles = s.mt ? tiles_of(s.mt, s.nt) : 257;
+        const float t = (all_cut ? 0.9f : 1.f) * (steps * s.step + s.fixed);
+        if (tiles > 256 || t >= (s.nt == 4 ? least : 0.94f * least)) continue;
+        if (s.nt != 4 && (steps < 24 || all_cut)) continue;
+        if (s.mt == 3 && s.nt == 3 && tiles_of(3, 4) > 192) continue;
+        least = *us = t;
+        if (!all_cut) best = {(m + 32 * s.mt - 1) / (32 * s.mt), (n + 64 * s.nt - 1) / (64 * s.nt), (int)tiles / 8 * 8, 1, steps, s.mt, s.nt};
+    }
+    return best;
 }
 
 // Grouped rows (experts): rows a group must average for tiles of 256 channels to replace 64-channel workgroups.  `least` is where
@@ -174,19 +188,21 @@ __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// 32 staged rows of up to 64 channels (144 bytes a row: 16-byte slots spread over the banks) to memory as whole 16-byte pieces
+// 32 staged rows of up to 16 * NT channels (16 bytes more a row: 16-byte slots spread over the banks) to memory as whole 16-byte pieces
 // of rows, by `threads` threads of which this is number t; the residual, read the same way, is added to the rounded values.
 // cols = row length of y, c0 = first channel, per = 16-byte pieces of a staged row.
 // STREAM: stores past the caches, see tg_group_stream.
-constexpr int TG_STAGE_ROW = 144;
-template <typename T, bool STREAM = false>
+template <int NT>
+constexpr int TG_STAGE_ROW = 32 * NT + 16;
+template <typename T, int NT, bool STREAM = false>
 __device__ __forceinline__ void tg_flush(uint16_t* y, const uint16_t* residual, const uint8_t* stage, int m0, int M, int c0,
                                          int cols, int per, bool aligned, int t, int threads) {
     const int row = t / per, c = c0 + 8 * (t - row * per), step = threads / per;
+    if (row >= step) return;                                  // threads past the last whole row
     for (int j = row; j < 32; j += step) {
         const int m = m0 + j;
         if (m >= M || c >= cols) continue;
-        u32x4 v = *(const u32x4*)(stage + j * TG_STAGE_ROW + 2 * (c - c0));
+        u32x4 v = *(const u32x4*)(stage + j * TG_STAGE_ROW<NT> + 2 * (c - c0));
         const int64_t at = (int64_t)m * cols + c;
         if (residual) {
             float f[8], g[8];

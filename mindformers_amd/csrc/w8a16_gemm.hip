@@ -515,15 +515,15 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 3 : 1) void w8a16_gemm4_ke
 }
 
 // ---- many rows ---------------------------------------------------------------------------------------------------------
-// More rows than two or three passes of the skinny kernel: tiles of 128 or 96 rows x 256 channels (w8a16_tile_gemm.h).
-// Output of one wave: 64 channels from n0 on, 32 rows at a time.  The channels of a row lie spread over the accumulators of
+// More rows than two or three passes of the skinny kernel: tiles of 128 or 96 rows x 256 or 192 channels (w8a16_tile_gemm.h).
+// Output of one wave: 16*NT channels from n0 on, 32 rows at a time.  The channels of a row lie spread over the accumulators of
 // four lanes, so the values (dequantised, with bias, gated where asked, rounded to T) go through LDS and leave as whole
-// 128-byte (gated: 64-byte) pieces of rows; the residual is read the same way.  Rounding points as in store4 / store_gated.
+// pieces of rows (128 bytes for 64 channels, gated 64); the residual is read the same way.  Rounding points as in store4 / store_gated.
 // (8-byte stores straight from the accumulators, each waiting for its own scales, on an earlier form of the tiles: 4096 x 4096 at 1536
 // rows 69.8 us against 54.3, 24576 x 1536 at 129 rows 42.3 against 25.6.)  N is a multiple of 16.
-template <typename T>
+template <typename T, int NT = 4>
 struct TileOut {
-    static constexpr int ROW = TG_STAGE_ROW;
+    static constexpr int ROW = TG_STAGE_ROW<NT>;
     uint16_t* y;
     const uint16_t *bias, *residual;
     int M, N, gated, aligned;
@@ -558,45 +558,46 @@ struct TileOut {
     // the 32 staged rows to memory, by `threads` threads of which this is number t
     template <bool STREAM = false>
     __device__ __forceinline__ void flush(int m0, int n0, const uint8_t* stage, int t, int threads) const {
-        tg_flush<T, STREAM>(y, residual, stage, m0, M, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? 4 : 8, aligned, t, threads);
+        tg_flush<T, NT, STREAM>(y, residual, stage, m0, M, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? NT : 2 * NT, aligned, t,
+                                threads);
     }
 };
 
-template <typename T, int MT>
+template <typename T, int MT, int NT>
 __global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
     uint16_t* __restrict__ y, float* __restrict__ partial, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp,
     const float* __restrict__ scale, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N,
     int K, int gated, int aligned, TileGrid g) {
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * 32 * MT * 128];
-    static_assert(tg::WAVES * 32 * TileOut<T>::ROW <= (int)sizeof(smem), "the output stage reuses the operand stages");
+    constexpr int OPS = 2 * 32 * MT * 128, OUT = tg::WAVES * 32 * TileOut<T, NT>::ROW;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];   // the output stage reuses the operand stages
     int mb, nb, part, slot;
     tg_locate(g, blockIdx.x, mb, nb, part, slot);
     const bool whole = blockIdx.x < g.full || g.split == 1;
     const int KS = K / tg::KSTEP, s0 = part * g.steps_per_split;
     const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = mb * 32 * MT, n0 = nb * tg::BN + 64 * wv;
-    float* pt = partial + (int64_t)slot * (32 * MT * tg::BN) + (wv * MT * 8 * 64 + lane) * 4;
-    const TileOut<T> out{y, bias, residual, M, N, gated, aligned};
-    f32x4 sc[4], bi[4];
-    uint8_t* stage = smem + wv * 32 * TileOut<T>::ROW;
-    tg::tile<T, MT, 0, false>(x, wp, M, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const f32x4 (&acc)[2][4]) {
+    const int m0 = mb * 32 * MT, n0 = nb * tg::BN_OF<NT> + 16 * NT * wv;
+    float* pt = partial + (int64_t)slot * (32 * MT * tg::BN_OF<NT>) + (wv * MT * 2 * NT * 64 + lane) * 4;
+    const TileOut<T, NT> out{y, bias, residual, M, N, gated, aligned};
+    f32x4 sc[NT], bi[NT];
+    uint8_t* stage = smem + wv * 32 * TileOut<T, NT>::ROW;
+    tg::tile<T, MT, NT, 0, false>(x, wp, M, K, m0, nb * (tg::BN_OF<NT> / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const f32x4 (&acc)[2][NT]) {
         constexpr int mt = decltype(mtc)::value;
         if (whole) {
             if (mt == 0) {
                 __syncthreads();                              // every wave has read its last operands
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt) out.load(scale, n0, nt, sc[nt], bi[nt]);
+                for (int nt = 0; nt < NT; ++nt) out.load(scale, n0, nt, sc[nt], bi[nt]);
             }
             wave_lds_order();
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                out.put(acc[e >> 2][e & 3], sc[e & 3], bi[e & 3], e >> 2, e & 3, stage);
+            for (int e = 0; e < 2 * NT; ++e)
+                out.put(acc[e / NT][e % NT], sc[e % NT], bi[e % NT], e / NT, e % NT, stage);
             wave_lds_order();
             out.flush(m0 + 32 * mt, n0, stage, lane, 64);
         } else {                                              // accumulator order: whole cache lines
 #pragma unroll
-            for (int e = 0; e < 8; ++e) *(f32x4*)(pt + (mt * 8 + e) * 256) = acc[e >> 2][e & 3];
+            for (int e = 0; e < 2 * NT; ++e) *(f32x4*)(pt + (mt * 2 * NT + e) * 256) = acc[e / NT][e % NT];
         }
     });
 }
@@ -691,7 +692,7 @@ __device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* xe
     const TileOut<T> out{y, nullptr, nullptr, rows, N, gated, aligned};
     f32x4 sc[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TileOut<T>::ROW;
-    tg::tile<T, MT, MT == 4 ? 2 : MT == 3 ? 0 : 2 * MT, NT>(xe, we, rows, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, 0, K / tg::KSTEP, smem,
+    tg::tile<T, MT, 4, MT == 4 ? 2 : MT == 3 ? 0 : 2 * MT, NT>(xe, we, rows, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, 0, K / tg::KSTEP, smem,
                     [&](auto mtc, const f32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
         if (mt == 0) {
@@ -1135,9 +1136,9 @@ struct GemmPlan {
 
 // Tile plan of the many-row kernel (4137 x 4096 x 14336: 16 of 528 tiles left over by whole rounds, 455 us uncut, 351 us in
 // 8 parts).
-constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f, 0.56f};
+constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f, {{3, 4, 7.8f, 0.6f}, {3, 3, 7.8f, 0.477f}, {4, 3, 8.5f, 0.556f}}};
 TileGrid plan_tiles(int m, int n, int k, float* us) {
-    return tg_plan(m, (n + tg::BN - 1) / tg::BN, k / tg::KSTEP, TG_COST, us);
+    return tg_plan(m, n, k / tg::KSTEP, TG_COST, us);
 }
 
 GemmPlan plan_w8a16(int m, int n, int k, int step_align = 1) {
@@ -1187,11 +1188,13 @@ void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale,
     float us;
     const TileGrid g = plan_tiles(m, n, k, &us);
     const int aligned = (((uintptr_t)y | (uintptr_t)residual) & 15) == 0;
-#define TG_LAUNCH(MT)                                                                                              \
-    hipLaunchKernelGGL((w8a16_tile_kernel<T, MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y, (float*)workspace, \
+#define TG_LAUNCH(MT, NT)                                                                                          \
+    hipLaunchKernelGGL((w8a16_tile_kernel<T, MT, NT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y, (float*)workspace, \
                        (const uint16_t*)x, wp, scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, gated, aligned, g)
-    if (g.mt == 3) TG_LAUNCH(3);
-    else TG_LAUNCH(4);
+    if (g.mt == 3 && g.nt == 3) TG_LAUNCH(3, 3);
+    else if (g.mt == 3) TG_LAUNCH(3, 4);
+    else if (g.nt == 3) TG_LAUNCH(4, 3);
+    else TG_LAUNCH(4, 4);
 #undef TG_LAUNCH
     if (g.split > 1)                                          // 128-row tiles
         hipLaunchKernelGGL((w8a16_tile_reduce_kernel<T, 4>), dim3((g.m_blocks * g.n_blocks - g.full) * tg::WAVES * 4), dim3(256), 0, st,
@@ -1369,7 +1372,7 @@ extern "C" size_t mf_w8a16_workspace_bytes(int m, int n, int k) {
     if (use_tiles(m, n, k)) {
         float us;
         const TileGrid g = plan_tiles(m, n, k, &us);
-        return g.split > 1 ? (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * g.mt * tg::BN) * sizeof(float) : 0;
+        return g.split > 1 ? (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (128 * tg::BN) * sizeof(float) : 0;
     }
     const GemmPlan p = plan_w8a16(m, n, k);
     return p.split_k > 1 ? (size_t)p.split_k * m * n * sizeof(float) : 0;

@@ -3,11 +3,11 @@
 #include "common.h"
 #include "tile_grid.h"
 
-// A workgroup of 4 waves (one per SIMD, two workgroups per compute unit) owns 32*MT rows x 256 channels; wave w owns channels
-// 64w .. 64w + 63 of all the rows, so that every weight byte of the tile is loaded and converted by exactly one wave and goes
+// A workgroup of 4 waves (one per SIMD, two workgroups per compute unit) owns 32*MT rows x 64*NT channels (MT and NT: 3 or 4, see
+// tg_plan); wave w owns the w-th quarter of the channels of all the rows, so that every weight byte of the tile is loaded and converted by exactly one wave and goes
 // from global memory straight into matrix operand registers, while the activation tile of a 64-wide k-step is staged in LDS
 // once and read by all four.  Weights are fetched two steps ahead by ordinary loads (the compiler counts them); the activations of a
-// step are written to the other of two LDS stages one step ahead.  A step is eight groups, (32 columns, 16 channels) each over all
+// step are written to the other of two LDS stages one step ahead.  A step is 2*NT groups, (32 columns, 16 channels) each over all
 // the rows: a group's 2*MT matrix instructions share one weight operand, and behind each of them goes a piece of what is needed
 // next (the conversion of the next group's weights, a row tile of the next 32 columns, a load), in the order written here; one
 // barrier per step, in front of the groups that begin to read the next one.
@@ -19,12 +19,14 @@
 //
 // What bounds it: the power budget.  4137 x 28672 x 4096: 782-797 us on 32x32x16, 714-724 here (1360 TFLOP/s); 4137 x 4096 x 14336:
 // 398 / 351-359; 2025 x 7168 x 16384: 424 / 350-360.  A lone workgroup on a compute unit (few tiles) is bound by issue: one wave starts a
-// vector instruction every 8 cycles, and a step has 96 beside 64 matrix instructions of 16 (0.7 to 0.9 us a step, two workgroups
-// together 1.55).
+// vector instruction every 8 cycles, and a step of 128 x 256 has 96 beside 64 matrix instructions of 16 (0.7 to 0.9 us a step, two
+// workgroups together 1.55; 96 x 256 0.60, 128 x 192 0.56, 96 x 192 0.48).
 namespace tg {
 
 constexpr int WAVES = 4;
-constexpr int BN = 64 * WAVES;                                // channels per workgroup
+template <int NT>
+constexpr int BN_OF = 16 * NT * WAVES;                       // channels per workgroup of NT 16-channel tiles a wave
+constexpr int BN = BN_OF<4>;
 constexpr int KSTEP = 64;
 constexpr int DW = 2;                                         // steps of weights in flight
 template <int MT>
@@ -35,9 +37,9 @@ constexpr int DX = MT == 4 ? 1 : 2;                           // steps of activa
 // chunks of two rows in both
 __device__ __forceinline__ int key(int row) { return ((row >> 1) & 1) | (((row >> 3) & 1) << 2); }
 
-// EARLY: 16-row tiles of a sub-step that are read behind the third channel tile of the one before; the others follow behind the
-// fourth, each into the registers of a tile that has just been used (0: half and half).  NT: weights that nobody else reads (non-temporal loads)
-template <typename T, int MT, int EARLY, bool NT, typename Epilogue>
+// EARLY: 16-row tiles of a sub-step that are read behind the last but one channel tile of the one before; the others follow behind the
+// last, each into the registers of a tile that has just been used (0: half and half).  STREAM: weights that nobody else reads (non-temporal loads)
+template <typename T, int MT, int NT, int EARLY, bool STREAM, typename Epilogue>
 __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, int M, int K, int m0,
                                      int tile0, int n_tiles, int s_begin, int s_end, uint8_t* smem, Epilogue&& epilogue) {
     using vec8 = typename T::vec8;
@@ -62,13 +64,13 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
         *(u32x4*)(smem + stage * STAGE + 4096 * i + xdst) = xreg[decltype(setc)::value][i];
     };
     // ---- weights: lane (r, g) of a packed 16-channel tile holds columns 16g .. 16g + 15 of channel r
-    const uint8_t* wbase[4];
+    const uint8_t* wbase[NT];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) wbase[nt] = wp + (int64_t)min(tile0 + 4 * wv + nt, n_tiles - 1) * 1024;
-    u32x4 wreg[DW][4];
+    for (int nt = 0; nt < NT; ++nt) wbase[nt] = wp + (int64_t)min(tile0 + NT * wv + nt, n_tiles - 1) * 1024;
+    u32x4 wreg[DW][NT];
     auto load_w = [&](auto setc, auto nc, int s) {
         constexpr int nt = decltype(nc)::value;
-        wreg[decltype(setc)::value][nt] = load16_at<NT>(wbase[nt] + (int64_t)min(s, s_last) * n_tiles * 1024, lane * 16);
+        wreg[decltype(setc)::value][nt] = load16_at<STREAM>(wbase[nt] + (int64_t)min(s, s_last) * n_tiles * 1024, lane * 16);
     };
     // ---- operands: a sub-step u of a step is 32 columns, 16g + 8u .. + 7 in lane (r, g).  The rows of a sub-step stay in registers
     // while the wave's four channel tiles pass by, converted one ahead
@@ -79,11 +81,11 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
         const int at = frow + (((2 * (lane >> 4) + U) ^ fkey) << 4);
         xf[U][m] = bitcast<vec8>(*(const u32x4*)(smem + stage * STAGE + 2048 * m + at));
     };
-    f32x4 acc[MT][2][4];                                      // [32-row block][16-row tile of it][16-channel tile]
+    f32x4 acc[MT][2][NT];                                     // [32-row block][16-row tile of it][16-channel tile]
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[mt][j >> 2][j & 3] = (f32x4)(0.f);
+        for (int j = 0; j < 2 * NT; ++j) acc[mt][j / NT][j % NT] = (f32x4)(0.f);
     using C0 = std::integral_constant<int, 0>;
     using C1 = std::integral_constant<int, 1>;
 
@@ -103,7 +105,7 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (xj > 0) static_for<MT>([&](auto ic) { load_x(std::integral_constant<int, xj % DX<MT>>{}, ic, s_first + xj); });
         __builtin_amdgcn_sched_barrier(0);
-        static_for<4>([&](auto nc) { load_w(jc, nc, max(s_first + j, s_begin)); });
+        static_for<NT>([&](auto nc) { load_w(jc, nc, max(s_first + j, s_begin)); });
         __builtin_amdgcn_sched_barrier(0);
     });
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -115,10 +117,10 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
     // group (u, nt): every row of sub-step u times channel tile nt, and behind each matrix instruction a piece of what the next
     // groups need
     auto group = [&](auto jsc, auto gc, int s) {
-        constexpr int J = decltype(jsc)::value, P = J & 1, G = decltype(gc)::value, U = G >> 2, nt = G & 3, NM = 2 * MT;
-        constexpr int NS = G == 7 ? (J + 1) % DW : J, NU = ((G + 1) >> 2) & 1, NN = (G + 1) & 3;      // the tile converted here
+        constexpr int J = decltype(jsc)::value, P = J & 1, G = decltype(gc)::value, U = G / NT, nt = G % NT, NM = 2 * MT;
+        constexpr int NS = G == 2 * NT - 1 ? (J + 1) % DW : J, NU = (G + 1) / NT & 1, NN = (G + 1) % NT;   // the tile converted here
         using CX = std::integral_constant<int, (J + 1) % DX<MT>>;                               // the next step's activations
-        if constexpr (G == 6) {                               // the other stage is written, this one has been read
+        if constexpr (G == 2 * NT - 2) {                            // the other stage is written, this one has been read
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
         }
@@ -134,8 +136,9 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
                 if constexpr (j * NM / 4 == m) w[j] = i8x2_to<T>(wreg[NS][NN][2 * NU + (j >> 1)], 16 * (j & 1));
             });
             // the next sub-step's rows: two halves behind every other instruction, or EARLY of them first and then one by one
-            constexpr int R = EARLY == 0 ? (m & 1 ? MT * (nt - 2) + m / 2 : NM) : nt == 2 ? (m < NM - EARLY ? NM : m - NM + EARLY) : EARLY + m;
-            if constexpr (nt >= 2 && R < NM)
+            constexpr int L = nt - (NT - 2);                  // the last two channel tiles
+            constexpr int R = EARLY == 0 ? (m & 1 ? MT * L + m / 2 : NM) : L == 0 ? (m < NM - EARLY ? NM : m - NM + EARLY) : EARLY + m;
+            if constexpr (L >= 0 && R < NM)
                 read_x(std::integral_constant<int, R>{}, U == 0 ? P : P ^ 1, std::integral_constant<int, U ^ 1>{});
             if constexpr (G == 0 && (m & 1) == 0) write_x(CX{}, std::integral_constant<int, m / 2>{}, P ^ 1);   // read before the last barrier
             if constexpr (G == 0 && (m & 1) == 1) load_x(CX{}, std::integral_constant<int, m / 2>{}, s + 1 + DX<MT>);
@@ -145,13 +148,13 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
         wf = bitcast<vec8>((u32x4){w[0], w[1], w[2], w[3]});
     };
     auto step = [&](auto jsc, int s) {                        // step J of a round over the weights' register sets, LDS stage J & 1
-        static_for<8>([&](auto gc) { group(jsc, gc, s); });
+        static_for<2 * NT>([&](auto gc) { group(jsc, gc, s); });
     };
     for (int s = s_first; s < s_end; s += DW) static_for<DW>([&](auto jc) { step(jc, s + decltype(jc)::value); });
-    asm volatile("s_nop 15" : "+a"(acc[MT - 1][1][3]));      // the last matrix instructions' results
-    static_for<8 * MT>([&](auto jc) {
+    asm volatile("s_nop 15" : "+a"(acc[MT - 1][1][NT - 1]));      // the last matrix instructions' results
+    static_for<2 * NT * MT>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
-        f32x4& a = acc[j >> 3][(j >> 2) & 1][j & 3];
+        f32x4& a = acc[j / (2 * NT)][j / NT & 1][j % NT];
         asm volatile("" : "+a"(a));
     });
     static_for<MT>([&](auto mtc) { epilogue(mtc, acc[decltype(mtc)::value]); });

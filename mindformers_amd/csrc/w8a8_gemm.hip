@@ -20,10 +20,10 @@
 // applied on the global-address side, which makes the operand reads bank-conflict free.
 // Small N cannot fill the chip with output tiles alone: K is then split across workgroups, which write exact
 // int32 partial tiles that a second kernel sums (integer sums do not depend on the order).
-// More kernels serve the shapes where that one is not the best: from 65 rows on with tiled activations 128 x 256 or 96 x 256
-// tiles with v_mfma_i32_16x16x64_i8 (w8a8_tile_kernel); where those leave a part of a round over, for narrow outputs and
+// More kernels serve the shapes where that one is not the best: from 65 rows on with tiled activations tiles of 128 or 96 rows x
+// 192, 256 or 320 channels with v_mfma_i32_16x16x64_i8 (w8a8_tile_kernel); where those leave a part of a round over, for narrow outputs and
 // few rows, a register-streaming kernel (w8a8_regs_kernel) and, for very wide outputs at 129+ rows (also where the tiles cannot
-// serve the call: accumulators asked for, N not a multiple of 16), 256 x 192 tiles on 8 waves with a coalesced, LDS-turned
+// serve the call: accumulators asked for, N not a multiple of 16; otherwise see plan_q_wide_tiles), 256 x 192 tiles on 8 waves with a coalesced, LDS-turned
 // epilogue (w8a8_wide_kernel).
 #include "common.h"
 #include "tile_grid.h"
@@ -757,10 +757,10 @@ __global__ __launch_bounds__(QRC_THREADS) void w8a8_reduce_rope_cache_kernel(
     }
 }
 
-// ---- many rows (tiled activations): 128 x 256 tiles, w8a8_tile_gemm.h ------------------------------------------------
-// Output of one wave, 32 rows x 64 channels at a time, through LDS as whole pieces of rows (tg_flush); rounding points as in
+// ---- many rows (tiled activations): w8a8_tile_gemm.h -----------------------------------------------------------------
+// Output of one wave, 32 rows x 16*NT channels at a time, through LDS as whole pieces of rows (tg_flush); rounding points as in
 // q2_store4.  N is a multiple of 16.
-template <typename T>
+template <typename T, int NT = 4>
 struct QTileOut {
     const float *x_scale, *w_scale;
     const uint16_t* bias;
@@ -777,19 +777,19 @@ struct QTileOut {
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = scaled_bias((float)a[i], xs, ws[i], true, bi[i], bias != nullptr);
-        uint8_t* row = stage + (16 * j + (threadIdx.x & 15)) * TG_STAGE_ROW;
+        uint8_t* row = stage + (16 * j + (threadIdx.x & 15)) * TG_STAGE_ROW<NT>;
         const int c = 16 * nt + 4 * ((threadIdx.x >> 4) & 3);
         if (gated) *(uint32_t*)(row + c) = q2_gated4<T>(v);
         else *(u32x2*)(row + 2 * c) = (u32x2){pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
     }
 };
 
-template <typename T, int MT>
-__global__ __launch_bounds__(256, 2) void w8a8_tile_kernel(
+template <typename T, int MT, int NT>
+__global__ __launch_bounds__(256, MT * NT > 16 ? 1 : 2) void w8a8_tile_kernel(
     uint16_t* __restrict__ y, int32_t* __restrict__ partial, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
     const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const uint16_t* __restrict__ bias,
     const uint16_t* __restrict__ residual, int M, int N, int K, int aligned, TileGrid g) {
-    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW, OPS = tq::LDS_BYTES<MT>;
+    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW<NT>, OPS = tq::LDS_BYTES<MT>;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
     int mb, nb, part, slot;
     tg_locate(g, blockIdx.x, mb, nb, part, slot);
@@ -797,32 +797,32 @@ __global__ __launch_bounds__(256, 2) void w8a8_tile_kernel(
     const int KS = (K + Q_KSTEP - 1) / Q_KSTEP, s0 = part * g.steps_per_split;
     const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = mb * 32 * MT, n0 = nb * tq::BN + 64 * wv;
-    int32_t* pt = partial + (int64_t)slot * (32 * MT * tq::BN) + (wv * MT * 8 * 64 + lane) * 4;
-    const QTileOut<T> out{x_scale, w_scale, bias, M, N, 0};
-    f32x4 ws[4], bi[4];
-    uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
+    const int m0 = mb * 32 * MT, n0 = nb * tq::BN_OF<NT> + 16 * NT * wv;
+    int32_t* pt = partial + (int64_t)slot * (32 * MT * tq::BN_OF<NT>) + (wv * MT * 2 * NT * 64 + lane) * 4;
+    const QTileOut<T, NT> out{x_scale, w_scale, bias, M, N, 0};
+    f32x4 ws[NT], bi[NT];
+    uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW<NT>;
     const tq::TiledRows<tq::XLOADS<MT>> rows((const uint8_t*)xq, m0 >> 4, (M + 15) >> 4, wv);
-    tq::tile<MT, false>(rows, wp, nb * (tq::BN / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const i32x4 (&acc)[2][4]) {
+    tq::tile<MT, NT, false>(rows, wp, nb * (tq::BN_OF<NT> / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const i32x4 (&acc)[2][NT]) {
         constexpr int mt = decltype(mtc)::value;
         if (whole) {
             if (mt == 0) {
                 __syncthreads();                              // every wave has read its last operands
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt) out.load(n0, nt, ws[nt], bi[nt]);
+                for (int nt = 0; nt < NT; ++nt) out.load(n0, nt, ws[nt], bi[nt]);
             }
             wave_lds_order();
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const float xs = x_scale[min(m0 + 32 * mt + 16 * j + (lane & 15), M - 1)];
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt) out.put(acc[j][nt], xs, ws[nt], bi[nt], j, nt, stage);
+                for (int nt = 0; nt < NT; ++nt) out.put(acc[j][nt], xs, ws[nt], bi[nt], j, nt, stage);
             }
             wave_lds_order();
-            tg_flush<T>(y, residual, stage, m0 + 32 * mt, M, n0, N, 8, aligned, lane, 64);
+            tg_flush<T, NT>(y, residual, stage, m0 + 32 * mt, M, n0, N, 2 * NT, aligned, lane, 64);
         } else {                                              // accumulator order: whole cache lines
 #pragma unroll
-            for (int e = 0; e < 8; ++e) *(i32x4*)(pt + (mt * 8 + e) * 256) = acc[e >> 2][e & 3];
+            for (int e = 0; e < 2 * NT; ++e) *(i32x4*)(pt + (mt * 2 * NT + e) * 256) = acc[e / NT][e % NT];
         }
     });
 }
@@ -833,7 +833,7 @@ __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
     uint16_t* __restrict__ y, const int32_t* __restrict__ partial, const float* __restrict__ x_scale,
     const float* __restrict__ w_scale, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N,
     int aligned, TileGrid g) {
-    __shared__ __attribute__((aligned(16))) uint8_t stage[32 * TG_STAGE_ROW];
+    __shared__ __attribute__((aligned(16))) uint8_t stage[32 * TG_STAGE_ROW<4>];
     constexpr int ITEMS = tq::WAVES * MT;                     // workgroups per tile
     constexpr int64_t PART = 32 * MT * tq::BN;
     const int tile = blockIdx.x / ITEMS, item = blockIdx.x - tile * ITEMS, wv = item / MT, mt = item - wv * MT;
@@ -856,7 +856,7 @@ __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
 #pragma unroll
     for (int e = 0; e < 2; ++e) out.put(v[e], xs, ws[e], bi[e], (e0 + e) >> 2, (e0 + e) & 3, stage);
     __syncthreads();
-    tg_flush<T>(y, residual, stage, m0, M, n0, N, 8, aligned, threadIdx.x, 256);
+    tg_flush<T, 4>(y, residual, stage, m0, M, n0, N, 8, aligned, threadIdx.x, 256);
 }
 
 // ---- grouped (experts): rows offsets[e] .. offsets[e+1] of the quantised activations use expert e's weights --------
@@ -1012,9 +1012,9 @@ __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, 
     const int n0 = nb * tq::BN + 64 * wv;
     const QTileOut<T> out{xs, ws, nullptr, rows, N, gated};
     f32x4 wsv[4], bi[4];
-    uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW;
+    uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW<4>;
     const tq::PlainRows<tq::XLOADS<MT>> src(xe, m0, rows, K, wv);
-    tq::tile<MT, NT>(src, we, nb * (tq::BN / 16), (N + 15) >> 4, 0, (K + Q_KSTEP - 1) / Q_KSTEP, smem,
+    tq::tile<MT, 4, NT>(src, we, nb * (tq::BN / 16), (N + 15) >> 4, 0, (K + Q_KSTEP - 1) / Q_KSTEP, smem,
                  [&](auto mtc, const i32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
         if (mt == 0) {
@@ -1030,7 +1030,7 @@ __device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, 
             for (int nt = 0; nt < 4; ++nt) out.put(acc[j][nt], x1, wsv[nt], bi[nt], j, nt, stage);
         }
         wave_lds_order();
-        tg_flush<T, STREAM>(y, nullptr, stage, m0 + 32 * mt, rows, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? 4 : 8, aligned,
+        tg_flush<T, 4, STREAM>(y, nullptr, stage, m0 + 32 * mt, rows, gated ? n0 >> 1 : n0, gated ? N >> 1 : N, gated ? 4 : 8, aligned,
                             lane, 64);
     });
 }
@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
     uint16_t* __restrict__ y, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
     const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const int32_t* __restrict__ offsets, int n_experts,
     int total_rows, int N, int K, int64_t expert_bytes, int gated, int aligned) {
-    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW, OPS = tq::LDS_BYTES<4>;
+    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW<4>, OPS = tq::LDS_BYTES<4>;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
     int e, m0, row0, rows, nb;
     if (!tg_group_locate(offsets, n_experts, total_rows, (N + tq::BN - 1) / tq::BN, e, m0, row0, rows, nb)) return;
@@ -1123,7 +1123,7 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
     return p;
 }
 
-// Many rows, tiled activations: 128 x 256 tiles against the kernels above.  Measured, a 64-wide step of a round of 256
+// Many rows, tiled activations: tiles (the figures: of 128 x 256, see tg_plan for the others) against the kernels above.  Measured, a 64-wide step of a round of 256
 // workgroups takes 0.32 us in the register-streaming kernel, 0.78 us in the wide one and 0.38 to 0.50 us in the LDS-staged one
 // (one workgroup on a compute unit; it starts and ends like a tile).  37888 x 3584 at 65 / 257 / 1531 rows runs in 35 / 54 / 182 us on
 // tiles against 51 / 86 / 232 (256 rows: 296 tiles, 40 more than units, 50 us against 48 on 198 wide tiles), 24576 x 1536 at 257 / 640
@@ -1131,11 +1131,11 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
 // against 33 / 33 / 55 (LDS-staged), 3584 x 18944 at 1531 rows in 113 against 172, 3584 x 3584 at 448 rows in 26 against 22.  `fused`: the
 // sum of the register-streaming and the wide kernel's parts carries what follows, which is a kernel of its own behind tiles (the
 // figures of the LDS-staged kernel have it in).
-constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f, 0.31f};
+constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f, {{3, 4, 6.6f, 0.346f}, {3, 3, 6.4f, 0.288f}, {4, 3, 9.5f, 0.3f}, {4, 5, 12.2f, 0.509f}}};
 bool plan_q_tiles(int m, int n, int k, bool fused, TileGrid& g) {
     if (m <= 64 || n % 16 != 0) return false;
     float us;
-    g = tg_plan(m, (n + tq::BN - 1) / tq::BN, (k + Q_KSTEP - 1) / Q_KSTEP, TQ_COST, &us);
+    g = tg_plan(m, n, (k + Q_KSTEP - 1) / Q_KSTEP, TQ_COST, &us);
     const QPlan p = plan_w8a8(m, n, k, true);
     const int rounds = (p.n_blocks * p.m_blocks * p.split_k + 255) / 256;
     const bool staged = !p.regs && !p.wide;
@@ -1144,16 +1144,30 @@ bool plan_q_tiles(int m, int n, int k, bool fused, TileGrid& g) {
     return us + (fused && p.split_k > 1 && !staged ? 6.f : 0.f) < old;
 }
 
+// Wide outputs at 129 to 256 rows: tiles of 128 x 320, each with a compute unit to itself, in place of the wide kernel's 256 x 192 where
+// there is one round of them (the k-loop is the shorter one, the start the longer).  256 x 37888 x 3584: 198 wide tiles 49.5 us, 238 of
+// these 43.2.
+bool plan_q_wide_tiles(const QPlan& p, int m, int n, int k, TileGrid& g) {
+    const int steps = (k + Q_KSTEP - 1) / Q_KSTEP, m_blocks = 2, n_blocks = (n + tq::BN_OF<5> - 1) / tq::BN_OF<5>, tiles = m_blocks * n_blocks;
+    if (!p.wide || p.split_k > 1 || m <= 128 || m > 256 || n % 16 != 0 || tiles > 256) return false;
+    const int rounds = (p.n_blocks * p.m_blocks + 255) / 256;
+    g = {m_blocks, n_blocks, tiles / 8 * 8, 1, steps, 4, 5};
+    return 12.2f + 0.509f * steps < 5.f + 0.78f * rounds * steps;
+}
+
 template <typename T>
 void launch_q_tiles(const TileGrid& g, void* y, const int8_t* xq, const float* x_scale, const uint8_t* wp,
                     const float* w_scale, const void* bias, const void* residual, int m, int n, int k, void* workspace,
                     hipStream_t st) {
     const int aligned = (((uintptr_t)y | (uintptr_t)residual) & 15) == 0;
-#define TQ_LAUNCH(MT)                                                                                              \
-    hipLaunchKernelGGL((w8a8_tile_kernel<T, MT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y, (int32_t*)workspace, xq, \
+#define TQ_LAUNCH(MT, NT)                                                                                          \
+    hipLaunchKernelGGL((w8a8_tile_kernel<T, MT, NT>), dim3(tg_workgroups(g)), dim3(256), 0, st, (uint16_t*)y, (int32_t*)workspace, xq, \
                        x_scale, wp, w_scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, aligned, g)
-    if (g.mt == 3) TQ_LAUNCH(3);
-    else TQ_LAUNCH(4);
+    if (g.mt == 3 && g.nt == 3) TQ_LAUNCH(3, 3);
+    else if (g.mt == 3) TQ_LAUNCH(3, 4);
+    else if (g.nt == 3) TQ_LAUNCH(4, 3);
+    else if (g.nt == 5) TQ_LAUNCH(4, 5);
+    else TQ_LAUNCH(4, 4);
 #undef TQ_LAUNCH
     if (g.split > 1)                                          // 128-row tiles
         hipLaunchKernelGGL((w8a8_tile_reduce_kernel<T, 4>), dim3((g.m_blocks * g.n_blocks - g.full) * tq::WAVES * 4),
@@ -1168,7 +1182,7 @@ int launch_w8a8(void* y, int32_t* acc_out, const int8_t* xq, const float* x_scal
                 const QRopeCacheArgs* rc = nullptr) {
     QPlan p = plan_w8a8(m, n, k, x_tiled);
     TileGrid g;
-    const bool tiles = x_tiled && y && !acc_out && plan_q_tiles(m, n, k, nq || rc, g);
+    const bool tiles = x_tiled && y && !acc_out && (plan_q_tiles(m, n, k, nq || rc, g) || plan_q_wide_tiles(p, m, n, k, g));
     if (tiles) p.split_k = 1;                                 // the tile kernel sums its own parts
     int32_t* partial = p.split_k > 1 ? (int32_t*)workspace : nullptr;
     dim3 grid(p.n_blocks, p.split_k, p.m_blocks);
@@ -1267,7 +1281,7 @@ extern "C" size_t mf_w8a8_workspace_bytes(int m, int n, int k) {
     }
     TileGrid g;
     if (plan_q_tiles(m, n, k, false, g) && g.split > 1) {     // enough for either kernel
-        const size_t b = (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (32 * g.mt * tq::BN) * sizeof(int32_t);
+        const size_t b = (size_t)(g.m_blocks * g.n_blocks - g.full) * g.split * (128 * tq::BN) * sizeof(int32_t);
         need = b > need ? b : need;
     }
     return need;
@@ -1284,6 +1298,11 @@ extern "C" int mf_w8a8_plan(int m, int n, int k, int fused, int* whole, int* cut
     }
     const QPlan p = plan_w8a8(m, n, k, true);
     *split = p.split_k;
+    if (plan_q_wide_tiles(p, m, n, k, g)) {
+        *whole = g.m_blocks * g.n_blocks;
+        *cut = 0;
+        return 2;
+    }
     *whole = p.split_k > 1 ? 0 : p.n_blocks * p.m_blocks;
     *cut = p.split_k > 1 ? p.n_blocks * p.m_blocks : 0;
     return p.wide ? 2 : p.regs ? 1 : 0;

@@ -3,7 +3,7 @@
 #include "common.h"
 #include "tile_grid.h"
 
-// A workgroup of 4 waves owns 32*MT rows x 256 channels, wave w channels 64w .. 64w + 63 of all the rows.  A packed weight tile is
+// A workgroup of 4 waves owns 32*MT rows x 64*NT channels (see tg_plan), wave w the w-th quarter of the channels of all the rows.  A packed weight tile is
 // the operand of v_mfma_i32_16x16x64_i8 as it lies, so weights go from global memory into operand registers and nowhere else; the
 // activations of a 64-wide step (tile order too) are staged in LDS once for the four waves.  Loads run three steps ahead of their use
 // in three register sets, the LDS stage of a step is written one step ahead, and the rows of half a step are read behind the
@@ -13,13 +13,15 @@
 // matrix pipe, and the smaller one, which reads and writes half the accumulators per operation, leaves the power budget more clock.
 // What bounds the kernel is the operand traffic out of L2 (24 KiB per 4.2 M operations a step, 171 op/B, about 12 TB/s) and that
 // budget: 4096 x 4096 x 16384 from warm caches 248 us on 32x32x32, 219 here (2515 TOP/s), 1531 x 37888 x 3584 with cold weights
-// 203 / 187, 2077 x 4096 x 7168 73 / 67, 1531 x 3584 x 18944 118 / 118 on 168 tiles of 128 rows, one on a compute unit (on the 224 of 96
-// rows that it runs on 113).  1531 x 37888 x 3584 on 256 x 192 tiles of 8 waves with both operands through an LDS ring: 232 to 275.  Row panels of 8 or 16 blocks instead of 4, or neighbouring
+// 203 / 187, 2077 x 4096 x 7168 73 / 67, 1531 x 3584 x 18944 118 / 118 on 168 tiles, one on a compute unit (on the 228 of
+// 128 x 192 that it runs on 104).  1531 x 37888 x 3584 on 256 x 192 tiles of 8 waves with both operands through an LDS ring: 232 to 275.  Row panels of 8 or 16 blocks instead of 4, or neighbouring
 // tiles paired on one compute unit, change nothing.
 namespace tq {
 
 constexpr int WAVES = 4;
-constexpr int BN = 64 * WAVES;
+template <int NT>
+constexpr int BN_OF = 16 * NT * WAVES;                       // channels per workgroup of NT 16-channel tiles a wave
+constexpr int BN = BN_OF<4>;
 constexpr int KSTEP = 64;
 constexpr int D = 3;                                          // register sets
 
@@ -62,14 +64,14 @@ struct PlainRows {                                            // rows m0 .. of `
 };
 
 // tile0: first 16-channel tile of the weights, n_tiles: tiles of a step
-// NT: weights that nobody else reads (non-temporal loads)
-template <int MT, bool NT, typename Rows, typename Epilogue>
+// STREAM: weights that nobody else reads (non-temporal loads)
+template <int MT, int NT, bool STREAM, typename Rows, typename Epilogue>
 __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ wp, int tile0, int n_tiles, int s_begin,
                                      int s_end, uint8_t* smem, Epilogue&& epilogue) {
     constexpr int XL = XLOADS<MT>, STAGE = 64 * XL * KSTEP;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int s_last = s_end - 1;
-    i32x4 xreg[D][XL], wreg[D][4];
+    i32x4 xreg[D][XL], wreg[D][NT];
     auto load_x = [&](auto setc, int s) {
 #pragma unroll
         for (int i = 0; i < XL; ++i) xreg[decltype(setc)::value][i] = x.load(i, min(s, s_last));
@@ -80,14 +82,14 @@ __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ 
             *(i32x4*)(smem + stage * STAGE + (4 * i + wv) * 1024 + lane * 16) = xreg[decltype(setc)::value][i];
     };
     // weights: a packed tile is the matrix operand of 16 channels x 64 columns; the tile addresses are the same in every lane
-    const uint8_t* wbase[4];
+    const uint8_t* wbase[NT];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) wbase[nt] = wp + (int64_t)min(tile0 + 4 * wv + nt, n_tiles - 1) * 1024;
+    for (int nt = 0; nt < NT; ++nt) wbase[nt] = wp + (int64_t)min(tile0 + NT * wv + nt, n_tiles - 1) * 1024;
     const uint32_t lane16 = lane * 16;
     auto load_w = [&](auto setc, int s) {
         const int64_t off = (int64_t)min(s, s_last) * n_tiles * 1024;
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) wreg[decltype(setc)::value][nt] = bitcast<i32x4>(load16_at<NT>(wbase[nt] + off, lane16));
+        for (int nt = 0; nt < NT; ++nt) wreg[decltype(setc)::value][nt] = bitcast<i32x4>(load16_at<STREAM>(wbase[nt] + off, lane16));
     };
     // activations of 16-row tile t: one KiB in operand order; tiles 0 .. MT - 1 make the first half of a step, the others the second
     i32x4 xf[2][MT];
@@ -96,24 +98,24 @@ __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ 
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) xf[B][mt] = *(const i32x4*)(smem + stage * STAGE + (B * MT + mt) * 1024 + lane16);
     };
-    i32x4 acc[MT][2][4];                                      // [32-row block][16-row tile of it][16-channel tile]
+    i32x4 acc[MT][2][NT];                                     // [32-row block][16-row tile of it][16-channel tile]
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[mt][j >> 2][j & 3] = (i32x4)(0);
+        for (int j = 0; j < 2 * NT; ++j) acc[mt][j / NT][j % NT] = (i32x4)(0);
     auto mul = [&](auto bufc, auto setc) {
         constexpr int B = decltype(bufc)::value, S = decltype(setc)::value;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) {
+            for (int nt = 0; nt < NT; ++nt) {
                 i32x4& a = acc[(B * MT + mt) >> 1][(B * MT + mt) & 1][nt];
                 a = __builtin_amdgcn_mfma_i32_16x16x64_i8(wreg[S][nt], xf[B][mt], a, 0, 0, 0);
             }
     };
     // one matrix instruction, then what hides behind it
     auto interleave = [&](auto writesc, auto loadsc) {
-        constexpr int NM = 4 * MT, R = MT, W = decltype(writesc)::value, L = decltype(loadsc)::value;
+        constexpr int NM = NT * MT, R = MT, W = decltype(writesc)::value, L = decltype(loadsc)::value;
         static_for<NM>([&](auto kc) {
             constexpr int k = decltype(kc)::value;
             constexpr int r = (k + 1) * R / NM - k * R / NM, w = (k + 1) * W / NM - k * W / NM, l = (k + 1) * L / NM - k * L / NM;

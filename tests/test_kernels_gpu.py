@@ -1272,6 +1272,17 @@ def test_w8a16_many_rows_on_96_row_tiles(dtype, m, n, k):
     test_w8a16_many_rows(dtype, m, n, k, False, True)
 
 
+@pytest.mark.parametrize("dtype,m,n,k,whole", [
+    (torch.bfloat16, 1048, 4000, 1600, 231), (torch.float16, 1057, 3872, 4160, 252),      # 96 x 192: ragged last blocks, odd numbers of k-steps
+    (torch.bfloat16, 2817, 2096, 1600, 253), (torch.float16, 2800, 2112, 4160, 242)])     # 128 x 192
+def test_w8a16_many_rows_on_192_channel_tiles(dtype, m, n, k, whole):
+    """The same at shapes that take tiles of 192 channels."""
+    out = [torch.zeros(1, dtype=torch.int32) for _ in range(3)]
+    assert ops._lib.load().mf_w8a16_plan(m, n, k, *[o.data_ptr() for o in out]) == 1 and [int(o) for o in out] == [whole, 0, 1]
+    test_w8a16_many_rows(dtype, m, n, k, True, False)
+    test_w8a16_many_rows(dtype, m, n, k, False, True)
+
+
 def test_w8a16_exact_on_integer_grid():
     """Power-of-two scales and small-integer activations make every product and sum exact: the kernel must
     return exactly the integer matmul (catches a dropped k-step, a wrong row/column or a transposed operand)."""
@@ -1552,6 +1563,18 @@ def test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, bias, residua
 def test_w8a8_many_rows_on_96_row_tiles(dtype, m, n, k):
     """The same at shapes that take the lower tiles: one row and one channel piece past whole ones, a short last k-step."""
     test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, True, True)
+
+
+@pytest.mark.parametrize("dtype,m,n,k,kind,whole", [
+    (torch.bfloat16, 1048, 4000, 2080, "tiles", 231), (torch.float16, 1057, 3872, 2064, "tiles", 252),     # 96 x 192, a short last k-step
+    (torch.bfloat16, 2817, 2096, 3344, "tiles", 253), (torch.float16, 130, 16400, 1744, "tiles", 172),     # 128 x 192
+    (torch.bfloat16, 2025, 5104, 3216, "tiles", 256), (torch.float16, 256, 37888, 1744, "tiles", 238),     # 128 x 320
+    (torch.bfloat16, 201, 37872, 3600, "wide", 238)])
+def test_w8a8_many_rows_on_192_and_320_channel_tiles(dtype, m, n, k, kind, whole):
+    """The same at shapes that take narrower and wider tiles."""
+    assert _w8a8_plan(m, n, k, False) == (kind, whole, 0, 1)
+    test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, True, True)
+    test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, False, False)
 
 
 @pytest.mark.parametrize("m,n,k", [(290, 24192, 1472), (300, 16392, 528)])
