@@ -508,6 +508,13 @@ int mf_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const float* x_sca
                  const float* w_scale, const void* bias, const void* residual, int m, int n, int k, int dtype,
                  int x_layout, void* workspace, size_t workspace_bytes, void* stream);
 
+/* mf_w8a8_gemm of a gate/up projection (w_packed and w_scale: N = 2F channels, [gate | up]) with silu(gate) * up in its
+ * epilogue: y [M, F], the bits of mf_w8a8_gemm followed by mf_silu_mul(layout 0); tiled activations.  Serves the sizes for
+ * which mf_w8a8_silu_mul_fused is 1, where it is the faster form. */
+int mf_w8a8_silu_mul_fused(int m, int n, int k);
+int mf_w8a8_gemm_silu_mul(void* y, const int8_t* xq, const float* x_scale, const void* w_packed, const float* w_scale,
+                          int m, int n, int k, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
 /* The row-parallel W8A8 projection (attention output, MLP down) together with what follows it in the layer: the
  * residual add and the RMSNorm whose only reader is the next per-token quantised projection
  * (llama_layer.py:195,225-228 behind the golden-stick QuantBatchMatmul of wo / w2).  h_out [M,N] =

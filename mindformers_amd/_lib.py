@@ -76,6 +76,8 @@ SIGNATURES = {
     "mf_rmsnorm_dynamic_quant": (_I, [_P, _P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _I, _I, _P]),
     "mf_silu_mul_dynamic_quant": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "mf_w8a8_workspace_bytes": (_Z, [_I, _I, _I]),
+    "mf_w8a8_silu_mul_fused": (_I, [_I, _I, _I]),
+    "mf_w8a8_gemm_silu_mul": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _Z, _P]),
     "mf_w8a8_plan": (_I, [_I, _I, _I, _I, _P, _P, _P]),
     "mf_w8a8_gemm": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _Z, _P]),
     "mf_w8a8_gemm_add_rmsnorm_quant": (_I, [_P] * 11 + [_F] + [_I] * 7 + [_P, _Z, _P]),

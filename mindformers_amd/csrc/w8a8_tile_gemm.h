@@ -63,10 +63,11 @@ struct PlainRows {                                            // rows m0 .. of `
     }
 };
 
-// tile0: first 16-channel tile of the weights, n_tiles: tiles of a step
+// tile0: first 16-channel tile of the weights, n_tiles: tiles of a step.  half (0: none): the second half of a wave's tiles are those
+// `half` tiles after the first half, the up projection's beside the gate's
 // STREAM: weights that nobody else reads (non-temporal loads)
 template <int MT, int NT, bool STREAM, typename Rows, typename Epilogue>
-__device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ wp, int tile0, int n_tiles, int s_begin,
+__device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ wp, int tile0, int n_tiles, int half, int s_begin,
                                      int s_end, uint8_t* smem, Epilogue&& epilogue) {
     constexpr int XL = XLOADS<MT>, STAGE = 64 * XL * KSTEP;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -84,7 +85,11 @@ __device__ __forceinline__ void tile(const Rows& x, const uint8_t* __restrict__ 
     // weights: a packed tile is the matrix operand of 16 channels x 64 columns; the tile addresses are the same in every lane
     const uint8_t* wbase[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) wbase[nt] = wp + (int64_t)min(tile0 + NT * wv + nt, n_tiles - 1) * 1024;
+    for (int nt = 0; nt < NT; ++nt) {
+        const int pair = tile0 + NT / 2 * wv + nt % (NT / 2);
+        const int t = half ? min(pair, half - 1) + (nt >= NT / 2 ? half : 0) : min(tile0 + NT * wv + nt, n_tiles - 1);
+        wbase[nt] = wp + (int64_t)t * 1024;
+    }
     const uint32_t lane16 = lane * 16;
     auto load_w = [&](auto setc, int s) {
         const int64_t off = (int64_t)min(s, s_last) * n_tiles * 1024;

@@ -183,8 +183,12 @@ class QuantDecodeLayer(nn.Module):
                 aq, a_s = ops.dynamic_quant(attn, self.wo_smooth, tiled=True)
             h, n2x, n2s = ops.w8a8_linear_add_rmsnorm_quant(aq, a_s, self._packed["wo"], x, self.ffn_norm, self.eps,
                                                             self.fc1_smooth, bias=self.wo_b)
-            actq = ops.silu_mul_dynamic_quant(self._linear(None, "fc1", quantized=(n2x, n2s)), self.fc2_smooth,
-                                              tiled=True)
+            fc1 = self._packed.get("fc1")
+            if self.fc1_b is None and ops.w8a8_gated_fused(n2s.numel(), fc1):
+                actq = ops.dynamic_quant(ops.w8a8_gated_linear(n2x, n2s, fc1, self.dtype), self.fc2_smooth, tiled=True)
+            else:
+                actq = ops.silu_mul_dynamic_quant(self._linear(None, "fc1", quantized=(n2x, n2s)), self.fc2_smooth,
+                                                  tiled=True)
             if next_norm is None:
                 return self._linear(None, "fc2", residual=h, quantized=actq)
             gamma, eps, smooth = next_norm

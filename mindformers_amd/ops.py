@@ -1115,6 +1115,30 @@ def _w8a8_operands(lib, xq, x_scale, w, what):
     return tiled, xshape, xdata, m
 
 
+def w8a8_gated_fused(rows, w):
+    """Whether ``w8a8_gated_linear`` serves this many rows of a gate/up projection: where the tile kernels are the faster ones."""
+    return rows > 64 and w is not None and not w.gated and w.experts is None and \
+        _lib.load().mf_w8a8_silu_mul_fused(rows, w.n, w.k) == 1
+
+
+def w8a8_gated_linear(xq, x_scale, w, out_dtype=torch.bfloat16):
+    """Gate/up projection with silu(gate) * up in its epilogue: xq TiledInt8Activations of [M, K], ``w`` packed with
+    ``pack_w8a16`` from [gate | up] rows; [M, F].  Bit-identical to w8a8_linear followed by silu_mul; for sizes that
+    ``w8a8_gated_fused`` names."""
+    lib = _lib.load()
+    _need(isinstance(xq, TiledInt8Activations), "xq must be tiled")
+    _, xshape, xdata, m = _w8a8_operands(lib, xq, x_scale, w, "w8a8_gated_linear")
+    dev = _dev_ok(xdata, x_scale)
+    _need(out_dtype in _ACT, "out_dtype must be bf16/fp16")
+    y = torch.empty(*xshape[:-1], w.n // 2, dtype=out_dtype, device=dev)
+    need = lib.mf_w8a8_workspace_bytes(m, w.n, w.k)
+    ws = workspace(need, dev, "gemm") if need else None
+    check(lib.mf_w8a8_gemm_silu_mul(ptr(y), ptr(xdata), ptr(x_scale), ptr(w.packed), ptr(w.scale), m, w.n, w.k,
+                                    dtype_code(out_dtype), ptr(ws), ws.numel() if ws is not None else 0, stream_ptr(dev)),
+          "mf_w8a8_gemm_silu_mul")
+    return y
+
+
 def w8a8_linear_add_rmsnorm_quant(xq, x_scale, w, residual, gamma, eps, smooth=None, bias=None, tiled_out=True):
     """Row-parallel W8A8 projection + residual add + the RMSNorm and per-token quantisation that feed the next
     quantised projection: returns (h, xq_next, scale_next) with h = x . w^T dequantised (+bias) + residual.

@@ -1577,6 +1577,26 @@ def test_w8a8_many_rows_on_192_and_320_channel_tiles(dtype, m, n, k, kind, whole
     test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, False, False)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,whole,cut", [
+    (129, 8224, 208, 66, 0),               # tiles of 128 x 256, one row past a whole one, a ragged last channel block, a short last k-step
+    (513, 3584, 9472, 0, 70),              # every tile cut along K
+    (1675, 9248, 1600, 512, 6),            # two rounds and six cut in four
+    (1153, 4640, 1040, 247, 0),            # tiles of 96 x 256
+    (257, 37888, 320, 444, 0)])
+def test_w8a8_gated_tiles_equal_unfused(dtype, m, n, k, whole, cut):
+    """silu(gate) * up in the tile kernels' epilogue and in the sum of their parts: the bits of the plain GEMM followed by silu_mul."""
+    assert _w8a8_plan(m, n, k, False)[:3] == ("tiles", whole, cut) and ops._lib.load().mf_w8a8_silu_mul_fused(m, n, k) == 1
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    w = torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+    ws = (torch.rand(n, generator=g, device="cuda") + 0.5) * (k ** -0.5 / 73)
+    packed = ops.pack_w8a16(w, ws)
+    xt, xs = ops.dynamic_quant(torch.randn(m, k, generator=g, device="cuda").to(dtype), None, tiled=True)
+    y = ops.w8a8_gated_linear(xt, xs, packed, dtype)
+    assert torch.equal(y, ops.silu_mul(ops.w8a8_linear(xt, xs, packed, out_dtype=dtype)))
+
+
 @pytest.mark.parametrize("m,n,k", [(290, 24192, 1472), (300, 16392, 528)])
 def test_w8a8_wide_kernel_past_256_rows(m, n, k):
     """Several row blocks of the wide kernel, with and without a ragged last piece of channels, at the same bounds."""
