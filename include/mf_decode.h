@@ -611,6 +611,28 @@ int mf_grouped_w8a8_gemm_silu_mul(void* y, const int8_t* xq, const float* x_scal
                                   const float* w_scale, const int32_t* offsets, int n_experts, int total_rows, int n, int k,
                                   int out_dtype, void* stream);
 
+/* A decode step of a weight-only layer (QuantDecodeLayer.forward with 16-bit caches and one token a sequence) from one call:
+ * the launches of mf_rmsnorm (unless `normed` brings the normed input), mf_w8a16_qkv_rope_and_cache, mf_paged_attention_decode,
+ * mf_w8a16_gemm_add_rmsnorm, mf_w8a16_gemm_silu_mul and mf_w8a16_gemm (with next_gamma: mf_w8a16_gemm_add_rmsnorm, whose norm goes to
+ * norm_out), the intermediate rows in `scratch` (16-byte aligned).  The rows of fc1_w are interleaved gate / up.  Every field is
+ * 8 bytes wide. */
+typedef struct {
+    const void *x, *normed, *attn_gamma, *ffn_gamma, *next_gamma;
+    const void *qkv_w, *wo_w, *fc1_w, *fc2_w;
+    const float *qkv_scale, *wo_scale, *fc1_scale, *fc2_scale;
+    const void *qkv_bias, *cos, *sin;
+    void *key_cache, *value_cache;
+    const int32_t *slot_mapping, *block_tables, *context_lens;
+    void *out, *norm_out, *scratch, *workspace, *attn_workspace, *stream;
+    int64_t rows, hidden, n_heads, n_kv_heads, head_dim, ffn, block_size, num_blocks, max_blocks;
+    int64_t dtype, table_dtype, attn_gamma_dtype, ffn_gamma_dtype, next_gamma_dtype;
+    int64_t scratch_bytes, workspace_bytes, attn_workspace_bytes;
+    double eps, next_eps, scale;
+} mf_decode_layer_args;
+size_t mf_decode_layer_scratch_bytes(int rows, int hidden, int n_heads, int n_kv_heads, int head_dim, int ffn);
+size_t mf_decode_layer_workspace_bytes(int rows, int hidden, int n_heads, int n_kv_heads, int head_dim, int ffn);
+int mf_decode_layer_step(const mf_decode_layer_args* args);
+
 /* MoeTokenUnpermute(permuted_tokens, sorted_indices, probs) — moe_layer.py:151-155.
  * out[t,:] = sum_j probs[t,j] * y[row_map[t*k+j],:] accumulated in fp32 in order j = 0..k-1
  * (+ shared[t,:] if shared != NULL, the shared-expert add of moe_layer.py:159-160). */

@@ -130,6 +130,14 @@ class QuantDecodeLayer(nn.Module):
         the kernel that finishes this layer's last projection (same bits, one launch fewer).  A W8A8 layer takes
         ``next_norm`` = (gamma, eps, smooth) with the next layer's QKV smoothing vector and hands over the quantised
         norm output (xq, scale), which is what a W8A8 layer accepts as ``normed``."""
+        if q_starts is None and not self.act_quant and self._plain():
+            packed, buffers = self._packed, self._buffers
+            step = ops.decode_layer_step(x, normed, buffers["attn_norm"], buffers["ffn_norm"], next_norm,
+                                         [packed.get(name) for name in self.NAMES], self.qkv_b, cos, sin, key_cache, value_cache,
+                                         slot_mapping, block_tables, batch_valid_length, self.n_head, self.n_kv_head,
+                                         self.head_dim, self.eps, self.scale_value)
+            if step is not None:
+                return step[0] if next_norm is None else step
         nq, nkv = self.n_head * self.head_dim, self.n_kv_head * self.head_dim
         if self.act_quant:                                    # W8A8: the norm feeds the quantised projection only
             if isinstance(normed, tuple):
@@ -209,6 +217,16 @@ class QuantDecodeLayer(nn.Module):
     @staticmethod
     def _chain(out, next_norm):
         return out if next_norm is None else (out, ops.rms_norm(out, next_norm[0], next_norm[1]))
+
+    def _plain(self):
+        """Whether a decode step may run as one native call: no bias but the fused projection's, and nothing that a subclass or an
+        instance has in place of the operators' order."""
+        d, buffers = self.__dict__, self._buffers
+        if type(self) is not QuantDecodeLayer or self.head_dim % 16 or "attend" in d or "gate_up" in d or "_linear" in d or "_chain" in d:
+            return False
+        if buffers.get("attn_norm") is None or buffers.get("ffn_norm") is None:
+            return False
+        return all(name in d and d[name] is None for name in ("wo_b", "fc1_b", "fc2_b"))
 
     def gate_up(self, n2):
         """silu(gate) * up of the MLP input projection: one fused kernel on the W8A16 path."""

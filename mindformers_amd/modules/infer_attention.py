@@ -97,9 +97,9 @@ class InferAttention(nn.Module):
             raise NotImplementedError("prefix_keys_values (p-tuning prefix) is not built")
         mgr = self.paged_attention_mgr
         shape = query.shape
-        q2 = query.reshape(-1, self.n_head * self.head_dim).contiguous()
-        k2 = key.reshape(-1, self.n_kv_head * self.head_dim).contiguous()
-        v2 = value.reshape(-1, self.n_kv_head * self.head_dim).contiguous()
+        q2 = ops.rows_of(query, self.n_head * self.head_dim).contiguous()
+        k2 = ops.rows_of(key, self.n_kv_head * self.head_dim).contiguous()
+        v2 = ops.rows_of(value, self.n_kv_head * self.head_dim).contiguous()
         if self.use_rope_rotary_emb and mgr.key_cache.dtype != torch.int8:
             # RoPE + scatter of the rotated key and of value in one launch (infer_attention.py:445,453);
             # same-stream ordering stands in for ops.depend (:454)
@@ -116,8 +116,8 @@ class InferAttention(nn.Module):
         if self.is_first_iteration:
             return self._prefill_attention(q2, k2, v2, attn_mask, alibi_mask, batch_valid_length,
                                            batch_valid_length, shape).reshape(shape)
-        return self._incre_attention(q2, batch_valid_length, block_tables, alibi_mask, attn_mask,
-                                     q_seq_lens).reshape(shape)
+        out = self._incre_attention(q2, batch_valid_length, block_tables, alibi_mask, attn_mask, q_seq_lens)
+        return out if out.shape == shape else out.reshape(shape)
 
     def _prefill_attention(self, query, key, value, attn_mask, alibi_mask, actual_seq_qlen=None,
                            actual_seq_kvlen=None, shape=None):

@@ -208,13 +208,14 @@ class WeightQuantLinearCell(_QuantLinearBase):
         return ops.w8a16_linear(x, self._packed, bias=self.bias, residual=residual)
 
     def forward(self, x, residual=None):
-        out_shape = tuple(x.shape[:-1]) + (self.out_channels,)
-        x2 = x.reshape(-1, self.in_channels)
+        x2 = ops.rows_of(x, self.in_channels)
         if x2.dtype != self.dtype:
             x2 = x2.to(self.dtype)
         if residual is not None:
-            residual = residual.reshape(-1, self.out_channels)
-        return self._matmul(x2.contiguous(), residual).reshape(out_shape)
+            residual = ops.rows_of(residual, self.out_channels)
+        y = self._matmul(x2.contiguous(), residual)
+        rows = x.dim() == 2 and x.shape[1] == self.in_channels
+        return y if rows else y.reshape(tuple(x.shape[:-1]) + (self.out_channels,))
 
     construct = forward
 

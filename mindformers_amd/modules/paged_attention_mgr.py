@@ -42,7 +42,7 @@ class PagedAttentionMgr(nn.Module):
         chunk_prefill every sequence brings q_seq_lens[b] new tokens, masked causally among themselves: `attn_mask` is
         taken to be that lower triangle (generation/parallel_decoding.py:73-80) and is not read."""
         shape = query.shape
-        q2 = query.reshape(-1, self.n_heads * self.head_dim)
+        q2 = ops.rows_of(query, self.n_heads * self.head_dim)
         if self.parallel_decoding or self.chunk_prefill:
             if q_seq_lens is None:
                 raise ValueError("parallel_decoding / chunk_prefill need q_seq_lens")
@@ -52,7 +52,7 @@ class PagedAttentionMgr(nn.Module):
         else:
             out = ops.paged_attention(q2, self.key_cache, self.value_cache, block_tables, batch_valid_length,
                                       self.n_heads, self.n_kv_heads, self.scale_value)
-        return out.reshape(shape)
+        return out if out.shape == shape else out.reshape(shape)
 
     def paged_attn_with_alibi(self, query, batch_valid_length, block_tables, alibi_tensor):
         """paged_attention_mgr.py:72-75 — no alibi model is on the built path."""

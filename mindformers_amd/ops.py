@@ -5,6 +5,7 @@ not expect can fault the GPU), allocates the output with torch (device-memory pl
 the kernel on torch's current stream.  Nothing is computed in Python.
 """
 import math
+import struct
 
 import torch
 
@@ -62,6 +63,11 @@ def _dev_of(*tensors):
         elif t.device != dev:
             raise ValueError("all tensors must be on the same device")
     return dev
+
+
+def rows_of(x, width):
+    """x as [rows, width]: the tensor itself where it is that (a reshape to its own shape costs a microsecond of a small step)."""
+    return x if x.dim() == 2 and x.shape[1] == width else x.reshape(-1, width)
 
 
 def workspace(nbytes, device, tag="default"):
@@ -134,7 +140,7 @@ def rope_rows(positions, inv_freq, dtype):
     dev = _dev_ok(positions, inv_freq)
     _need(positions.dtype == torch.int32 and inv_freq.dtype == torch.float32 and dtype in _ACT, "rope_rows dtypes")
     t, d = positions.numel(), 2 * inv_freq.numel()
-    cos = torch.empty(t, d, dtype=dtype, device=dev)
+    cos = inv_freq.new_empty((t, d), dtype=dtype)
     sin = torch.empty_like(cos)
     check(lib.mf_rope_rows(ptr(cos), ptr(sin), ptr(positions), ptr(inv_freq), t, d, dtype_code(dtype), stream_ptr(dev)),
           "mf_rope_rows")
@@ -187,7 +193,7 @@ def paged_attention(query, key_cache, value_cache, block_tables, context_lens, n
         raise ValueError(f"query has {query.numel()} elements, expected {b}*{n_heads}*{d}")
     max_blocks = block_tables.shape[1]
     if out is None:
-        out = torch.empty(query.shape, dtype=query.dtype, device=dev)
+        out = query.new_empty(query.shape)
     else:
         _need(out.shape == query.shape and out.dtype == query.dtype, "out mismatch")
     need = lib.mf_paged_attention_workspace_bytes(b, n_heads, d, max_blocks * bs)
@@ -669,7 +675,7 @@ def silu_mul(gate_up, interleaved=False):
     _need(gate_up.dtype in _ACT and gate_up.shape[-1] % 2 == 0, "gate_up must be bf16/fp16 with an even last dim")
     cols = gate_up.shape[-1] // 2
     rows = gate_up.numel() // (2 * cols)
-    out = torch.empty(*gate_up.shape[:-1], cols, dtype=gate_up.dtype, device=dev)
+    out = gate_up.new_empty((*gate_up.shape[:-1], cols))
     check(lib.mf_silu_mul(ptr(out), ptr(gate_up), rows, cols, 1 if interleaved else 0, dtype_code(gate_up.dtype),
                           stream_ptr(dev)), "mf_silu_mul")
     return out
@@ -742,7 +748,7 @@ def w8a16_linear(x, w, scale=None, bias=None, residual=None):
     if x.shape[-1] != k:
         raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
-    y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=dev)
+    y = x.new_empty((*x.shape[:-1], n))
     _need(bias is None or (bias.dtype == x.dtype and bias.numel() == n), "bias mismatch")
     _need(residual is None or (residual.dtype == x.dtype and residual.shape == y.shape), "residual mismatch")
     need = lib.mf_w8a16_workspace_bytes(m, n, k)
@@ -813,7 +819,7 @@ def w4a16_linear(x, w, bias=None, residual=None):
     if x.shape[-1] != k:
         raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
-    y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=dev)
+    y = x.new_empty((*x.shape[:-1], n))
     _need(bias is None or (bias.dtype == x.dtype and bias.numel() == n), "bias mismatch")
     _need(residual is None or (residual.dtype == x.dtype and residual.shape == y.shape), "residual mismatch")
     need = lib.mf_w4a16_workspace_bytes(m, n, k, w.group_size)
@@ -951,7 +957,7 @@ def w8a16_gated_linear(x, w, bias=None):
     if x.shape[-1] != k:
         raise ValueError(f"x has {x.shape[-1]} input channels, weight expects {k}")
     m = x.numel() // k
-    y = torch.empty(*x.shape[:-1], n // 2, dtype=x.dtype, device=dev)
+    y = x.new_empty((*x.shape[:-1], n // 2))
     _need(bias is None or (bias.dtype == x.dtype and bias.numel() == n), "bias mismatch")
     need = lib.mf_w8a16_workspace_bytes(m, n, k)
     ws = workspace(need, dev, "gemm") if need else None
@@ -1309,6 +1315,71 @@ def grouped_w8a8_linear(xq, x_scale, w, offsets, out_dtype=torch.bfloat16, retur
     check(lib.mf_grouped_w8a8_gemm(ptr(y), ptr(acc), ptr(xq), ptr(x_scale), ptr(w.packed), ptr(w.scale), ptr(offsets), e,
                                    xq.shape[0], n, k, dtype_code(out_dtype), stream_ptr(dev)), "mf_grouped_w8a8_gemm")
     return (y, acc) if return_acc else y
+
+
+_STEP = struct.Struct("@27P17q3d")                            # mf_decode_layer_args
+
+
+def decode_layer_step(x, normed, attn_norm, ffn_norm, next_norm, weights, qkv_bias, cos, sin, key_cache, value_cache, slots, tables,
+                      lens, n_heads, n_kv_heads, head_dim, eps, scale):
+    """A decode step of a weight-only layer in one native call, or None where an operand is not of the plain form that it takes (the
+    caller then goes through the separate operators, which say what is wrong or take the other form).  x [T, hidden]; ``weights``:
+    the packed (qkv, wo, fc1, fc2), fc1 gated; ``next_norm`` None or (gamma, eps).  Returns (out, normed output or None)."""
+    dt, dev = x.dtype, x.get_device()
+    rows = lens.numel()
+    if dt not in _ACT or dev < 0 or x.dim() != 2 or rows == 0 or key_cache.dim() != 4:
+        return None
+    hidden = x.shape[1]
+    nb, bs, n_kv, d = key_cache.shape
+    nq, nqkv = n_heads * head_dim, (n_heads + 2 * n_kv_heads) * head_dim
+    qkv, wo, fc1, fc2 = weights
+    if not all(isinstance(w, PackedInt8Weight) and w.scale.get_device() == w.packed.get_device() == dev for w in weights):
+        return None
+    ffn = fc2.k
+    if qkv.shape != (nqkv, hidden) or wo.shape != (hidden, nq) or fc1.shape != (2 * ffn, hidden) or fc2.n != hidden \
+            or fc2.experts is not None or qkv.gated or wo.gated or fc2.gated or not fc1.gated:
+        return None
+    if x.shape[0] != rows or n_kv != n_kv_heads or d != head_dim or value_cache.shape != key_cache.shape or value_cache.dtype != dt \
+            or key_cache.dtype != dt or tables.dim() != 2 or tables.shape[0] != rows or lens.dim() != 1 or slots.numel() != rows \
+            or tables.dtype != torch.int32 or lens.dtype != torch.int32 or slots.dtype != torch.int32 \
+            or cos.numel() != rows * d or sin.numel() != rows * d or sin.dtype != cos.dtype \
+            or attn_norm.numel() != hidden or ffn_norm.numel() != hidden:
+        return None
+    if normed is not None and (normed.shape != x.shape or normed.dtype != dt):
+        return None
+    if qkv_bias is not None and (qkv_bias.dtype != dt or qkv_bias.numel() != nqkv):
+        return None
+    gamma, next_eps = (None, 0.0) if next_norm is None else (next_norm[0], next_norm[1])
+    if gamma is not None and gamma.numel() != hidden:
+        return None
+    for t in (x, normed, attn_norm, ffn_norm, gamma, qkv_bias, cos, sin, key_cache, value_cache, slots, tables, lens):
+        if t is not None and not (type(t) is torch.Tensor and t.get_device() == dev and t.is_contiguous()):
+            return None
+    lib = _lib.load()
+    device = x.device
+    sizes = (rows, hidden, n_heads, n_kv, d, ffn)
+    need = lib.mf_decode_layer_workspace_bytes(*sizes)
+    ws = workspace(need, device, "gemm") if need else None
+    need = lib.mf_paged_attention_workspace_bytes(rows, n_heads, d, tables.shape[1] * bs)
+    pws = workspace(need, device, "pa") if need else None
+    scratch_bytes = lib.mf_decode_layer_scratch_bytes(*sizes)
+    scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=device)
+    out = torch.empty_like(x)
+    norm_out = None if gamma is None else torch.empty_like(x)
+    args = _STEP.pack(
+        x.data_ptr(), 0 if normed is None else normed.data_ptr(), attn_norm.data_ptr(), ffn_norm.data_ptr(),
+        0 if gamma is None else gamma.data_ptr(), qkv.packed.data_ptr(), wo.packed.data_ptr(), fc1.packed.data_ptr(),
+        fc2.packed.data_ptr(), qkv.scale.data_ptr(), wo.scale.data_ptr(), fc1.scale.data_ptr(), fc2.scale.data_ptr(),
+        0 if qkv_bias is None else qkv_bias.data_ptr(), cos.data_ptr(), sin.data_ptr(), key_cache.data_ptr(),
+        value_cache.data_ptr(), slots.data_ptr(), tables.data_ptr(), lens.data_ptr(), out.data_ptr(),
+        0 if norm_out is None else norm_out.data_ptr(), scratch.data_ptr(), 0 if ws is None else ws.data_ptr(),
+        0 if pws is None else pws.data_ptr(), stream_ptr(device),
+        rows, hidden, n_heads, n_kv, d, ffn, bs, nb, tables.shape[1],
+        dtype_code(dt), dtype_code(cos.dtype), dtype_code(attn_norm.dtype), dtype_code(ffn_norm.dtype),
+        0 if gamma is None else dtype_code(gamma.dtype), scratch_bytes, 0 if ws is None else ws.numel(),
+        0 if pws is None else pws.numel(), float(eps), float(next_eps), float(scale))
+    check(lib.mf_decode_layer_step(args), "mf_decode_layer_step")
+    return out, norm_out
 
 
 def moe_unpermute(y, row_map, probs, shared=None):

@@ -311,3 +311,52 @@ def test_step_under_a_cuda_default_device():
         finally:
             torch.set_default_device(None)
     assert np.array_equal(*outs)
+
+
+@pytest.mark.parametrize("dtype,hidden,nh,nkv,d,ffn,batch,bias", [
+    (torch.float16, 512, 8, 2, 64, 1376, 4, False), (torch.bfloat16, 512, 8, 8, 64, 1024, 1, True),
+    (torch.bfloat16, 1024, 12, 4, 128, 2048, 70, False),     # past 64 rows
+])
+def test_a_native_decode_step_has_the_bits_of_the_separate_operators(dtype, hidden, nh, nkv, d, ffn, batch, bias):
+    """A weight-only decode step in one native call and through the operators one by one (an instance with an ``attend`` of its own
+    takes those): outputs, handed-over norms and caches, with and without either end of a chain; operands in another form are
+    taken or refused as by the operators."""
+    from mindformers_amd import synthetic
+    from mindformers_amd.decode_layer import QuantDecodeLayer
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(batch)
+    layer = synthetic.fill_layer(QuantDecodeLayer(hidden, nh, nkv, d, ffn, 1e-5, dtype, qkv_bias=bias), gen)
+    if bias:
+        layer.qkv_b.copy_(torch.randn(layer.qkv_b.shape, generator=gen, device="cuda"))
+    rng, bs = np.random.default_rng(3), 16
+    lens = rng.integers(1, 200, batch).astype(np.int32)
+    need = (lens + bs - 1) // bs
+    tables = -np.ones((batch, int(need.max())), np.int32)
+    ids = rng.permutation(int(need.sum()) + 1).astype(np.int32)
+    for i, n in enumerate(need):
+        tables[i, :n], ids = ids[:n], ids[n:]
+    slots = np.array([tables[i, (l - 1) // bs] * bs + (l - 1) % bs for i, l in enumerate(lens)], np.int32)
+    shape = (int(need.sum()) + 1, bs, nkv, d)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(dtype)
+    x, kc, vc, cos, sin = rand(batch, hidden), rand(*shape), rand(*shape), rand(batch, d), rand(batch, d)
+    tb, ln, sl = (torch.from_numpy(a).cuda() for a in (tables, lens, slots))
+    gamma = torch.rand(hidden, generator=gen, device="cuda")
+
+    def steps(x, tb):
+        out = []
+        for normed, nxt in ((None, None), (None, (gamma, 1e-6)), (rand(batch, hidden), None)):
+            gen.manual_seed(9)
+            k, v = kc.clone(), vc.clone()
+            y = layer(x, k, v, tb, ln, sl, cos, sin, normed=None if normed is None else rand(batch, hidden), next_norm=nxt)
+            out += [k, v] + (list(y) if isinstance(y, tuple) else [y])
+        return out
+    native = steps(x, tb)
+    wide = torch.cat((tb, tb), 1)[:, :tb.shape[1]] if batch > 1 else None                # rows not contiguous
+    layer.attend = lambda *a, **kw: QuantDecodeLayer.attend(layer, *a, **kw)
+    separate = steps(x, tb)
+    del layer.attend
+    assert len(native) == 10 and all(torch.equal(a, b) for a, b in zip(native, separate))
+    for bad_x, bad_tb in ((x.float(), tb), (x, tb.long()), (x[:, :-8], tb), (x, wide)):
+        if bad_tb is not None:
+            with pytest.raises(ValueError):
+                steps(bad_x, bad_tb)
