@@ -579,6 +579,12 @@ int mf_moe_permute_int8(int8_t* permuted_x, float* permuted_scale, int32_t* row_
                         const int8_t* x, const float* x_scale, const int32_t* expert_index, int tokens, int k,
                         int n_experts, int hidden, void* stream);
 
+/* mf_moe_permute without the copies, for the grouped GEMMs that read rows through an index: sources [T*k], the token that each permuted
+ * row is a copy of (entries past offsets[E] are not written).  x_scale [tokens] (may be NULL, permuted_scale with it) goes to
+ * permuted_scale [T*k] as in mf_moe_permute_int8. */
+int mf_moe_sort(int32_t* row_map, int32_t* sources, float* permuted_scale, int64_t* counts, int32_t* offsets,
+                const float* x_scale, const int32_t* expert_index, int tokens, int k, int n_experts, void* stream);
+
 /* GroupedMatmulV4(split_item=3, group_type=0, group_list_type=1) with int8 expert weights —
  * mindformers/parallel_core/inference/transformer/moe/experts.py:116-117,136-137.
  * Rows offsets[e]..offsets[e+1] of x use expert e: y = (x . w[e]^T) * scale[e].  w_packed holds the E experts
@@ -610,6 +616,18 @@ int mf_grouped_w8a8_gemm(void* y, int32_t* acc_out, const int8_t* xq, const floa
 int mf_grouped_w8a8_gemm_silu_mul(void* y, const int8_t* xq, const float* x_scale, const void* w_packed,
                                   const float* w_scale, const int32_t* offsets, int n_experts, int total_rows, int n, int k,
                                   int out_dtype, void* stream);
+
+/* The gated grouped GEMMs on rows that lie elsewhere: row i of the total_rows permuted ones is row sources[i] of the n_sources rows of x
+ * (mf_moe_sort; clamped to them), same bits as on the copied rows.  x_scale is that of the permuted rows.  Served where
+ * mf_grouped_*_reads_sources says so: prompt-sized groups, up to 4 GiB of rows. */
+int mf_grouped_w8a16_reads_sources(int n_sources, int n_experts, int total_rows, int n, int k);
+int mf_grouped_w8a8_reads_sources(int n_sources, int n_experts, int total_rows, int n, int k);
+int mf_grouped_w8a16_gemm_silu_mul_sources(void* y, const void* x, const int32_t* sources, int n_sources,
+                                           const void* w_packed, const float* scale, const int32_t* offsets, int n_experts,
+                                           int total_rows, int n, int k, int dtype, void* stream);
+int mf_grouped_w8a8_gemm_silu_mul_sources(void* y, const int8_t* xq, const float* x_scale, const int32_t* sources,
+                                          int n_sources, const void* w_packed, const float* w_scale, const int32_t* offsets,
+                                          int n_experts, int total_rows, int n, int k, int out_dtype, void* stream);
 
 /* A decode step of a weight-only layer (QuantDecodeLayer.forward with 16-bit caches and one token a sequence) from one call:
  * the launches of mf_rmsnorm (unless `normed` brings the normed input), mf_w8a16_qkv_rope_and_cache, mf_paged_attention_decode,

@@ -93,6 +93,11 @@ SIGNATURES = {
     "mf_grouped_w8a16_gemm_silu_mul": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "mf_grouped_w8a8_gemm": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "mf_grouped_w8a8_gemm_silu_mul": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
+    "mf_grouped_w8a16_reads_sources": (_I, [_I] * 5),
+    "mf_grouped_w8a8_reads_sources": (_I, [_I] * 5),
+    "mf_grouped_w8a16_gemm_silu_mul_sources": (_I, [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
+    "mf_grouped_w8a8_gemm_silu_mul_sources": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
+    "mf_moe_sort": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "mf_decode_layer_scratch_bytes": (_Z, [_I] * 6),
     "mf_decode_layer_workspace_bytes": (_Z, [_I] * 6),
     "mf_decode_layer_step": (_I, [ctypes.c_char_p]),

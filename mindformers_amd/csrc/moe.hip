@@ -136,10 +136,16 @@ __global__ __launch_bounds__(64) void moe_route_kernel(uint16_t* __restrict__ we
 // What bounds it: the latency of a few dependent passes.  16616 pairs on 256 experts: 129 us in one workgroup that
 // walked the pairs 64 at a time, 8 us here.  (The scan with a run of experts per lane of one wave: 1.6 us more at 1024 experts.)
 constexpr int SORT_CHUNK = 1024;
+struct SortRows {                                             // where the rows are not copied: token (of k pairs each) and scale of each
+    int32_t* sources;
+    float* scale;
+    const float* x_scale;
+    int k;
+};
 __global__ __launch_bounds__(SORT_CHUNK) void moe_sort_kernel(int32_t* __restrict__ row_map, int64_t* __restrict__ counts,
                                                               int32_t* __restrict__ offsets,
                                                               const int32_t* __restrict__ expert_index, int pairs,
-                                                              int E) {
+                                                              int E, SortRows rows) {
     __shared__ int s_before[RT_MAX_E], s_rest[RT_MAX_E], s_cur[RT_MAX_E];
     __shared__ __attribute__((aligned(16))) uint8_t s_wave[SORT_CHUNK / 64][RT_MAX_E];   // pairs of the wave: at most 64
     __shared__ int s_total[SORT_CHUNK / 64];
@@ -203,6 +209,11 @@ __global__ __launch_bounds__(SORT_CHUNK) void moe_sort_kernel(int32_t* __restric
         for (int w = 0; w < wv; ++w) dst += s_wave[w][e];
     }
     row_map[p] = dst;
+    if (rows.sources && dst >= 0) {
+        const int token = p / rows.k;
+        rows.sources[dst] = token;
+        if (rows.x_scale) rows.scale[dst] = rows.x_scale[token];
+    }
 }
 
 // permuted_x[row_map[p]] = x[p / k]; one workgroup per pair.  Rows of int8 values come as `hidden` pairs of them, with their
@@ -484,15 +495,21 @@ GatePlan plan_router_gate(int tokens, int E, int H) {
     return p;
 }
 
-int permute(uint16_t* permuted, float* permuted_scale, int32_t* row_map, int64_t* counts, int32_t* offsets, const uint16_t* x,
-            const float* x_scale, const int32_t* expert_index, int tokens, int k, int n_experts, int hidden,
-            hipStream_t stream) {
-    const int pairs = tokens * k, chunks = pairs > SORT_CHUNK ? (pairs + SORT_CHUNK - 1) / SORT_CHUNK : 1;
+int sort_pairs(int32_t* row_map, int64_t* counts, int32_t* offsets, const int32_t* expert_index, int pairs, int n_experts,
+               const SortRows& rows, hipStream_t stream) {
+    const int chunks = pairs > SORT_CHUNK ? (pairs + SORT_CHUNK - 1) / SORT_CHUNK : 1;
     // one chunk: fewer waves meet at the barriers sooner (1 token on 8 experts: 5.4 us with the gather in 16 waves, 4.7 in one)
     const int most = pairs > n_experts ? pairs : n_experts, threads = most < SORT_CHUNK ? (most + 63) / 64 * 64 : SORT_CHUNK;
     hipLaunchKernelGGL(moe_sort_kernel, dim3(chunks), dim3(threads), 0, stream, row_map, counts, offsets, expert_index,
-                       pairs, n_experts);
-    int rc = MF_LAUNCH_CHECK();
+                       pairs, n_experts, rows);
+    return MF_LAUNCH_CHECK();
+}
+
+int permute(uint16_t* permuted, float* permuted_scale, int32_t* row_map, int64_t* counts, int32_t* offsets, const uint16_t* x,
+            const float* x_scale, const int32_t* expert_index, int tokens, int k, int n_experts, int hidden,
+            hipStream_t stream) {
+    const int pairs = tokens * k;
+    int rc = sort_pairs(row_map, counts, offsets, expert_index, pairs, n_experts, {nullptr, nullptr, nullptr, k}, stream);
     if (rc || pairs == 0) return rc;
     hipLaunchKernelGGL(moe_gather_kernel, dim3(pairs), dim3(256), 0, stream, permuted, permuted_scale, x, x_scale, row_map, k,
                        hidden, pairs);
@@ -581,6 +598,15 @@ extern "C" int mf_moe_permute(void* permuted_x, int32_t* row_map, int64_t* count
     MF_REQUIRE((((uintptr_t)permuted_x | (uintptr_t)x) & 15) == 0, "moe_permute: rows must be 16-byte aligned");
     return permute((uint16_t*)permuted_x, nullptr, row_map, counts, offsets, (const uint16_t*)x, nullptr, expert_index, tokens,
                    k, n_experts, hidden, (hipStream_t)stream);
+}
+
+extern "C" int mf_moe_sort(int32_t* row_map, int32_t* sources, float* permuted_scale, int64_t* counts, int32_t* offsets,
+                           const float* x_scale, const int32_t* expert_index, int tokens, int k, int n_experts, void* stream) {
+    MF_REQUIRE(row_map && sources && counts && offsets && expert_index && !permuted_scale == !x_scale, "moe_sort: null argument");
+    MF_REQUIRE(n_experts > 0 && n_experts <= RT_MAX_E, "moe_sort: n_experts (%d) must be in 1..%d", n_experts, RT_MAX_E);
+    MF_REQUIRE(tokens >= 0 && k > 0 && (int64_t)tokens * k <= 65536, "moe_sort: tokens*k must be <= 65536");
+    return sort_pairs(row_map, counts, offsets, expert_index, tokens * k, n_experts, {sources, permuted_scale, x_scale, k},
+                      (hipStream_t)stream);
 }
 
 extern "C" int mf_moe_permute_int8(int8_t* permuted_x, float* permuted_scale, int32_t* row_map, int64_t* counts,

@@ -581,7 +581,8 @@ __global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
     const TileOut<T, NT> out{y, bias, residual, M, N, gated, aligned};
     f32x4 sc[NT], bi[NT];
     uint8_t* stage = smem + wv * 32 * TileOut<T, NT>::ROW;
-    tg::tile<T, MT, NT, 0, false>(x, wp, M, K, m0, nb * (tg::BN_OF<NT> / 16), (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const f32x4 (&acc)[2][NT]) {
+    tg::tile<T, MT, NT, 0, false>(x + (int64_t)m0 * K, [&](int r) { return min(r, M - 1 - m0); }, wp, K, nb * (tg::BN_OF<NT> / 16),
+                                  (N + 15) >> 4, s0, s_end, smem, [&](auto mtc, const f32x4 (&acc)[2][NT]) {
         constexpr int mt = decltype(mtc)::value;
         if (whole) {
             if (mt == 0) {
@@ -685,14 +686,20 @@ __global__ __launch_bounds__(GW_WAVES * 64, 2) void w8a16_grouped_kernel(
 // more rows gain nothing (7168 x 2048 at 65 rows 679 / 704), and an expert's further blocks share the weights through L2 (200 rows:
 // 1257 / 1420).  Up to 16 bytes of scratch a lane, outside the k-loops.
 template <typename T, int MT, bool NT, bool STREAM>
-__device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* xe, const uint8_t* we, const float* se, int rows,
-                                                 int m0, int nb, int N, int K, int gated, int aligned, uint8_t* smem) {
+__device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* x, const TileSources& src, const uint8_t* we,
+                                                 const float* se, int row0, int rows, int m0, int nb, int N, int K, int gated,
+                                                 int aligned, uint8_t* smem) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = nb * tg::BN + 64 * wv;
     const TileOut<T> out{y, nullptr, nullptr, rows, N, gated, aligned};
     f32x4 sc[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TileOut<T>::ROW;
-    tg::tile<T, MT, 4, MT == 4 ? 2 : MT == 3 ? 0 : 2 * MT, NT>(xe, we, rows, K, m0, nb * (tg::BN / 16), (N + 15) >> 4, 0, K / tg::KSTEP, smem,
+    const uint16_t* xb = src.sources ? x : x + (int64_t)(row0 + m0) * K;
+    const auto row_of = [&](int r) {
+        const int in = min(r, rows - 1 - m0);
+        return src.sources ? src.of(row0 + m0 + in) : in;
+    };
+    tg::tile<T, MT, 4, MT == 4 ? 2 : MT == 3 ? 0 : 2 * MT, NT>(xb, row_of, we, K, nb * (tg::BN / 16), (N + 15) >> 4, 0, K / tg::KSTEP, smem,
                     [&](auto mtc, const f32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
         if (mt == 0) {
@@ -713,17 +720,16 @@ template <typename T, bool STREAM>
 __global__ __launch_bounds__(256, 2) void w8a16_group_tile_kernel(
     uint16_t* __restrict__ y, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, const float* __restrict__ scale,
     const int32_t* __restrict__ offsets, int n_experts, int total_rows, int N, int K, int64_t expert_bytes, int gated,
-    int aligned) {
+    int aligned, TileSources src) {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * 128 * 128];
     static_assert(tg::WAVES * 32 * TileOut<T>::ROW <= (int)sizeof(smem), "the output stage reuses the operand stages");
     int e, m0, row0, rows, nb;
     if (!tg_group_locate(offsets, n_experts, total_rows, (N + tg::BN - 1) / tg::BN, e, m0, row0, rows, nb)) return;
     uint16_t* ye = y + (int64_t)row0 * (gated ? N >> 1 : N);
-    const uint16_t* xe = x + (int64_t)row0 * K;
     const uint8_t* we = wp + (int64_t)e * expert_bytes;
     const float* se = scale + (int64_t)e * N;
     const int left = rows - m0;
-#define GT(MT, NT) w8a16_group_tile<T, MT, NT, STREAM>(ye, xe, we, se, rows, m0, nb, N, K, gated, aligned, smem)
+#define GT(MT, NT) w8a16_group_tile<T, MT, NT, STREAM>(ye, x, src, we, se, row0, rows, m0, nb, N, K, gated, aligned, smem)
     if (left <= 32) {
         if (m0 == 0) GT(1, true);                             // nobody else reads these weights
         else GT(1, false);
@@ -1550,9 +1556,19 @@ extern "C" int mf_w8a16_gemm_silu_mul(void* y, const void* x, const void* w_pack
                             workspace_bytes, stream);
 }
 
+static bool gw_group_tiles(int n_experts, int total_rows, int n, int k) {
+    return n % 16 == 0 && k % tg::KSTEP == 0 && k <= (1 << 24) &&   // K: the tiles' 32-bit offsets reach over 128 rows
+           total_rows > gw_group_tile_rows(n_experts, n, k) * (int64_t)n_experts;
+}
+
+extern "C" int mf_grouped_w8a16_reads_sources(int n_sources, int n_experts, int total_rows, int n, int k) {
+    if (n_sources <= 0 || n_experts <= 0 || total_rows <= 0 || n <= 0 || k <= 0) return 0;
+    return (int64_t)n_sources * k < (1LL << 31) && gw_group_tiles(n_experts, total_rows, n, k);   // the tiles' row offsets have 32 bits
+}
+
 static int grouped_w8a16_entry(const char* who, void* y, const void* x, const void* w_packed, const float* scale,
                                const int32_t* offsets, int n_experts, int total_rows, int n, int k, int dtype, int gated,
-                               void* stream) {
+                               void* stream, TileSources src = {nullptr, 0}) {
     MF_REQUIRE(dtype == MF_BF16 || dtype == MF_FP16, "%s: dtype must be bf16 or fp16", who);
     if (total_rows == 0) return 0;
     MF_REQUIRE(y && x && w_packed && scale && offsets, "%s: null argument", who);
@@ -1561,15 +1577,16 @@ static int grouped_w8a16_entry(const char* who, void* y, const void* x, const vo
     MF_REQUIRE(!gated || n % 4 == 0, "%s: N (%d) must be a multiple of 4 (gate / up pairs)", who, n);
     MF_REQUIRE((((uintptr_t)x | (uintptr_t)w_packed) & 15) == 0, "%s: x and w_packed must be 16-byte aligned", who);
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
-    if (n % 16 == 0 && k % tg::KSTEP == 0 && k <= (1 << 24) &&   // K: the tiles' 32-bit offsets reach over 128 rows
-        total_rows > gw_group_tile_rows(n_experts, n, k) * (int64_t)n_experts) {
+    MF_REQUIRE(!src.sources || mf_grouped_w8a16_reads_sources(src.n_sources, n_experts, total_rows, n, k),
+               "%s: %d rows for %d experts of %d x %d are not read through an index", who, total_rows, n_experts, n, k);
+    if (gw_group_tiles(n_experts, total_rows, n, k)) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tg::BN - 1) / tg::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;
         const bool stream_out = tg_group_stream(n_experts, expert_bytes);
 #define GGT_LAUNCH(TT, ST)                                                                                        \
     hipLaunchKernelGGL((w8a16_group_tile_kernel<TT, ST>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y,        \
                        (const uint16_t*)x, (const uint8_t*)w_packed, scale, offsets, n_experts, total_rows, n, k,    \
-                       expert_bytes, gated, aligned)
+                       expert_bytes, gated, aligned, src)
         if (dtype == MF_BF16) { if (stream_out) GGT_LAUNCH(BF16, true); else GGT_LAUNCH(BF16, false); }
         else { if (stream_out) GGT_LAUNCH(FP16, true); else GGT_LAUNCH(FP16, false); }
 #undef GGT_LAUNCH
@@ -1599,6 +1616,14 @@ extern "C" int mf_grouped_w8a16_gemm_silu_mul(void* y, const void* x, const void
                                               int dtype, void* stream) {
     return grouped_w8a16_entry("grouped_w8a16_gemm_silu_mul", y, x, w_packed, scale, offsets, n_experts, total_rows, n,
                                k, dtype, 1, stream);
+}
+
+extern "C" int mf_grouped_w8a16_gemm_silu_mul_sources(void* y, const void* x, const int32_t* sources, int n_sources,
+                                                      const void* w_packed, const float* scale, const int32_t* offsets,
+                                                      int n_experts, int total_rows, int n, int k, int dtype, void* stream) {
+    MF_REQUIRE(sources && n_sources > 0, "grouped_w8a16_gemm_silu_mul_sources: no rows");
+    return grouped_w8a16_entry("grouped_w8a16_gemm_silu_mul_sources", y, x, w_packed, scale, offsets, n_experts, total_rows, n, k,
+                               dtype, 1, stream, {sources, n_sources});
 }
 
 // ---- 4-bit weights ---------------------------------------------------------------------------------------------------

@@ -39,8 +39,9 @@ __device__ __forceinline__ int key(int row) { return ((row >> 1) & 1) | (((row >
 
 // EARLY: 16-row tiles of a sub-step that are read behind the last but one channel tile of the one before; the others follow behind the
 // last, each into the registers of a tile that has just been used (0: half and half).  STREAM: weights that nobody else reads (non-temporal loads)
-template <typename T, int MT, int NT, int EARLY, bool STREAM, typename Epilogue>
-__device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, int M, int K, int m0,
+// row_of(r): the row of x that is row r of the tile (the last one where the tile has no such row), within 32-bit byte offsets
+template <typename T, int MT, int NT, int EARLY, bool STREAM, typename RowOf, typename Epilogue>
+__device__ __forceinline__ void tile(const uint16_t* __restrict__ x, RowOf&& row_of, const uint8_t* __restrict__ wp, int K,
                                      int tile0, int n_tiles, int s_begin, int s_end, uint8_t* smem, Epilogue&& epilogue) {
     using vec8 = typename T::vec8;
     constexpr int STAGE = 32 * MT * 128;
@@ -49,10 +50,10 @@ __device__ __forceinline__ void tile(const uint16_t* __restrict__ x, const uint8
 
     // ---- activations: load i of a thread is chunk (t & 7) of row 32i + (t >> 3)
     const int xr = threadIdx.x >> 3, xc = threadIdx.x & 7;
-    const uint8_t* xbase = (const uint8_t*)(x + (int64_t)m0 * K);
+    const uint8_t* xbase = (const uint8_t*)x;
     uint32_t xoff[MT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) xoff[i] = (uint32_t)min(32 * i + xr, M - 1 - m0) * (uint32_t)K * 2u + 16u * xc;
+    for (int i = 0; i < MT; ++i) xoff[i] = (uint32_t)row_of(32 * i + xr) * (uint32_t)K * 2u + 16u * xc;
     const uint32_t xdst = xr * 128 + ((xc ^ key(xr)) << 4);   // + 4096 per i (the key has no bit above 3)
     u32x4 xreg[DX<MT>][MT];
     auto load_x = [&](auto setc, auto ic, int s) {

@@ -1045,15 +1045,15 @@ __global__ __launch_bounds__(QG_WAVES * 64, 2) void w8a8_grouped_kernel(
 // more rows it depends on the number of experts (64 of 2816 x 2048 at 100 rows 95 / 83, a layer of 256 experts at 65 rows 2545 / 2632),
 // and an expert's further blocks share the weights through L2 (200 rows: 928 / 1276 us).
 template <typename T, int MT, bool NT, bool STREAM>
-__device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* xe, const float* xs, const uint8_t* we,
-                                                const float* ws, int rows, int m0, int nb, int N, int K, int gated,
+__device__ __forceinline__ void w8a8_group_tile(uint16_t* y, const uint8_t* x, const TileSources& from, const float* xs,
+                                                const uint8_t* we, const float* ws, int row0, int rows, int m0, int nb, int N, int K, int gated,
                                                 int aligned, uint8_t* smem) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = nb * tq::BN + 64 * wv;
     const QTileOut<T> out{xs, ws, nullptr, rows, N, gated};
     f32x4 wsv[4], bi[4];
     uint8_t* stage = smem + wv * 32 * TG_STAGE_ROW<4>;
-    const tq::PlainRows<tq::XLOADS<MT>> src(xe, m0, rows, K, wv);
+    const tq::PlainRows<tq::XLOADS<MT>> src(x, from, row0, m0, rows, K, wv);
     tq::tile<MT, 4, NT>(src, we, nb * (tq::BN / 16), (N + 15) >> 4, 0, 0, (K + Q_KSTEP - 1) / Q_KSTEP, smem,
                  [&](auto mtc, const i32x4 (&acc)[2][4]) {
         constexpr int mt = decltype(mtc)::value;
@@ -1079,16 +1079,16 @@ template <typename T, bool STREAM>
 __global__ __launch_bounds__(256, 2) void w8a8_group_tile_kernel(
     uint16_t* __restrict__ y, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
     const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const int32_t* __restrict__ offsets, int n_experts,
-    int total_rows, int N, int K, int64_t expert_bytes, int gated, int aligned) {
+    int total_rows, int N, int K, int64_t expert_bytes, int gated, int aligned, TileSources from) {
     constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW<4>, OPS = tq::LDS_BYTES<4>;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
     int e, m0, row0, rows, nb;
     if (!tg_group_locate(offsets, n_experts, total_rows, (N + tq::BN - 1) / tq::BN, e, m0, row0, rows, nb)) return;
     uint16_t* ye = y + (int64_t)row0 * (gated ? N >> 1 : N);
-    const uint8_t *xe = (const uint8_t*)xq + (int64_t)row0 * K, *we = wp + (int64_t)e * expert_bytes;
+    const uint8_t *x = (const uint8_t*)xq, *we = wp + (int64_t)e * expert_bytes;
     const float *xs = x_scale + row0, *ws = w_scale + (int64_t)e * N;
     const int left = rows - m0;
-#define GT(MT, NT) w8a8_group_tile<T, MT, NT, STREAM>(ye, xe, xs, we, ws, rows, m0, nb, N, K, gated, aligned, smem)
+#define GT(MT, NT) w8a8_group_tile<T, MT, NT, STREAM>(ye, x, from, xs, we, ws, row0, rows, m0, nb, N, K, gated, aligned, smem)
     if (left <= 64) {
         if (m0 == 0) GT(2, true);                             // nobody else reads these weights
         else GT(2, false);
@@ -1470,9 +1470,19 @@ extern "C" int mf_w8a8_qkv_rope_and_cache(void* qkv, const int8_t* xq, const flo
                              x_layout == 1, workspace, (hipStream_t)stream, nullptr, &rc);
 }
 
+static bool qg_group_tiles(int n_experts, int total_rows, int n, int k) {
+    return n % 16 == 0 && k <= (1 << 25) &&                   // K: the tiles' 32-bit offsets reach over 128 rows
+           total_rows > tg_group_min_rows(n_experts, (n + tq::BN - 1) / tq::BN, k, QG_TILE_ROWS) * (int64_t)n_experts;
+}
+
+extern "C" int mf_grouped_w8a8_reads_sources(int n_sources, int n_experts, int total_rows, int n, int k) {
+    if (n_sources <= 0 || n_experts <= 0 || total_rows <= 0 || n <= 0 || k <= 0) return 0;
+    return (int64_t)n_sources * k < (1LL << 32) && qg_group_tiles(n_experts, total_rows, n, k);   // the tiles' row offsets have 32 bits
+}
+
 static int grouped_w8a8_entry(const char* who, void* y, int32_t* acc_out, const int8_t* xq, const float* x_scale,
                               const void* w_packed, const float* w_scale, const int32_t* offsets, int n_experts, int total_rows,
-                              int n, int k, int out_dtype, int gated, void* stream) {
+                              int n, int k, int out_dtype, int gated, void* stream, TileSources src = {nullptr, 0}) {
     MF_REQUIRE(out_dtype == MF_BF16 || out_dtype == MF_FP16, "%s: out_dtype must be bf16 or fp16", who);
     if (total_rows == 0) return 0;
     MF_REQUIRE((y || acc_out) && xq && x_scale && w_packed && w_scale && offsets, "%s: null argument", who);
@@ -1483,16 +1493,16 @@ static int grouped_w8a8_entry(const char* who, void* y, int32_t* acc_out, const 
     MF_REQUIRE((((uintptr_t)xq | (uintptr_t)w_packed) & 15) == 0, "%s: xq and w_packed must be 16-byte aligned", who);
     const int64_t expert_bytes = (int64_t)mf_w8a16_packed_bytes(n, k);
     dim3 grid((n + QG_BN - 1) / QG_BN, n_experts);
-    // (K: the tiles' 32-bit offsets reach over 128 rows)
-    if (y && !acc_out && n % 16 == 0 && k <= (1 << 25) &&
-        total_rows > tg_group_min_rows(n_experts, (n + tq::BN - 1) / tq::BN, k, QG_TILE_ROWS) * (int64_t)n_experts) {
+    MF_REQUIRE(!src.sources || mf_grouped_w8a8_reads_sources(src.n_sources, n_experts, total_rows, n, k),
+               "%s: %d rows for %d experts of %d x %d are not read through an index", who, total_rows, n_experts, n, k);
+    if (y && !acc_out && qg_group_tiles(n_experts, total_rows, n, k)) {
         const dim3 tiles(tg_group_workgroups(total_rows, n_experts, (n + tq::BN - 1) / tq::BN));
         const int aligned = ((uintptr_t)y & 15) == 0;
         const bool stream_out = tg_group_stream(n_experts, expert_bytes);
 #define QGT_LAUNCH(TT, ST)                                                                                       \
     hipLaunchKernelGGL((w8a8_group_tile_kernel<TT, ST>), tiles, dim3(256), 0, (hipStream_t)stream, (uint16_t*)y, xq, x_scale, \
                        (const uint8_t*)w_packed, w_scale, offsets, n_experts, total_rows, n, k, expert_bytes, gated, \
-                       aligned)
+                       aligned, src)
         if (out_dtype == MF_BF16) { if (stream_out) QGT_LAUNCH(BF16, true); else QGT_LAUNCH(BF16, false); }
         else { if (stream_out) QGT_LAUNCH(FP16, true); else QGT_LAUNCH(FP16, false); }
 #undef QGT_LAUNCH
@@ -1527,4 +1537,13 @@ extern "C" int mf_grouped_w8a8_gemm_silu_mul(void* y, const int8_t* xq, const fl
                                              int k, int out_dtype, void* stream) {
     return grouped_w8a8_entry("grouped_w8a8_gemm_silu_mul", y, nullptr, xq, x_scale, w_packed, w_scale, offsets, n_experts,
                               total_rows, n, k, out_dtype, 1, stream);
+}
+
+extern "C" int mf_grouped_w8a8_gemm_silu_mul_sources(void* y, const int8_t* xq, const float* x_scale, const int32_t* sources,
+                                                     int n_sources, const void* w_packed, const float* w_scale,
+                                                     const int32_t* offsets, int n_experts, int total_rows, int n, int k,
+                                                     int out_dtype, void* stream) {
+    MF_REQUIRE(sources && n_sources > 0, "grouped_w8a8_gemm_silu_mul_sources: no rows");
+    return grouped_w8a8_entry("grouped_w8a8_gemm_silu_mul_sources", y, nullptr, xq, x_scale, w_packed, w_scale, offsets, n_experts,
+                              total_rows, n, k, out_dtype, 1, stream, {sources, n_sources});
 }

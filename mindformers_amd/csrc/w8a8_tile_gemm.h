@@ -47,16 +47,19 @@ struct TiledRows {                                            // tile order: who
     }
 };
 template <int XL>
-struct PlainRows {                                            // rows m0 .. of `rows` rows of K (a multiple of 16) bytes
+struct PlainRows {                                            // rows m0 .. of a group of `rows` rows from row0 on, of K (a multiple of 16) bytes
     const uint8_t* p;
     uint32_t row[XL];
     int c, last;                                              // columns past K are clamped: their weights are zero
-    __device__ __forceinline__ PlainRows(const uint8_t* xq, int m0, int rows, int K, int wv) : p(xq + (int64_t)m0 * K) {
+    __device__ __forceinline__ PlainRows(const uint8_t* xq, const TileSources& src, int row0, int m0, int rows, int K, int wv)
+        : p(src.sources ? xq : xq + (int64_t)(row0 + m0) * K) {
         c = 16 * ((threadIdx.x >> 4) & 3);
         last = K - 16;
 #pragma unroll
-        for (int i = 0; i < XL; ++i)
-            row[i] = (uint32_t)min(16 * (4 * i + wv) + (int)(threadIdx.x & 15), rows - 1 - m0) * (uint32_t)K;
+        for (int i = 0; i < XL; ++i) {
+            const int in = min(16 * (4 * i + wv) + (int)(threadIdx.x & 15), rows - 1 - m0);
+            row[i] = (uint32_t)(src.sources ? src.of(row0 + m0 + in) : in) * (uint32_t)K;
+        }
     }
     __device__ __forceinline__ i32x4 load(int i, int s) const {
         return bitcast<i32x4>(load16_at(p, row[i] + (uint32_t)min(s * KSTEP + c, last)));

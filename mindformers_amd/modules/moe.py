@@ -170,16 +170,23 @@ class QuantGroupedMLP(nn.Module):
             return None
         return self._quant(x, self.act_scale1)
 
-    def forward(self, hidden_states, group_list=None, offsets=None, row_scale=None, out_dtype=None):
+    def reads_sources(self, x, total_rows):
+        """Whether the first projection reads the tokens x (as ``quantize_tokens`` returns them, or as they are) through the sort's
+        index, so that they need not be copied ``total_rows`` times."""
+        if self._p1 is None:
+            self.prepare()
+        return (x.dtype == torch.int8) == bool(self.act_quant) and ops.grouped_reads_sources(x, self._p1, total_rows)
+
+    def forward(self, hidden_states, group_list=None, offsets=None, row_scale=None, out_dtype=None, sources=None):
         """``row_scale`` (fp32, one per row): hidden_states are the permuted integers of ``quantize_tokens``; the result
-        is of ``out_dtype``."""
+        is of ``out_dtype``.  ``sources`` (where ``reads_sources``): hidden_states are the tokens, and these name a row's."""
         if self._p1 is None:
             self.prepare()
         if offsets is None:
             offsets = torch.zeros(self.num_experts + 1, dtype=torch.int32, device=hidden_states.device)
             offsets[1:] = torch.cumsum(group_list, 0).to(torch.int32)
         if not self.act_quant:
-            a = ops.grouped_w8a16_linear(hidden_states, self._p1, offsets)       # silu(gate) * hidden included
+            a = ops.grouped_w8a16_linear(hidden_states, self._p1, offsets, sources=sources)   # silu(gate) * hidden included
             return ops.grouped_w8a16_linear(a, self._p2, offsets)
         dt = out_dtype or hidden_states.dtype
         if row_scale is not None:
@@ -188,7 +195,7 @@ class QuantGroupedMLP(nn.Module):
             xq, xs = ops.dynamic_quant(hidden_states.contiguous(), self.smooth_scale1, offsets=offsets)
         else:
             xq, xs = self._quant(hidden_states.contiguous(), self.act_scale1)
-        a = ops.grouped_w8a8_linear(xq, xs, self._p1, offsets, out_dtype=dt)      # silu(gate) * hidden included
+        a = ops.grouped_w8a8_linear(xq, xs, self._p1, offsets, out_dtype=dt, sources=sources)   # silu(gate) * hidden included
         if self.act_quant == "per_tensor":
             aq, a_s = ops.static_quant(a, self.act_scale2)
         elif self.smooth_scale2 is not None:
@@ -246,7 +253,12 @@ class MoELayer(nn.Module):
         expert_weight, routing_map = self.router(x)
         early = isinstance(self.experts, QuantGroupedMLP) and self.experts.takes_quantized_rows()
         quantized = self.experts.quantize_tokens(x) if early else None
-        if quantized is not None:
+        rows = quantized[0] if quantized is not None else x
+        if early and self.experts.reads_sources(rows, routing_map.numel()):
+            sources, ps, row_map, counts, offsets = ops.moe_sort(routing_map, self.num_experts,
+                                                                 None if quantized is None else quantized[1])
+            y = self.experts(rows, counts, offsets=offsets, row_scale=ps, out_dtype=x.dtype, sources=sources)
+        elif quantized is not None:
             px, ps, row_map, counts, offsets = ops.moe_permute_int8(*quantized, routing_map, self.num_experts)
             y = self.experts(px, counts, offsets=offsets, row_scale=ps, out_dtype=x.dtype)
         else:

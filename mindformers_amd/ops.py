@@ -1272,18 +1272,51 @@ def moe_permute_int8(xq, x_scale, expert_index, n_experts):
     return px, ps, row_map, counts, offsets
 
 
-def grouped_w8a16_linear(x, w, offsets, scale=None):
+def moe_sort(expert_index, n_experts, x_scale=None):
+    """``moe_permute`` without the copies: returns (sources int32 [T*k], the token of each permuted row, permuted_scale (of
+    ``x_scale`` fp32 [T]) or None, row_map, counts, offsets), for the grouped GEMMs with ``sources``."""
+    lib = _lib.load()
+    dev = _dev_ok(expert_index, x_scale)
+    _need(expert_index.dtype == torch.int32 and expert_index.dim() == 2, "expert_index must be int32 [T, k]")
+    t, k = expert_index.shape
+    _need(x_scale is None or (x_scale.dtype == torch.float32 and x_scale.numel() == t), "x_scale must be fp32 [T]")
+    maps = torch.empty(2, t * k, dtype=torch.int32, device=dev)
+    ps = None if x_scale is None else torch.empty(t * k, dtype=torch.float32, device=dev)
+    counts = torch.empty(n_experts, dtype=torch.int64, device=dev)
+    offsets = torch.empty(n_experts + 1, dtype=torch.int32, device=dev)
+    check(lib.mf_moe_sort(ptr(maps[0]), ptr(maps[1]), ptr(ps), ptr(counts), ptr(offsets), ptr(x_scale), ptr(expert_index), t, k,
+                          n_experts, stream_ptr(dev)), "mf_moe_sort")
+    return maps[1], ps, maps[0], counts, offsets
+
+
+def grouped_reads_sources(x, w, total_rows):
+    """Whether the grouped GEMM of the gated expert weights ``w`` reads the rows of x (int8 or 16-bit) through an index where
+    there are ``total_rows`` permuted ones: groups of prompt size."""
+    lib = _lib.load()
+    fn = lib.mf_grouped_w8a8_reads_sources if x.dtype == torch.int8 else lib.mf_grouped_w8a16_reads_sources
+    return bool(w.gated and fn(x.shape[0], w.experts, total_rows, w.n, w.k))
+
+
+def grouped_w8a16_linear(x, w, offsets, scale=None, sources=None):
     """GroupedMatmulV4 over expert row groups.  x [R, K]; ``w`` a PackedInt8Weight of [E, N, K] (or a raw int8
     [E, N, K] tensor with ``scale`` [E, N], packed on every call); offsets int32 [E+1].  A weight packed with
-    ``pack_w8a16_gated`` runs with silu(gate) * up in the epilogue and returns [R, N/2]."""
+    ``pack_w8a16_gated`` runs with silu(gate) * up in the epilogue and returns [R, N/2].  ``sources`` (int32 [R], of
+    ``moe_sort``; gated, where ``grouped_reads_sources``): x [T, K] are the rows that they name."""
     lib = _lib.load()
     if not isinstance(w, PackedInt8Weight):
         w = pack_w8a16(w, scale)
     _need(w.experts is not None, "grouped_w8a16_linear needs stacked expert weights [E, N, K]")
-    dev = _dev_ok(x, offsets)
+    dev = _dev_ok(x, offsets, sources)
     e, n, k = w.experts, w.n, w.k
     _need(x.dtype in _ACT and x.dim() == 2 and x.shape[1] == k, "x must be bf16/fp16 [R, K]")
     _need(offsets.dtype == torch.int32 and offsets.numel() == e + 1, "offsets must be int32 [E+1]")
+    if sources is not None:
+        _need(w.gated and sources.dtype == torch.int32 and sources.dim() == 1, "sources (int32 [R]) go with gated weights")
+        y = torch.empty(sources.numel(), n // 2, dtype=x.dtype, device=dev)
+        check(lib.mf_grouped_w8a16_gemm_silu_mul_sources(ptr(y), ptr(x), ptr(sources), x.shape[0], ptr(w.packed), ptr(w.scale),
+                                                         ptr(offsets), e, sources.numel(), n, k, dtype_code(x.dtype),
+                                                         stream_ptr(dev)), "mf_grouped_w8a16_gemm_silu_mul_sources")
+        return y
     y = torch.empty(x.shape[0], n // 2 if w.gated else n, dtype=x.dtype, device=dev)
     fn = lib.mf_grouped_w8a16_gemm_silu_mul if w.gated else lib.mf_grouped_w8a16_gemm
     check(fn(ptr(y), ptr(x), ptr(w.packed), ptr(w.scale), ptr(offsets), e, x.shape[0], n, k, dtype_code(x.dtype),
@@ -1291,21 +1324,28 @@ def grouped_w8a16_linear(x, w, offsets, scale=None):
     return y
 
 
-def grouped_w8a8_linear(xq, x_scale, w, offsets, out_dtype=torch.bfloat16, return_acc=False):
+def grouped_w8a8_linear(xq, x_scale, w, offsets, out_dtype=torch.bfloat16, return_acc=False, sources=None):
     """GroupedMatmulV4 on int8 operands: xq int8 [R, K] row-major with per-row scales (``dynamic_quant`` of the permuted
     rows), ``w`` a PackedInt8Weight of [E, N, K], offsets int32 [E+1].  Exact int32 accumulators, dequantised to
     out_dtype; with ``return_acc`` also the int32 [R, N] accumulators.  A weight packed with ``pack_w8a16_gated`` runs with
-    silu(gate) * up in the epilogue and returns [R, N/2]."""
+    silu(gate) * up in the epilogue and returns [R, N/2].  ``sources``: as in ``grouped_w8a16_linear``; x_scale stays [R]."""
     lib = _lib.load()
     _need(isinstance(w, PackedInt8Weight) and w.experts is not None and not (w.gated and return_acc),
           "grouped_w8a8_linear needs stacked expert weights [E, N, K] (not gated where the accumulators are wanted)")
-    dev = _dev_ok(xq, x_scale, offsets)
+    dev = _dev_ok(xq, x_scale, offsets, sources)
     e, n, k = w.experts, w.n, w.k
+    rows = xq.shape[0] if sources is None else sources.numel()
     _need(xq.dtype == torch.int8 and xq.dim() == 2 and xq.shape[1] == k, "xq must be int8 [R, K]")
-    _need(x_scale.dtype == torch.float32 and x_scale.numel() == xq.shape[0], "x_scale must be fp32 [R]")
+    _need(x_scale.dtype == torch.float32 and x_scale.numel() == rows, "x_scale must be fp32 [R]")
     _need(offsets.dtype == torch.int32 and offsets.numel() == e + 1, "offsets must be int32 [E+1]")
     _need(out_dtype in _ACT, "out_dtype must be bf16/fp16")
-    y = torch.empty(xq.shape[0], n // 2 if w.gated else n, dtype=out_dtype, device=dev)
+    y = torch.empty(rows, n // 2 if w.gated else n, dtype=out_dtype, device=dev)
+    if sources is not None:
+        _need(w.gated and sources.dtype == torch.int32 and sources.dim() == 1, "sources (int32 [R]) go with gated weights")
+        check(lib.mf_grouped_w8a8_gemm_silu_mul_sources(ptr(y), ptr(xq), ptr(x_scale), ptr(sources), xq.shape[0], ptr(w.packed),
+                                                        ptr(w.scale), ptr(offsets), e, rows, n, k, dtype_code(out_dtype),
+                                                        stream_ptr(dev)), "mf_grouped_w8a8_gemm_silu_mul_sources")
+        return y
     if w.gated:
         check(lib.mf_grouped_w8a8_gemm_silu_mul(ptr(y), ptr(xq), ptr(x_scale), ptr(w.packed), ptr(w.scale), ptr(offsets), e,
                                                 xq.shape[0], n, k, dtype_code(out_dtype), stream_ptr(dev)),

@@ -2163,6 +2163,37 @@ def test_grouped_w8a8_gated_equals_unfused(counts, n, k, dtype):
     assert fused.shape == (rows, n // 2) and torch.equal(fused[:, :c], ref)
 
 
+@pytest.mark.parametrize("tokens,e,k,n,h,dtype", [
+    (129, 5, 3, 96, 128, torch.float16), (700, 64, 4, 512, 1024, torch.bfloat16), (1, 1, 21, 32, 64, torch.bfloat16),
+    (900, 20, 8, 160, 192, torch.bfloat16),                  # row blocks of 128 and what is left over
+])
+def test_grouped_gemms_read_rows_through_the_index(tokens, e, k, n, h, dtype):
+    """The tokens through ``sources`` have the bits of their gathered copies; experts without rows and pairs without an expert."""
+    rng = np.random.default_rng(tokens)
+    idx = rng.integers(0, e, (tokens, k)).astype(np.int32)
+    idx[rng.random(idx.shape) < 0.05] = e + 3
+    idx[idx == e // 2] = 0
+    x = dev(rounded(rng.normal(size=(tokens, h)), dtype), dtype)
+    w = ops.pack_w8a16_gated(torch.from_numpy(rng.integers(-127, 128, (e, n, h)).astype(np.int8)).cuda(),
+                             torch.from_numpy(rng.uniform(0.01, 0.02, (e, n)).astype(np.float32)).cuda(), "halves")
+    di = torch.from_numpy(idx).cuda()
+    px, row_map, counts, offsets = ops.moe_permute(x, di, e)
+    xq, xs = ops.dynamic_quant(x)
+    pq, ps, *_ = ops.moe_permute_int8(xq, xs, di, e)
+    sources, scale, *maps = ops.moe_sort(di, e, xs)
+    live = int(offsets[-1])
+    assert all(torch.equal(a, b) for a, b in zip(maps, (row_map, counts, offsets)))
+    assert torch.equal(x[sources[:live].long()], px[:live]) and torch.equal(scale[:live], ps[:live])
+    assert ops.grouped_reads_sources(x, w, tokens * k) and ops.grouped_reads_sources(xq, w, tokens * k)
+    a = ops.grouped_w8a16_linear(px, w, offsets)[:live]
+    assert torch.equal(ops.grouped_w8a16_linear(x, w, offsets, sources=sources)[:live], a)
+    b = ops.grouped_w8a8_linear(pq, ps, w, offsets, out_dtype=dtype)[:live]
+    assert torch.equal(ops.grouped_w8a8_linear(xq, scale, w, offsets, out_dtype=dtype, sources=sources)[:live], b)
+    assert not ops.grouped_reads_sources(x, w, e)            # few rows an expert: the kernels that read them side by side
+    with pytest.raises(Exception, match="not read through an index"):
+        ops.grouped_w8a16_linear(x, w, offsets, sources=sources[:e])
+
+
 @pytest.mark.parametrize("counts,n", [
     ([50, 80, 62], 48), ([65, 64, 66], 48),                     # few tiles: up to 64 rows a group the passes, above it tiles
     ([20] * 255 + [8], 32), ([21] * 200 + [22] * 56, 32),       # tiles enough: 20 rows (16-bit activations; 12 with int8 ones)
