@@ -8,15 +8,20 @@
 struct TileGrid {
     int m_blocks, n_blocks, full, split, steps_per_split;
     int mt, nt;                                               // rows of a block / 32, channels of a block / 64
+    int tail;                                                 // tiles of a last row block with fewer 32-row pieces (not in m_blocks)
 };
 constexpr int TG_PANEL = 4;                                   // row blocks walked together along the channels
 __device__ __forceinline__ void tg_locate(const TileGrid& g, int id, int& mb, int& nb, int& part, int& slot) {
     int t;
+    part = slot = 0;
     if (id < g.full) {
         t = (id & 7) * (g.full >> 3) + (id >> 3);
-        part = slot = 0;
+    } else if (id < g.full + g.tail) {
+        nb = id - g.full;
+        mb = g.m_blocks;
+        return;
     } else {
-        slot = id - g.full;
+        slot = id - g.full - g.tail;
         t = g.full + slot / g.split;
         part = slot % g.split;
     }
@@ -25,13 +30,14 @@ __device__ __forceinline__ void tg_locate(const TileGrid& g, int id, int& mb, in
     nb = in / rows;
     mb = panel * TG_PANEL + in - nb * rows;
 }
-inline int tg_workgroups(const TileGrid& g) { return g.full + (g.m_blocks * g.n_blocks - g.full) * g.split; }
+inline int tg_workgroups(const TileGrid& g) { return g.full + g.tail + (g.m_blocks * g.n_blocks - g.full) * g.split; }
 
 // Measured times (us): a k-step of a tile on a compute unit of its own, of a pair of tiles on one compute unit (the clock
 // follows the power draw), what a launch and a tile's start and end take, the reduce launch, and one part's share of
 // writing and summing the parts.
 struct TileCost {
     float alone, pair, fixed, reduce, part;
+    float tail;                                               // a k-step of a tile of up to 64 rows
     // other shapes of tile (32*mt rows, 64*nt channels), each on a compute unit of its own: a launch, a k-step
     struct { int mt, nt; float fixed, step; } once[4];
 };
@@ -43,6 +49,7 @@ inline TileGrid tg_plan_rounds(int m, int n, int steps, const TileCost& c, float
     g.mt = g.nt = 4;
     g.m_blocks = m_blocks;
     g.n_blocks = n_blocks;
+    g.tail = 0;
     const int tiles = m_blocks * n_blocks, rounds = tiles / 256, rem = tiles % 256;
     float best = 0.f;
     g.split = 1;
@@ -71,6 +78,27 @@ inline TileGrid tg_plan_rounds(int m, int n, int steps, const TileCost& c, float
     return g;
 }
 
+// A last row block of up to 64 rows behind two rounds and more of whole tiles: tiles of just its 32-row pieces, dealt last and one after
+// the other over the XCDs.  Beside whole tiles, in places that would be empty, they cost what they compute; where they overflow the
+// last round they add their own length.  They replace matrix instructions on rows that are not there, which cost the power of those
+// that are.  us on whole tiles | with a tail: W8A16 1048 x 28672 x 4096 230 | 224, 2080 x 28672 x 4096 393 | 381, 1057 x 37888 x 3584 254 |
+// 246, 1300 x 24576 x 1536 97 | 89, W8A8 1048 x 37888 x 3584 164 | 159, 1340 x 37888 x 3584 186 | 182, 1300 x 24576 x 1536 67 | 62;
+// overflowing 4137 x 4096 x 14336 366 | 425.  Pieces of 65 to 96 rows gain nothing (1632 x 28672 x 4096 311 | 314), nor do tiles of 96 rows
+// throughout (1048 x 28672 x 4096 231 | 234, 2080 rows 398 | 420), and the few tiles of a narrow output are shorter cut along K
+// (4137 x 6144 x 4096 168 | 171).
+inline bool tg_plan_tail(int m, int n, int steps, const TileCost& c, float* us, TileGrid& g) {
+    const int rows = m % 128, n_blocks = (n + 255) / 256, tiles = m / 128 * n_blocks, last = tiles % 512;
+    if (rows == 0 || rows > 64 || tiles < 512 || n_blocks < 48) return false;
+    const float whole = tiles / 512 * c.pair + (last == 0 ? 0.f : last <= 256 ? c.alone : c.pair);
+    const float tail = last > 0 && last + n_blocks <= 512 ? c.tail * n_blocks / 256 : c.tail;
+    const bool room = last > 256 && last + n_blocks <= 512;   // the round that the whole tiles would have them in takes as long
+    const float t = c.fixed + steps * (whole + (room ? 0.f : tail));
+    if (t > *us) return false;
+    *us = t;
+    g = {m / 128, n_blocks, tiles / 8 * 8, 1, steps, 4, 4, n_blocks};
+    return true;
+}
+
 // Tiles of 128 x 256, or of another shape where those are all resident at once, each on a compute unit of its own, and the shape is
 // the shortest: more units then share the work, or fewer rows and channels are padding.  A tile of fewer channels pays more for its
 // activations a matrix instruction, a wider one needs all the registers of a compute unit, so neither gains where the device is full for
@@ -86,6 +114,8 @@ inline TileGrid tg_plan_rounds(int m, int n, int steps, const TileCost& c, float
 // leave a quarter of the units idle, and more of them are wanted (2025 x 2112 x 7168, 198 tiles of 96 x 256, would gain a seventh as well).
 inline TileGrid tg_plan(int m, int n, int steps, const TileCost& c, float* us) {
     const TileGrid g = tg_plan_rounds(m, n, steps, c, us);
+    TileGrid t;
+    if (tg_plan_tail(m, n, steps, c, us, t)) return t;
     if (m <= 128 || steps < 16) return g;
     const bool all_cut = g.split > 1 && g.full == 0;
     const auto tiles_of = [&](int mt, int nt) { return (int64_t)((m + 32 * mt - 1) / (32 * mt)) * ((n + 64 * nt - 1) / (64 * nt)); };
@@ -98,7 +128,7 @@ inline TileGrid tg_plan(int m, int n, int steps, const TileCost& c, float* us) {
         if (s.nt != 4 && (steps < 24 || all_cut)) continue;
         if (s.mt == 3 && s.nt == 3 && tiles_of(3, 4) > 192) continue;
         least = *us = t;
-        if (!all_cut) best = {(m + 32 * s.mt - 1) / (32 * s.mt), (n + 64 * s.nt - 1) / (64 * s.nt), (int)tiles / 8 * 8, 1, steps, s.mt, s.nt};
+        if (!all_cut) best = {(m + 32 * s.mt - 1) / (32 * s.mt), (n + 64 * s.nt - 1) / (64 * s.nt), (int)tiles / 8 * 8, 1, steps, s.mt, s.nt, 0};
     }
     return best;
 }

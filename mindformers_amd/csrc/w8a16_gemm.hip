@@ -563,20 +563,13 @@ struct TileOut {
     }
 };
 
+// one tile of 32*MT rows from row m0 on
 template <typename T, int MT, int NT>
-__global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
-    uint16_t* __restrict__ y, float* __restrict__ partial, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp,
-    const float* __restrict__ scale, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N,
-    int K, int gated, int aligned, TileGrid g) {
-    constexpr int OPS = 2 * 32 * MT * 128, OUT = tg::WAVES * 32 * TileOut<T, NT>::ROW;
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];   // the output stage reuses the operand stages
-    int mb, nb, part, slot;
-    tg_locate(g, blockIdx.x, mb, nb, part, slot);
-    const bool whole = blockIdx.x < g.full || g.split == 1;
-    const int KS = K / tg::KSTEP, s0 = part * g.steps_per_split;
-    const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
+__device__ __forceinline__ void w8a16_tile_of(uint16_t* y, float* partial, const uint16_t* x, const uint8_t* wp, const float* scale,
+                                              const uint16_t* bias, const uint16_t* residual, int M, int N, int K, int gated,
+                                              int aligned, int m0, int nb, int slot, bool whole, int s0, int s_end, uint8_t* smem) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = mb * 32 * MT, n0 = nb * tg::BN_OF<NT> + 16 * NT * wv;
+    const int n0 = nb * tg::BN_OF<NT> + 16 * NT * wv;
     float* pt = partial + (int64_t)slot * (32 * MT * tg::BN_OF<NT>) + (wv * MT * 2 * NT * 64 + lane) * 4;
     const TileOut<T, NT> out{y, bias, residual, M, N, gated, aligned};
     f32x4 sc[NT], bi[NT];
@@ -603,6 +596,32 @@ __global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
     });
 }
 
+template <typename T, int MT, int NT>
+__global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
+    uint16_t* __restrict__ y, float* __restrict__ partial, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp,
+    const float* __restrict__ scale, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N,
+    int K, int gated, int aligned, TileGrid g) {
+    constexpr int OPS = 2 * 32 * MT * 128, OUT = tg::WAVES * 32 * TileOut<T, NT>::ROW;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];   // the output stage reuses the operand stages
+    int mb, nb, part, slot;
+    tg_locate(g, blockIdx.x, mb, nb, part, slot);
+    const bool whole = blockIdx.x < g.full + g.tail || g.split == 1;
+    const int KS = K / tg::KSTEP, s0 = part * g.steps_per_split, m0 = mb * 32 * MT;
+    const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
+#define TILE_OF(MTV) \
+    w8a16_tile_of<T, MTV, NT>(y, partial, x, wp, scale, bias, residual, M, N, K, gated, aligned, m0, nb, slot, whole, s0, s_end, smem)
+    if constexpr (MT == 4 && NT == 4) {                       // a plan with a tail
+        const int left = g.tail && mb == g.m_blocks ? M - m0 : 128;
+        if (left <= 32) TILE_OF(1);
+        else if (left <= 64) TILE_OF(2);
+        else if (left <= 96) TILE_OF(3);
+        else TILE_OF(4);
+    } else {
+        TILE_OF(MT);
+    }
+#undef TILE_OF
+}
+
 // Sums the parts of the tiles that were cut along K, in order: a workgroup per 32 rows x 64 channels, a quarter of the
 // channels per wave.
 template <typename T, int MT>
@@ -614,7 +633,7 @@ __global__ __launch_bounds__(256) void w8a16_tile_reduce_kernel(
     constexpr int64_t PART = 32 * MT * tg::BN;
     const int tile = blockIdx.x / ITEMS, item = blockIdx.x - tile * ITEMS, wv = item / MT, mt = item - wv * MT;
     int mb, nb, part, slot;
-    tg_locate(g, g.full + tile * g.split, mb, nb, part, slot);
+    tg_locate(g, g.full + g.tail + tile * g.split, mb, nb, part, slot);
     const int m0 = mb * 32 * MT + 32 * mt, n0 = nb * tg::BN + 64 * wv;
     if (m0 >= M || n0 >= N) return;
     const int lane = threadIdx.x & 63, e0 = 2 * (threadIdx.x >> 6);
@@ -1142,7 +1161,7 @@ struct GemmPlan {
 
 // Tile plan of the many-row kernel (4137 x 4096 x 14336: 16 of 528 tiles left over by whole rounds, 455 us uncut, 351 us in
 // 8 parts).
-constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f, {{3, 4, 7.8f, 0.6f}, {3, 3, 7.8f, 0.477f}, {4, 3, 8.5f, 0.556f}}};
+constexpr TileCost TG_COST = {0.75f, 1.58f, 6.f, 5.f, 0.065f, 0.38f, {{3, 4, 7.8f, 0.6f}, {3, 3, 7.8f, 0.477f}, {4, 3, 8.5f, 0.556f}}};
 TileGrid plan_tiles(int m, int n, int k, float* us) {
     return tg_plan(m, n, k / tg::KSTEP, TG_COST, us);
 }
@@ -1390,8 +1409,8 @@ extern "C" int mf_w8a16_plan(int m, int n, int k, int* whole, int* cut, int* spl
         float us;
         const TileGrid g = plan_tiles(m, n, k, &us);
         *split = g.split;
-        *whole = g.split > 1 ? g.full : g.m_blocks * g.n_blocks;
-        *cut = g.m_blocks * g.n_blocks - *whole;
+        *whole = g.tail + (g.split > 1 ? g.full : g.m_blocks * g.n_blocks);
+        *cut = g.m_blocks * g.n_blocks + g.tail - *whole;
         return 1;
     }
     const GemmPlan p = plan_w8a16(m, n, k);

@@ -810,20 +810,13 @@ struct QTileGated {
 // GATED: N = 2F channels, [gate | up]; y [M, F] = silu(gate) * up (no bias, no residual).  It halves what is written here and read by the
 // quantisation behind it: a layer step with 37888 x 3584 on 100 / 600 / 1531 / 4100 rows 132.5 / 286 / 481 / 1124 us with a kernel for
 // silu * up and quantisation, 131.1 / 277.5 / 471 / 1081 here.
-template <typename T, int MT, int NT, bool GATED = false>
-__global__ __launch_bounds__(256, MT * NT > 16 ? 1 : 2) void w8a8_tile_kernel(
-    uint16_t* __restrict__ y, int32_t* __restrict__ partial, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
-    const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const uint16_t* __restrict__ bias,
-    const uint16_t* __restrict__ residual, int M, int N, int K, int aligned, TileGrid g) {
-    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW<NT>, OPS = tq::LDS_BYTES<MT>;
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
-    int mb, nb, part, slot;
-    tg_locate(g, blockIdx.x, mb, nb, part, slot);
-    const bool whole = blockIdx.x < g.full || g.split == 1;
-    const int KS = (K + Q_KSTEP - 1) / Q_KSTEP, s0 = part * g.steps_per_split;
-    const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
+// One tile of 32*MT rows from row m0 on.
+template <typename T, int MT, int NT, bool GATED>
+__device__ __forceinline__ void w8a8_tile_of(uint16_t* y, int32_t* partial, const int8_t* xq, const float* x_scale, const uint8_t* wp,
+                                             const float* w_scale, const uint16_t* bias, const uint16_t* residual, int M, int N, int aligned,
+                                             int m0, int nb, int slot, bool whole, int s0, int s_end, uint8_t* smem) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = mb * 32 * MT, n0 = (nb * tq::BN_OF<NT> + 16 * NT * wv) >> GATED;   // first channel of the output
+    const int n0 = (nb * tq::BN_OF<NT> + 16 * NT * wv) >> GATED;   // first channel of the output
     int32_t* pt = partial + (int64_t)slot * (32 * MT * tq::BN_OF<NT>) + (wv * MT * 2 * NT * 64 + lane) * 4;
     const QTileOut<T, NT> out{x_scale, w_scale, bias, M, N, 0};
     const QTileGated<T, NT> gout{x_scale, w_scale, M, N >> 1};
@@ -860,6 +853,32 @@ __global__ __launch_bounds__(256, MT * NT > 16 ? 1 : 2) void w8a8_tile_kernel(
     });
 }
 
+template <typename T, int MT, int NT, bool GATED = false>
+__global__ __launch_bounds__(256, MT * NT > 16 ? 1 : 2) void w8a8_tile_kernel(
+    uint16_t* __restrict__ y, int32_t* __restrict__ partial, const int8_t* __restrict__ xq, const float* __restrict__ x_scale,
+    const uint8_t* __restrict__ wp, const float* __restrict__ w_scale, const uint16_t* __restrict__ bias,
+    const uint16_t* __restrict__ residual, int M, int N, int K, int aligned, TileGrid g) {
+    constexpr int OUT = tq::WAVES * 32 * TG_STAGE_ROW<NT>, OPS = tq::LDS_BYTES<MT>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[OUT > OPS ? OUT : OPS];
+    int mb, nb, part, slot;
+    tg_locate(g, blockIdx.x, mb, nb, part, slot);
+    const bool whole = blockIdx.x < g.full + g.tail || g.split == 1;
+    const int KS = (K + Q_KSTEP - 1) / Q_KSTEP, s0 = part * g.steps_per_split, m0 = mb * 32 * MT;
+    const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
+#define TILE_OF(MTV) \
+    w8a8_tile_of<T, MTV, NT, GATED>(y, partial, xq, x_scale, wp, w_scale, bias, residual, M, N, aligned, m0, nb, slot, whole, s0, s_end, \
+                                    smem)
+    if constexpr (MT == 4 && NT == 4) {                       // a plan with a tail
+        const int left = g.tail && mb == g.m_blocks ? M - m0 : 128;
+        if (left <= 64) TILE_OF(2);
+        else if (left <= 96) TILE_OF(3);
+        else TILE_OF(4);
+    } else {
+        TILE_OF(MT);
+    }
+#undef TILE_OF
+}
+
 // Sums the parts of the tiles that were cut along K: a workgroup per 32 rows x 64 channels, a quarter of them per wave.
 template <typename T, int MT, bool GATED = false>
 __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
@@ -871,7 +890,7 @@ __global__ __launch_bounds__(256) void w8a8_tile_reduce_kernel(
     constexpr int64_t PART = 32 * MT * tq::BN;
     const int tile = blockIdx.x / ITEMS, item = blockIdx.x - tile * ITEMS, wv = item / MT, mt = item - wv * MT;
     int mb, nb, part, slot;
-    tg_locate(g, g.full + tile * g.split, mb, nb, part, slot);
+    tg_locate(g, g.full + g.tail + tile * g.split, mb, nb, part, slot);
     const int m0 = mb * 32 * MT + 32 * mt, n0 = (nb * tq::BN + 64 * wv) >> GATED;
     if (m0 >= M || n0 >= N >> GATED) return;
     // 16-row tile j, channel tiles nt and nt + 2
@@ -1171,7 +1190,7 @@ QPlan plan_w8a8(int m, int n, int k, bool x_tiled) {
 // against 33 / 33 / 55 (LDS-staged), 3584 x 18944 at 1531 rows in 113 against 172, 3584 x 3584 at 448 rows in 26 against 22.  `fused`: the
 // sum of the register-streaming and the wide kernel's parts carries what follows, which is a kernel of its own behind tiles (the
 // figures of the LDS-staged kernel have it in).
-constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f, {{3, 4, 6.6f, 0.346f}, {3, 3, 6.4f, 0.288f}, {4, 3, 9.5f, 0.3f}, {4, 5, 12.2f, 0.509f}}};
+constexpr TileCost TQ_COST = {0.40f, 0.93f, 6.f, 5.f, 0.065f, 0.25f, {{3, 4, 6.6f, 0.346f}, {3, 3, 6.4f, 0.288f}, {4, 3, 9.5f, 0.3f}, {4, 5, 12.2f, 0.509f}}};
 bool plan_q_tiles(int m, int n, int k, bool fused, TileGrid& g) {
     if (m <= 64 || n % 16 != 0) return false;
     float us;
@@ -1191,7 +1210,7 @@ bool plan_q_wide_tiles(const QPlan& p, int m, int n, int k, TileGrid& g) {
     const int steps = (k + Q_KSTEP - 1) / Q_KSTEP, m_blocks = 2, n_blocks = (n + tq::BN_OF<5> - 1) / tq::BN_OF<5>, tiles = m_blocks * n_blocks;
     if (!p.wide || p.split_k > 1 || m <= 128 || m > 256 || n % 16 != 0 || tiles > 256) return false;
     const int rounds = (p.n_blocks * p.m_blocks + 255) / 256;
-    g = {m_blocks, n_blocks, tiles / 8 * 8, 1, steps, 4, 5};
+    g = {m_blocks, n_blocks, tiles / 8 * 8, 1, steps, 4, 5, 0};
     return 12.2f + 0.509f * steps < 5.f + 0.78f * rounds * steps;
 }
 
@@ -1339,8 +1358,8 @@ extern "C" int mf_w8a8_plan(int m, int n, int k, int fused, int* whole, int* cut
     TileGrid g;
     if (plan_q_tiles(m, n, k, fused != 0, g)) {
         *split = g.split;
-        *whole = g.split > 1 ? g.full : g.m_blocks * g.n_blocks;
-        *cut = g.m_blocks * g.n_blocks - *whole;
+        *whole = g.tail + (g.split > 1 ? g.full : g.m_blocks * g.n_blocks);
+        *cut = g.m_blocks * g.n_blocks + g.tail - *whole;
         return 3;
     }
     const QPlan p = plan_w8a8(m, n, k, true);

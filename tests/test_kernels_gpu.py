@@ -1283,6 +1283,19 @@ def test_w8a16_many_rows_on_192_channel_tiles(dtype, m, n, k, whole):
     test_w8a16_many_rows(dtype, m, n, k, False, True)
 
 
+TAILS = [(1025, 16400, 1088), (1056, 16656, 1024), (1057, 16400, 1152), (1088, 16416, 1024), (1300, 24576, 1536)]
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.bfloat16 if i % 2 else torch.float16, *shape) for i, shape in enumerate(TAILS)])
+def test_w8a16_many_rows_with_a_short_last_row_block(dtype, m, n, k):
+    """The same at shapes of more than two rounds whose last row block has tiles of one or two 32-row pieces (1, 32, 33, 64 and 20 rows)."""
+    out = [torch.zeros(1, dtype=torch.int32) for _ in range(3)]
+    assert ops._lib.load().mf_w8a16_plan(m, n, k, *[o.data_ptr() for o in out]) == 1
+    assert [int(o) for o in out] == [(m + 127) // 128 * ((n + 255) // 256), 0, 1]           # none is cut along K
+    test_w8a16_many_rows(dtype, m, n, k, True, False)
+    test_w8a16_many_rows(dtype, m, n, k, False, True)
+
+
 def test_w8a16_exact_on_integer_grid():
     """Power-of-two scales and small-integer activations make every product and sum exact: the kernel must
     return exactly the integer matmul (catches a dropped k-step, a wrong row/column or a transposed operand)."""
@@ -1575,6 +1588,16 @@ def test_w8a8_many_rows_on_192_and_320_channel_tiles(dtype, m, n, k, kind, whole
     assert _w8a8_plan(m, n, k, False) == (kind, whole, 0, 1)
     test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, True, True)
     test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, False, False)
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.float16 if i % 2 else torch.bfloat16, m, n // 32 * 32, k + 16)
+                                         for i, (m, n, k) in enumerate(TAILS)])
+def test_w8a8_many_rows_with_a_short_last_row_block(dtype, m, n, k):
+    """The same at shapes of more than two rounds whose last row block has tiles of two 32-row pieces, gated too."""
+    whole = (m + 127) // 128 * ((n + 255) // 256)
+    assert _w8a8_plan(m, n, k, False) == ("tiles", whole, 0, 1)
+    test_w8a8_many_rows_equal_the_row_major_kernel(dtype, m, n, k, True, True)
+    test_w8a8_gated_tiles_equal_unfused(dtype, m, n, k, whole, 0)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
