@@ -1227,6 +1227,88 @@ void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale,
                            n, gated, aligned, g);
 }
 
+// ---- up to 16 rows, few channels, a short K -------------------------------------------------------------------------------------
+// A workgroup owns 16 channels, its W waves cut K between them and meet in LDS: no staged activations and no barrier in the k-loop, where
+// gemm4 has four waves of 16 channels each walk all of K.  What bounds it: latency, of the launch and of three or four rounds of loads.
+// us, the other kernel | here, cold weights: 4 rows 512 x 512 4.3 | 3.1, 512 x 1376 9.4 | 3.7, 2752 x 512 4.6 | 3.3, 4096 x 1024 6.2 |
+// 3.6; 16 rows 512 x 1376 10.0 | 4.9, 4096 x 1024 6.2 | 3.9.
+template <typename T, bool KTAIL, int W>
+__global__ __launch_bounds__(64 * W) void w8a16_rows_kernel(
+    uint16_t* __restrict__ y, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, const float* __restrict__ scale,
+    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N, int K, int steps_per_wave, int gated) {
+    using vec8 = typename T::vec8;
+    constexpr int D = 3;                                      // steps in flight
+    __shared__ f32x4 red[W][64];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int KS = (K + GW_KSTEP - 1) / GW_KSTEP, s_begin = wv * steps_per_wave, s_end = min(KS, s_begin + steps_per_wave);
+    const int n_tiles = (N + 15) >> 4;
+    const uint8_t* wbase = wp + (int64_t)blockIdx.x * GW_TILE_BYTES;
+    // rows past the last and columns past K read as zeros without a fetch: their offsets lie behind the buffer's end
+    const auto xbuf = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00027000);
+    constexpr int NOWHERE = 0x7ffff000;
+    const int xrow = r < M ? r * K * 2 + 32 * g : NOWHERE;
+    u32x4 wreg[D], xreg[D][2];
+    auto load = [&](auto setc, int s) {
+        constexpr int S = decltype(setc)::value;
+        const int sc = min(s, s_end - 1);
+        wreg[S] = gw_stream_load<u32x4>(wbase + (int64_t)sc * n_tiles * GW_TILE_BYTES + lane * 16);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool in = !KTAIL || sc * GW_KSTEP + 16 * g + 8 * u < K;
+            xreg[S][u] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, in ? xrow + 16 * u : NOWHERE, sc * (2 * GW_KSTEP), 0);
+        }
+    };
+    f32x4 acc = (f32x4)(0.f);
+    auto step = [&](auto jc, int s) {
+        constexpr int J = decltype(jc)::value;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            acc = T::mfma16(dequant8<T>(wreg[J][2 * u], wreg[J][2 * u + 1]), bitcast<vec8>(xreg[J][u]), acc);
+        __builtin_amdgcn_sched_barrier(0);                    // the set is free: all of it has been used
+        load(jc, s + D);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (s_begin < s_end) {
+        static_for<D>([&](auto dc) { load(dc, s_begin + decltype(dc)::value); });
+        int s = s_begin;
+        for (; s + D <= s_end; s += D) static_for<D>([&](auto jc) { step(jc, s + decltype(jc)::value); });
+        static_for<D - 1>([&](auto jc) {
+            if (s + decltype(jc)::value < s_end) step(jc, s + decltype(jc)::value);
+        });
+    }
+    red[wv][lane] = acc;
+    __syncthreads();
+    if (wv != 0) return;
+    f32x4 sum = red[0][lane];                                 // the waves' parts in order
+#pragma unroll
+    for (int w = 1; w < W; ++w) sum += red[w][lane];
+    const int n = 16 * blockIdx.x + 4 * g;
+    if (r >= M || n >= N) return;
+    if (gated) store_gated<T>(y, bias, scale, r, n, N, sum);
+    else store4<T>(y, bias, residual, scale, (int64_t)r * N, n, N, sum);
+}
+
+// Where the other kernel does not cut K (its parts are summed by what follows, which the reduction then carries: 6144 x 4096 at 8 rows 10.0
+// | 12.1, 4096 x 14336 15.0 | 18.2) and the lanes' own reads of the rows stay few.  us, the other kernel | this one: 4 rows 16384 x
+// 1024 6.8 | 5.9, 24576 x 1536 10.1 | 13.6; 8 rows 8192 x 1472 7.9 | 7.1; 16 rows 6144 x 1472 7.8 | 8.3, 16384 x 1024 6.9 | 7.5, 32768 x
+// 512 6.4 | 11.1.
+bool use_rows(const GemmPlan& p, int m, int n, int k) {
+    const int64_t tiles = (n + 15) / 16, steps = (k + GW_KSTEP - 1) / GW_KSTEP;
+    return m <= 16 && p.split_k == 1 && k < (1 << 24) && tiles * steps * (m + 4) <= 160000;   // K: 32-bit offsets
+}
+template <typename T>
+void launch_rows(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias, const void* residual, int m, int n,
+                 int k, int gated, hipStream_t st) {
+    const int steps = (k + GW_KSTEP - 1) / GW_KSTEP;
+#define W8R(KT, W)                                                                                               \
+    hipLaunchKernelGGL((w8a16_rows_kernel<T, KT, W>), dim3((n + 15) / 16), dim3(64 * W), 0, st, (uint16_t*)y, (const uint16_t*)x, wp, \
+                       scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, (steps + W - 1) / W, gated)
+    if (k % GW_KSTEP) W8R(true, 8);
+    else W8R(false, 8);
+#undef W8R
+}
+
 // Every lane group reads the activations itself, so the rows have to be few.  The other kernel cuts K between workgroups, so it wins where
 // the channel tiles are too few for the compute units and K is long, and with groups of 64 (twice the scale loads) where the workgroups
 // fill their last round to five eighths at most or the many short workgroups of wide outputs start and end more than they work.
@@ -1293,7 +1375,8 @@ void launch_skinny(const GemmPlan& p, void* y, float* partial, const void* x, co
 #define GW4_W4_BY_GROUP(MTV, WV)                                                                                 \
     { if (w4_group == 0) GW4_LAUNCH_W4(MTV, WV, 0); else if (w4_group == 64) GW4_LAUNCH_W4(MTV, WV, 64);          \
       else GW4_LAUNCH_W4(MTV, WV, 128); }
-    if (w4_group >= 0) {
+    if (w4_group < 0 && use_rows(p, m, n, k)) launch_rows<T>(y, x, wp, scale, bias, residual, m, n, k, gated, st);
+    else if (w4_group >= 0) {
         if (p.mt == 1) GW4_W4_BY_GROUP(1, 4)
         else if (p.mt == 2) GW4_W4_BY_GROUP(2, 4)
         else GW4_W4_BY_GROUP(4, 8)
