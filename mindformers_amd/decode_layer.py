@@ -130,7 +130,8 @@ class QuantDecodeLayer(nn.Module):
         the kernel that finishes this layer's last projection (same bits, one launch fewer).  A W8A8 layer takes
         ``next_norm`` = (gamma, eps, smooth) with the next layer's QKV smoothing vector and hands over the quantised
         norm output (xq, scale), which is what a W8A8 layer accepts as ``normed``."""
-        if q_starts is None and not self.act_quant and self._plain():
+        # (int8 caches: asked first, so that a step which waits for the host does not pay for checks that end in the operators)
+        if q_starts is None and not self.act_quant and key_cache.dtype is x.dtype and self._plain():
             packed, buffers = self._packed, self._buffers
             step = ops.decode_layer_step(x, normed, buffers["attn_norm"], buffers["ffn_norm"], next_norm,
                                          [packed.get(name) for name in self.NAMES], self.qkv_b, cos, sin, key_cache, value_cache,

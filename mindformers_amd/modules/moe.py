@@ -173,6 +173,8 @@ class QuantGroupedMLP(nn.Module):
     def reads_sources(self, x, total_rows):
         """Whether the first projection reads the tokens x (as ``quantize_tokens`` returns them, or as they are) through the sort's
         index, so that they need not be copied ``total_rows`` times."""
+        if total_rows <= self.num_experts:                        # far from prompt size: a step of few tokens waits for the host
+            return False
         if self._p1 is None:
             self.prepare()
         return (x.dtype == torch.int8) == bool(self.act_quant) and ops.grouped_reads_sources(x, self._p1, total_rows)
