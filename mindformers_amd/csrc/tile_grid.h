@@ -4,7 +4,8 @@
 
 // Workgroup id -> (row block, channel block, part of K).  Ids below `full` are whole tiles: ids go to the XCDs in turn, so
 // XCD j is given the tiles [j * full / 8, (j + 1) * full / 8) and the workgroups that run on it at one time share row and
-// channel blocks in its L2.  The tiles left over are cut into `split` parts of K each.
+// channel blocks in its L2.  Then come the `tail` tiles of a short last row block, side by side along the channels, and the tiles left
+// over, cut into `split` parts of K each.
 struct TileGrid {
     int m_blocks, n_blocks, full, split, steps_per_split;
     int mt, nt;                                               // rows of a block / 32, channels of a block / 64

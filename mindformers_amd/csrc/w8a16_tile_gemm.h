@@ -4,7 +4,7 @@
 #include "tile_grid.h"
 
 // A workgroup of 4 waves (one per SIMD, two workgroups per compute unit) owns 32*MT rows x 64*NT channels (MT and NT: 3 or 4, see
-// tg_plan); wave w owns the w-th quarter of the channels of all the rows, so that every weight byte of the tile is loaded and converted by exactly one wave and goes
+// tg_plan; fewer rows in a group's or a plan's last block); wave w owns the w-th quarter of the channels of all the rows, so that every weight byte of the tile is loaded and converted by exactly one wave and goes
 // from global memory straight into matrix operand registers, while the activation tile of a 64-wide k-step is staged in LDS
 // once and read by all four.  Weights are fetched two steps ahead by ordinary loads (the compiler counts them); the activations of a
 // step are written to the other of two LDS stages one step ahead.  A step is 2*NT groups, (32 columns, 16 channels) each over all
