@@ -1228,20 +1228,25 @@ void launch_tiles(void* y, const void* x, const uint8_t* wp, const float* scale,
 }
 
 // ---- up to 16 rows, few channels, a short K -------------------------------------------------------------------------------------
-// A workgroup owns 16 channels, its W waves cut K between them and meet in LDS: no staged activations and no barrier in the k-loop, where
-// gemm4 has four waves of 16 channels each walk all of K.  What bounds it: latency, of the launch and of three or four rounds of loads.
-// us, the other kernel | here, cold weights: 4 rows 512 x 512 4.3 | 3.1, 512 x 1376 9.4 | 3.7, 2752 x 512 4.6 | 3.3, 4096 x 1024 6.2 |
-// 3.6; 16 rows 512 x 1376 10.0 | 4.9, 4096 x 1024 6.2 | 3.9.
-template <typename T, bool KTAIL, int W>
-__global__ __launch_bounds__(64 * W) void w8a16_rows_kernel(
+// A workgroup owns 16 channels, its waves cut K between them: each has its steps' loads in flight from the start and converts them,
+// then the waves continue one chain of matrix instructions in turn, handing the sums on through LDS.  No staged activations and one
+// barrier a turn, where gemm4 has four waves of 16 channels each walk all of K behind a barrier a step.  The chain is gemm4's, so the
+// sums have its bits: a row's result does not depend on which of the two a call with more or fewer rows takes.  What bounds it: latency, of
+// the launch, of one or two rounds of loads and of the chain.  us, the other kernel | here, cold weights: 4 rows 512 x 512 3.8 | 2.9, 512 x
+// 1376 10.2 | 5.0, 2752 x 512 4.7 | 3.6, 4096 x 1024 6.2 | 4.5; 16 rows 512 x 1376 10.8 | 5.5, 4096 x 1024 6.2 | 4.7.  With a sum in every one of
+// eight waves, added at the end, 2.8, 3.8, 3.4 and 3.7 at 4 rows, in bits of its own.  Fewer waves with longer turns (3 of 8 steps) are up
+// to 0.7 us faster at K = 1376 and up to 1 us slower past 8192 channels.
+constexpr int ROWS_WAVES = 4, ROWS_STEPS = 4;                 // waves, steps of a wave's turn
+template <typename T, bool KTAIL>
+__global__ __launch_bounds__(64 * ROWS_WAVES) void w8a16_rows_kernel(
     uint16_t* __restrict__ y, const uint16_t* __restrict__ x, const uint8_t* __restrict__ wp, const float* __restrict__ scale,
-    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N, int K, int steps_per_wave, int gated) {
+    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual, int M, int N, int K, int gated) {
     using vec8 = typename T::vec8;
-    constexpr int D = 3;                                      // steps in flight
-    __shared__ f32x4 red[W][64];
+    constexpr int W = ROWS_WAVES, D = ROWS_STEPS;
+    __shared__ f32x4 sums[64];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4;
-    const int KS = (K + GW_KSTEP - 1) / GW_KSTEP, s_begin = wv * steps_per_wave, s_end = min(KS, s_begin + steps_per_wave);
+    const int KS = (K + GW_KSTEP - 1) / GW_KSTEP;
     const int n_tiles = (N + 15) >> 4;
     const uint8_t* wbase = wp + (int64_t)blockIdx.x * GW_TILE_BYTES;
     // rows past the last and columns past K read as zeros without a fetch: their offsets lie behind the buffer's end
@@ -1249,63 +1254,60 @@ __global__ __launch_bounds__(64 * W) void w8a16_rows_kernel(
     constexpr int NOWHERE = 0x7ffff000;
     const int xrow = r < M ? r * K * 2 + 32 * g : NOWHERE;
     u32x4 wreg[D], xreg[D][2];
-    auto load = [&](auto setc, int s) {
-        constexpr int S = decltype(setc)::value;
-        const int sc = min(s, s_end - 1);
-        wreg[S] = gw_stream_load<u32x4>(wbase + (int64_t)sc * n_tiles * GW_TILE_BYTES + lane * 16);
+    auto load = [&](int s0) {                                 // steps past the last: the last one again, not used
+        static_for<D>([&](auto dc) {
+            constexpr int S = decltype(dc)::value;
+            const int sc = min(s0 + S, KS - 1);
+            wreg[S] = gw_stream_load<u32x4>(wbase + (int64_t)sc * n_tiles * GW_TILE_BYTES + lane * 16);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const bool in = !KTAIL || sc * GW_KSTEP + 16 * g + 8 * u < K;
-            xreg[S][u] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, in ? xrow + 16 * u : NOWHERE, sc * (2 * GW_KSTEP), 0);
-        }
+            for (int u = 0; u < 2; ++u) {
+                const bool in = !KTAIL || sc * GW_KSTEP + 16 * g + 8 * u < K;
+                xreg[S][u] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, in ? xrow + 16 * u : NOWHERE, sc * (2 * GW_KSTEP), 0);
+            }
+        });
     };
     f32x4 acc = (f32x4)(0.f);
-    auto step = [&](auto jc, int s) {
-        constexpr int J = decltype(jc)::value;
+    load(wv * D);
+    for (int turn = 0, s0 = 0;; ++turn, s0 += D) {            // the same in every wave: steps s0 .. s0 + D - 1 are wave turn % W's
+        if (wv == turn % W) {
+            if (turn > 0) acc = sums[lane];
+            static_for<D>([&](auto dc) {
+                constexpr int S = decltype(dc)::value;
+                if (s0 + S < KS) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-            acc = T::mfma16(dequant8<T>(wreg[J][2 * u], wreg[J][2 * u + 1]), bitcast<vec8>(xreg[J][u]), acc);
-        __builtin_amdgcn_sched_barrier(0);                    // the set is free: all of it has been used
-        load(jc, s + D);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    if (s_begin < s_end) {
-        static_for<D>([&](auto dc) { load(dc, s_begin + decltype(dc)::value); });
-        int s = s_begin;
-        for (; s + D <= s_end; s += D) static_for<D>([&](auto jc) { step(jc, s + decltype(jc)::value); });
-        static_for<D - 1>([&](auto jc) {
-            if (s + decltype(jc)::value < s_end) step(jc, s + decltype(jc)::value);
-        });
+                    for (int u = 0; u < 2; ++u)
+                        acc = T::mfma16(dequant8<T>(wreg[S][2 * u], wreg[S][2 * u + 1]), bitcast<vec8>(xreg[S][u]), acc);
+                }
+            });
+            if (s0 + D >= KS) break;
+            sums[lane] = acc;
+            if (s0 + W * D < KS) load(s0 + W * D);
+        } else if (s0 + D >= KS) {
+            return;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
     }
-    red[wv][lane] = acc;
-    __syncthreads();
-    if (wv != 0) return;
-    f32x4 sum = red[0][lane];                                 // the waves' parts in order
-#pragma unroll
-    for (int w = 1; w < W; ++w) sum += red[w][lane];
     const int n = 16 * blockIdx.x + 4 * g;
     if (r >= M || n >= N) return;
-    if (gated) store_gated<T>(y, bias, scale, r, n, N, sum);
-    else store4<T>(y, bias, residual, scale, (int64_t)r * N, n, N, sum);
+    if (gated) store_gated<T>(y, bias, scale, r, n, N, acc);
+    else store4<T>(y, bias, residual, scale, (int64_t)r * N, n, N, acc);
 }
 
 // Where the other kernel does not cut K (its parts are summed by what follows, which the reduction then carries: 6144 x 4096 at 8 rows 10.0
-// | 12.1, 4096 x 14336 15.0 | 18.2) and the lanes' own reads of the rows stay few.  us, the other kernel | this one: 4 rows 16384 x
-// 1024 6.8 | 5.9, 24576 x 1536 10.1 | 13.6; 8 rows 8192 x 1472 7.9 | 7.1; 16 rows 6144 x 1472 7.8 | 8.3, 16384 x 1024 6.9 | 7.5, 32768 x
-// 512 6.4 | 11.1.
-bool use_rows(const GemmPlan& p, int m, int n, int k) {
-    const int64_t tiles = (n + 15) / 16, steps = (k + GW_KSTEP - 1) / GW_KSTEP;
-    return m <= 16 && p.split_k == 1 && k < (1 << 24) && tiles * steps * (m + 4) <= 160000;   // K: 32-bit offsets
-}
+// us there, 12.1 on eight waves of a workgroup; so K has fewer than 24 steps) and the lanes' own reads of the rows stay few: two workgroups
+// a compute unit, three for up to 8 rows.  us, the other kernel | this one: 8 rows 8192 x 512 4.6 | 4.3, 12288 x 512 4.9 | 5.0, 12288 x 1472
+// 8.2 | 7.6, 16384 x 512 5.0 | 5.8, 16384 x 1472 8.7 | 9.2; 16 rows 8192 x 512 4.7 | 5.0, 8192 x 1472 8.0 | 7.2, 10240 x 512 4.8 | 6.0, 10240 x
+// 1472 8.1 | 8.6.
+bool use_rows(const GemmPlan& p, int m, int n) { return m <= 16 && p.split_k == 1 && (n + 15) / 16 <= (m <= 8 ? 768 : 512); }
 template <typename T>
 void launch_rows(void* y, const void* x, const uint8_t* wp, const float* scale, const void* bias, const void* residual, int m, int n,
                  int k, int gated, hipStream_t st) {
-    const int steps = (k + GW_KSTEP - 1) / GW_KSTEP;
-#define W8R(KT, W)                                                                                               \
-    hipLaunchKernelGGL((w8a16_rows_kernel<T, KT, W>), dim3((n + 15) / 16), dim3(64 * W), 0, st, (uint16_t*)y, (const uint16_t*)x, wp, \
-                       scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, (steps + W - 1) / W, gated)
-    if (k % GW_KSTEP) W8R(true, 8);
-    else W8R(false, 8);
+#define W8R(KT)                                                                                                  \
+    hipLaunchKernelGGL((w8a16_rows_kernel<T, KT>), dim3((n + 15) / 16), dim3(64 * ROWS_WAVES), 0, st, (uint16_t*)y, \
+                       (const uint16_t*)x, wp, scale, (const uint16_t*)bias, (const uint16_t*)residual, m, n, k, gated)
+    if (k % GW_KSTEP) W8R(true);
+    else W8R(false);
 #undef W8R
 }
 
@@ -1375,7 +1377,7 @@ void launch_skinny(const GemmPlan& p, void* y, float* partial, const void* x, co
 #define GW4_W4_BY_GROUP(MTV, WV)                                                                                 \
     { if (w4_group == 0) GW4_LAUNCH_W4(MTV, WV, 0); else if (w4_group == 64) GW4_LAUNCH_W4(MTV, WV, 64);          \
       else GW4_LAUNCH_W4(MTV, WV, 128); }
-    if (w4_group < 0 && use_rows(p, m, n, k)) launch_rows<T>(y, x, wp, scale, bias, residual, m, n, k, gated, st);
+    if (w4_group < 0 && use_rows(p, m, n)) launch_rows<T>(y, x, wp, scale, bias, residual, m, n, k, gated, st);
     else if (w4_group >= 0) {
         if (p.mt == 1) GW4_W4_BY_GROUP(1, 4)
         else if (p.mt == 2) GW4_W4_BY_GROUP(2, 4)

@@ -1292,6 +1292,24 @@ def test_w8a16_few_rows_and_channels(dtype, m, n, k):
     test_w8a16_many_rows(dtype, m, n, k, False, True)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k", [(64, 200), (512, 1376), (4096, 1024), (8192, 1472), (12288, 520), (16384, 1024)])
+def test_w8a16_a_row_does_not_depend_on_the_rows_beside_it(dtype, n, k):
+    """K that is not cut between workgroups: up to 32 rows every kernel sums a row's products in one chain in the order of K, so the
+    same row has the same bits in a call of any of these sizes (1 to 3 turns of the waves, short last ones, both sides of the line)."""
+    assert ops._lib.load().mf_w8a16_workspace_bytes(32, n, k) == 0
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    w = torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+    packed = ops.pack_w8a16(w, (torch.rand(n, generator=g, device="cuda") + 0.5) * (k ** -0.5 / 73))
+    gated = ops.pack_w8a16_gated(w, packed.scale, "halves")
+    x = torch.randn(32, k, generator=g, device="cuda").to(dtype)
+    y, z = ops.w8a16_linear(x, packed), ops.w8a16_gated_linear(x, gated)
+    for m in (1, 4, 8, 9, 16, 17):
+        assert torch.equal(ops.w8a16_linear(x[:m], packed), y[:m])
+        assert torch.equal(ops.w8a16_gated_linear(x[:m], gated), z[:m])
+
+
 TAILS = [(1025, 16400, 1088), (1056, 16656, 1024), (1057, 16400, 1152), (1088, 16416, 1024), (1300, 24576, 1536)]
 
 
