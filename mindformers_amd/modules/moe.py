@@ -258,7 +258,7 @@ class MoELayer(nn.Module):
         rows = quantized[0] if quantized is not None else x
         if early and self.experts.reads_sources(rows, routing_map.numel()):
             sources, ps, row_map, counts, offsets = ops.moe_sort(routing_map, self.num_experts,
-                                                                 None if quantized is None else quantized[1])
+                                                                 None if quantized is None else quantized[1], tokens=rows.shape[0])
             y = self.experts(rows, counts, offsets=offsets, row_scale=ps, out_dtype=x.dtype, sources=sources)
         elif quantized is not None:
             px, ps, row_map, counts, offsets = ops.moe_permute_int8(*quantized, routing_map, self.num_experts)

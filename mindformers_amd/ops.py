@@ -1272,12 +1272,14 @@ def moe_permute_int8(xq, x_scale, expert_index, n_experts):
     return px, ps, row_map, counts, offsets
 
 
-def moe_sort(expert_index, n_experts, x_scale=None):
+def moe_sort(expert_index, n_experts, x_scale=None, tokens=None):
     """``moe_permute`` without the copies: returns (sources int32 [T*k], the token of each permuted row, permuted_scale (of
-    ``x_scale`` fp32 [T]) or None, row_map, counts, offsets), for the grouped GEMMs with ``sources``."""
+    ``x_scale`` fp32 [T]) or None, row_map, counts, offsets), for the grouped GEMMs with ``sources``.  ``tokens``: rows of the
+    tensor that they will name, refused where T is another number (the GEMMs would clamp to it)."""
     lib = _lib.load()
     dev = _dev_ok(expert_index, x_scale)
-    _need(expert_index.dtype == torch.int32 and expert_index.dim() == 2, "expert_index must be int32 [T, k]")
+    _need(expert_index.dtype == torch.int32 and expert_index.dim() == 2 and tokens in (None, expert_index.shape[0]),
+          "expert_index must be int32 [T, k]")
     t, k = expert_index.shape
     _need(x_scale is None or (x_scale.dtype == torch.float32 and x_scale.numel() == t), "x_scale must be fp32 [T]")
     maps = torch.empty(2, t * k, dtype=torch.int32, device=dev)

@@ -1309,3 +1309,32 @@ def test_moe_experts_with_a_forward_or_hooks_of_their_own_see_the_tokens_type():
     net.experts = Experts(8, cfg, act_quant="per_token").quantize_from_float(w1, w2)
     assert torch.equal(net(x), ref)
     assert seen == [BF] * 3
+
+
+def _prompt_sized_moe(act_quant, tokens=300):
+    """A small layer with enough rows an expert for the grouped GEMMs that read them through the sort's index, and its tokens."""
+    from mindformers_amd.modules import MoELayer, QuantGroupedMLP
+    from mindformers_amd.transformer_config import TransformerConfig
+    cfg = TransformerConfig(num_layers=1, num_attention_heads=8, hidden_size=128, hidden_act="silu", num_moe_experts=8,
+                            moe_router_topk=2, shared_expert_num=0, moe_shared_expert_intermediate_size=None,
+                            moe_ffn_hidden_size=96, moe_router_group_topk=2, moe_router_num_groups=4, add_bias_linear=False,
+                            gated_linear_unit=True, compute_dtype="bfloat16", params_dtype="bfloat16",
+                            moe_router_dtype="bfloat16", moe_router_enable_expert_bias=True,
+                            moe_router_score_function="sigmoid")
+    torch.manual_seed(11)
+    net = MoELayer(cfg)
+    net.router.weight.data.normal_(0, 0.3)
+    w1, w2 = torch.randn(8, 128, 192, device="cuda") * 0.2, torch.randn(8, 96, 128, device="cuda") * 0.2
+    net.experts = QuantGroupedMLP(8, cfg, act_quant=act_quant).quantize_from_float(w1, w2)
+    return net, torch.randn(tokens, 128, device="cuda").to(BF)
+
+
+@pytest.mark.parametrize("act_quant", [None, "per_token"])
+def test_moe_layer_refuses_a_routing_of_another_number_of_tokens(act_quant):
+    """Also where the experts read the tokens through the sort's index, which the GEMMs would clamp to the rows that there are."""
+    net, x = _prompt_sized_moe(act_quant)
+    router = net.router.forward
+    for rows in (slice(0, 290), slice(None)):
+        net.router.forward = lambda h: tuple(t[rows].contiguous() for t in router(torch.cat((h, h[:7]))))
+        with pytest.raises(ValueError, match="expert_index must be int32"):
+            net(x)
