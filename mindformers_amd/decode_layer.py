@@ -193,7 +193,7 @@ class QuantDecodeLayer(nn.Module):
             h, n2x, n2s = ops.w8a8_linear_add_rmsnorm_quant(aq, a_s, self._packed["wo"], x, self.ffn_norm, self.eps,
                                                             self.fc1_smooth, bias=self.wo_b)
             fc1 = self._packed.get("fc1")
-            if self.fc1_b is None and ops.w8a8_gated_fused(n2s.numel(), fc1):
+            if self.fc1_b is None and self._own("_linear") and ops.w8a8_gated_fused(n2s.numel(), fc1):
                 actq = ops.dynamic_quant(ops.w8a8_gated_linear(n2x, n2s, fc1, self.dtype), self.fc2_smooth, tiled=True)
             else:
                 actq = ops.silu_mul_dynamic_quant(self._linear(None, "fc1", quantized=(n2x, n2s)), self.fc2_smooth,
@@ -218,6 +218,11 @@ class QuantDecodeLayer(nn.Module):
     @staticmethod
     def _chain(out, next_norm):
         return out if next_norm is None else (out, ops.rms_norm(out, next_norm[0], next_norm[1]))
+
+    def _own(self, *names):
+        """Whether these methods are the ones below, of no subclass and no instance: only then may their work go another way."""
+        cls, d = type(self), self.__dict__
+        return all(name not in d and getattr(cls, name) is getattr(QuantDecodeLayer, name) for name in names)
 
     def _plain(self):
         """Whether a decode step may run as one native call: no bias but the fused projection's, and nothing that a subclass or an

@@ -360,3 +360,38 @@ def test_a_native_decode_step_has_the_bits_of_the_separate_operators(dtype, hidd
         if bad_tb is not None:
             with pytest.raises(ValueError):
                 steps(bad_x, bad_tb)
+
+
+def _step_inputs(batch, hidden, nkv, d, dtype, gen):
+    """Operands of a decode step of sequences of 5 to 30 tokens in caches of 16-token blocks."""
+    lens = torch.arange(batch, dtype=torch.int32) % 26 + 5
+    tables = torch.arange(2 * batch, dtype=torch.int32).view(batch, 2)
+    slots = tables.gather(1, ((lens - 1) // 16).long()[:, None])[:, 0] * 16 + (lens - 1) % 16
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(dtype)
+    return (rand(batch, hidden), rand(2 * batch, 16, nkv, d), rand(2 * batch, 16, nkv, d), tables.cuda(), lens.cuda(),
+            slots.to(torch.int32).cuda(), rand(batch, d), rand(batch, d))
+
+
+def test_a_w8a8_layer_asks_a_projection_of_its_own():
+    """A layer whose ``_linear`` is a subclass's or an instance's is asked for the gate/up projection at every number of rows, also where
+    the layer's own is fused with the activation behind it."""
+    from mindformers_amd import ops, synthetic
+    from mindformers_amd.decode_layer import QuantDecodeLayer
+
+    class Asked(QuantDecodeLayer):
+        def _linear(self, x, name, **kw):
+            seen.append(name)
+            return super()._linear(x, name, **kw)
+
+    gen, args = torch.Generator(device="cuda"), (320, 4, 2, 64, 4112, 1e-5, torch.bfloat16)
+    for rows in (40, 129):
+        outs, seen = [], []
+        for cls in (QuantDecodeLayer, QuantDecodeLayer, Asked):
+            gen.manual_seed(rows)
+            layer = synthetic.fill_layer(cls(*args, act_quant=True), gen)
+            if len(outs) == 1:
+                layer._linear = lambda x, name, **kw: (seen.append(name), QuantDecodeLayer._linear(layer, x, name, **kw))[1]
+            outs.append(layer(*_step_inputs(rows, 320, 2, 64, torch.bfloat16, gen)))
+            fused = ops.w8a8_gated_fused(rows, layer._packed["fc1"])
+        assert fused == (rows == 129) and seen == ["fc1", "fc2"] * 2
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
