@@ -220,15 +220,19 @@ class QuantDecodeLayer(nn.Module):
         return out if next_norm is None else (out, ops.rms_norm(out, next_norm[0], next_norm[1]))
 
     def _own(self, *names):
-        """Whether these methods are the ones below, of no subclass and no instance: only then may their work go another way."""
+        """Whether these methods are the ones defined here, and no subclass's or instance's nor put in their place on the class: only
+        then may their work go another way."""
         cls, d = type(self), self.__dict__
-        return all(name not in d and getattr(cls, name) is getattr(QuantDecodeLayer, name) for name in names)
+        for name in names:
+            if name in d or getattr(cls, name) is not _METHODS[name]:
+                return False
+        return True
 
     def _plain(self):
-        """Whether a decode step may run as one native call: no bias but the fused projection's, and nothing that a subclass or an
-        instance has in place of the operators' order."""
+        """Whether a decode step may run as one native call: no bias but the fused projection's, and nothing in place of the
+        operators' order."""
         d, buffers = self.__dict__, self._buffers
-        if type(self) is not QuantDecodeLayer or self.head_dim % 16 or "attend" in d or "gate_up" in d or "_linear" in d or "_chain" in d:
+        if type(self) is not QuantDecodeLayer or self.head_dim % 16 or not self._own("attend", "gate_up", "_linear", "_chain"):
             return False
         if buffers.get("attn_norm") is None or buffers.get("ffn_norm") is None:
             return False
@@ -245,3 +249,6 @@ class QuantDecodeLayer(nn.Module):
 
     def weight_bytes(self):
         return sum(getattr(self, f"{n}_w").numel() for n in self.NAMES)
+
+
+_METHODS = {name: getattr(QuantDecodeLayer, name) for name in ("attend", "gate_up", "_linear", "_chain")}

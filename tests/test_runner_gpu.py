@@ -395,3 +395,20 @@ def test_a_w8a8_layer_asks_a_projection_of_its_own():
             fused = ops.w8a8_gated_fused(rows, layer._packed["fc1"])
         assert fused == (rows == 129) and seen == ["fc1", "fc2"] * 2
         assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("name", ["attend", "gate_up", "_linear", "_chain"])
+def test_a_method_put_on_the_layer_class_is_asked(name, monkeypatch):
+    """A method of QuantDecodeLayer that is replaced on the class itself is asked in a decode step, with the same bits."""
+    from mindformers_amd import synthetic
+    from mindformers_amd.decode_layer import QuantDecodeLayer
+    gen, seen = torch.Generator(device="cuda"), []
+    gen.manual_seed(5)
+    layer = synthetic.fill_layer(QuantDecodeLayer(512, 8, 2, 64, 1376, 1e-5, torch.float16), gen)
+    args = _step_inputs(4, 512, 2, 64, torch.float16, gen)
+    ref = layer(*args)
+    original = QuantDecodeLayer.__dict__[name]
+    call = original.__func__ if isinstance(original, staticmethod) else original
+    replaced = lambda *a, **kw: (seen.append(name), call(*a, **kw))[1]
+    monkeypatch.setattr(QuantDecodeLayer, name, staticmethod(replaced) if call is not original else replaced)
+    assert torch.equal(layer(*args), ref) and seen
