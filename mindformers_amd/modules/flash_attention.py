@@ -115,10 +115,10 @@ class FlashAttention(nn.Module):
         return ops.q_starts_from_actual_seq_len(torch.as_tensor(actual_seq_qlen, device=query.device), query.shape[0])
 
     def takes_key_parts(self):
-        """Whether ``prefill_shared_rope`` stands for ``forward``: not where a subclass or an instance brings its own ``forward``,
-        nor under forward hooks, which are shown the joined keys."""
+        """Whether ``prefill_shared_rope`` stands for ``forward``: not where a subclass, an instance or a replaced method brings its
+        own ``forward``, nor under forward hooks, which are shown the joined keys."""
         hooks = torch.nn.modules.module
-        return type(self).forward is FlashAttention.forward and "forward" not in self.__dict__ and not (
+        return type(self).forward is _FORWARD and "forward" not in self.__dict__ and not (
             self._forward_hooks or self._forward_pre_hooks or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
 
     def prefill_shared_rope(self, query, key_nope, key_rope, value, actual_seq_qlen=None, actual_seq_kvlen=None):
@@ -127,3 +127,6 @@ class FlashAttention(nn.Module):
         return ops.causal_attention_shared_rope(query, key_nope, key_rope, value,
                                                 self._starts(query, actual_seq_qlen, actual_seq_kvlen), self.head_num,
                                                 self.scale_value)
+
+
+_FORWARD = FlashAttention.forward

@@ -1338,3 +1338,18 @@ def test_moe_layer_refuses_a_routing_of_another_number_of_tokens(act_quant):
         net.router.forward = lambda h: tuple(t[rows].contiguous() for t in router(torch.cat((h, h[:7]))))
         with pytest.raises(ValueError, match="expert_index must be int32"):
             net(x)
+
+
+def test_mla_prefill_asks_a_forward_put_on_the_attention_class(monkeypatch):
+    """A ``forward`` that is replaced on FlashAttention itself gets the joined keys too."""
+    from mindformers_amd.modules import FlashAttention
+    rng = np.random.default_rng(6)
+    net = _mla_module_and_params(rng, 512, 4, None, rope_type="rope")[0]
+    t, seen = 33, []
+    x = dev(rounded(rng.normal(size=(t, 512)), BF), BF)
+    cos, sin = net.rotary_pos_emb.get_cos_sin_for_decode(torch.arange(t).cuda())
+    args = dict(rotary_pos_cos=cos, rotary_pos_sin=sin, actual_seq_qlen=torch.tensor([t], dtype=torch.int32, device="cuda"))
+    ref, original = net(x, None, **args), FlashAttention.forward
+    monkeypatch.setattr(FlashAttention, "forward", lambda self, q, k, *a, **kw: (
+        seen.append(tuple(k.shape)), original(self, q, k, *a, **kw))[1])
+    assert torch.equal(net(x, None, **args), ref) and seen == [(t, 4 * 192)]
