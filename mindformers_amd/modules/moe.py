@@ -209,13 +209,16 @@ class QuantGroupedMLP(nn.Module):
     construct = forward
 
     def takes_quantized_rows(self):
-        """Whether the rows may arrive as the integers of ``quantize_tokens``: not where a subclass or an instance brings its own
-        ``forward`` or quantisation (it expects the tokens' type and the three arguments that it names), nor under forward
-        hooks, which are shown the rows."""
-        own = type(self).forward is QuantGroupedMLP.forward and type(self)._quant is QuantGroupedMLP._quant
+        """Whether the rows may arrive as the integers of ``quantize_tokens`` or as an index of the tokens: not where a subclass, an
+        instance or a replaced method brings its own ``forward`` or quantisation (it expects the permuted rows, of the tokens' type,
+        and the three arguments that it names), nor under forward hooks, which are shown the rows."""
+        own = type(self).forward is _EXPERTS_FORWARD and type(self)._quant is _EXPERTS_QUANT
         hooks = torch.nn.modules.module
         return own and "forward" not in self.__dict__ and not (
             self._forward_hooks or self._forward_pre_hooks or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
+
+
+_EXPERTS_FORWARD, _EXPERTS_QUANT = QuantGroupedMLP.forward, QuantGroupedMLP._quant
 
 
 class SharedExpertMLP(MLP):

@@ -1353,3 +1353,14 @@ def test_mla_prefill_asks_a_forward_put_on_the_attention_class(monkeypatch):
     monkeypatch.setattr(FlashAttention, "forward", lambda self, q, k, *a, **kw: (
         seen.append(tuple(k.shape)), original(self, q, k, *a, **kw))[1])
     assert torch.equal(net(x, None, **args), ref) and seen == [(t, 4 * 192)]
+
+
+@pytest.mark.parametrize("act_quant", [None, "per_token"])
+def test_moe_layer_asks_a_forward_put_on_the_experts_class(act_quant, monkeypatch):
+    """A ``forward`` that is replaced on QuantGroupedMLP itself gets the permuted 16-bit rows."""
+    from mindformers_amd.modules import QuantGroupedMLP
+    net, x = _prompt_sized_moe(act_quant)
+    ref, original, seen = net(x), QuantGroupedMLP.forward, []
+    monkeypatch.setattr(QuantGroupedMLP, "forward", lambda self, h, *a, **kw: (
+        seen.append((tuple(h.shape), h.dtype, kw.get("sources"))), original(self, h, *a, **kw))[1])
+    assert torch.equal(net(x), ref) and seen == [((600, 128), BF, None)]
