@@ -115,10 +115,10 @@ class FlashAttention(nn.Module):
         return ops.q_starts_from_actual_seq_len(torch.as_tensor(actual_seq_qlen, device=query.device), query.shape[0])
 
     def takes_key_parts(self):
-        """Whether ``prefill_shared_rope`` stands for ``forward``: not where a subclass, an instance or a replaced method brings its
-        own ``forward``, nor under forward hooks, which are shown the joined keys."""
+        """Whether ``prefill_shared_rope`` stands for ``forward``: not where that would write the keys into a cache (no latent one), a
+        subclass, an instance or a replaced method brings its own ``forward``, nor under forward hooks, which are shown the joined keys."""
         hooks = torch.nn.modules.module
-        return type(self).forward is _FORWARD and "forward" not in self.__dict__ and not (
+        return self.use_multi_latent_attention and type(self).forward is _FORWARD and "forward" not in self.__dict__ and not (
             self._forward_hooks or self._forward_pre_hooks or hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
 
     def prefill_shared_rope(self, query, key_nope, key_rope, value, actual_seq_qlen=None, actual_seq_kvlen=None):

@@ -1364,3 +1364,21 @@ def test_moe_layer_asks_a_forward_put_on_the_experts_class(act_quant, monkeypatc
     monkeypatch.setattr(QuantGroupedMLP, "forward", lambda self, h, *a, **kw: (
         seen.append((tuple(h.shape), h.dtype, kw.get("sources"))), original(self, h, *a, **kw))[1])
     assert torch.equal(net(x), ref) and seen == [((600, 128), BF, None)]
+
+
+def test_mla_prefill_refuses_a_core_attention_without_a_latent_cache():
+    """A core attention that writes keys and values of its own into the caches does not take a latent one."""
+    from mindformers_amd.modules import FlashAttention
+    net = _mla_module_and_params(np.random.default_rng(8), 512, 4, None, rope_type="rope")[0]
+    t = 6
+    cos, sin = net.rotary_pos_emb.get_cos_sin_for_decode(torch.arange(t).cuda())
+    args = dict(rotary_pos_cos=cos, rotary_pos_sin=sin, actual_seq_qlen=torch.tensor([t], dtype=torch.int32, device="cuda"),
+                slot_mapping=torch.arange(t, dtype=torch.int32, device="cuda"),
+                key_cache=torch.zeros(2, 16, 1, 576, dtype=BF, device="cuda"))
+    x = torch.ones(t, 512, dtype=BF, device="cuda")
+    net(x, None, **args)
+    core = net.core_attention
+    net.core_attention = FlashAttention(core.head_num, core.hidden_size_per_attention_head, core.kv_head_num,
+                                        scale_value=core.scale_value)
+    with pytest.raises(ValueError):
+        net(x, None, **args)
