@@ -1392,7 +1392,7 @@ def decode_layer_step(x, normed, attn_norm, ffn_norm, next_norm, weights, qkv_bi
     if qkv_bias is not None and (qkv_bias.dtype != dt or qkv_bias.numel() != nqkv):
         return None
     gamma, next_eps = (None, 0.0) if next_norm is None else (next_norm[0], next_norm[1])
-    if gamma is not None and gamma.numel() != hidden:
+    if next_norm is not None and (gamma is None or gamma.numel() != hidden):
         return None
     for t in (x, normed, attn_norm, ffn_norm, gamma, qkv_bias, cos, sin, key_cache, value_cache, slots, tables, lens):
         if t is not None and not (type(t) is torch.Tensor and t.get_device() == dev and t.is_contiguous()):

@@ -412,3 +412,12 @@ def test_a_method_put_on_the_layer_class_is_asked(name, monkeypatch):
     replaced = lambda *a, **kw: (seen.append(name), call(*a, **kw))[1]
     monkeypatch.setattr(QuantDecodeLayer, name, staticmethod(replaced) if call is not original else replaced)
     assert torch.equal(layer(*args), ref) and seen
+
+
+def test_a_decode_step_refuses_a_next_norm_without_a_gamma():
+    from mindformers_amd import synthetic
+    from mindformers_amd.decode_layer import QuantDecodeLayer
+    gen = torch.Generator(device="cuda")
+    layer = synthetic.fill_layer(QuantDecodeLayer(512, 8, 2, 64, 1376, 1e-5, torch.float16), gen)
+    with pytest.raises(AttributeError):
+        layer(*_step_inputs(4, 512, 2, 64, torch.float16, gen), next_norm=(None, 1e-5))
