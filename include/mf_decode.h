@@ -647,6 +647,7 @@ typedef struct {
     int64_t scratch_bytes, workspace_bytes, attn_workspace_bytes;
     double eps, next_eps, scale;
 } mf_decode_layer_args;
+size_t mf_decode_layer_args_bytes(void);                     /* what this library takes the struct to be */
 size_t mf_decode_layer_scratch_bytes(int rows, int hidden, int n_heads, int n_kv_heads, int head_dim, int ffn);
 size_t mf_decode_layer_workspace_bytes(int rows, int hidden, int n_heads, int n_kv_heads, int head_dim, int ffn);
 int mf_decode_layer_step(const mf_decode_layer_args* args);

@@ -4,6 +4,7 @@ The library is the product: if it has not been built, loading fails loudly — t
 """
 import ctypes
 import os
+import struct
 
 import torch
 
@@ -98,11 +99,24 @@ SIGNATURES = {
     "mf_grouped_w8a16_gemm_silu_mul_sources": (_I, [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "mf_grouped_w8a8_gemm_silu_mul_sources": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "mf_moe_sort": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
+    "mf_decode_layer_args_bytes": (_Z, []),
     "mf_decode_layer_scratch_bytes": (_Z, [_I] * 6),
     "mf_decode_layer_workspace_bytes": (_Z, [_I] * 6),
     "mf_decode_layer_step": (_I, [ctypes.c_char_p]),
     "mf_moe_unpermute": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
 }
+
+# mf_decode_layer_args, field by field: pointers, int64, doubles
+DECODE_LAYER_FIELDS = {
+    "P": ("x", "normed", "attn_gamma", "ffn_gamma", "next_gamma", "qkv_w", "wo_w", "fc1_w", "fc2_w", "qkv_scale", "wo_scale",
+          "fc1_scale", "fc2_scale", "qkv_bias", "cos", "sin", "key_cache", "value_cache", "slot_mapping", "block_tables",
+          "context_lens", "out", "norm_out", "scratch", "workspace", "attn_workspace", "stream"),
+    "q": ("rows", "hidden", "n_heads", "n_kv_heads", "head_dim", "ffn", "block_size", "num_blocks", "max_blocks", "dtype",
+          "table_dtype", "attn_gamma_dtype", "ffn_gamma_dtype", "next_gamma_dtype", "scratch_bytes", "workspace_bytes",
+          "attn_workspace_bytes"),
+    "d": ("eps", "next_eps", "scale"),
+}
+DECODE_LAYER_ARGS = struct.Struct("@" + "".join(f"{len(names)}{kind}" for kind, names in DECODE_LAYER_FIELDS.items()))
 
 _lib = None
 
@@ -125,6 +139,9 @@ def load():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    if lib.mf_decode_layer_args_bytes() != DECODE_LAYER_ARGS.size:    # a library of another state of the header
+        raise ImportError(f"{LIB_PATH} takes mf_decode_layer_args of {lib.mf_decode_layer_args_bytes()} bytes, this package packs "
+                          f"{DECODE_LAYER_ARGS.size}: build it again (python mindformers_amd/build.py)")
     _lib = lib
     return lib
 

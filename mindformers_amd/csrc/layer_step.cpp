@@ -24,6 +24,8 @@ struct Scratch {
 };
 }  // namespace
 
+extern "C" size_t mf_decode_layer_args_bytes(void) { return sizeof(mf_decode_layer_args); }
+
 extern "C" size_t mf_decode_layer_scratch_bytes(int rows, int hidden, int n_heads, int n_kv_heads, int head_dim, int ffn) {
     if (rows <= 0 || hidden <= 0 || n_heads <= 0 || n_kv_heads <= 0 || head_dim <= 0 || ffn <= 0) return 0;
     return Scratch(rows, hidden, (int64_t)n_heads * head_dim, (int64_t)n_kv_heads * head_dim, ffn).end;

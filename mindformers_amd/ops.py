@@ -5,12 +5,11 @@ not expect can fault the GPU), allocates the output with torch (device-memory pl
 the kernel on torch's current stream.  Nothing is computed in Python.
 """
 import math
-import struct
 
 import torch
 
 from . import _lib
-from ._lib import check, dtype_code, ptr, stream_ptr
+from ._lib import DECODE_LAYER_ARGS, check, dtype_code, ptr, stream_ptr
 
 _ACT = (torch.bfloat16, torch.float16)
 _workspaces = {}
@@ -1359,9 +1358,6 @@ def grouped_w8a8_linear(xq, x_scale, w, offsets, out_dtype=torch.bfloat16, retur
     return (y, acc) if return_acc else y
 
 
-_STEP = struct.Struct("@27P17q3d")                            # mf_decode_layer_args
-
-
 def decode_layer_step(x, normed, attn_norm, ffn_norm, next_norm, weights, qkv_bias, cos, sin, key_cache, value_cache, slots, tables,
                       lens, n_heads, n_kv_heads, head_dim, eps, scale):
     """A decode step of a weight-only layer in one native call, or None where an operand is not of the plain form that it takes (the
@@ -1408,7 +1404,7 @@ def decode_layer_step(x, normed, attn_norm, ffn_norm, next_norm, weights, qkv_bi
     scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=device)
     out = torch.empty_like(x)
     norm_out = None if gamma is None else torch.empty_like(x)
-    args = _STEP.pack(
+    args = DECODE_LAYER_ARGS.pack(                            # in the order of _lib.DECODE_LAYER_FIELDS
         x.data_ptr(), 0 if normed is None else normed.data_ptr(), attn_norm.data_ptr(), ffn_norm.data_ptr(),
         0 if gamma is None else gamma.data_ptr(), qkv.packed.data_ptr(), wo.packed.data_ptr(), fc1.packed.data_ptr(),
         fc2.packed.data_ptr(), qkv.scale.data_ptr(), wo.scale.data_ptr(), fc1.scale.data_ptr(), fc2.scale.data_ptr(),

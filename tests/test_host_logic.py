@@ -44,6 +44,24 @@ def test_library_exports_every_declared_symbol():
     assert loaded.mf_w8a16_workspace_bytes(0, 10, 16) == 0
 
 
+def test_the_decode_step_packs_the_struct_that_the_header_declares(monkeypatch):
+    """Names and kinds of mf_decode_layer_args in their order, its size on both sides, and a library with another one refused."""
+    from mindformers_amd import _lib
+    text = open(os.path.join(ROOT, "include", "mf_decode.h")).read()
+    body = re.search(r"typedef struct \{([^}]*)\} mf_decode_layer_args;", text).group(1)
+    fields = []
+    for decl in filter(None, (d.strip() for d in body.split(";"))):
+        kind = "P" if "*" in decl else {"int64_t": "q", "double": "d"}[decl.split()[0]]
+        fields += [(kind, name) for name in re.findall(r"(\w+)\s*(?:,|$)", decl)]
+    assert fields == [(kind, name) for kind, names in _lib.DECODE_LAYER_FIELDS.items() for name in names]
+    lib = _lib.load()
+    assert lib.mf_decode_layer_args_bytes() == _lib.DECODE_LAYER_ARGS.size == 8 * len(fields)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "DECODE_LAYER_ARGS", _lib.struct.Struct("@28P17q3d"))
+    with pytest.raises(ImportError, match="build it again"):
+        _lib.load()
+
+
 def test_argument_errors_are_reported_without_a_gpu():
     from mindformers_amd import _lib
     lib = _lib.load()
