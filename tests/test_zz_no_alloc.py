@@ -28,12 +28,13 @@ def _both(lib, rng, b, nh, nkv, d, bs, lens, max_blocks, dtype):
           "mf_paged_attention_decode")
     out = torch.full((b, nh * d), -5.0, dtype=dtype, device="cuda")
     torch.cuda.synchronize()
-    before = torch.cuda.memory_allocated()
+    made = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]      # all that were ever made: what is freed meanwhile does not count
+    before = made()
     check(lib.mf_paged_attention_decode_static(ptr(out), ptr(q), ptr(kc), ptr(vc), ptr(tb), ptr(ln), b, nh, nkv, d, bs,
                                                max_blocks, nb, scale, 0, dtype_code(dtype), st),
           "mf_paged_attention_decode_static")
     torch.cuda.synchronize()
-    assert torch.cuda.memory_allocated() == before
+    assert made() == before
     return out, ref, need
 
 
