@@ -111,8 +111,9 @@ inline bool tg_plan_tail(int m, int n, int steps, const TileCost& c, float* us, 
 // measured from there on and have to be 6 % shorter, about what the prices err by).  Nor does a plan all of whose tiles are cut along K: its parts are all resident too, and the model prices
 // parts that run at once too high (0.015 us each there, not c.part); against other kernels it counts a tenth less than 96 x 256 tiles would.
 // 96 x 256 | 128 x 256 in two parts: W8A16 777 x 4096 x 4096 44.0 | 37.6, 513 x 6144 x 4096 44.5 | 38.5, W8A8 448 x 5120 x 5120 29.8 |
-// 27.4.  Where only what is left over by whole rounds is cut, another shape has to be a fifth shorter.  96 x 192 where 96 x 256 would
-// leave a quarter of the units idle, and more of them are wanted (2025 x 2112 x 7168, 198 tiles of 96 x 256, would gain a seventh as well).
+// 27.4.  Where only what is left over by whole rounds is cut, another shape has to be a fifth shorter.  96 x 256 | 96 x 192 on shapes that
+// fill less than a round with either: W8A16 2025 x 2112 x 7168 75.3 | 64.0, 1042 x 4416 x 1600 23.2 | 20.7, 1216 x 3648 x 14336 138 |
+// 123, W8A8 2025 x 2112 x 7168 45.0 | 40.0, 3322 x 1312 x 1600 14.8 | 13.4 (102 of 102 shapes of 1040 to 4416 channels, by 6 to 24 %).
 inline TileGrid tg_plan(int m, int n, int steps, const TileCost& c, float* us) {
     const TileGrid g = tg_plan_rounds(m, n, steps, c, us);
     TileGrid t;
@@ -127,7 +128,6 @@ inline TileGrid tg_plan(int m, int n, int steps, const TileCost& c, float* us) {
         const float t = (all_cut ? 0.9f : 1.f) * (steps * s.step + s.fixed);
         if (tiles > 256 || t >= (s.nt == 4 ? least : 0.94f * least)) continue;
         if (s.nt != 4 && (steps < 24 || all_cut)) continue;
-        if (s.mt == 3 && s.nt == 3 && tiles_of(3, 4) > 192) continue;
         least = *us = t;
         if (!all_cut) best = {(m + 32 * s.mt - 1) / (32 * s.mt), (n + 64 * s.nt - 1) / (64 * s.nt), (int)tiles / 8 * 8, 1, steps, s.mt, s.nt, 0};
     }

@@ -140,9 +140,18 @@ def test_plans_of_the_shapes_that_the_96_row_tiles_are_tested_at():
     """Tiles of 96 rows where they fit the device at once: their number is not that of 128-row tiles, and nothing is cut along K."""
     from mindformers_amd import _lib
     lib, tiles8, tiles16 = _lib.load(), 3, 1
-    for (m, n, k), whole in {(1153, 4112, 1216): 221, (1048, 4096, 1088): 176, (2025, 2112, 7168): 198}.items():
+    for (m, n, k), whole in {(1153, 4112, 1216): 221, (1048, 4096, 1088): 176, (1300, 4608, 1600): 252}.items():
         assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, whole, 0, 1), (m, n, k)
     for (m, n, k), whole in {(1531, 3584, 3600): 224, (1300, 4608, 1040): 252, (1153, 4624, 1040): 247}.items():
+        assert _plan(lib.mf_w8a8_plan, m, n, k, 0) == (tiles8, whole, 0, 1), (m, n, k)
+
+
+def test_plans_that_fill_less_than_a_round_take_the_tiles_that_fill_more_of_it():
+    """96 x 192 where 96 x 256 would leave units idle, up to the last of them: the faster one at every shape measured."""
+    from mindformers_amd import _lib
+    lib, tiles8, tiles16 = _lib.load(), 3, 1
+    for (m, n, k), whole in {(2025, 2112, 7168): 242, (2665, 1600, 2560): 252, (1042, 4416, 1600): 253, (1216, 3648, 14336): 247}.items():
+        assert _plan(lib.mf_w8a16_plan, m, n, k) == (tiles16, whole, 0, 1), (m, n, k)
         assert _plan(lib.mf_w8a8_plan, m, n, k, 0) == (tiles8, whole, 0, 1), (m, n, k)
 
 

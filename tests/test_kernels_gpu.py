@@ -1265,7 +1265,7 @@ def test_w8a16_many_rows(dtype, m, n, k, bias, residual):
 @pytest.mark.parametrize("dtype,m,n,k", [
     (torch.bfloat16, 1153, 4112, 1216),    # 96-row tiles: one row and one 16-channel piece past whole ones, an odd number of k-steps
     (torch.float16, 1048, 4096, 1088),
-    (torch.bfloat16, 2025, 2112, 7168)])
+    (torch.bfloat16, 1300, 4608, 1600)])
 def test_w8a16_many_rows_on_96_row_tiles(dtype, m, n, k):
     """The same at shapes that take the lower tiles."""
     test_w8a16_many_rows(dtype, m, n, k, True, False)
@@ -1274,6 +1274,7 @@ def test_w8a16_many_rows_on_96_row_tiles(dtype, m, n, k):
 
 @pytest.mark.parametrize("dtype,m,n,k,whole", [
     (torch.bfloat16, 1048, 4000, 1600, 231), (torch.float16, 1057, 3872, 4160, 252),      # 96 x 192: ragged last blocks, odd numbers of k-steps
+    (torch.bfloat16, 2025, 2112, 7168, 242),                                              # and more than three quarters of a round of 96 x 256
     (torch.bfloat16, 2817, 2096, 1600, 253), (torch.float16, 2800, 2112, 4160, 242)])     # 128 x 192
 def test_w8a16_many_rows_on_192_channel_tiles(dtype, m, n, k, whole):
     """The same at shapes that take tiles of 192 channels."""
@@ -1607,6 +1608,7 @@ def test_w8a8_many_rows_on_96_row_tiles(dtype, m, n, k):
 
 @pytest.mark.parametrize("dtype,m,n,k,kind,whole", [
     (torch.bfloat16, 1048, 4000, 2080, "tiles", 231), (torch.float16, 1057, 3872, 2064, "tiles", 252),     # 96 x 192, a short last k-step
+    (torch.bfloat16, 2025, 2112, 1616, "tiles", 242),
     (torch.bfloat16, 2817, 2096, 3344, "tiles", 253), (torch.float16, 130, 16400, 1744, "tiles", 172),     # 128 x 192
     (torch.bfloat16, 2025, 5104, 3216, "tiles", 256), (torch.float16, 256, 37888, 1744, "tiles", 238),     # 128 x 320
     (torch.bfloat16, 201, 37872, 3600, "wide", 238)])
