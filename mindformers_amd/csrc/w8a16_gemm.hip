@@ -610,11 +610,10 @@ __global__ __launch_bounds__(256, 2) void w8a16_tile_kernel(
     const int s_end = whole ? KS : min(KS, s0 + g.steps_per_split);
 #define TILE_OF(MTV) \
     w8a16_tile_of<T, MTV, NT>(y, partial, x, wp, scale, bias, residual, M, N, K, gated, aligned, m0, nb, slot, whole, s0, s_end, smem)
-    if constexpr (MT == 4 && NT == 4) {                       // a plan with a tail
+    if constexpr (MT == 4 && NT == 4) {                       // a plan with a tail, of up to 64 rows
         const int left = g.tail && mb == g.m_blocks ? M - m0 : 128;
         if (left <= 32) TILE_OF(1);
         else if (left <= 64) TILE_OF(2);
-        else if (left <= 96) TILE_OF(3);
         else TILE_OF(4);
     } else {
         TILE_OF(MT);

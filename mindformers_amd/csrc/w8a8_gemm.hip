@@ -868,10 +868,9 @@ __global__ __launch_bounds__(256, MT * NT > 16 ? 1 : 2) void w8a8_tile_kernel(
 #define TILE_OF(MTV) \
     w8a8_tile_of<T, MTV, NT, GATED>(y, partial, xq, x_scale, wp, w_scale, bias, residual, M, N, aligned, m0, nb, slot, whole, s0, s_end, \
                                     smem)
-    if constexpr (MT == 4 && NT == 4) {                       // a plan with a tail
+    if constexpr (MT == 4 && NT == 4) {                       // a plan with a tail, of up to 64 rows
         const int left = g.tail && mb == g.m_blocks ? M - m0 : 128;
         if (left <= 64) TILE_OF(2);
-        else if (left <= 96) TILE_OF(3);
         else TILE_OF(4);
     } else {
         TILE_OF(MT);
