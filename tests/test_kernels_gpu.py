@@ -2246,6 +2246,44 @@ def test_grouped_gemms_read_rows_through_the_index(tokens, e, k, n, h, dtype):
         ops.grouped_w8a16_linear(x, w, offsets, sources=sources[:e])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("act_quant", [False, True])
+def test_grouped_gemms_behind_a_long_weight_stream(act_quant, dtype):
+    """Prompt-sized groups on more than 1 GiB of expert weights, where the outputs are stored past the caches: the bits of the same
+    kernel on either half of the experts, which stores them as usual; plain and gated, rows side by side and through an index."""
+    e, n, k = 40, 4096, 7168
+    lib, g = ops._lib.load(), torch.Generator(device="cuda")
+    assert (e // 2) * lib.mf_w8a16_packed_bytes(n, k) <= 1 << 30 < e * lib.mf_w8a16_packed_bytes(n, k)
+    g.manual_seed(e + act_quant)
+    w = torch.randint(-127, 128, (e, n, k), generator=g, device="cuda", dtype=torch.int8)
+    ws = (torch.rand(e, n, generator=g, device="cuda") + 0.5) * (k ** -0.5 / 73)
+    counts = np.array([0, 1, 32, 33, 64, 65, 96, 97, 129] + [5] * 11)
+    counts = np.concatenate((counts, counts[::-1]))
+    off, rows = np.concatenate(([0], np.cumsum(counts))).astype(np.int32), int(counts.sum())
+    x = torch.randn(200, k, generator=g, device="cuda").to(dtype)
+    sources = torch.randint(0, 200, (rows,), generator=g, device="cuda", dtype=torch.int32)
+    xq, xs = ops.dynamic_quant(x)
+    if act_quant:
+        def linear(p, at, idx):
+            i = idx.long()
+            return [ops.grouped_w8a8_linear(xq[i], xs[i], p, at, out_dtype=dtype)] + (
+                [ops.grouped_w8a8_linear(xq, xs[i], p, at, out_dtype=dtype, sources=idx)] if p.gated else [])
+        reads = lib.mf_grouped_w8a8_reads_sources
+    else:
+        def linear(p, at, idx):
+            return [ops.grouped_w8a16_linear(x[idx.long()], p, at)] + (
+                [ops.grouped_w8a16_linear(x, p, at, sources=idx)] if p.gated else [])
+        reads = lib.mf_grouped_w8a16_reads_sources
+    assert reads(200, e, rows, n, k) and reads(200, e // 2, rows // 2, n, k)         # the tile kernels, of all and of half the experts
+    h, mid = e // 2, rows // 2
+    for pack in (ops.pack_w8a16, lambda w, s: ops.pack_w8a16_gated(w, s, "halves")):
+        out = linear(pack(w, ws), torch.from_numpy(off).cuda(), sources)
+        lo = linear(pack(w[:h], ws[:h]), torch.from_numpy(off[:h + 1]).cuda(), sources[:mid])
+        hi = linear(pack(w[h:], ws[h:]), torch.from_numpy(off[h:] - mid).cuda(), sources[mid:])
+        for y, a, b in zip(out, lo, hi):
+            assert y.shape[0] == rows and torch.equal(y, torch.cat((a, b))) and torch.equal(y, out[0])
+
+
 @pytest.mark.parametrize("counts,n", [
     ([50, 80, 62], 48), ([65, 64, 66], 48),                     # few tiles: up to 64 rows a group the passes, above it tiles
     ([20] * 255 + [8], 32), ([21] * 200 + [22] * 56, 32),       # tiles enough: 20 rows (16-bit activations; 12 with int8 ones)
