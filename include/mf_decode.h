@@ -359,7 +359,7 @@ size_t mf_w8a16_packed_bytes(int n, int k);
 int mf_w8a16_pack_weight(void* packed, const int8_t* w, int n, int k, void* stream);
 
 size_t mf_w8a16_workspace_bytes(int m, int n, int k);
-/* The kernel that serves an [m, k] x [n, k] product: 0 = passes of up to 64 rows, 1 = 128 x 256 tiles; *whole and *cut = its
+/* The kernel that serves an [m, k] x [n, k] product: 0 = passes of up to 64 rows, 1 = tiles; *whole and *cut = its
  * output blocks with all of K and those cut into *split parts of it.  Host arithmetic only, for tests and tools. */
 int mf_w8a16_plan(int m, int n, int k, int* whole, int* cut, int* split);
 

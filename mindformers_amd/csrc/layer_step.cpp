@@ -2,7 +2,7 @@
 //
 // A step is seven to nine launches of about 3 us of host time each; reaching every one of them through its own wrapper (checks,
 // an allocation, a call with 12 to 20 arguments) took another 40 us a layer, which is what a step of few sequences waits for: two layers of
-// 512 x 1376 at 4 sequences, through the serving runner, 178 to 187 us, 119 with this call (80 on the device).  Every entry point
+// 512 x 1376 at 4 sequences, through the serving runner, 178 to 187 us, 119 with this call (80 on the device then, 64 now).  Every entry point
 // called here checks its own arguments.
 #include "../../include/mf_decode.h"
 

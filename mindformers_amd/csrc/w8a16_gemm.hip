@@ -10,10 +10,10 @@
 // from the row-major matrix makes every group of lanes touch 16 different cache lines per instruction and
 // ran at about a third of the bandwidth.)
 //
-// Three kernels share the format.  Many rows run on tiles (w8a16_tile_kernel).  The skinny dense kernel (w8a16_gemm4_kernel, described where it is defined) loads weight
-// tiles straight into MFMA operand registers, shares one LDS-staged activation tile among the waves of a workgroup
-// and serves the decode layer's projections; its epilogue, or the split-K reduce kernels, carry the fused variants
-// (gate/up + SiLU*mul, residual + RMSNorm,
+// Four kernels share the format.  Many rows run on tiles (w8a16_tile_kernel), up to 16 rows on few channels with a short K on one wave's
+// tile a workgroup (w8a16_rows_kernel).  The skinny dense kernel (w8a16_gemm4_kernel, described where it is defined) loads weight tiles
+// straight into MFMA operand registers, shares one LDS-staged activation tile among the waves of a workgroup and serves the decode
+// layer's projections; its epilogue, or the split-K reduce kernels, carry the fused variants (gate/up + SiLU*mul, residual + RMSNorm,
 // QKV + RoPE + cache scatter).  The grouped kernel (experts) keeps the earlier register-streaming tile routine
 // w8a16_tile: a workgroup of 4 waves owns 64 output channels (4 n-tiles) for up to 64 rows of x; the waves
 // interleave the 64-wide k-steps of the workgroup's k-range, each streams its tiles HBM -> registers two steps
@@ -563,7 +563,7 @@ struct TileOut {
     }
 };
 
-// one tile of 32*MT rows from row m0 on
+// one tile of 32*MT rows from row m0 on (128 x 256: a pair of registers waits in scratch, 12 bytes a lane, while the k-loop runs)
 template <typename T, int MT, int NT>
 __device__ __forceinline__ void w8a16_tile_of(uint16_t* y, float* partial, const uint16_t* x, const uint8_t* wp, const float* scale,
                                               const uint16_t* bias, const uint16_t* residual, int M, int N, int K, int gated,
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(GW_WAVES * 64, 2) void w8a16_grouped_kernel(
 // Weights of an expert with one block of up to 64 rows are read past the caches, where they would push out the rows that all
 // channel blocks read: 109 experts of 4096 x 7168 at 33 rows 551 us cached, 511 so, 8 of 28672 x 4096 at 33 rows 178 / 163; blocks of
 // more rows gain nothing (7168 x 2048 at 65 rows 679 / 704), and an expert's further blocks share the weights through L2 (200 rows:
-// 1257 / 1420).  Up to 16 bytes of scratch a lane, outside the k-loops.
+// 1257 / 1420).
 template <typename T, int MT, bool NT, bool STREAM>
 __device__ __forceinline__ void w8a16_group_tile(uint16_t* y, const uint16_t* x, const TileSources& src, const uint8_t* we,
                                                  const float* se, int row0, int rows, int m0, int nb, int N, int K, int gated,

@@ -1288,7 +1288,8 @@ def test_w8a16_many_rows_on_192_channel_tiles(dtype, m, n, k, whole):
     (torch.bfloat16, 1, 16, 8), (torch.float16, 16, 48, 64), (torch.bfloat16, 5, 88, 1528), (torch.float16, 16, 512, 1376),
     (torch.bfloat16, 4, 2752, 512), (torch.float16, 4, 16384, 1024), (torch.bfloat16, 16, 6144, 1472)])
 def test_w8a16_few_rows_and_channels(dtype, m, n, k):
-    """The same with K cut between a workgroup's waves: fewer steps than waves, short last steps and channel tiles, and the other side of the line."""
+    """The same where a workgroup's waves take turns along K: one to six turns, short last ones, steps and channel tiles, and the other
+    side of the line."""
     test_w8a16_many_rows(dtype, m, n, k, True, n % 16 != 0)     # (silu_mul takes multiples of 8 columns)
     test_w8a16_many_rows(dtype, m, n, k, False, True)
 
