@@ -193,7 +193,8 @@ class QuantDecodeLayer(nn.Module):
             h, n2x, n2s = ops.w8a8_linear_add_rmsnorm_quant(aq, a_s, self._packed["wo"], x, self.ffn_norm, self.eps,
                                                             self.fc1_smooth, bias=self.wo_b)
             fc1 = self._packed.get("fc1")
-            if self.fc1_b is None and self._own("_linear") and ops.w8a8_gated_fused(n2s.numel(), fc1):
+            own = "_linear" not in self.__dict__ and type(self)._linear is _LINEAR
+            if own and self.fc1_b is None and ops.w8a8_gated_fused(n2s.numel(), fc1):
                 actq = ops.dynamic_quant(ops.w8a8_gated_linear(n2x, n2s, fc1, self.dtype), self.fc2_smooth, tiled=True)
             else:
                 actq = ops.silu_mul_dynamic_quant(self._linear(None, "fc1", quantized=(n2x, n2s)), self.fc2_smooth,
@@ -219,20 +220,13 @@ class QuantDecodeLayer(nn.Module):
     def _chain(out, next_norm):
         return out if next_norm is None else (out, ops.rms_norm(out, next_norm[0], next_norm[1]))
 
-    def _own(self, *names):
-        """Whether these methods are the ones defined here, and no subclass's or instance's nor put in their place on the class: only
-        then may their work go another way."""
-        cls, d = type(self), self.__dict__
-        for name in names:
-            if name in d or getattr(cls, name) is not _METHODS[name]:
-                return False
-        return True
-
     def _plain(self):
-        """Whether a decode step may run as one native call: no bias but the fused projection's, and nothing in place of the
-        operators' order."""
-        d, buffers = self.__dict__, self._buffers
-        if type(self) is not QuantDecodeLayer or self.head_dim % 16 or not self._own("attend", "gate_up", "_linear", "_chain"):
+        """Whether a decode step may run as one native call: no bias but the fused projection's, and nothing that a subclass or an
+        instance has in place of the operators' order, or that was put in their place on the class."""
+        d, buffers, cls = self.__dict__, self._buffers, QuantDecodeLayer
+        if type(self) is not cls or self.head_dim % 16 or "attend" in d or "gate_up" in d or "_linear" in d or "_chain" in d:
+            return False
+        if cls.attend is not _ATTEND or cls.gate_up is not _GATE_UP or cls._linear is not _LINEAR or cls._chain is not _CHAIN:
             return False
         if buffers.get("attn_norm") is None or buffers.get("ffn_norm") is None:
             return False
@@ -251,4 +245,5 @@ class QuantDecodeLayer(nn.Module):
         return sum(getattr(self, f"{n}_w").numel() for n in self.NAMES)
 
 
-_METHODS = {name: getattr(QuantDecodeLayer, name) for name in ("attend", "gate_up", "_linear", "_chain")}
+_ATTEND, _GATE_UP, _LINEAR, _CHAIN = (QuantDecodeLayer.attend, QuantDecodeLayer.gate_up, QuantDecodeLayer._linear,
+                                      QuantDecodeLayer._chain)
