@@ -336,7 +336,7 @@ def int8_gemm_roofline(layer, x, torch, ops, iters):
         weight_bytes += shapes[name].n * shapes[name].k
     total_us = sum(us.values())
     ach = total_ops / (total_us * 1e-6) / 1e12
-    return dict(bound="mfma", kernel="int8 GEMMs of the layer step (w8a8_wide_kernel / w8a8_gemm_kernel / w8a8_regs_kernel "
+    return dict(bound="mfma", kernel="int8 GEMMs of the layer step (w8a8_tile_kernel / w8a8_regs_kernel "
                                      "+ split-K reduce): qkv, wo, gate/up, down", achieved=round(ach, 1),
                 peak=INT8_PEAK_TOPS, unit="TOP/s", frac=round(ach / INT8_PEAK_TOPS, 4), traffic=None,
                 ops_per_step=total_ops, avg_launch_us=round(total_us, 2), per_gemm_us=us,
