@@ -1284,8 +1284,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void w8a16_rows_kernel(
         } else if (s0 + D >= KS) {
             return;
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
+        __syncthreads();
     }
     const int n = 16 * blockIdx.x + 4 * g;
     if (r >= M || n >= N) return;
